@@ -36,14 +36,6 @@ constexpr int kTile = 128;      // column tile of the weighted outer-product GEM
 constexpr int kRowTile = 64;    // image rows per workgroup of the weights GEMM
 constexpr int kMaxChains = 8;   // perturbations applied in one batched call
 constexpr int kPartBlocks = 1024;  // blocks of the grid-wide maxima in the split prep
-// waves per work-group of the FP64 outer-product GEMM (4: 64 x 64 per wave,
-// two work-groups per CU; 8: 64 x 32 per wave, two work-groups and four
-// waves per SIMD, measured 17.6 ms against 22.6 ms at the 128-atom
-// workload); its launches use 64 * this many threads
-#ifndef TDS_F64_OUTER_WAVES
-#define TDS_F64_OUTER_WAVES 8
-#endif
-constexpr int kF64OuterThreads = 64 * TDS_F64_OUTER_WAVES;
 
 inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
 inline long round_up_l(long x, long m) { return (x + m - 1) / m * m; }
@@ -209,5 +201,27 @@ struct Ctx {
 };
 
 int ensure_split(Ctx* c, int prec);
+
+// FP64 GEMM launches (pa_fp64.hip), shared by every caller of the kernels
+struct F64Tiles {
+  int ntile;  // column tiles
+  int cb;     // columns of a tile / 16
+};
+F64Tiles f64_tiles(int n);
+struct F64Rows {
+  const double* U;    // [Mp, np] image rows
+  const double* F;    // [Mp, np]
+  const double* rho;  // [Mp]
+  long Mp;
+};
+void launch_weights_f64(const F64Rows& r, int n, int np, int nc, const double* Y1,
+                        const double* R1, const double* fy, const double* fpsi, int apply_d4,
+                        long tile0, long tile1, long row_lo, long row_hi, double* coef,
+                        hipStream_t s);
+void launch_outer_f64(const F64Rows& r, int n, int np, int nc, const double* coef,
+                      const double* fy, int ksplit, long kb, long ke, long rps, int accumulate,
+                      double* zpart, double* fpart, hipStream_t s);
+void launch_reduce_f64(int n, int np, int nc, int ksplit, const double* zpart,
+                       const double* fpart, double* zsum, double* f, double norm, hipStream_t s);
 
 }  // namespace tdscha

@@ -15,13 +15,6 @@
 
 namespace tdscha {
 
-__global__ void weights_f64(const double*, const double*, const double*, const double*,
-                            const double*, const double*, const double*, int, long, int, long,
-                            long, long, long, int, double*);
-__global__ void outer_f64(const double*, const double*, const double*, const double*, int, long,
-                          int, int, long, long, long, int, int, double*, double*);
-__global__ void reduce_ksplit(const double*, const double*, int, int, double*, double*, double);
-
 // 64 MiB, held by every device the library runs on until the process ends
 constexpr long kScratchDoubles = 8L * 1024 * 1024;
 static __device__ __align__(256) double scratch[kScratchDoubles];
@@ -253,7 +246,7 @@ int tdscha_perturb_averages_noalloc(int n_modes, int n_configs, const double* X,
   hipLaunchKernelGGL(na_prep, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, w, T, R1, Y1,
                      n_modes, np, fy, fpsi, R1p, Y1p);
   hipLaunchKernelGGL(na_neff, dim3(1), dim3(256), 0, s, rho, n_configs, neff);
-  const int ntile = np / kTile;
+  const F64Rows rows{U, F, rimg, L.Mc};
   const long Mc = L.Mc;
   const long rps = Mc / L.ks;   // a multiple of 16
   int chunk = 0;
@@ -261,16 +254,12 @@ int tdscha_perturb_averages_noalloc(int n_modes, int n_configs, const double* X,
     hipLaunchKernelGGL(na_expand, dim3((unsigned)Mc, (np + 127) / 128), dim3(128), 0, s, X, Y,
                        rho, syms, n_degeneracy, degenerate_space, sym_block_id, n_modes, np,
                        n_syms, n_blocks, dmax, b0, lo, hi, U, F, rimg);
-    // one chain: work-group id = row tile (Mc / 64 tiles)
-    hipLaunchKernelGGL(weights_f64, dim3((unsigned)(Mc / 64)), dim3(256), 0, s, U, F, Y1p, R1p,
-                       fy, fpsi, rimg, np, Mc, apply_d4, 0L, Mc / 64, 0L, Mc, 1, coef);
-    hipLaunchKernelGGL(outer_f64, dim3((unsigned)(ntile * ntile * L.ks)), dim3(kF64OuterThreads),
-                       0, s, U, F,
-                       coef, fy, np, Mc, L.ks, ntile, 0L, Mc, rps, chunk > 0 ? 1 : 0, 1, zpart,
-                       fpart);
+    launch_weights_f64(rows, n_modes, np, 1, Y1p, R1p, fy, fpsi, apply_d4, 0L, Mc / 64, 0L, Mc,
+                       coef, s);
+    launch_outer_f64(rows, n_modes, np, 1, coef, fy, L.ks, 0L, Mc, rps, chunk > 0 ? 1 : 0, zpart,
+                     fpart, s);
   }
-  hipLaunchKernelGGL(reduce_ksplit, dim3((unsigned)((nn + 255) / 256), 1), dim3(256), 0, s, zpart,
-                     fpart, np, L.ks, zsum, fsum, 1.0);
+  launch_reduce_f64(n_modes, np, 1, L.ks, zpart, fpart, zsum, fsum, 1.0, s);
   const long n2 = (long)n_modes * n_modes;
   hipLaunchKernelGGL(na_finish, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, s, zsum, fsum,
                      fy, neff, n_modes, np, n_syms, f_out, d2v_out);

@@ -1,4 +1,4 @@
-// FP64 ensemble-averaged D3/D4 application on MFMA (v_mfma_f64_16x16x4f64).
+// FP64 ensemble-averaged D3/D4 application on MFMA (v_mfma_f64_4x4x4_4b_f64).
 //
 // The per-image algebra of CModules/LanczosFunctions.c:2082-2754 is regrouped
 // into three passes over the device-resident symmetric image ensemble
@@ -14,10 +14,28 @@
 //   reduce        d2v = fY Z + (fY Z)^T, f = sum of partials, scaled by
 //                 1/(N_eff N_sym); fixed summation order (deterministic).
 //
-// MFMA f64 16x16x4 operand layout (one double per lane):
-//   A[i][k]: i = lane % 16, k = lane / 16;  B[k][j]: j = lane % 16, k = lane / 16
-//   D[i][j]: j = lane % 16, i = 4 * r + lane / 16  (r = register 0..3; note the
-//   row interleave, unlike the FP32-output MFMAs whose row is 4 * (lane / 16) + r)
+// Both GEMMs are bound by the FP64 matrix rate.  The 4x4x4 instruction (four
+// independent 4x4x4 products) sustains 72 TF/s with constant operands on
+// MI355X, at one wave per SIMD already (70-72 with both operands read from LDS
+// each step); the 16x16x4 one 35 TF/s at one wave per SIMD and 49 TF/s at eight
+// in the same loop.  Measured at 381 modes, 960,000 images, 3 chains: weights
+// 14.0 ms, outer 14.1 ms (60 TF/s each; with the 16x16x4 instruction and
+// register prefetch 18.6 and 17.4 ms), at 159 modes and 240,000 images 0.88 and
+// 0.82 ms (2.35 and 1.94 ms with 128-column tiles).
+//
+// Operand layout of the 4x4x4 MFMA (one double per lane, block q = lane / 4 % 4):
+//   A[i][k]: i = lane % 4, k = lane / 16;  B[k][j]: j = lane % 4, k = lane / 16
+//   D[i][j]: j = lane % 4, i = lane / 16
+// The four blocks of A hold 16 rows (row 4 q + i of a group: lane % 16).  B holds
+// either the same 4 columns in all four blocks (its lanes read one LDS address:
+// a broadcast), or 16 columns, rotated by r blocks (a DPP row rotation) in four
+// MFMAs so that block q meets the columns of block q - r.  FP64 vector
+// instructions take matrix time here, so a B that is built (the outer product)
+// is built once per value and rotated: built four-fold for the broadcast form
+// the outer product ran at 44 TF/s instead of 57.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace tdscha {
@@ -60,25 +78,92 @@ __global__ void expand_images(const double* __restrict__ X, const double* __rest
 // Work-group order of both GEMMs: the hardware deals work-groups to the 8
 // XCDs in turn (id % 8), so the chains of one tile get ids 8 apart and run on
 // one XCD at about the same time, sharing its L2 for the image rows.
+//
+// Tiles: n modes are covered by ceil(n / 128) equal column tiles of 16 CB
+// columns (CB = 1 .. 8), so that little is computed for padding (159 modes: two
+// tiles of 80 columns, where whole 128-column tiles would do 1.6 times the
+// work of a GEMM side and 2.6 times that of the outer product).
 // ---------------------------------------------------------------------------
+static __device__ __forceinline__ double mfma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
 
-// weights: one work-group = 64 image rows x a 128-column pass; K = np in
-// chunks of 16, double-buffered: the next chunk's global loads are in
-// flight while the MFMAs consume the current one (one barrier per chunk)
+// CB consecutive doubles from p[o] on (16-byte pieces where CB is even).  The
+// LDS reads of both kernels form each address with one index: the compiler
+// knows which LDS array a read may touch only through short pointer
+// chains, and otherwise waits for every copy in flight.
+template <int CB>
+static __device__ __forceinline__ void read_run(const double* p, long o, double (&v)[CB]) {
+  if constexpr (CB % 2 == 0) {
+#pragma unroll
+    for (int c = 0; c < CB; c += 2) {
+      const double2 t = *reinterpret_cast<const double2*>(p + (o + c));
+      v[c] = t.x;
+      v[c + 1] = t.y;
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < CB; ++c) v[c] = p[o + c];
+  }
+}
+
+// LDS addresses of the copies are formed in the LDS address space: a generic
+// pointer at a constant offset would count as any array
+typedef __attribute__((address_space(3))) double* lds_d;
+static __device__ __forceinline__ void copy16(const double* g, lds_d l) {
+  __builtin_amdgcn_global_load_lds((gbl_ptr_t)g, (lds_ptr_t)l, 16, 0, 0);
+}
+
+// v of the lane 4 R lanes before, cyclic within a row of 16 lanes
+template <int R>
+static __device__ __forceinline__ double rot4(double v) {
+  if constexpr (R == 0) return v;
+  constexpr int ctrl = 0x120 + 4 * R;   // row_ror:4R
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// acc[i][r] += A_i x B, 16 rows per i: block q of lane's column group q - r
+template <int NA>
+static __device__ __forceinline__ void mfma_rot(const double (&a)[NA], double b,
+                                                double (&acc)[NA][4]) {
+  const double b1 = rot4<1>(b), b2 = rot4<2>(b), b3 = rot4<3>(b);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) acc[i][0] = mfma4(a[i], b, acc[i][0]);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) acc[i][1] = mfma4(a[i], b1, acc[i][1]);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) acc[i][2] = mfma4(a[i], b2, acc[i][2]);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) acc[i][3] = mfma4(a[i], b3, acc[i][3]);
+}
+
+// Both kernels run 4 waves per work-group, two work-groups per CU (3 of the outer
+// product up to CB = 5), and stream their K chunks through a ring of 3 LDS slots
+// (separate arrays, slot fixed at compile time by a 3-fold unroll) filled by
+// direct-to-LDS copies issued two chunks ahead; with the next chunk held in
+// registers (one chunk ahead) the latency of the loads showed (50 and 34 TF/s).
+
+// weights: one work-group = 64 image rows, column tiles of 16 CB one after the
+// other (wave w: columns 4 CB w .. of the tile for all 64 rows), K in chunks of
+// 16 modes.  A lane reads two successive modes of a row at once (16 bytes): within 8 modes the first MFMA takes the even ones and the
+// second the odd ones, in A and B alike.  The 16-byte pieces of a row are
+// stored XOR-ed with the row (the copies permute their source), so that the 8
+// rows a read serves per cycle sit in 8 distinct bank groups.  The first chunks
+// of the next column tile are requested before a tile's epilogue.
 constexpr int WA_KC = 16;
-// LDS row padding (doubles) of the K-chunk tiles: 16 puts the four 16-lane
-// groups of an MFMA operand read in distinct bank halves
-#ifndef TDS_F64_PAD
-#define TDS_F64_PAD 16
-#endif
-constexpr int kPad = TDS_F64_PAD;
 
+template <int CB>
 __global__ __launch_bounds__(256, 2) void weights_f64(
     const double* __restrict__ U, const double* __restrict__ F,
     const double* __restrict__ Y1all, const double* __restrict__ R1all,
     const double* __restrict__ fy, const double* __restrict__ fpsi,
-    const double* __restrict__ rho_img, int np, long Mp, int apply_d4, long tile0, long tile1,
-    long row_lo, long row_hi, int nc, double* __restrict__ coef_all) {
+    const double* __restrict__ rho_img, int np, int nk, int ntile, long Mp, int apply_d4,
+    long tile0, long tile1, long row_lo, long row_hi, int nc, double* __restrict__ coef_all) {
+  constexpr int W = 16 * CB;
+  constexpr int kCY = (2 * CB + 3) / 4;   // copies of Y1 per wave and chunk
+  constexpr int kLoads = 2 + kCY;
   const int xcd = blockIdx.x & 7;
   const int jj = blockIdx.x >> 3;
   const int chain = jj % nc;
@@ -90,160 +175,176 @@ __global__ __launch_bounds__(256, 2) void weights_f64(
   const long r0 = tile * 64;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int lr = lane & 15;   // lane within a 16-group
-  const int lg = lane >> 4;   // 16-group index
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4, lq = lane & 3;
+  const int drow = (lane & 12) + lg;   // row of a 16-row group this lane's results belong to
 
-  __shared__ double sU[2][64][WA_KC + 1];
-  __shared__ double sY[2][WA_KC][kTile + kPad];
-  __shared__ double red[4][64][4];
-  __shared__ double rowsum[64][4];
+  constexpr int kU = 64 * WA_KC, kSlot = kU + WA_KC * W;
+  __shared__ __align__(16) double s0[kSlot];
+  __shared__ __align__(16) double s1[kSlot];
+  __shared__ __align__(16) double s2[kSlot];
+  static_assert(1024 <= kSlot, "the row-dot partials fit a slot");
+  double(*const red)[64][4] = reinterpret_cast<double(*)[64][4]>(s2);   // [4][64][4]
 
-  rowsum[tid >> 2][tid & 3] = 0.0;
+  // copy chunk kc of column tile c0, 64 pieces of 16 bytes per copy, dealt to
+  // the waves (every wave and lane takes part in each, so that the number of
+  // copies in flight is known; those beyond the last repeat it): 8 copies of 8
+  // U rows (128 bytes of a row each), 2 CB copies of Y1
+  const double* pu = U + (r0 + 16 * wave + (lane >> 3)) * np + 2 * ((lane & 7) ^ (lane >> 3));
+  int yoff[kCY];
+#pragma unroll
+  for (int e = 0; e < kCY; ++e) {
+    const int p = 64 * min(wave + 4 * e, 2 * CB - 1) + lane;
+    yoff[e] = p / (W / 2) * np + 2 * (p % (W / 2));
+  }
+  auto issue = [&](lds_d slot, int c0, int kc) {
+    const int k0 = kc * WA_KC;
+    copy16(pu + k0, slot + 16 * wave * WA_KC);
+    copy16(pu + 8L * np + k0, slot + (16 * wave + 8) * WA_KC);
+    const double* py = Y1 + (long)k0 * np + c0;
+#pragma unroll
+    for (int e = 0; e < kCY; ++e)
+      copy16(py + yoff[e], slot + kU + 128 * min(wave + 4 * e, 2 * CB - 1));
+  };
 
-  double ru[4], ry[8];
-  for (int c0 = 0; c0 < np; c0 += kTile) {
-    v4d acc[4][2];
+  double acc[4][CB];
+  auto compute = [&](const double* cur) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int k8 = 0; k8 < WA_KC; k8 += 8) {
+      double2 a[4];
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
-
-    // U[r0:r0+64, k0:k0+16] (4 per thread) and Y1[k0:k0+16, c0:c0+128] (8 per thread)
-    auto load = [&](int k0) {
+      for (int rb = 0; rb < 4; ++rb)
+        a[rb] = *reinterpret_cast<const double2*>(
+            cur + ((16 * rb + lr) * WA_KC + 2 * ((k8 / 2 + lg) ^ (lr & 7))));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int idx = tid + 256 * e;
-        ru[e] = U[(r0 + (idx >> 4)) * np + k0 + (idx & 15)];
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int idx = tid + 256 * e;
-        ry[e] = Y1[(long)(k0 + (idx >> 7)) * np + c0 + (idx & 127)];
-      }
-    };
-    auto store = [&](int b) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int idx = tid + 256 * e;
-        sU[b][idx >> 4][idx & 15] = ru[e];
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int idx = tid + 256 * e;
-        sY[b][idx >> 7][idx & 127] = ry[e];
-      }
-    };
-    load(0);
-    store(0);
-    __syncthreads();
-    int cur = 0;
-    for (int k0 = 0; k0 < np; k0 += WA_KC) {
-      const bool more = k0 + WA_KC < np;
-      if (more) load(k0 + WA_KC);
-#pragma unroll
-      for (int kk = 0; kk < WA_KC; kk += 4) {
-        double a[4], b[2];
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) a[rb] = sU[cur][16 * rb + lr][kk + lg];
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) b[cb] = sY[cur][kk + lg][32 * wave + 16 * cb + lr];
+      for (int t = 0; t < 2; ++t) {
+        double b[CB];
+        read_run<CB>(cur, kU + (k8 + 2 * lg + t) * W + 4 * CB * wave + CB * lq, b);
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-          for (int cb = 0; cb < 2; ++cb)
-            acc[rb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rb], b[cb], acc[rb][cb], 0, 0, 0);
+          for (int cb = 0; cb < CB; ++cb)
+            acc[rb][cb] = mfma4(t ? a[rb].y : a[rb].x, b[cb], acc[rb][cb]);
       }
-      if (more) store(cur ^ 1);
-      __syncthreads();
-      cur ^= 1;
+    }
+  };
+  // chunk kc: its copies (all but the youngest kLoads) have landed and every
+  // wave is done with chunk kc - 1, whose slot takes chunk kc + 2
+  auto step = [&](const double* cur, double* nxt, int c0, int kc) {
+    TDS_WAIT_VMCNT(kLoads);
+    lds_barrier();
+    issue((lds_d)nxt, c0, kc + 2);
+    compute(cur);
+  };
+  // the last two chunks
+  auto tail = [&](const double* a, const double* b) {
+    TDS_WAIT_VMCNT(kLoads);
+    lds_barrier();
+    compute(a);
+    TDS_WAIT_VMCNT(0);
+    lds_barrier();
+    compute(b);
+  };
+
+  // tid = 4 row + quantity: running row-dot sums over the column tiles
+  const int urow = tid >> 2;
+  double rowsum = 0.0;
+  const int nkc = nk / WA_KC;
+  issue((lds_d)s0, 0, 0);
+  issue((lds_d)s1, 0, 1);
+  for (int c0 = 0; c0 < ntile * W; c0 += W) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < CB; ++b) acc[a][b] = 0.0;
+    int kc = 0;
+    for (; kc + 5 <= nkc; kc += 3) {
+      step(s0, s2, c0, kc);
+      step(s1, s0, c0, kc + 1);
+      step(s2, s1, c0, kc + 2);
+    }
+    if (nkc - kc == 2) {
+      tail(s0, s1);
+    } else if (nkc - kc == 3) {
+      step(s0, s2, c0, kc);
+      tail(s1, s2);
+    } else {
+      step(s0, s2, c0, kc);
+      step(s1, s0, c0, kc + 1);
+      tail(s2, s0);
+    }
+    lds_barrier();   // every slot is free
+    if (c0 + W < ntile * W) {
+      issue((lds_d)s0, c0 + W, 0);
+      issue((lds_d)s1, c0 + W, 1);
     }
 
-    // fused epilogue: partial row dots over this wave's 32 columns
+    // fused epilogue: row dots over this lane's CB columns, then over the four
+    // lanes of the row
+    const int col = c0 + 4 * CB * wave + CB * lq;
+    double fyr[CB], fpc[CB], r1c[CB];
+    read_run<CB>(fy, col, fyr);
+    read_run<CB>(fpsi, col, fpc);
+    read_run<CB>(R1, col, r1c);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) fyr[cb] *= r1c[cb];
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
-      double p[4][4];
+      const long o = (r0 + 16 * rb + drow) * np + col;
+      double u[CB], f[CB];
+      read_run<CB>(U, o, u);
+      read_run<CB>(F, o, f);
+      double p[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) p[r][q] = 0.0;
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        const int col = c0 + 32 * wave + 16 * cb + lr;
-        const double fyc = fy[col], fpc = fpsi[col], r1c = R1[col];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const long row = r0 + 16 * rb + 4 * r + lg;
-          const double u = U[row * np + col];
-          const double f = F[row * np + col];
-          const double v = acc[rb][cb][r];
-          p[r][0] += v * u;
-          p[r][1] += v * f * fpc;
-          p[r][2] += u * fyc * r1c;
-          p[r][3] += f * r1c;
-        }
+      for (int cb = 0; cb < CB; ++cb) {
+        p[0] += acc[rb][cb] * u[cb];
+        p[1] += acc[rb][cb] * (f[cb] * fpc[cb]);
+        p[2] += u[cb] * fyr[cb];
+        p[3] += f[cb] * r1c[cb];
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          double v = p[r][q];
-          v += __shfl_xor(v, 1);
-          v += __shfl_xor(v, 2);
-          v += __shfl_xor(v, 4);
-          v += __shfl_xor(v, 8);
-          p[r][q] = v;
-        }
-      if (lr == 0) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) red[wave][16 * rb + 4 * r + lg][q] = p[r][q];
+      for (int q = 0; q < 4; ++q) {
+        p[q] += __shfl_xor(p[q], 1);
+        p[q] += __shfl_xor(p[q], 2);
       }
+      red[wave][16 * rb + drow][lq] = lq < 2 ? (lq ? p[1] : p[0]) : (lq == 2 ? p[2] : p[3]);
     }
-    __syncthreads();
-    {
-      const int rr = tid >> 2, q = tid & 3;
-      rowsum[rr][q] += (red[0][rr][q] + red[1][rr][q]) + (red[2][rr][q] + red[3][rr][q]);
-    }
+    lds_barrier();
+    rowsum += (red[0][urow][lq] + red[1][urow][lq]) + (red[2][urow][lq] + red[3][urow][lq]);
+    // (slot 2 is filled again after the next tile's first barrier)
   }
-  __syncthreads();
-  if (tid < 64) {
-    const long row = r0 + tid;
-    const double s1 = rowsum[tid][0];  // u.Y1.u
-    const double s2 = rowsum[tid][1];  // u.Y1.g  (Y1 symmetrised on upload)
-    const double s3 = rowsum[tid][2];  // a.R1
-    const double s4 = rowsum[tid][3];  // f.R1
-    // images outside [row_lo, row_hi) carry no weight (image-range calls)
-    const double rho = (row >= row_lo && row < row_hi) ? rho_img[row] : 0.0;
-    double* c = coef + row * 4;
-    c[0] = rho * (-s3 / 3.0 + apply_d4 * s1 / 8.0);
-    c[1] = rho * (-s4 / 3.0 + apply_d4 * s2 / 4.0);
-    c[2] = -rho * s1 / 6.0;
-    c[3] = -rho * s2 / 3.0;
-  }
+  // the row's four lanes share its sums; lane q writes coefficient q
+  const int base = lane & 60;
+  const double s_1 = __shfl(rowsum, base);       // u.Y1.u
+  const double s_2 = __shfl(rowsum, base + 1);   // u.Y1.g  (Y1 symmetrised on upload)
+  const double s_3 = __shfl(rowsum, base + 2);   // a.R1
+  const double s_4 = __shfl(rowsum, base + 3);   // f.R1
+  const long row = r0 + urow;
+  // images outside [row_lo, row_hi) carry no weight (image-range calls)
+  const double rho = (row >= row_lo && row < row_hi) ? rho_img[row] : 0.0;
+  const double c1 = rho * (-s_3 / 3.0 + apply_d4 * s_1 / 8.0);
+  const double c2 = rho * (-s_4 / 3.0 + apply_d4 * s_2 / 4.0);
+  coef[row * 4 + lq] = lq < 2 ? (lq ? c2 : c1) : (lq == 2 ? -rho * s_1 / 6.0 : -rho * s_2 / 3.0);
 }
 
 // ---------------------------------------------------------------------------
 // outer: split-K Z[mu, nu] = sum_b U[b, mu] B[b, nu] over a range of images,
-// 128 x 128 tiles, 4 waves of 64 x 64; K in chunks of 8 images,
-// double-buffered like the weights GEMM (raw U, F and coefficients of the
-// next chunk in registers during the MFMAs, B built when they are stored).
-// Two work-groups per CU: one's barrier overlaps the other's MFMAs.
+// T x T tiles (T = 16 CB), wave w on all T rows and the columns 4 CB w .., chunks
+// of 8 images.  A slot holds the images' U of the mu columns, F and (off the
+// diagonal) U of the nu columns and the coefficients; a wave builds the B values
+// of its own columns in registers as it reads them, 16 columns at a time in the
+// rotated form and the CB % 4 groups of 4 that remain in the broadcast form.
 // ---------------------------------------------------------------------------
 constexpr int WB_KC = 8;
-constexpr int kOW = TDS_F64_OUTER_WAVES;   // 4 (64 x 64 per wave) or 8 (64 x 32 per wave)
-constexpr int kOT = kF64OuterThreads;      // threads
-constexpr int kWN = kOW == 4 ? 64 : 32;    // columns per wave
-constexpr int kNJ = kWN / 16;              // 16-column blocks per wave
-constexpr int kRS = kOT / kTile;           // image rows staged per pass of the threads
-constexpr int kRE = WB_KC / kRS;           // rows per thread and chunk
 
-__global__ __launch_bounds__(kOT, kOW == 8 ? 4 : 2) void outer_f64(
+template <int CB>
+__global__ __launch_bounds__(256, CB > 5 ? 2 : 3) void outer_f64(
     const double* __restrict__ U, const double* __restrict__ F,
     const double* __restrict__ coef_all, const double* __restrict__ fy, int np, long Mp,
     int ksplit, int ntile, long kbase, long kend, long rows_per_split, int accumulate, int nc,
     double* __restrict__ zpart_all, double* __restrict__ fpart_all) {
+  constexpr int T = 16 * CB;
+  constexpr int NF = CB / 4, NQ = CB % 4;   // rotated 16-column and broadcast 4-column operands
   const int xcd = blockIdx.x & 7;
   const int jj = blockIdx.x >> 3;
   const int chain = jj % nc;
@@ -255,175 +356,287 @@ __global__ __launch_bounds__(kOT, kOW == 8 ? 4 : 2) void outer_f64(
   const double* coef = coef_all + (long)chain * Mp * 4;
   double* zpart = zpart_all + ((long)chain * ksplit + ks) * np * np;
   double* fpart = fpart_all + ((long)chain * ksplit + ks) * np;
-  const int mu0 = tm * kTile, nu0 = tn * kTile;
-  const bool diag = (tm == tn);
+  const int mu0 = tm * T, nu0 = tn * T;
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int lr = lane & 15, lg = lane >> 4;
-  const int wm = wave / (kTile / kWN), wn = wave % (kTile / kWN);   // 64 rows x kWN columns
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4, lq = lane & 3, lb = (lane >> 2) & 3;
 
-  __shared__ double sA[2][WB_KC][kTile + kPad];
-  __shared__ double sB[2][WB_KC][kTile + kPad];
-  __shared__ double sF[kRS][kTile];
+  constexpr int kM = WB_KC * T, kSlot = 3 * kM + 128;
+  __shared__ __align__(16) double s0[kSlot];
+  __shared__ __align__(16) double s1[kSlot];
+  __shared__ __align__(16) double s2[kSlot];
 
-  v4d acc[4][kNJ];
+  double acc[NF > 0 ? NF : 1][CB][4], aq[NQ > 0 ? NQ : 1][CB];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int i = 0; i < CB; ++i) {
 #pragma unroll
-    for (int b = 0; b < kNJ; ++b) acc[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
+    for (int g = 0; g < NF; ++g) acc[g][i][0] = acc[g][i][1] = acc[g][i][2] = acc[g][i][3] = 0.0;
+#pragma unroll
+    for (int g = 0; g < NQ; ++g) aq[g][i] = 0.0;
+  }
 
   const long kb = kbase + (long)ks * rows_per_split;
-  long ke = kb + rows_per_split;
-  if (ke > kend) ke = kend;
-  const int col = tid & 127;
-  const int rsub = tid >> 7;  // rows rsub, rsub + kRS, ... of a chunk
-  const double fyn = fy[nu0 + col];
-  double fl = 0.0;
-  // next chunk's raw values; on diagonal tiles U of the nu columns is the
-  // A value itself, and rx, ry carry alpha, beta instead
-  double rc1[kRE], rc2[kRE], rum[kRE], rfn[kRE], rx[kRE], ry[kRE];
-  const long rstride = (long)kRS * np;       // between a thread's rows
-  auto load = [&](long k0) {
-    const long row0 = k0 + rsub;
-    const double* pu = U + row0 * np + col;
-    const double* pf = F + row0 * np + nu0 + col;
-    const double* pc = coef + row0 * 4;
+  const long ke = kb + rows_per_split < kend ? kb + rows_per_split : kend;
+  const int nch = ke > kb ? (int)((ke - kb) / WB_KC) : 0;
+  // this lane's B columns: 16 g + lr of the rotated operands, 4 g + lq of the others
+  const int wcol = 4 * CB * wave + lr, qcol = 4 * CB * wave + 16 * NF + lq;
+  double hf[NF > 0 ? NF : 1], hq[NQ > 0 ? NQ : 1], fa[NF + 1], fb[NF + 1];
 #pragma unroll
-    for (int e = 0; e < kRE; ++e) {
-      rc1[e] = pc[4 * kRS * e];
-      rc2[e] = pc[4 * kRS * e + 1];
-      rum[e] = pu[e * rstride + mu0];
-      rfn[e] = pf[e * rstride];
-      if (diag) {
-        rx[e] = pc[4 * kRS * e + 2];
-        ry[e] = pc[4 * kRS * e + 3];
-      } else {
-        rx[e] = pu[e * rstride + nu0];
+  for (int g = 0; g < NF; ++g) hf[g] = 0.5 * fy[nu0 + wcol + 16 * g];
+#pragma unroll
+  for (int g = 0; g < NQ; ++g) hq[g] = 0.5 * fy[nu0 + qcol + 4 * g];
+#pragma unroll
+  for (int g = 0; g <= NF; ++g) fa[g] = fb[g] = 0.0;   // sums of alpha f, beta u (diagonal tiles)
+  // column of the tile whose f sum a lane holds in fa[NF]: 16 NF + lr of the wave's 4 CB
+  const int lcol = 4 * CB * wave + 16 * NF + (lr < 4 * NQ ? lr : 0);
+
+  auto run = [&](auto is_diag) {
+    constexpr bool DIAG = decltype(is_diag)::value;
+    constexpr int kC = (CB + 3) / 4;                  // copies per matrix, wave and chunk
+    constexpr int kLoads = kC * (DIAG ? 2 : 3) + 1;
+    constexpr int oUn = DIAG ? 0 : 2 * kM;            // U of the nu columns
+    // 64 pieces of 16 bytes per copy, CB copies per matrix, dealt to the waves
+    // (every wave and lane takes part in each, so that the number of copies in
+    // flight is known; those beyond the last repeat it)
+    int off[kC];
+#pragma unroll
+    for (int e = 0; e < kC; ++e) {
+      const int p = 64 * min(wave + 4 * e, CB - 1) + lane;
+      off[e] = p / (T / 2) * np + 2 * (p % (T / 2));
+    }
+    const int coff = 2 * (lane & 15);   // 8 images of 4 coefficients, four times over
+    auto issue = [&](lds_d slot, int ch) {
+      const long row = kb + (long)ch * WB_KC;
+      const double* pu = U + row * np;
+      const double* pf = F + row * np + nu0;
+#pragma unroll
+      for (int e = 0; e < kC; ++e) {
+        const lds_d d = slot + 128 * min(wave + 4 * e, CB - 1);
+        copy16(pu + mu0 + off[e], d);
+        copy16(pf + off[e], d + kM);
+        if (!DIAG) copy16(pu + nu0 + off[e], d + 2 * kM);
       }
+      copy16(coef + row * 4 + coff, slot + 3 * kM);
+    };
+    // chunk ch: its copies (all but the youngest kLoads) have landed and every
+    // wave is done with chunk ch - 1, whose slot takes chunk ch + 2 (the last
+    // one again beyond the end)
+    auto step = [&](const double* cur, double* nxt, int ch) {
+      TDS_WAIT_VMCNT(kLoads);
+      lds_barrier();
+      issue((lds_d)nxt, min(ch + 2, nch - 1));
+#pragma unroll
+      for (int k4 = 0; k4 < WB_KC; k4 += 4) {
+        const int k = k4 + lg;
+        double a[CB];
+        // rows 16 i + lane % 16, or (CB even) rows 32 i + 2 (lane % 16) + 0, 1
+        if constexpr (CB % 2 == 0) {
+#pragma unroll
+          for (int i = 0; i < CB; i += 2) {
+            const double2 t = *reinterpret_cast<const double2*>(cur + (k * T + 16 * i + 2 * lr));
+            a[i] = t.x;
+            a[i + 1] = t.y;
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < CB; ++i) a[i] = cur[k * T + 16 * i + lr];
+        }
+        const int of = kM + k * T, on = oUn + k * T;
+        const double2 c12 = *reinterpret_cast<const double2*>(cur + (3 * kM + 4 * k));
+        double2 ab;
+        if constexpr (DIAG) ab = *reinterpret_cast<const double2*>(cur + (3 * kM + 4 * k + 2));
+#pragma unroll
+        for (int g = 0; g < NF; ++g) {
+          const double f = cur[of + wcol + 16 * g], u = cur[on + wcol + 16 * g];
+          mfma_rot<CB>(a, c12.x * f + c12.y * (hf[g] * u), acc[g]);
+          if constexpr (DIAG) {
+            fa[g] += ab.x * f;
+            fb[g] += ab.y * u;
+          }
+        }
+#pragma unroll
+        for (int g = 0; g < NQ; ++g) {
+          const double b =
+              c12.x * cur[of + qcol + 4 * g] + c12.y * (hq[g] * cur[on + qcol + 4 * g]);
+#pragma unroll
+          for (int i = 0; i < CB; ++i) aq[g][i] = mfma4(a[i], b, aq[g][i]);
+        }
+        if constexpr (DIAG && NQ > 0) {
+          fa[NF] += ab.x * cur[of + lcol];
+          fb[NF] += ab.y * cur[on + lcol];
+        }
+      }
+    };
+    issue((lds_d)s0, 0);
+    issue((lds_d)s1, min(1, nch - 1));
+    for (int ch = 0;;) {
+      step(s0, s2, ch);
+      if (++ch == nch) break;
+      step(s1, s0, ch);
+      if (++ch == nch) break;
+      step(s2, s1, ch);
+      if (++ch == nch) break;
     }
+    TDS_WAIT_VMCNT(0);   // the copies past the end land before the LDS is released
   };
-  auto store = [&](int b) {
-#pragma unroll
-    for (int e = 0; e < kRE; ++e) {
-      const int kk = rsub + kRS * e;
-      const double un = diag ? rum[e] : rx[e];
-      sA[b][kk][col] = rum[e];
-      sB[b][kk][col] = rc1[e] * rfn[e] + 0.5 * rc2[e] * fyn * un;
-      if (diag) fl += rx[e] * rfn[e] + ry[e] * fyn * un;
-    }
-  };
-  if (kb < ke) {
-    load(kb);
-    store(0);
+  if (nch > 0) {
+    if (tm == tn)
+      run(std::true_type{});
+    else
+      run(std::false_type{});
   }
-  __syncthreads();
-  int cur = 0;
-  for (long k0 = kb; k0 < ke; k0 += WB_KC) {
-    const bool more = k0 + WB_KC < ke;
-    if (more) load(k0 + WB_KC);
+
+  // write the partial tile; accumulate: add to the partial of earlier image
+  // chunks (each element has one writer, chunks run in order)
+  const int drow = 4 * lb + lg;
 #pragma unroll
-    for (int kk = 0; kk < WB_KC; kk += 4) {
-      double a[4], b[kNJ];
+  for (int i = 0; i < CB; ++i) {
+    const int mu = mu0 + (CB % 2 ? 16 * i + drow : 16 * (i & ~1) + 2 * drow + (i & 1));
+    double* z = zpart + (long)mu * np + nu0 + 4 * CB * wave + lq;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = sA[cur][kk + lg][64 * wm + 16 * i + lr];
-#pragma unroll
-      for (int j = 0; j < kNJ; ++j) b[j] = sB[cur][kk + lg][kWN * wn + 16 * j + lr];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < kNJ; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    if (more) store(cur ^ 1);
-    __syncthreads();
-    cur ^= 1;
-  }
-  // write the partial tile
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < kNJ; ++j)
+    for (int g = 0; g < NF; ++g)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int mu = mu0 + 64 * wm + 16 * i + 4 * r + lg;
-        const int nu = nu0 + kWN * wn + 16 * j + lr;
-        // accumulate: add to the partial of earlier image chunks (each
-        // element has one writer, chunks run in order)
-        const double prev = accumulate ? zpart[(long)mu * np + nu] : 0.0;
-        zpart[(long)mu * np + nu] = prev + acc[i][j][r];
+        double* p = z + 16 * g + 4 * ((lb - r) & 3);
+        *p = (accumulate ? *p : 0.0) + acc[g][i][r];
       }
-  if (diag) {
-    sF[rsub][col] = fl;
-    __syncthreads();
-    if (tid < kTile) {
-      double sum = 0.0;
 #pragma unroll
-      for (int q = 0; q < kRS; ++q) sum += sF[q][tid];
-      const double prev = accumulate ? fpart[nu0 + tid] : 0.0;
-      fpart[nu0 + tid] = prev + sum;
+    for (int g = 0; g < NQ; ++g) {
+      double* p = z + 16 * NF + 4 * g;
+      *p = (accumulate ? *p : 0.0) + aq[g][i];
+    }
+  }
+  if (tm == tn) {
+#pragma unroll
+    for (int g = 0; g < NF + (NQ > 0); ++g) {
+      const int c = g < NF ? wcol + 16 * g : lcol;
+      double v = fa[g] + fy[nu0 + c] * fb[g];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      if (lg == 0 && (g < NF || lr < 4 * NQ)) {
+        double* p = fpart + nu0 + c;
+        *p = (accumulate ? *p : 0.0) + v;
+      }
     }
   }
 }
 
-// sum the K-split partials (fixed order): zsum[mu, nu], f
-__global__ void reduce_ksplit(const double* __restrict__ zpart_all,
-                              const double* __restrict__ fpart_all, int np, int ksplit,
-                              double* __restrict__ zsum_all, double* __restrict__ f_all,
-                              double norm) {
-  const int chain = blockIdx.y;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// sum the K-split partials in a fixed order, rows and columns below n: 64
+// elements per work-group, the partials in 4 slices of 8 loads in flight each,
+// combined in LDS; grid (ceil(n / 64), n + 1, chains), the last row the f sums
+__global__ __launch_bounds__(256) void reduce_ksplit(const double* __restrict__ zpart_all,
+                                                     const double* __restrict__ fpart_all, int n,
+                                                     int np, int ksplit,
+                                                     double* __restrict__ zsum_all,
+                                                     double* __restrict__ f_all, double norm) {
+  const int chain = blockIdx.z, row = blockIdx.y;
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;
   const long nn = (long)np * np;
-  const double* zp = zpart_all + (long)chain * ksplit * nn;
-  if (e < nn) {
-    // eight loads in flight, summed in the same order as one at a time
-    double s = 0.0;
-    int k = 0;
-    for (; k + 8 <= ksplit; k += 8) {
+  const bool isf = row == n;
+  const long stride = isf ? np : nn;
+  const double* p = isf ? fpart_all + (long)chain * ksplit * np + c
+                        : zpart_all + (long)chain * ksplit * nn + (long)row * np + c;
+  const int per = (ksplit + 3) / 4;
+  const int lo = sl * per, hi = lo + per < ksplit ? lo + per : ksplit;
+  double s = 0.0;
+  if (c < n) {
+    int k = lo;
+    for (; k + 8 <= hi; k += 8) {
       double v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = zp[(long)(k + j) * nn + e];
+      for (int j = 0; j < 8; ++j) v[j] = p[(k + j) * stride];
 #pragma unroll
       for (int j = 0; j < 8; ++j) s += v[j];
     }
-    for (; k < ksplit; ++k) s += zp[(long)k * nn + e];
-    zsum_all[(long)chain * nn + e] = s;
+    for (; k < hi; ++k) s += p[k * stride];
   }
-  if (e < np) {
-    const double* fp = fpart_all + (long)chain * ksplit * np;
-    double s = 0.0;
-    for (int k = 0; k < ksplit; ++k) s += fp[(long)k * np + e];
-    f_all[(long)chain * np + e] = s * norm;
+  __shared__ double red[4][64];
+  red[sl][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (sl == 0 && c < n) {
+    const double t = (red[0][c & 63] + red[1][c & 63]) + (red[2][c & 63] + red[3][c & 63]);
+    if (isf)
+      f_all[(long)chain * np + c] = t * norm;
+    else
+      zsum_all[(long)chain * nn + (long)row * np + c] = t;
   }
 }
 
+// column tiles of n modes: ceil(n / 128) of them, 16 CB columns each
+F64Tiles f64_tiles(int n) {
+  const int t = (n + kTile - 1) / kTile;
+  return {t, ((n + t - 1) / t + 15) / 16};
+}
+
+template <typename Fn>
+static void with_cb(int cb, Fn fn) {
+  switch (cb) {
+    case 1: fn(std::integral_constant<int, 1>{}); break;
+    case 2: fn(std::integral_constant<int, 2>{}); break;
+    case 3: fn(std::integral_constant<int, 3>{}); break;
+    case 4: fn(std::integral_constant<int, 4>{}); break;
+    case 5: fn(std::integral_constant<int, 5>{}); break;
+    case 6: fn(std::integral_constant<int, 6>{}); break;
+    case 7: fn(std::integral_constant<int, 7>{}); break;
+    default: fn(std::integral_constant<int, 8>{}); break;
+  }
+}
+
+// rows [64 tile0, 64 tile1) of U, F; coefficients of images outside
+// [row_lo, row_hi) are zero
+void launch_weights_f64(const F64Rows& r, int n, int np, int nc, const double* Y1,
+                        const double* R1, const double* fy, const double* fpsi, int apply_d4,
+                        long tile0, long tile1, long row_lo, long row_hi, double* coef,
+                        hipStream_t s) {
+  const F64Tiles t = f64_tiles(n);
+  const int nk = std::max(2 * WA_KC, round_up(n, WA_KC));   // the ring starts with two chunks
+  // tiles dealt 8 at a time (one per XCD), every chain of a tile on its XCD
+  const long g = round_up_l(tile1 - tile0, 8) * nc;
+  with_cb(t.cb, [&](auto cb) {
+    hipLaunchKernelGGL(weights_f64<decltype(cb)::value>, dim3((unsigned)g), dim3(256), 0, s, r.U,
+                       r.F, Y1, R1, fy, fpsi, r.rho, np, nk, t.ntile, r.Mp,
+                       apply_d4, tile0, tile1, row_lo, row_hi, nc, coef);
+  });
+}
+
+void launch_outer_f64(const F64Rows& r, int n, int np, int nc, const double* coef,
+                      const double* fy, int ksplit, long kb, long ke, long rps, int accumulate,
+                      double* zpart, double* fpart, hipStream_t s) {
+  const F64Tiles t = f64_tiles(n);
+  const long g = (long)t.ntile * t.ntile * ksplit * nc;
+  with_cb(t.cb, [&](auto cb) {
+    hipLaunchKernelGGL(outer_f64<decltype(cb)::value>, dim3((unsigned)g), dim3(256), 0, s, r.U,
+                       r.F, coef, fy, np, r.Mp, ksplit, t.ntile, kb, ke, rps, accumulate, nc,
+                       zpart, fpart);
+  });
+}
+
+void launch_reduce_f64(int n, int np, int nc, int ksplit, const double* zpart,
+                       const double* fpart, double* zsum, double* f, double norm, hipStream_t s) {
+  hipLaunchKernelGGL(reduce_ksplit, dim3((n + 63) / 64, n + 1, nc), dim3(256), 0, s, zpart, fpart,
+                     n, np, ksplit, zsum, f, norm);
+}
+
 int launch_pa_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev) {
-  const int ntile = c->np / kTile;
+  const F64Rows rows{c->U, c->F, c->rho_img, c->Mp};
   // image range [row_lo, row_hi): whole 64-row tiles of the weights kernel
   // (rows outside the range get zero coefficients), and the outer GEMM's K
-  // range from the 16-row step below row_lo to the step above row_hi
+  // range from the 8-row step below row_lo to the step above row_hi
   const long t0 = c->row_lo / 64, t1 = (c->row_hi + 63) / 64;
-  // tiles dealt 8 at a time (one per XCD), every chain of a tile on its XCD
-  const long ga = round_up_l(t1 - t0, 8) * nc;
   if (ev) (void)hipEventRecord(ev[0], s);
-  hipLaunchKernelGGL(weights_f64, dim3((unsigned)ga), dim3(256), 0, s, c->U, c->F, c->Y1, c->R1,
-                     c->fy, c->fpsi, c->rho_img, c->np, c->Mp, apply_d4, t0, t1, c->row_lo,
-                     c->row_hi, nc, c->coef);
+  launch_weights_f64(rows, c->n, c->np, nc, c->Y1, c->R1, c->fy, c->fpsi, apply_d4, t0, t1,
+                     c->row_lo, c->row_hi, c->coef, s);
   if (ev) (void)hipEventRecord(ev[1], s);
   const long kb = c->row_lo / WB_KC * WB_KC;
   const long ke = round_up_l(c->row_hi, WB_KC);
   const long rps = round_up_l((ke - kb + c->ksplit - 1) / c->ksplit, WB_KC);
-  const long gb = (long)ntile * ntile * c->ksplit * nc;
-  hipLaunchKernelGGL(outer_f64, dim3((unsigned)gb), dim3(kOT), 0, s, c->U, c->F, c->coef, c->fy,
-                     c->np, c->Mp, c->ksplit, ntile, kb, ke, rps, 0, nc, c->zpart, c->fpart);
+  launch_outer_f64(rows, c->n, c->np, nc, c->coef, c->fy, c->ksplit, kb, ke, rps, 0, c->zpart,
+                   c->fpart, s);
   if (ev) (void)hipEventRecord(ev[2], s);
-  const long nn = (long)c->np * c->np;
-  const double norm = 1.0 / (c->n_eff * c->n_syms);
   // zsum -> c->d2v_out (padded), normalised f -> c->f_out
-  dim3 gr((unsigned)((nn + 255) / 256), nc);
-  hipLaunchKernelGGL(reduce_ksplit, gr, dim3(256), 0, s, c->zpart, c->fpart, c->np, c->ksplit,
-                     c->d2v_out, c->f_out, norm);
+  launch_reduce_f64(c->n, c->np, nc, c->ksplit, c->zpart, c->fpart, c->d2v_out, c->f_out,
+                    1.0 / (c->n_eff * c->n_syms), s);
   if (ev) (void)hipEventRecord(ev[3], s);
   return 0;
 }
