@@ -882,37 +882,46 @@ __global__ __launch_bounds__(512, 1) void outer_split(
   }
 }
 
-// FP64 sum of the FP32 partial tiles (fixed order), scales undone:
-// zsum[mu, nu] = sum_k zpart[k, mu, nu] / (su[mu] sb[nu])
-__global__ void reduce_ksplit_s32(const float* __restrict__ zpart_all,
-                                  const double* __restrict__ fpart_all,
-                                  const double* __restrict__ su, const double* __restrict__ sb_all,
-                                  int np, int ksplit, double* __restrict__ zsum_all,
-                                  double* __restrict__ f_all, double norm) {
-  const int chain = blockIdx.y;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// FP64 sum of the FP32 partial tiles (fixed order), scales undone, below n:
+// zsum[mu, nu] = sum_k zpart[k, mu, nu] / (su[mu] sb[nu]); 64 elements per
+// work-group, the partials in 4 slices of 8 loads in flight each, combined in LDS;
+// grid (ceil(n / 64), n + 1, chains), the last row the f sums.  Bound by latency:
+// one thread per element with the f sums behind its first rows took 31 us for two
+// chains of 381 modes (48 partials), 25 us now.
+__global__ __launch_bounds__(256) void reduce_ksplit_s32(
+    const float* __restrict__ zpart_all, const double* __restrict__ fpart_all,
+    const double* __restrict__ su, const double* __restrict__ sb_all, int n, int np, int ksplit,
+    double* __restrict__ zsum_all, double* __restrict__ f_all, double norm) {
+  const int chain = blockIdx.z, row = blockIdx.y;
+  const int t = threadIdx.x & 63, c = blockIdx.x * 64 + t, sl = threadIdx.x >> 6;
   const long nn = (long)np * np;
-  const float* zp = zpart_all + (long)chain * ksplit * nn;
-  if (e < nn) {
-    // eight loads in flight, summed in the same order as one at a time
-    double s = 0.0;
-    int k = 0;
-    for (; k + 8 <= ksplit; k += 8) {
-      float v[8];
+  const bool isf = row == n;
+  const float* zp = zpart_all + (long)chain * ksplit * nn + (long)row * np + c;
+  const double* fp = fpart_all + (long)chain * ksplit * np + c;
+  const int per = (ksplit + 3) / 4;
+  const int lo = sl * per, hi = lo + per < ksplit ? lo + per : ksplit;
+  double s = 0.0;
+  if (c < n) {
+    int k = lo;
+    for (; k + 8 <= hi; k += 8) {
+      double v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = zp[(long)(k + j) * nn + e];
+      for (int j = 0; j < 8; ++j) v[j] = isf ? fp[(long)(k + j) * np] : (double)zp[(k + j) * nn];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += (double)v[j];
+      for (int j = 0; j < 8; ++j) s += v[j];
     }
-    for (; k < ksplit; ++k) s += (double)zp[(long)k * nn + e];
-    const int mu = (int)(e / np), nu = (int)(e % np);
-    zsum_all[(long)chain * nn + e] = s / (su[mu] * sb_all[(long)chain * np + nu]);
+    for (; k < hi; ++k) s += isf ? fp[(long)k * np] : (double)zp[k * nn];
   }
-  if (e < np) {
-    const double* fp = fpart_all + (long)chain * ksplit * np;
-    double s = 0.0;
-    for (int k = 0; k < ksplit; ++k) s += fp[(long)k * np + e];
-    f_all[(long)chain * np + e] = s * norm;
+  __shared__ double red[4][64];
+  red[sl][t] = s;
+  __syncthreads();
+  if (sl == 0 && c < n) {
+    const double v = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+    if (isf)
+      f_all[(long)chain * np + c] = v * norm;
+    else
+      zsum_all[(long)chain * nn + (long)row * np + c] =
+          v / (su[row] * sb_all[(long)chain * np + c]);
   }
 }
 
@@ -1081,8 +1090,8 @@ static int launch_all(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* e
   if (ev) (void)hipEventRecord(ev[2], s);
   const long nn = (long)np * np;
   const double norm = 1.0 / (c->n_eff * c->n_syms);
-  hipLaunchKernelGGL(reduce_ksplit_s32, dim3((unsigned)((nn + 255) / 256), nc), dim3(256), 0, s,
-                     c->zpart32, c->fpart_s, st.su, c->sbsc, np, c->ksplit_s, c->d2v_out,
+  hipLaunchKernelGGL(reduce_ksplit_s32, dim3((c->n + 63) / 64, c->n + 1, nc), dim3(256), 0, s,
+                     c->zpart32, c->fpart_s, st.su, c->sbsc, c->n, np, c->ksplit_s, c->d2v_out,
                      c->f_out, norm);
   if (ev) (void)hipEventRecord(ev[3], s);
   TDS_CHECK_HIP(hipGetLastError());
