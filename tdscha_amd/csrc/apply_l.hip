@@ -18,6 +18,8 @@
 namespace tdscha {
 
 int run_pa(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_dev, hipStream_t s);
+bool orbit_translations(Ctx* c, int n_cart, const double* pols, int n_cells, const int* inv_perms,
+                        const double* proj);
 
 // coefficient rows of c->std_coef
 enum { SC_X = 0, SC_Y = 1, SC_X1 = 2, SC_Y1 = 3 };
@@ -412,21 +414,37 @@ __global__ void assemble_out(const double* __restrict__ psi_all, long len, int n
   out_all[chain * len + e] = v + shift * psi[e];
 }
 
+// R1, Y1 of the vectors, padded, into c->R1, c->Y1
+void launch_prepare_pert(Ctx* c, int nc, const double* psi, int use_wigner, int transpose,
+                         hipStream_t s) {
+  const long nn = (long)c->np * c->np, len = c->n + (long)c->n * (c->n + 1);
+  hipLaunchKernelGGL(prepare_pert, dim3((unsigned)((nn + 255) / 256), nc), dim3(256), 0, s, psi,
+                     len, c->n, c->np, c->pair_ca, c->pair_cb, c->yw, c->reaw, use_wigner,
+                     transpose, c->R1, c->Y1);
+}
+
+// plan: the orbit form of these vectors (a Lanczos run's); psi_host: the host's copy
+// of psi, where one may be looked for (waits for the stream)
 int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, int transpose,
                 int ignore_harmonic, int ignore_v3, int ignore_v4, int reverse, double shift,
-                int precision, hipStream_t s) {
+                int precision, hipStream_t s, const OrbPlan* plan,
+                const double* psi_host) {
   int rc = setup_pairs(c);
   if (rc) return rc;
-  const int n = c->n, np = c->np;
+  const int n = c->n;
   const long P = (long)n * (n + 1) / 2;
   const long len = n + 2 * P;
   const int anharmonic = ignore_v3 ? 0 : 1;
   if (anharmonic) {
-    const long nn = (long)np * np;
-    hipLaunchKernelGGL(prepare_pert, dim3((unsigned)((nn + 255) / 256), nc), dim3(256), 0, s, psi,
-                       len, n, np, c->pair_ca, c->pair_cb, c->yw, c->reaw, use_wigner, transpose,
-                       c->R1, c->Y1);
-    rc = run_pa(c, nc, ignore_v4 ? 0 : 1, precision, c->f_fin, c->d2v_fin, s);
+    launch_prepare_pert(c, nc, psi, use_wigner, transpose, s);
+    const int d4 = ignore_v4 ? 0 : 1;
+    if (!plan && psi_host && orbit_worth(c, nc, precision, psi_host, len)) {
+      rc = orbit_plan(c, nc, precision, s, c->orb.plan[0]);
+      if (rc) return rc;
+      plan = &c->orb.plan[0];
+    }
+    rc = plan && plan->ok ? run_pa_orbit(c, *plan, d4, c->f_fin, c->d2v_fin, s)
+                          : run_pa(c, nc, d4, precision, c->f_fin, c->d2v_fin, s);
     if (rc) return rc;
     if (c->n_cells > 0) {
       rc = project_translations(c, nc, s);
@@ -637,6 +655,8 @@ int tdscha_set_translations(tdscha_ctx* ctx, int n_cart, const double* pols, int
   TDS_CHECK_HIP(hipMemcpy(c->tproj, tT.data(), sizeof(double) * (long)n * n,
                           hipMemcpyHostToDevice));
   c->n_cells = n_cells;
+  c->orb.trans_ok = c->orb.usable && c->orb.group &&
+                    orbit_translations(c, n_cart, pols, n_cells, inv_perms, trans_projector);
   return 0;
 }
 
@@ -651,7 +671,7 @@ int tdscha_apply_L_dev(tdscha_ctx* ctx, int n_vec, const double* psi_dev, double
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : c->stream;
   return apply_L_dev(c, n_vec, psi_dev, out_dev, use_wigner, transpose, ignore_harmonic, ignore_v3,
-                     ignore_v4, reverse, shift, precision, s);
+                     ignore_v4, reverse, shift, precision, s, nullptr, nullptr);
 }
 
 int tdscha_apply_L(tdscha_ctx* ctx, int n_vec, const double* psi, double* out, int use_wigner,
@@ -666,9 +686,9 @@ int tdscha_apply_L(tdscha_ctx* ctx, int n_vec, const double* psi, double* out, i
   const long len = c->n + (long)c->n * (c->n + 1);
   TDS_CHECK_HIP(hipMemcpyAsync(c->psi_dev, psi, sizeof(double) * n_vec * len,
                                hipMemcpyHostToDevice, c->stream));
-  rc = tdscha_apply_L_dev(ctx, n_vec, c->psi_dev, c->psi_out_dev, use_wigner, transpose,
-                          ignore_harmonic, ignore_v3, ignore_v4, reverse, shift, precision,
-                          c->stream);
+  TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0, 1 or 2");
+  rc = apply_L_dev(c, n_vec, c->psi_dev, c->psi_out_dev, use_wigner, transpose, ignore_harmonic,
+                   ignore_v3, ignore_v4, reverse, shift, precision, c->stream, nullptr, psi);
   if (rc) return rc;
   TDS_CHECK_HIP(hipMemcpyAsync(out, c->psi_out_dev, sizeof(double) * n_vec * len,
                                hipMemcpyDeviceToHost, c->stream));

@@ -89,6 +89,53 @@ struct SplitStore {
   bool ready = false;
 };
 
+// Orbit form of the averages (orbit.hip)
+constexpr int kProbe = 8;            // probe configurations of the rank search
+constexpr int kOrbRank = 6;          // largest orbit of a chain
+constexpr int kOrbPairs = 24;        // rotated perturbations of one pass
+constexpr double kOrbTol = 1e-12;    // accuracy of the relation
+constexpr int kOrbClean = 3;         // Lanczos steps between projections on the sector
+// shortest general form (microseconds, estimated) for which the search, a wait
+// for the host of about 40 us and the rotations are worth trying
+constexpr double kOrbWorthUs = 500.0;
+
+struct OrbPlan {
+  bool ok = false;
+  int nc = 0, npairs = 0;
+  struct Round {
+    int chain0, chains, first, count;
+  };
+  std::vector<Round> rounds;   // passes of the clean-up
+  std::vector<char> host;
+  void* dev = nullptr;
+  size_t cap = 0;
+  int4 *mats = nullptr, *cmats = nullptr;
+  int2 *pairs = nullptr, *clean = nullptr;
+  double* C = nullptr;
+};
+
+struct Orbit {
+  bool usable = false;     // tables built
+  bool group = false;      // the symmetries are closed under multiplication
+  bool trans_ok = false;   // the translation average commutes with them
+  int nsym = 1, npanel = 0, rows = 0;
+  long Mp = 0;
+  std::vector<double> syms;               // host copy of the symmetry blocks
+  std::vector<int> gens;                  // generators of the group
+  double* arena = nullptr;                // holds start, S, ST, pu, pf (and U, F, rho)
+  int* start = nullptr;                   // [npanel + 1]
+  double *S = nullptr, *ST = nullptr;     // [npanel, nsym, 32, 32] panels of S_j, transposed
+  double *U = nullptr, *F = nullptr, *rho = nullptr;       // [Mp, np] the configurations
+  double *pu = nullptr, *pf = nullptr, *pones = nullptr;   // [rows, np] probe images
+  double* work = nullptr;                 // holds the workspaces below
+  double *ppart = nullptr;                // partial sums of the probe
+  double* pout = nullptr;                 // pinned host memory: its results
+  double *R1 = nullptr, *Y1 = nullptr;    // [kOrbPairs, np(, np)] rotated inputs
+  double *Rb = nullptr, *Yb = nullptr;    // [2 kMaxChains, np(, np)] unpacked vectors
+  double *coef = nullptr, *zpart = nullptr, *fpart = nullptr, *z = nullptr, *f = nullptr;
+  OrbPlan plan[1];                        // of the synchronous entries
+};
+
 // ------------------------------------------------------------- context
 struct Ctx {
   int device = 0;
@@ -198,9 +245,18 @@ struct Ctx {
   double* rot_t1 = nullptr;    // [kMaxChains, np, np] rotation intermediates
   double* rot_t2 = nullptr;
   double* rot_f = nullptr;     // [kMaxChains, np]
+  Orbit orb;
 };
 
 int ensure_split(Ctx* c, int prec);
+
+void orbit_plan_free(OrbPlan& p);
+bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld);
+int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p);
+int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
+                 hipStream_t s);
+int orbit_clean(Ctx* c, const OrbPlan& p, double* x, const int* kk, const int* active,
+                hipStream_t s);
 
 // FP64 GEMM launches (pa_fp64.hip), shared by every caller of the kernels
 struct F64Tiles {

@@ -25,6 +25,11 @@ bool rot_panels_fit(int dmax);
 int rot_panels(const int* bs, const int* d, int n, int np, int* start, int* nreal);
 int run_pa_rot(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_dev,
                hipStream_t s);
+int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const int* block_modes,
+                const std::vector<double>& syms, const double* X_dev, const double* Y_dev,
+                const double* rho_dev, const int* d_mb, const int* d_mp, const int* d_bd,
+                const int* d_bmo, const long* d_bso, const int* d_bm, const double* d_syms);
+void orbit_free(Ctx* c);
 
 // pad R1 (n) -> (np) and Y1 (n,n) -> symmetric (np,np); zero outside
 __global__ void pad_inputs(const double* __restrict__ R1, const double* __restrict__ Y1, int n,
@@ -85,6 +90,24 @@ int run_pa(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_de
                      norm, f_dev, d2v_dev);
   TDS_CHECK_HIP(hipGetLastError());
   return 0;
+}
+
+// R_host: the host's copy of R1, where a small orbit of the perturbations may be
+// looked for (waits for the stream)
+static int perturb_averages_dev(Ctx* c, int nc, const double* R1_dev, const double* Y1_dev,
+                                int apply_d4, int prec, double* f_dev, double* d2v_dev,
+                                hipStream_t s, const double* R_host) {
+  const long nn = (long)c->np * c->np;
+  dim3 g((unsigned)((nn + 255) / 256), nc);
+  hipLaunchKernelGGL(pad_inputs, g, dim3(256), 0, s, R1_dev, Y1_dev, c->n, c->np, c->R1, c->Y1);
+  TDS_CHECK_HIP(hipGetLastError());
+  if (R_host && orbit_worth(c, nc, prec, R_host, c->n)) {
+    OrbPlan& p = c->orb.plan[0];
+    const int rc = orbit_plan(c, nc, prec, s, p);
+    if (rc) return rc;
+    if (p.ok) return run_pa_orbit(c, p, apply_d4, f_dev, d2v_dev, s);
+  }
+  return run_pa(c, nc, apply_d4, prec, f_dev, d2v_dev, s);
 }
 
 }  // namespace tdscha
@@ -301,6 +324,8 @@ int tdscha_ctx_create(tdscha_ctx** out, int n_modes, int n_configs, const double
                        c->rho_img);
     ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess;
   }
+  ok = ok && orbit_setup(c, n_syms, n_blocks, block_dim, block_modes, hsyms, d_X, d_Y, d_rho, d_mb,
+                         d_mp, d_bd, d_bmo, d_bso, d_bm, d_syms) == 0;
   hipFree(d_mb); hipFree(d_mp); hipFree(d_bd); hipFree(d_bmo); hipFree(d_bm); hipFree(d_bso);
   hipFree(d_syms); hipFree(d_X); hipFree(d_Y); hipFree(d_rho);
   if (!ok) {
@@ -332,6 +357,7 @@ void tdscha_ctx_destroy(tdscha_ctx* ctx) {
     for (void* p : sp)
       if (p) hipFree(p);
   }
+  orbit_free(c);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
 }
@@ -361,11 +387,8 @@ int tdscha_perturb_averages_dev(tdscha_ctx* ctx, int n_chains, const double* R1_
   TDS_REQUIRE(R1_dev && Y1_dev && f_dev && d2v_dev, 2, "tdscha_perturb_averages_dev: NULL pointer");
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : c->stream;
-  const long nn = (long)c->np * c->np;
-  dim3 g((unsigned)((nn + 255) / 256), n_chains);
-  hipLaunchKernelGGL(pad_inputs, g, dim3(256), 0, s, R1_dev, Y1_dev, c->n, c->np, c->R1, c->Y1);
-  TDS_CHECK_HIP(hipGetLastError());
-  return run_pa(c, n_chains, apply_d4, precision, f_dev, d2v_dev, s);
+  return perturb_averages_dev(c, n_chains, R1_dev, Y1_dev, apply_d4, precision, f_dev, d2v_dev, s,
+                              nullptr);
 }
 
 int tdscha_perturb_averages_range(tdscha_ctx* ctx, int n_chains, const double* R1_dev,
@@ -409,7 +432,9 @@ int tdscha_perturb_averages_batched(tdscha_ctx* ctx, int n_chains, const double*
   double* dd = c->stage_out + (size_t)n_chains * n;
   TDS_CHECK_HIP(hipMemcpyAsync(dR, R1, sizeof(double) * n_chains * n, hipMemcpyHostToDevice, c->stream));
   TDS_CHECK_HIP(hipMemcpyAsync(dY, Y1, sizeof(double) * n_chains * nn, hipMemcpyHostToDevice, c->stream));
-  int rc = tdscha_perturb_averages_dev(ctx, n_chains, dR, dY, apply_d4, precision, df, dd, c->stream);
+  TDS_REQUIRE(apply_d4 == 0 || apply_d4 == 1, 2, "the apply_d4 value passed must be either 0 or 1");
+  TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0 (FP64), 1 (FP16x2) or 2 (BF16x2)");
+  int rc = perturb_averages_dev(c, n_chains, dR, dY, apply_d4, precision, df, dd, c->stream, R1);
   if (rc) return rc;
   TDS_CHECK_HIP(hipMemcpyAsync(f_out, df, sizeof(double) * n_chains * n, hipMemcpyDeviceToHost, c->stream));
   TDS_CHECK_HIP(hipMemcpyAsync(d2v_out, dd, sizeof(double) * n_chains * nn, hipMemcpyDeviceToHost, c->stream));

@@ -10,6 +10,7 @@
 // one step is a fixed kernel sequence: captured once as a hipGraph and
 // replayed, or the whole run captured and launched once.  Reductions are
 // two-stage with a fixed order (deterministic).
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -20,7 +21,10 @@ namespace tdscha {
 
 int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, int transpose,
                 int ignore_harmonic, int ignore_v3, int ignore_v4, int reverse, double shift,
-                int precision, hipStream_t s);
+                int precision, hipStream_t s, const OrbPlan* plan,
+                const double* psi_host);
+void launch_prepare_pert(Ctx* c, int nc, const double* psi, int use_wigner, int transpose,
+                         hipStream_t s);
 int setup_pairs(Ctx* c);
 
 constexpr int kRedBlocks = 128;   // blocks per chain in the partial reductions
@@ -28,15 +32,16 @@ constexpr int kRedThreads = 256;
 constexpr int kMaxRunChains = 64; // chains of one device Lanczos run
 
 // L applied to nc chains of the run, kMaxChains at a time (the perturbed
-// averages take up to kMaxChains per pass)
+// averages take up to kMaxChains per pass); plans: the groups' orbit forms
 static void apply_L_groups(Ctx* c, int nc, long len, const double* in, double* out,
                            int use_wigner, int transpose, int ignore_harmonic, int ignore_v3,
                            int ignore_v4, int reverse, double shift, int precision,
-                           hipStream_t s) {
+                           hipStream_t s, const std::vector<OrbPlan>* plans = nullptr) {
   for (int c0 = 0; c0 < nc; c0 += kMaxChains) {
     const int g = nc - c0 < kMaxChains ? nc - c0 : kMaxChains;
     apply_L_dev(c, g, in + (long)c0 * len, out + (long)c0 * len, use_wigner, transpose,
-                ignore_harmonic, ignore_v3, ignore_v4, reverse, shift, precision, s);
+                ignore_harmonic, ignore_v3, ignore_v4, reverse, shift, precision, s,
+                plans ? &(*plans)[c0 / kMaxChains] : nullptr, nullptr);
   }
 }
 
@@ -58,6 +63,8 @@ struct LanczosState {
   int* act2 = nullptr;       // [nc] chains whose second Gram-Schmidt pass runs
   int* cap = nullptr;        // [nc]
   int* ndone = nullptr;      // [nc] number of a coefficients
+  int* stepno = nullptr;     // steps taken by the run
+  std::vector<OrbPlan> plans;  // per group of kMaxChains chains (empty: general form)
   double* upart = nullptr;   // [nc, jsplit, len] basis-range partial updates (short vectors)
   int nslice = 1;            // element slices of the projections
   int jsplit = 1;            // basis-vector ranges of the update
@@ -66,9 +73,10 @@ struct LanczosState {
 
 static void free_state(LanczosState& s) {
   void* p[] = {s.Q, s.qcur, s.Lq, s.r, s.mask, s.part, s.coef, s.a, s.b, s.scal, s.k, s.active,
-               s.cap, s.ndone, s.upart, s.act2};
+               s.cap, s.ndone, s.upart, s.act2, s.stepno};
   for (void* x : p)
     if (x) (void)hipFree(x);
+  for (OrbPlan& q : s.plans) orbit_plan_free(q);
 }
 
 __global__ void build_mask(int n, long len, double* __restrict__ mask) {
@@ -279,8 +287,9 @@ __global__ void lanczos_advance(const double* __restrict__ part, long ps, long l
 __global__ void lanczos_commit(const double* __restrict__ part, long ps, int kmax, double tol,
                                int* __restrict__ kk, int* __restrict__ active,
                                const int* __restrict__ cap, int* __restrict__ ndone,
-                               double* __restrict__ b) {
+                               double* __restrict__ b, int* __restrict__ stepno) {
   const int c = threadIdx.x;
+  if (c == 0) stepno[0] += 1;
   if (!active[c]) return;
   const int k = kk[c];
   const double bk = sqrt(sum_partials(part + c * ps));
@@ -315,11 +324,15 @@ static void lanczos_step(Ctx* c, LanczosState& st, int reorth, int precision, in
   const dim3 gv((unsigned)((len + 255) / 256), nc);
   const dim3 gr(kRedBlocks, nc);
   apply_L_groups(c, nc, len, st.qcur, st.Lq, 1, 0, ignore_harmonic, ignore_v3, ignore_v4, 0,
-                 0.0, precision, s);
+                 0.0, precision, s, st.plans.empty() ? nullptr : &st.plans);
   hipLaunchKernelGGL(dot_partial, gr, dim3(kRedThreads), 0, s, st.qcur, len, st.Lq, len, st.mask,
                      len, st.part, ps, 0);
   hipLaunchKernelGGL(lanczos_residual, gv, dim3(256), 0, s, st.part, ps, st.Q, st.qcur, st.Lq,
                      len, kmax, st.k, st.active, st.a, st.b, st.scal, st.r);
+  for (size_t g = 0; g < st.plans.size(); ++g)
+    if (st.plans[g].ok)
+      orbit_clean(c, st.plans[g], st.r + (long)g * kMaxChains * len, st.stepno,
+                  st.active + g * kMaxChains, s);
   if (reorth) {
     // classical Gram-Schmidt against the whole basis; the second pass runs
     // for the chains whose first pass failed the norm test (flags in act2).
@@ -353,7 +366,7 @@ static void lanczos_step(Ctx* c, LanczosState& st, int reorth, int precision, in
   hipLaunchKernelGGL(lanczos_advance, gv, dim3(256), 0, s, st.part, ps, len, kmax, tol, st.k,
                      st.active, st.cap, st.ndone, st.b, st.r, st.Q, st.qcur);
   hipLaunchKernelGGL(lanczos_commit, dim3(1, 1), dim3(nc), 0, s, st.part, ps, kmax, tol, st.k,
-                     st.active, st.cap, st.ndone, st.b);
+                     st.active, st.cap, st.ndone, st.b, st.stepno);
 }
 
 __global__ void fill_int(int* p, int n, int v) {
@@ -698,10 +711,6 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   int rc = setup_pairs(c);
   if (rc) return rc;
-  if (precision != PREC_FP64) {
-    rc = ensure_split(c, precision);  // allocations must precede graph capture
-    if (rc) return rc;
-  }
   const int n = c->n;
   LanczosState st;
   st.nc = n_chains;
@@ -723,7 +732,8 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
             hipMalloc((void**)&st.active, sizeof(int) * n_chains) == hipSuccess &&
             hipMalloc((void**)&st.act2, sizeof(int) * n_chains) == hipSuccess &&
             hipMalloc((void**)&st.cap, sizeof(int) * n_chains) == hipSuccess &&
-            hipMalloc((void**)&st.ndone, sizeof(int) * n_chains) == hipSuccess;
+            hipMalloc((void**)&st.ndone, sizeof(int) * n_chains) == hipSuccess &&
+            hipMalloc((void**)&st.stepno, sizeof(int)) == hipSuccess;
   // projections: element slices of >= 4096 entries (at most 64); updates of
   // short vectors split over ranges of basis vectors so that enough
   // work-groups run
@@ -759,6 +769,7 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
       hipMemcpyAsync(st.r, psi0, sizeof(double) * n_chains * len, hipMemcpyHostToDevice, s) != hipSuccess)
     return fail("upload failed");
   hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, s, st.k, n_chains, 0);
+  hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, s, st.stepno, 1, 0);
   hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, s, st.active, n_chains, 1);
   hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, s, st.ndone, n_chains, 0);
   // a chain that stops on |b| < tol leaves its last b slot unwritten: the
@@ -777,6 +788,30 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
                      st.part, ps, st.r, len, n_steps, st.Q, st.qcur);
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
     return fail("initialisation failed");
+  // orbit form per group of chains, from the start vectors: an operator that
+  // commutes with the symmetry group keeps their relation
+  const bool sector = !ignore_v3 && c->orb.group && (c->n_cells == 0 || c->orb.trans_ok);
+  bool general = !sector;
+  if (sector)
+    for (int c0 = 0; c0 < n_chains; c0 += kMaxChains) {
+      const int g = std::min(kMaxChains, n_chains - c0);
+      st.plans.emplace_back();
+      if (orbit_worth(c, g, precision, psi0 + (long)c0 * len, len)) {
+        launch_prepare_pert(c, g, st.qcur + (long)c0 * len, 1, 0, s);
+        if (orbit_plan(c, g, precision, s, st.plans.back())) {
+          free_state(st);
+          return -1;
+        }
+      }
+      general = general || !st.plans.back().ok;
+    }
+  if (general && precision != PREC_FP64) {
+    rc = ensure_split(c, precision);  // allocations must precede graph capture
+    if (rc) {
+      free_state(st);
+      return rc;
+    }
+  }
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
     return fail("event creation failed");
   // use_graph 1: one step captured and replayed; 2: the whole run captured

@@ -1,0 +1,947 @@
+// Symmetrised perturbed averages from the orbit of the perturbation.
+//
+// With the S_j block diagonal over degenerate modes (on which fY and fpsi are
+// constant), the average over all images is
+//   T_sym(v) = (1 / n_syms) sum_j S_j T(S_j^T v),
+// T the average over the configurations alone and v = (R1, Y1) with S^T v =
+// (S^T R1, S^T Y1 S), S (f, d2v) = (S f, S d2v S^T) (rotate.hip).  T is
+// linear, so when the n_syms rotated perturbations span only r dimensions,
+//   S_j^T v = sum_k C_jk S_jk^T v   (k = 1 .. r),
+//   T_sym(v) = (1 / n_syms) sum_j S_j sum_k C_jk T(S_jk^T v):
+// r averages over the N configurations instead of one over N n_syms images.
+// The perturbations of linear response have small orbits: r = 3 for an IR
+// (vector) perturbation of a cubic crystal, at most 6 for a Raman (tensor) one,
+// against 48 images.
+//
+// The rank is found for each call from the perturbation itself, not assumed: the
+// row-dots of the averages (s1 = u.Y1.u, s2 = u.Y1.(fpsi f), s3 = (fY u).R1,
+// s4 = f.R1) are evaluated on all images of kProbe random configurations of the
+// thermal amplitudes; a relation C that holds for these 4 kProbe functionals
+// to kOrbTol holds for the perturbation (random functionals: a remainder that
+// all of them miss has probability zero, and one that the 26 beyond the rank
+// understate tenfold 1e-26).  Otherwise the general form is used.  kOrbTol is the accuracy
+// to which the symmetry tables themselves are a representation (1e-12 on 381
+// modes).
+//
+// A Lanczos run whose operator commutes with the symmetries (they form a group
+// and the translation average commutes with them, both checked numerically)
+// keeps the relation C of its start vector.  Rounding leaves that sector and
+// the three-term recurrence amplifies it (about 5-fold per step), so the residual is
+// projected back every kOrbClean steps with the same two kernels.
+//
+// Measured, three IR vectors, one application of L in FP64 (host arrays in and out):
+// 128 atoms x 20000 configurations x 48: 9 averages over 20,096 rows instead of
+// three over 960,000 images, 29.1 -> 2.73 ms (weights 1.04, outer 1.03, rotations
+// 0.20 ms); 54 atoms x 5000 x 48: 1.70 -> 0.47 ms.
+#include <algorithm>
+#include <cmath>
+#include <random>
+#include <vector>
+
+#include "common.hpp"
+
+namespace tdscha {
+
+__global__ void expand_images(const double*, const double*, const double*, const int*, const int*,
+                              const int*, const int*, const long*, const int*, const double*, int,
+                              int, int, long, double*, double*, double*);
+__global__ void rot_copy_configs(const double* X, const double* Y, const double* rho, int n, int np,
+                                 long N, long Mp, double* U, double* F, double* rho_img);
+int rot_panels(const int* bs, const int* d, int n, int np, int* start, int* nreal);
+
+constexpr int kOP = 32;          // modes of a panel (whole blocks)
+constexpr int kOLd = kOP + 1;
+
+static __device__ __forceinline__ double mfma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+
+// v of the lane 4 R lanes before, cyclic within a row of 16 lanes
+template <int R>
+static __device__ __forceinline__ double rot4(double v) {
+  if constexpr (R == 0) return v;
+  constexpr int ctrl = 0x120 + 4 * R;   // row_ror:4R
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// acc += A B for a 16 x 16 block, 4 of the K index: A[i][k] i = lane % 16,
+// B[k][j] j = lane % 16, k = lane / 16; acc[r] of a lane is the element of row
+// 4 q + lane / 16, column 4 ((q - r) % 4) + lane % 4 (q = lane / 4 % 4)
+static __device__ __forceinline__ void mma16(double a, double b, double (&acc)[4]) {
+  acc[0] = mfma4(a, b, acc[0]);
+  acc[1] = mfma4(a, rot4<1>(b), acc[1]);
+  acc[2] = mfma4(a, rot4<2>(b), acc[2]);
+  acc[3] = mfma4(a, rot4<3>(b), acc[3]);
+}
+
+// ------------------------------------------------------------------- the probe
+// row-dots of 16 probe rows over 16 columns of V = U Y1, a quarter of the K index
+// per wave (the dots are linear in V); grid (rows / 16, ceil(n / 16), chains):
+// many short work-groups, since the host waits for the result (31 us for three
+// chains of 381 modes, 60 us with 64 rows to a work-group)
+__global__ __launch_bounds__(256) void orb_probe(const double* __restrict__ U,
+                                                 const double* __restrict__ F,
+                                                 const double* __restrict__ Y1all,
+                                                 const double* __restrict__ R1all,
+                                                 const double* __restrict__ fy,
+                                                 const double* __restrict__ fpsi, int np, int nk,
+                                                 int rows, double* __restrict__ part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lr = lane & 15, lg = lane >> 4, lq = lane & 3, lb = (lane >> 2) & 3;
+  const int r0 = blockIdx.x * 16, c0 = blockIdx.y * 16, chain = blockIdx.z;
+  const double* pu = U + (long)(r0 + lr) * np + lg;
+  const double* py = Y1all + (long)chain * np * np + (long)lg * np + c0 + lr;
+  const double* R1 = R1all + (long)chain * np;
+  __shared__ double red[4][16][4];
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int k0 = 16 * wave; k0 < nk; k0 += 64) {
+    double a[4], b[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      a[k] = pu[k0 + 4 * k];
+      b[k] = py[(long)(k0 + 4 * k) * np];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mma16(a[k], b[k], acc);
+  }
+  const int row = r0 + 4 * lb + lg;
+  double p[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int col = c0 + 4 * ((lb - r) & 3) + lq;
+    const double u = U[(long)row * np + col], f = F[(long)row * np + col], r1 = R1[col];
+    p[0] += acc[r] * u;
+    p[1] += acc[r] * (f * fpsi[col]);
+    if (wave == 0) {
+      p[2] += u * (fy[col] * r1);
+      p[3] += f * r1;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    p[q] += __shfl_xor(p[q], 1);
+    p[q] += __shfl_xor(p[q], 2);
+  }
+  red[wave][4 * lb + lg][lq] = lq < 2 ? (lq ? p[1] : p[0]) : (lq == 2 ? p[2] : p[3]);
+  __syncthreads();
+  if (wave == 0) {
+    const int rr = lane >> 2;
+    part[(((long)chain * gridDim.y + blockIdx.y) * rows + r0 + rr) * 4 + lq] =
+        (red[0][rr][lq] + red[1][rr][lq]) + (red[2][rr][lq] + red[3][rr][lq]);
+  }
+}
+
+__global__ void orb_probe_sum(const double* __restrict__ part, int ncol, int rows4,
+                              double* __restrict__ out) {
+  const int chain = blockIdx.y, e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows4) return;
+  double s = 0.0;
+#pragma unroll 8
+  for (int c = 0; c < ncol; ++c) s += part[((long)chain * ncol + c) * rows4 + e];
+  out[(long)chain * rows4 + e] = s;
+}
+
+// --------------------------------------------------------------- rotations
+// Tiles of the panels (whole degenerate blocks, at most 32 modes): S_j is block
+// diagonal, so a tile of S_j^T A S_j (or S_j A S_j^T) is a product of the tile of A
+// with the two panels' diagonal parts of S_j, from tables padded with zeros to
+// 32 x 32.  Four waves, one 16 x 16 quadrant each.
+struct OrbPanels {
+  const int* start;   // [npanel + 1]
+  int npanel;
+  int nsym;
+  const double* S;    // [npanel, nsym, 32, 32]
+  const double* ST;   // the same, transposed
+};
+
+// pair p = (source matrix, symmetry j): Yo[p] = S_j^T Y[src] S_j, Ro[p] =
+// S_j^T R[src] (modes below n; the padding of Yo, Ro stays zero).  skip: see
+// orb_out.
+__global__ __launch_bounds__(256) void orb_in(OrbPanels pn, const int2* __restrict__ pairs,
+                                              const double* __restrict__ Yb,
+                                              const double* __restrict__ Rb, int np,
+                                              const int* __restrict__ kk, int every,
+                                              double* __restrict__ Yo, double* __restrict__ Ro) {
+  if (every && (kk[0] % every) != every - 1) return;
+  const int pi = blockIdx.x / pn.npanel, pj = blockIdx.x % pn.npanel, p = blockIdx.y;
+  const int src = pairs[p].x, j = pairs[p].y;
+  const int r0 = pn.start[pi], h = pn.start[pi + 1] - r0;
+  const int q0 = pn.start[pj], w = pn.start[pj + 1] - q0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wr = 16 * (wave >> 1), wc = 16 * (wave & 1);
+  const int lr = lane & 15, lg = lane >> 4, lq = lane & 3, lb = (lane >> 2) & 3;
+  __shared__ double T[kOP][kOLd];
+  const double* Si = pn.S + ((long)pi * pn.nsym + j) * kOP * kOP;
+  const double* Sj = pn.S + ((long)pj * pn.nsym + j) * kOP * kOP;
+  const double* Y = Yb + (long)src * np * np;
+  double a[8], b[8], s[8];
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) {
+    const int k = 4 * ks + lg;
+    a[ks] = Si[k * kOP + wr + lr];
+    const bool in = k < h && wc + lr < w;
+    b[ks] = in ? Y[(long)(r0 + k) * np + q0 + wc + lr] : 0.0;
+    s[ks] = Sj[k * kOP + wc + lr];
+  }
+  double t[4] = {0.0, 0.0, 0.0, 0.0}, o[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) mma16(a[ks], b[ks], t);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) T[wr + 4 * lb + lg][wc + 4 * ((lb - r) & 3) + lq] = t[r];
+  __syncthreads();
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) mma16(T[wr + lr][4 * ks + lg], s[ks], o);
+  const int row = wr + 4 * lb + lg;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int col = wc + 4 * ((lb - r) & 3) + lq;
+    if (row < h && col < w) Yo[(long)p * np * np + (long)(r0 + row) * np + q0 + col] = o[r];
+  }
+  if (pj == 0 && (int)threadIdx.x < h) {
+    const double* R = Rb + (long)src * np + r0;
+    double v = 0.0;
+    for (int m = 0; m < h; ++m) v += Si[m * kOP + threadIdx.x] * R[m];
+    Ro[(long)p * np + r0 + threadIdx.x] = v;
+  }
+}
+
+// Matrix m = (first pair, rank, relation): sum_j S_j (sum_k C_jk D_k) S_j^T and
+// sum_j S_j sum_k C_jk f_k.  AVG: D_k = fY Z_k + (fY Z_k)^T of the raw outer
+// sums, results to f_out, d_out (both halves).  Else D_k the symmetric inputs,
+// results to the packed vectors x [chain][n + 2 P] (matrix m = 2 chain + sector; R
+// with sector 0), in which case the kernel runs only on every `every`-th step.
+// grid (panel pairs pi <= pj, matrices); per symmetry a wave combines D in
+// registers (its 16 rows), and the product with S_pj^T passes through LDS.  Bound by
+// the latency of that chain over the symmetries (few tiles): two groups of four waves
+// take every other one, 97 instead of 128 us at 159 modes, 185 (171) us at 381.
+template <bool AVG>
+__global__ __launch_bounds__(512) void orb_out(
+    OrbPanels pn, const int4* __restrict__ mats, const double* __restrict__ C,
+    const double* __restrict__ Zb, const double* __restrict__ fb, const double* __restrict__ fy,
+    int n, int np, double normf, double normd, const int* __restrict__ kk, int every,
+    const int* __restrict__ active, double* __restrict__ f_out, double* __restrict__ d_out) {
+  if (every && (kk[0] % every) != every - 1) return;
+  const int m = blockIdx.y;
+  const int4 mt = mats[m];
+  if (!AVG && !active[m >> 1]) return;
+  int pj = 0, pi = blockIdx.x;
+  while (pi > pj) pi -= ++pj;   // pair (pi, pj), pi <= pj
+  const int r0 = pn.start[pi], h = pn.start[pi + 1] - r0;
+  const int q0 = pn.start[pj], w = pn.start[pj + 1] - q0;
+  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, half = threadIdx.x >> 8;
+  const int wr = 16 * (wave >> 1), wc = 16 * (wave & 1);
+  const int lr = lane & 15, lg = lane >> 4, lq = lane & 3, lb = (lane >> 2) & 3;
+  __shared__ double T[2][2][kOP][kOLd];
+  const long nn = (long)np * np;
+  const int rank = mt.y;
+  double d[kOrbRank][8];
+#pragma unroll
+  for (int k = 0; k < kOrbRank; ++k)
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      const int a = wr + lr, b = 4 * ks + lg;
+      double v = 0.0;
+      if (k < rank && a < h && b < w) {
+        const double* z = Zb + (long)(mt.x + k) * nn;
+        v = z[(long)(r0 + a) * np + q0 + b];
+        if (AVG) v = fy[r0 + a] * v + fy[q0 + b] * z[(long)(q0 + b) * np + r0 + a];
+      }
+      d[k][ks] = v;
+    }
+  const double* Cm = C + (long)mt.z * pn.nsym * kOrbRank;
+  const double* Ti = pn.ST + (long)pi * pn.nsym * kOP * kOP + wr + lr;
+  const double* Tj = pn.ST + (long)pj * pn.nsym * kOP * kOP + wc + lr;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int jj = 0; jj < pn.nsym; jj += 2) {
+    // the halves take every other symmetry (weight zero past the last)
+    const bool in = jj + half < pn.nsym;
+    const int j = in ? jj + half : 0;
+    double sj[8], si[8], mm[8];
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      sj[ks] = Tj[(long)j * kOP * kOP + (4 * ks + lg) * kOP];
+      si[ks] = Ti[(long)j * kOP * kOP + (4 * ks + lg) * kOP];
+      mm[ks] = 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < kOrbRank; ++k)
+      if (k < rank) {
+        const double c = in ? Cm[j * kOrbRank + k] : 0.0;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) mm[ks] += c * d[k][ks];
+      }
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) mma16(mm[ks], sj[ks], t);
+    double(*Tb)[kOLd] = T[half][(jj >> 1) & 1];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) Tb[wr + 4 * lb + lg][wc + 4 * ((lb - r) & 3) + lq] = t[r];
+    __syncthreads();   // (the other buffer was last read before this barrier)
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) mma16(si[ks], Tb[4 * ks + lg][wc + lr], acc);
+  }
+  __syncthreads();
+  double(*sum)[kOP * kOP / 4] = reinterpret_cast<double(*)[kOP * kOP / 4]>(&T[0][0][0][0]);
+  if (half)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sum[r][threadIdx.x & 255] = acc[r];
+  __syncthreads();
+  if (!half)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] += sum[r][threadIdx.x];
+  const int row = wr + 4 * lb + lg;
+  const long P = (long)n * (n + 1) / 2, len = n + 2 * P;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int col = wc + 4 * ((lb - r) & 3) + lq;
+    if (half || row >= h || col >= w) continue;
+    const int gr = r0 + row, gc = q0 + col;
+    const double v = normd * acc[r];
+    if (AVG) {
+      if (gr > gc) continue;   // exactly symmetric
+      double* o = d_out + (long)m * n * n;
+      o[(long)gr * n + gc] = v;
+      o[(long)gc * n + gr] = v;
+    } else if (gr <= gc) {
+      const long p = (long)gr * n - (long)gr * (gr - 1) / 2 + (gc - gr);
+      d_out[(m >> 1) * len + n + (m & 1) * P + p] = v;
+    }
+  }
+  if (pi != pj || !(AVG || (m & 1) == 0)) return;
+  // f of the panel: thread = (mode, every sixteenth symmetry), f_k in LDS
+  __syncthreads();
+  double(*fs)[kOP] = reinterpret_cast<double(*)[kOP]>(&T[0][0][0][0]);   // [kOrbRank][32]
+  double(*part)[kOP] = reinterpret_cast<double(*)[kOP]>(&T[1][0][0][0]); // [16][32]
+  const int t = threadIdx.x & 31, sl = threadIdx.x >> 5;
+  if (sl < rank) fs[sl][t] = t < h ? fb[(long)(mt.x + sl) * np + r0 + t] : 0.0;
+  __syncthreads();
+  const double* St = pn.ST + (long)pi * pn.nsym * kOP * kOP + t;
+  double v = 0.0;
+  for (int j = sl; j < pn.nsym; j += 16) {
+    double g[kOrbRank];
+#pragma unroll
+    for (int k = 0; k < kOrbRank; ++k) g[k] = 0.0;
+#pragma unroll 8
+    for (int b = 0; b < kOP; ++b) {
+      const double st = St[((long)j * kOP + b) * kOP];
+#pragma unroll
+      for (int k = 0; k < kOrbRank; ++k)
+        if (k < rank) g[k] += st * fs[k][b];
+    }
+#pragma unroll
+    for (int k = 0; k < kOrbRank; ++k)
+      if (k < rank) v += Cm[j * kOrbRank + k] * g[k];
+  }
+  part[sl][t] = v;
+  __syncthreads();
+  if ((int)threadIdx.x < h) {
+    double f = 0.0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) f += part[q][t];
+    if (AVG)
+      f_out[(long)m * n + r0 + t] = normf * f;
+    else
+      d_out[(m >> 1) * len + r0 + t] = normf * f;
+  }
+}
+
+// packed vectors -> symmetric padded matrices [2 chain + sector] and R (zero for
+// sector 1)
+__global__ void orb_unpack(const double* __restrict__ x, int n, int np,
+                           const int* __restrict__ kk, int every, double* __restrict__ Yb,
+                           double* __restrict__ Rb) {
+  if (every && (kk[0] % every) != every - 1) return;
+  const int m = blockIdx.y;
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= (long)np * np) return;
+  const int a = (int)(e / np), b = (int)(e % np);
+  const long P = (long)n * (n + 1) / 2, len = n + 2 * P;
+  const double* v = x + (m >> 1) * len;
+  double y = 0.0;
+  if (a < n && b < n) {
+    const int r = a < b ? a : b, c = a < b ? b : a;
+    y = v[n + (m & 1) * P + (long)r * n - (long)r * (r - 1) / 2 + (c - r)];
+  }
+  Yb[(long)m * np * np + e] = y;
+  if (e < np) Rb[(long)m * np + e] = (e < n && (m & 1) == 0) ? v[e] : 0.0;
+}
+
+// --------------------------------------------------------------------- tables
+// panel parts of S_j, and transposed: grid (panels, symmetries), 1024 threads
+__global__ void orb_tables(const int* __restrict__ start, const int* __restrict__ mode_block,
+                           const int* __restrict__ mode_pos, const int* __restrict__ block_dim,
+                           const long* __restrict__ block_soff, const double* __restrict__ syms,
+                           int nsym, double* __restrict__ S, double* __restrict__ ST) {
+  const int q = blockIdx.x, j = blockIdx.y, x = threadIdx.x >> 5, y = threadIdx.x & 31;
+  const int r = start[q] + x, c = start[q] + y, e = start[q + 1];
+  double v = 0.0;
+  if (r < e && c < e && mode_block[r] == mode_block[c]) {
+    const int b = mode_block[r], d = block_dim[b];
+    v = syms[block_soff[b] + ((long)j * d + mode_pos[r]) * d + mode_pos[c]];
+  }
+  const long base = ((long)q * nsym + j) * kOP * kOP;
+  S[base + x * kOP + y] = v;
+  ST[base + y * kOP + x] = v;
+}
+
+// Whether the tables allow the orbit form: blocks of consecutive modes (at most
+// 32) on which fY and fpsi are constant to 1e-13.
+static bool blocks_fit(const Ctx* c, int n_blocks, const int* block_dim, const int* block_modes,
+                       const std::vector<double>& fy) {
+  int off = 0;
+  for (int b = 0; b < n_blocks; ++b) {
+    const int d = block_dim[b];
+    if (d > kOP) return false;
+    double lo = 1e300, hi = 0.0;
+    for (int k = 0; k < d; ++k) {
+      if (block_modes[off + k] != block_modes[off] + k) return false;
+      lo = std::min(lo, fy[block_modes[off + k]]);
+      hi = std::max(hi, fy[block_modes[off + k]]);
+    }
+    if (!(hi - lo <= 1e-13 * hi)) return false;
+    off += d;
+  }
+  return true;
+}
+
+// S_j z (or S_j^T z)
+static void apply_s(const Ctx* c, const std::vector<double>& syms, int j, bool transpose,
+                    const double* z, double* out) {
+  const Orbit& o = c->orb;
+  long so = 0;
+  int off = 0;
+  for (int d : c->block_dim) {
+    const double* S = syms.data() + so + (long)j * d * d;
+    const int m0 = c->block_modes[off];
+    for (int a = 0; a < d; ++a) {
+      double v = 0.0;
+      for (int b = 0; b < d; ++b) v += (transpose ? S[b * d + a] : S[a * d + b]) * z[m0 + b];
+      out[m0 + a] = v;
+    }
+    so += (long)o.nsym * d * d;
+    off += d;
+  }
+}
+
+static double dot(const double* x, const double* y, int n) {
+  double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  int m = 0;
+  for (; m + 8 <= n; m += 8)
+    for (int k = 0; k < 8; ++k) s[k] += x[m + k] * y[m + k];
+  for (; m < n; ++m) s[0] += x[m] * y[m];
+  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
+// Whether the S_j are closed under multiplication: p.S_i S_j z equals p.S_k z for
+// one k for two independent random pairs (p, z), to 1e-9 of their size.  Fills
+// the list of generators.
+static bool closed(Ctx* c) {
+  Orbit& o = c->orb;
+  const int ns = o.nsym, n = c->n;
+  std::mt19937_64 g(12345);
+  std::normal_distribution<double> nd;
+  std::vector<double> A[2], B[2], ref(2 * (size_t)ns);
+  for (int t = 0; t < 2; ++t) {
+    std::vector<double> p(n), z(n);
+    for (double& v : p) v = nd(g);
+    for (double& v : z) v = nd(g);
+    A[t].resize((size_t)ns * n);
+    B[t].resize((size_t)ns * n);
+    for (int j = 0; j < ns; ++j) {
+      apply_s(c, o.syms, j, true, p.data(), A[t].data() + (size_t)j * n);
+      apply_s(c, o.syms, j, false, z.data(), B[t].data() + (size_t)j * n);
+      ref[2 * (size_t)j + t] = dot(p.data(), B[t].data() + (size_t)j * n, n);
+    }
+  }
+  const double tol = 1e-9 * n;
+  std::vector<int> order(ns), table((size_t)ns * ns);
+  for (int j = 0; j < ns; ++j) order[j] = j;
+  std::sort(order.begin(), order.end(),
+            [&](int a, int b) { return ref[2 * (size_t)a] < ref[2 * (size_t)b]; });
+  for (int i = 0; i < ns; ++i)
+    for (int j = 0; j < ns; ++j) {
+      double v[2];
+      for (int t = 0; t < 2; ++t)
+        v[t] = dot(A[t].data() + (size_t)i * n, B[t].data() + (size_t)j * n, n);
+      auto it = std::lower_bound(order.begin(), order.end(), v[0] - tol,
+                                 [&](int a, double x) { return ref[2 * (size_t)a] < x; });
+      int hit = -1;
+      for (; it != order.end() && ref[2 * (size_t)*it] <= v[0] + tol && hit < 0; ++it)
+        if (std::fabs(ref[2 * (size_t)*it + 1] - v[1]) <= tol) hit = *it;
+      if (hit < 0) return false;
+      table[(size_t)i * ns + j] = hit;
+    }
+  // generators: add elements until their products reach the whole list
+  std::vector<char> in(ns, 0);
+  std::vector<int> sub;
+  o.gens.clear();
+  for (int j = 0; j < ns; ++j) {
+    if (in[j]) continue;
+    o.gens.push_back(j);
+    in[j] = 1;
+    sub.push_back(j);
+    for (size_t a = 0; a < sub.size(); ++a)
+      for (int q : o.gens)
+        for (int k : {table[(size_t)sub[a] * ns + q], table[(size_t)q * ns + sub[a]]})
+          if (!in[k]) {
+            in[k] = 1;
+            sub.push_back(k);
+          }
+  }
+  return true;
+}
+
+// Whether the translation average commutes with the group's generators, on random
+// vectors: the mean projector (proj z against its rotation), and the second
+// moment over the permutations that the average of d2v applies.
+bool orbit_translations(Ctx* c, int n_cart, const double* pols, int n_cells, const int* inv_perms,
+                        const double* proj) {
+  const Orbit& o = c->orb;
+  const int n = c->n;
+  std::mt19937_64 g(777);
+  std::normal_distribution<double> nd;
+  std::vector<double> z(n), p(n), sz(n), sp(n), u(n), v(n), t(n);
+  std::vector<double> cz(n_cart), cp(n_cart), csz(n_cart), csp(n_cart);
+  for (double& x : z) x = nd(g);
+  for (double& x : p) x = nd(g);
+  auto matvec = [&](const double* M, int rows, const std::vector<double>& x,
+                    std::vector<double>& y) {
+    for (int a = 0; a < rows; ++a) y[a] = dot(M + (size_t)a * n, x.data(), n);
+  };
+  // sum over t of (p . T_t z)^2, T_t = pols^T P_t pols: (P_t x)[a] = x[inv_perm_t[a]]
+  auto second = [&](const std::vector<double>& pc, const std::vector<double>& zc) {
+    double s = 0.0;
+    for (int q = 0; q < n_cells; ++q) {
+      double d = 0.0;
+      for (int a = 0; a < n_cart; ++a) d += pc[a] * zc[inv_perms[(size_t)q * n_cart + a]];
+      s += d * d;
+    }
+    return s;
+  };
+  matvec(proj, n, z, t);
+  matvec(pols, n_cart, z, cz);
+  matvec(pols, n_cart, p, cp);
+  double scale = 0.0;
+  for (int m = 0; m < n; ++m) scale = std::max(scale, std::fabs(z[m]));
+  for (int j : o.gens) {
+    apply_s(c, o.syms, j, false, z.data(), sz.data());
+    apply_s(c, o.syms, j, false, t.data(), v.data());
+    apply_s(c, o.syms, j, true, p.data(), sp.data());
+    matvec(proj, n, sz, u);
+    for (int m = 0; m < n; ++m)
+      if (!(std::fabs(u[m] - v[m]) <= 1e-9 * scale)) return false;
+    matvec(pols, n_cart, sz, csz);
+    matvec(pols, n_cart, sp, csp);
+    const double s1 = second(cp, csz), s2 = second(csp, cz);
+    if (!(std::fabs(s1 - s2) <= 1e-9 * (std::fabs(s1) + std::fabs(s2)))) return false;
+  }
+  return true;
+}
+
+static double estimate_us(double flop, int prec) {
+  // sustained rates of the GEMM pairs: 55 TF/s in FP64, 300 TF/s (counted once,
+  // not three times) in the split precisions
+  return flop / (prec == PREC_FP64 ? 5.5e7 : 3e8);
+}
+
+static double pass_flop(const Ctx* c, double rows) {
+  const double n16 = round_up(c->n, 16);
+  return 4.0 * rows * n16 * n16;
+}
+
+// The configurations, panel tables and probe rows; called at context creation
+// with the configurations still on the device.  Leaves c->orb.usable false where
+// the form does not apply or cannot pay (the general form of 8 chains under
+// kOrbWorthUs), or with more than 512 symmetries (the tables and the closure check
+// grow with their number and its square).
+int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const int* block_modes,
+                const std::vector<double>& syms, const double* X_dev, const double* Y_dev,
+                const double* rho_dev, const int* d_mb, const int* d_mp, const int* d_bd,
+                const int* d_bmo, const long* d_bso, const int* d_bm, const double* d_syms) {
+  Orbit& o = c->orb;
+  o.nsym = n_syms;
+  const double images = (double)c->N * n_syms;
+  if (n_syms < 4 || n_syms > 512 || estimate_us(8 * pass_flop(c, images), PREC_FP64) < kOrbWorthUs) return 0;
+  const int n = c->n, np = c->np;
+  std::vector<double> fy(np);
+  TDS_CHECK_HIP(hipMemcpy(fy.data(), c->fy, sizeof(double) * np, hipMemcpyDeviceToHost));
+  if (!blocks_fit(c, n_blocks, block_dim, block_modes, fy)) return 0;
+  // panels
+  std::vector<int> bs(n), dd(n), start(n + 2);
+  {
+    int off = 0;
+    for (int b = 0; b < n_blocks; ++b)
+      for (int k = 0, o0 = off; k < block_dim[b]; ++k, ++off) {
+        bs[block_modes[off]] = block_modes[o0];
+        dd[block_modes[off]] = block_dim[b];
+      }
+  }
+  int nreal = 0;
+  rot_panels(bs.data(), dd.data(), n, np, start.data(), &nreal);
+  o.npanel = nreal;
+  start[nreal] = n;
+  const size_t ntab = (size_t)nreal * n_syms * kOP * kOP;
+  o.syms = syms;
+  o.group = closed(c);
+  // probe configurations: thermal amplitudes for x; forces of the same weight
+  // in s2 = u.Y1.(fpsi f) as x has in s1
+  std::mt19937_64 g(2024);
+  std::normal_distribution<double> nd;
+  std::vector<double> px((size_t)kProbe * n), py(px.size()), ones(kProbe, 1.0);
+  for (int i = 0; i < kProbe; ++i)
+    for (int m = 0; m < n; ++m) {
+      px[(size_t)i * n + m] = nd(g) / std::sqrt(fy[m]);
+      py[(size_t)i * n + m] = nd(g) * std::sqrt(fy[m]);
+    }
+  o.rows = round_up(kProbe * n_syms, 16);
+  // one allocation: tables, probe rows, and the inputs of the kernels that fill them
+  size_t at = 0;
+  auto place = [&](size_t count) {
+    const size_t here = at;
+    at += (count + 31) / 32 * 32;
+    return here;
+  };
+  o.Mp = c->rotate ? c->Mp : round_up_l(c->N, 128);
+  const size_t np_rows = (size_t)o.rows * np, own = c->rotate ? 0 : (size_t)o.Mp;
+  const size_t aS = place(ntab), aST = place(ntab), apu = place(np_rows), apf = place(np_rows),
+               apo = place(o.rows), adx = place(px.size()), ady = place(py.size()),
+               ad1 = place(ones.size()), ast = place(nreal + 1), aU = place(own * np),
+               aF = place(own * np), arho = place(own);
+  auto up = [](void* dst, const void* src, size_t bytes) {
+    return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess;
+  };
+  if (hipMalloc((void**)&o.arena, sizeof(double) * at) != hipSuccess) {
+    (void)hipGetLastError();   // no room: the general form serves every call
+    return 0;
+  }
+  o.S = o.arena + aS; o.ST = o.arena + aST;
+  o.pu = o.arena + apu; o.pf = o.arena + apf; o.pones = o.arena + apo;
+  o.start = reinterpret_cast<int*>(o.arena + ast);
+  double *dx = o.arena + adx, *dy = o.arena + ady, *d1 = o.arena + ad1;
+  bool ok = up(dx, px.data(), sizeof(double) * px.size()) &&
+       up(dy, py.data(), sizeof(double) * py.size()) &&
+       up(d1, ones.data(), sizeof(double) * ones.size()) &&
+       up(o.start, start.data(), sizeof(int) * (nreal + 1));
+  if (ok) {
+    hipLaunchKernelGGL(orb_tables, dim3(nreal, n_syms), dim3(1024), 0, c->stream, o.start, d_mb,
+                       d_mp, d_bd, d_bso, d_syms, n_syms, o.S, o.ST);
+    hipLaunchKernelGGL(expand_images, dim3((unsigned)o.rows, (np + 127) / 128), dim3(128), 0,
+                       c->stream, dx, dy, d1, d_mb, d_mp, d_bd, d_bmo, d_bso, d_bm, d_syms, n, np,
+                       n_syms, (long)kProbe * n_syms, o.pu, o.pf, o.pones);
+    if (c->rotate) {   // its rows are the configurations
+      o.U = c->U;
+      o.F = c->F;
+      o.rho = c->rho_img;
+    } else {
+      o.U = o.arena + aU;
+      o.F = o.arena + aF;
+      o.rho = o.arena + arho;
+      const long count = o.Mp * np;
+      hipLaunchKernelGGL(rot_copy_configs, dim3((unsigned)((count + 255) / 256)), dim3(256), 0,
+                         c->stream, X_dev, Y_dev, rho_dev, n, np, (long)c->N, o.Mp, o.U, o.F,
+                         o.rho);
+    }
+  }
+  ok = ok && hipGetLastError() == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess;
+  if (!ok) {
+    set_error("tdscha_ctx_create: tables of the orbit form failed");
+    return -1;
+  }
+  o.usable = true;
+  return 0;
+}
+
+void orbit_free(Ctx* c) {
+  Orbit& o = c->orb;
+  if (o.arena) (void)hipFree(o.arena);
+  if (o.work) (void)hipFree(o.work);
+  if (o.pout) (void)hipHostFree(o.pout);
+  for (OrbPlan& pl : o.plan) orbit_plan_free(pl);
+}
+
+void orbit_plan_free(OrbPlan& p) {
+  if (p.dev) (void)hipFree(p.dev);
+  p.dev = nullptr;
+  p.ok = false;
+}
+
+// K split of the outer product over the configurations: the same whatever the
+// number of pairs, so that a chain's sums do not depend on its batch
+static int orb_ksplit(const Ctx* c) {
+  const int t = f64_tiles(c->n).ntile;
+  int ks = std::min(24, round_up((2048 + 3 * t * t - 1) / (3 * t * t), 8));
+  while (ks > 8 && (long)ks * 128 > c->orb.Mp) ks -= 8;
+  return ks;
+}
+
+// workspaces of the orbit form, at its first use; false = no room (the general form
+// serves this and every later call)
+static bool ensure(Ctx* c) {
+  Orbit& o = c->orb;
+  if (o.work) return true;
+  const size_t np = c->np, nn = np * np;
+  const int ks = orb_ksplit(c), ncol = (c->n + 15) / 16;
+  const size_t count[] = {(size_t)kMaxChains * ncol * o.rows * 4,
+                          kOrbPairs * np, kOrbPairs * nn,
+                          2 * kMaxChains * np, 2 * kMaxChains * nn,
+                          kOrbPairs * (size_t)o.Mp * 4,
+                          kOrbPairs * ks * nn, kOrbPairs * ks * np,
+                          kOrbPairs * nn, kOrbPairs * np};
+  double** dst[] = {&o.ppart, &o.R1, &o.Y1, &o.Rb, &o.Yb, &o.coef, &o.zpart, &o.fpart, &o.z, &o.f};
+  size_t at = 0;
+  for (size_t k : count) at += (k + 31) / 32 * 32;
+  const size_t nout = (size_t)kMaxChains * o.rows * 4;
+  if (hipMalloc((void**)&o.work, sizeof(double) * at) != hipSuccess) o.work = nullptr;
+  if (o.work && hipHostMalloc((void**)&o.pout, sizeof(double) * nout) != hipSuccess) {
+    (void)hipFree(o.work);
+    o.work = o.pout = nullptr;
+  }
+  if (!o.work) {
+    (void)hipGetLastError();
+    o.usable = false;
+    return false;
+  }
+  at = 0;
+  for (size_t k = 0; k < sizeof(count) / sizeof(count[0]); ++k) {
+    *dst[k] = o.work + at;
+    at += (count[k] + 31) / 32 * 32;
+  }
+  return true;
+}
+
+// ----------------------------------------------------------------- the relation
+// Rank and relation of one chain from its row-dots s[rows][4]: rows j of W hold
+// the 4 kProbe functionals, scaled so that what weighs F (s1, s3) and what weighs
+// U (s2, s4) have unit size.  Pivoted Gram-Schmidt; rank 0 = no use.
+static int relation(const double* s, int ns, std::vector<int>& piv, std::vector<double>& C) {
+  constexpr int K = 4 * kProbe;
+  std::vector<double> W((size_t)ns * K);
+  double g[2] = {0.0, 0.0};
+  for (int j = 0; j < ns; ++j)
+    for (int i = 0; i < kProbe; ++i) {
+      const double* q = s + ((size_t)i * ns + j) * 4;
+      double* w = W.data() + (size_t)j * K + 4 * i;
+      w[0] = q[0] / 6.0;
+      w[1] = q[2] / 3.0;
+      w[2] = q[1] / 3.0;
+      w[3] = q[3] / 3.0;
+      g[0] += w[0] * w[0] + w[1] * w[1];
+      g[1] += w[2] * w[2] + w[3] * w[3];
+    }
+  if (!(g[0] > 0.0) || !(g[1] > 0.0) || !std::isfinite(g[0]) || !std::isfinite(g[1])) return 0;
+  for (int j = 0; j < ns; ++j)
+    for (int e = 0; e < K; ++e) W[(size_t)j * K + e] /= std::sqrt(g[(e & 3) >> 1] / ns);
+  std::vector<double> V = W, Q;
+  piv.clear();
+  double top = 0.0;
+  std::vector<double> nrm(ns);
+  for (;;) {
+    int best = 0;
+    for (int j = 0; j < ns; ++j) {
+      nrm[j] = std::sqrt(dot(V.data() + (size_t)j * K, V.data() + (size_t)j * K, K));
+      if (nrm[j] > nrm[best]) best = j;
+    }
+    if (piv.empty()) top = nrm[best];
+    if (nrm[best] <= kOrbTol * top) break;
+    // a direction this weak would enter the relation with large factors
+    if (nrm[best] < 1e-3 * top || (int)piv.size() == kOrbRank) return 0;
+    piv.push_back(best);
+    const size_t r = piv.size() - 1;
+    Q.resize((r + 1) * K);
+    double* q = Q.data() + r * K;
+    for (int e = 0; e < K; ++e) q[e] = V[(size_t)best * K + e] / nrm[best];
+    for (int j = 0; j < ns; ++j)   // twice: the second pass takes what rounding left
+      for (int pass = 0; pass < 2; ++pass) {
+        double* v = V.data() + (size_t)j * K;
+        const double t = dot(v, q, K);
+        for (int e = 0; e < K; ++e) v[e] -= t * q[e];
+      }
+  }
+  // W_j = sum_k C_jk W_piv[k]: with W Q^T = A, C A_piv = A (A_piv lower triangular)
+  const int r = (int)piv.size();
+  std::vector<double> A((size_t)ns * r);
+  for (int j = 0; j < ns; ++j)
+    for (int k = 0; k < r; ++k) {
+      A[(size_t)j * r + k] = dot(W.data() + (size_t)j * K, Q.data() + (size_t)k * K, K);
+    }
+  C.assign((size_t)ns * kOrbRank, 0.0);
+  for (int j = 0; j < ns; ++j)
+    for (int k = r - 1; k >= 0; --k) {
+      double t = A[(size_t)j * r + k];
+      for (int l = k + 1; l < r; ++l) t -= C[(size_t)j * kOrbRank + l] * A[(size_t)piv[l] * r + k];
+      C[(size_t)j * kOrbRank + k] = t / A[(size_t)piv[k] * r + k];
+    }
+  return r;
+}
+
+// Whether to look for a plan: the general form is long enough, and the R vectors
+// (host, `ld` apart) do not rule it out: more than kOrbRank independent rotations
+// of one among the first symmetries.  This keeps the probe and the wait for it
+// away from perturbations of no symmetry (10 us of host work under the upload, for
+// 50 us).
+bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld) {
+  const Orbit& o = c->orb;
+  if (!o.usable || c->row_lo != 0 || c->row_hi != c->M ||
+      !(estimate_us(nc * pass_flop(c, (double)c->N * o.nsym), prec) > kOrbWorthUs))
+    return false;
+  const int n = c->n;
+  std::vector<double> Q((size_t)(kOrbRank + 1) * n);
+  for (int ch = 0; R && ch < nc; ++ch) {
+    int r = 0;
+    for (int j = 0; j < std::min(o.nsym, kOrbRank + 2) && r <= kOrbRank; ++j) {
+      double* v = Q.data() + (size_t)r * n;
+      apply_s(c, o.syms, j, true, R + ch * ld, v);
+      const double whole = dot(v, v, n);
+      for (int k = 0; k < r; ++k) {
+        const double* q = Q.data() + (size_t)k * n;
+        const double t = dot(v, q, n);
+        for (int m = 0; m < n; ++m) v[m] -= t * q[m];
+      }
+      const double rest = dot(v, v, n);
+      if (!(rest > 1e-12 * whole)) continue;   // (NaN: left to the probe)
+      const double inv = 1.0 / std::sqrt(rest);
+      for (int m = 0; m < n; ++m) v[m] *= inv;
+      ++r;
+    }
+    if (r > kOrbRank) return false;
+  }
+  return true;
+}
+
+// Plan of nc chains whose padded inputs are in c->R1, c->Y1 (waits for the
+// stream): p.ok false = use the general form.
+int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p) {
+  Orbit& o = c->orb;
+  p.ok = false;
+  const bool first = !o.work;
+  if (!ensure(c)) return 0;
+  if (first) {   // the padding of the rotated inputs is never written
+    TDS_CHECK_HIP(hipMemsetAsync(o.R1, 0, sizeof(double) * kOrbPairs * c->np, s));
+    TDS_CHECK_HIP(hipMemsetAsync(o.Y1, 0, sizeof(double) * kOrbPairs * (size_t)c->np * c->np, s));
+    TDS_CHECK_HIP(hipStreamSynchronize(s));
+  }
+  const int ncol = (c->n + 15) / 16, rows4 = o.rows * 4, ns = o.nsym;
+  std::vector<int> piv;
+  std::vector<double> C, Call;
+  hipLaunchKernelGGL(orb_probe, dim3(o.rows / 16, ncol, nc), dim3(256), 0, s, o.pu, o.pf, c->Y1,
+                     c->R1, c->fy, c->fpsi, c->np, round_up(c->n, 16), o.rows, o.ppart);
+  hipLaunchKernelGGL(orb_probe_sum, dim3((rows4 + 255) / 256, nc), dim3(256), 0, s, o.ppart, ncol,
+                     rows4, o.pout);
+  TDS_CHECK_HIP(hipGetLastError());
+  TDS_CHECK_HIP(hipStreamSynchronize(s));
+  std::vector<int2> pairs, clean;
+  std::vector<int4> mats, cmats;
+  for (int ch = 0; ch < nc; ++ch) {
+    const int r = relation(o.pout + (size_t)ch * rows4, ns, piv, C);
+    if (r == 0 || (int)pairs.size() + r > kOrbPairs) return 0;
+    mats.push_back(int4{(int)pairs.size(), r, ch, 0});
+    for (int k = 0; k < r; ++k) pairs.push_back(int2{ch, piv[k]});
+    for (int sec = 0; sec < 2; ++sec) {
+      // pairs of the clean-up, in rounds of whole chains (orbit_clean)
+      cmats.push_back(int4{0, r, ch, 0});
+      for (int k = 0; k < r; ++k) clean.push_back(int2{2 * ch + sec, piv[k]});
+    }
+    Call.insert(Call.end(), C.begin(), C.end());
+  }
+  const double full = estimate_us(nc * pass_flop(c, (double)c->N * ns), prec);
+  const double orb = estimate_us(pairs.size() * pass_flop(c, c->N), PREC_FP64) + 150.0;
+  if (orb > 0.8 * full) return 0;
+  p.nc = nc;
+  p.npairs = (int)pairs.size();
+  // rounds of the clean-up: whole chains, at most kOrbPairs pairs each
+  p.rounds.clear();
+  for (int ch = 0, at = 0; ch < nc;) {
+    int used = 0, c0 = ch;
+    while (ch < nc && used + 2 * mats[ch].y <= kOrbPairs) {
+      for (int sec = 0; sec < 2; ++sec) {
+        cmats[2 * ch + sec].x = used;
+        used += mats[ch].y;
+      }
+      ++ch;
+    }
+    p.rounds.push_back({c0, ch - c0, at, used});
+    at += used;
+  }
+  const size_t b0 = sizeof(int4) * (mats.size() + cmats.size()),
+               b1 = sizeof(int2) * (pairs.size() + clean.size()), b2 = sizeof(double) * Call.size();
+  const size_t need = b0 + b1 + b2;
+  if (p.cap < need) {
+    orbit_plan_free(p);
+    p.cap = 0;
+    const size_t most = sizeof(int4) * 3 * kMaxChains + sizeof(int2) * 3 * kOrbPairs +
+                        sizeof(double) * kMaxChains * (size_t)ns * kOrbRank;
+    TDS_CHECK_HIP(hipMalloc(&p.dev, std::max(most, need)));
+    p.cap = std::max(most, need);
+  }
+  p.host.resize(need);
+  char* h = p.host.data();
+  std::copy(mats.begin(), mats.end(), reinterpret_cast<int4*>(h));
+  std::copy(cmats.begin(), cmats.end(), reinterpret_cast<int4*>(h) + mats.size());
+  std::copy(Call.begin(), Call.end(), reinterpret_cast<double*>(h + b0));
+  std::copy(pairs.begin(), pairs.end(), reinterpret_cast<int2*>(h + b0 + b2));
+  std::copy(clean.begin(), clean.end(), reinterpret_cast<int2*>(h + b0 + b2) + pairs.size());
+  TDS_CHECK_HIP(hipMemcpyAsync(p.dev, h, need, hipMemcpyHostToDevice, s));
+  char* d = static_cast<char*>(p.dev);
+  p.mats = reinterpret_cast<int4*>(d);
+  p.cmats = p.mats + mats.size();
+  p.C = reinterpret_cast<double*>(d + b0);
+  p.pairs = reinterpret_cast<int2*>(d + b0 + b2);
+  p.clean = p.pairs + pairs.size();
+  p.ok = true;
+  return 0;
+}
+
+static OrbPanels panels(const Ctx* c) {
+  const Orbit& o = c->orb;
+  return OrbPanels{o.start, o.npanel, o.nsym, o.S, o.ST};
+}
+
+// the perturbed averages of the plan's chains (inputs in c->R1, c->Y1)
+int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
+                 hipStream_t s) {
+  Orbit& o = c->orb;
+  const int n = c->n, np = c->np, P = p.npairs, ks = orb_ksplit(c);
+  const OrbPanels pn = panels(c);
+  hipLaunchKernelGGL(orb_in, dim3(o.npanel * o.npanel, P), dim3(256), 0, s, pn, p.pairs, c->Y1,
+                     c->R1, np, (const int*)nullptr, 0, o.Y1, o.R1);
+  const F64Rows rows{o.U, o.F, o.rho, o.Mp};
+  launch_weights_f64(rows, n, np, P, o.Y1, o.R1, c->fy, c->fpsi, apply_d4, 0,
+                     (c->N + 63) / 64, 0, c->N, o.coef, s);
+  const long ke = round_up_l(c->N, 8);
+  launch_outer_f64(rows, n, np, P, o.coef, c->fy, ks, 0, ke, round_up_l((ke + ks - 1) / ks, 8), 0,
+                   o.zpart, o.fpart, s);
+  launch_reduce_f64(n, np, P, ks, o.zpart, o.fpart, o.z, o.f, 1.0 / c->n_eff, s);
+  hipLaunchKernelGGL(orb_out<true>, dim3(o.npanel * (o.npanel + 1) / 2, p.nc), dim3(512), 0, s, pn,
+                     p.mats, p.C, o.z, o.f, c->fy, n, np, 1.0 / o.nsym,
+                     1.0 / (c->n_eff * o.nsym), (const int*)nullptr, 0, (const int*)nullptr, f_dev,
+                     d2v_dev);
+  TDS_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+
+// project the packed vectors x of the plan's chains on their sector, on every
+// kOrbClean-th step (kk: the chains' common step counter on the device)
+int orbit_clean(Ctx* c, const OrbPlan& p, double* x, const int* kk, const int* active,
+                hipStream_t s) {
+  Orbit& o = c->orb;
+  const int n = c->n, np = c->np;
+  const long nn = (long)np * np;
+  const OrbPanels pn = panels(c);
+  hipLaunchKernelGGL(orb_unpack, dim3((unsigned)((nn + 255) / 256), 2 * p.nc), dim3(256), 0, s, x,
+                     n, np, kk, kOrbClean, o.Yb, o.Rb);
+  const long len = n + (long)n * (n + 1);
+  for (const OrbPlan::Round& r : p.rounds) {
+    hipLaunchKernelGGL(orb_in, dim3(o.npanel * o.npanel, r.count), dim3(256), 0, s, pn,
+                       p.clean + r.first, o.Yb, o.Rb, np, kk, kOrbClean, o.Y1, o.R1);
+    hipLaunchKernelGGL(orb_out<false>, dim3(o.npanel * (o.npanel + 1) / 2, 2 * r.chains),
+                       dim3(512), 0, s, pn, p.cmats + 2 * r.chain0, p.C, o.Y1, o.R1, c->fy, n, np,
+                       1.0 / o.nsym, 1.0 / o.nsym, kk, kOrbClean, active + r.chain0,
+                       (double*)nullptr, x + r.chain0 * len);
+  }
+  TDS_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+
+}  // namespace tdscha
