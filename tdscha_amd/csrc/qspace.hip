@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -41,7 +42,7 @@ namespace tdscha {
 constexpr int kQMaxChains = 256;
 constexpr int kQMaxQ = 512;
 constexpr int kQWeightsChains = 2;   // chains per q_weights workgroup
-constexpr int kD2vChains = 16;       // chains per slab q_d2v workgroup
+constexpr int kD2vChains = 15;       // chains per slab q_d2v workgroup
 constexpr int kSlabBytes = 65536;    // LDS of one slab q_d2v workgroup (two buffers)
 constexpr int kD2vThreads = 256;     // threads (items) per slab q_d2v workgroup
 
@@ -426,37 +427,48 @@ __global__ void q_slab_build(const double2* __restrict__ X, const double2* __res
 // slab k.  The two buffers are distinct arrays and each half of the unrolled
 // loop names its own, so that the compiler sees that the reads of one do not
 // depend on the copies into the other.  Each thread accumulates the 6x6
-// block of one (chain, pair) item, in configuration order.  The item blocks
-// of one chunk run on one XCD and share the chunk through its L2.
+// block of one (chain, pair) item, in configuration order; on small grids (long
+// slabs, few items) ns threads take an item, every ns-th configuration each, and
+// their blocks are added in LDS at the end (36 items at 8 chains on 2x2x2: 124 us with
+// one thread each, 61 us).  ns follows from the grid alone, so that a chain's
+// sums do not depend on its batch.  The item blocks
+// of one chunk run on one XCD and share the chunk through its L2.  T is known at
+// compile time so that the LDS offsets are immediates (64 chains on 4x4x4: 934 us
+// with a run-time T, 859 us).
 constexpr int kSlabUnits = kSlabBytes / 2 / (int)sizeof(double2);
+constexpr int d2v_slices(int T) { return T > 2 ? T / 2 : 1; }
 
-template <int NB>
+template <int NB, int T>
 __global__ void __launch_bounds__(kD2vThreads) __attribute__((amdgpu_waves_per_eu(2))) q_d2v_slab(
     const double2* __restrict__ S, int N, int nq, const int* __restrict__ active,
     const int4* __restrict__ items, const int* __restrict__ blk_start, int nib, int MP,
-    const double2* __restrict__ wc, const double2* __restrict__ wd, int lgT, int chunk, int nch,
+    const double2* __restrict__ wc, const double2* __restrict__ wd, int chunk, int nch,
     double2* __restrict__ dpart) {
   __shared__ double2 bufA[kSlabUnits], bufB[kSlabUnits];
   int ch, ib;
   if (!xcd_tile(blockIdx.x, nib, nch, ch, ib)) return;
-  const int T = 1 << lgT, SR = NB * T + 1, U = 2 * nq * SR;
+  constexpr int SR = NB * T + 1;
+  const int U = 2 * nq * SR;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nwave = blockDim.x >> 6;
   const int i0 = blk_start[ib], i1 = blk_start[ib + 1];
   const int c_lo = items[i0].x, ncb = items[i1 - 1].x - c_lo + 1;
   bool any = false;
   for (int k = 0; k < ncb; ++k) any |= active[c_lo + k] != 0;
   if (!any) return;
+  const int ni = i1 - i0;
+  constexpr int ns = d2v_slices(T);
+  const int sl = t / ni, at = t - sl * ni;
   int4 it = make_int4(0, 0, 0, 0);
-  bool mine = i0 + t < i1;
+  bool mine = sl < ns;
   if (mine) {
-    it = items[i0 + t];
+    it = items[i0 + at];
     mine = active[it.x] != 0;
   }
-  const int cw = (it.x - c_lo) << (lgT + 1);
-  const int nW = ncb << (lgT + 1);
+  const int cw = (it.x - c_lo) * 2 * T;
+  const int nW = ncb * 2 * T;
   const int lo = ch * chunk, hi = min(N, lo + chunk);
   auto issue = [&](int s0, double2* dst) {
-    const long sl = s0 >> lgT;
+    const long sl = s0 / T;
     const double2* src = S + sl * U;
     for (int k = wave; k * 64 < U; k += nwave)
       if (k * 64 + lane < U) dma16(src + k * 64 + lane, dst + k * 64);
@@ -465,7 +477,7 @@ __global__ void __launch_bounds__(kD2vThreads) __attribute__((amdgpu_waves_per_e
     for (int k = wave; k * 64 < nW; k += nwave) {
       const int e = k * 64 + lane;
       if (e < nW) {
-        const int j = e & (T - 1), h = (e >> lgT) & 1, c = c_lo + (e >> (lgT + 1));
+        const int j = e % T, h = (e / T) & 1, c = c_lo + e / (2 * T);
         dma16((h ? wd : wc) + (long)c * N + min(s0 + j, N - 1), dst + U + k * 64);
       }
     }
@@ -477,7 +489,7 @@ __global__ void __launch_bounds__(kD2vThreads) __attribute__((amdgpu_waves_per_e
     for (int b = 0; b < NB; ++b) acc[a][b] = make_double2(0.0, 0.0);
   auto accumulate = [&](const double2* img) {
     if (!mine) return;
-    for (int j = 0; j < T; ++j) {
+    for (int j = sl; j < T; j += ns) {
       const double2 wci = img[U + cw + j], wdi = img[U + cw + T + j];
       const double2* x1 = img + it.z * SR + j;
       const double2* y1 = img + (nq + it.z) * SR + j;
@@ -512,13 +524,63 @@ __global__ void __launch_bounds__(kD2vThreads) __attribute__((amdgpu_waves_per_e
     if (s0 + 2 * T < hi) issue(s0 + 2 * T, bufA);
     accumulate(bufB);
   }
-  if (mine) {
-    double2* o = dpart + (((long)it.x * MP + it.y) * nch + ch) * NB * NB;
+  if constexpr (ns == 1) {
+    if (mine) {
+      double2* o = dpart + (((long)it.x * MP + it.y) * nch + ch) * NB * NB;
 #pragma unroll
-    for (int a = 0; a < NB; ++a)
+      for (int a = 0; a < NB; ++a)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) o[a * NB + b] = make_double2(-acc[a][b].x, -acc[a][b].y);
+        for (int b = 0; b < NB; ++b) o[a * NB + b] = make_double2(-acc[a][b].x, -acc[a][b].y);
+    }
+    return;
   }
+  // one row of the blocks at a time: [slice][item][b] (ns ni <= 256 threads)
+#pragma unroll
+  for (int a = 0; a < NB; ++a) {
+    lds_barrier();
+    if (sl < ns)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) bufA[t * NB + b] = acc[a][b];
+    lds_barrier();
+    for (int e = t; e < ni * NB; e += kD2vThreads) {
+      const int4 w = items[i0 + e / NB];
+      if (!active[w.x]) continue;
+      double2 v = make_double2(0.0, 0.0);
+      for (int k = 0; k < ns; ++k) v = cadd(v, bufA[k * ni * NB + e]);
+      dpart[((((long)w.x * MP + w.y) * nch + ch) * NB + a) * NB + e % NB] =
+          make_double2(-v.x, -v.y);
+    }
+  }
+}
+
+// Sum over k of p[k W + t], k < n, for t < W of a 256-thread workgroup: the
+// entries in 256 / W slices, four loads in flight each, the slices added in LDS in
+// a fixed order.
+template <int W>
+__device__ __forceinline__ double2 slice_sum(const double2* __restrict__ p, int n) {
+  constexpr int S = 256 / W, step = S * W;
+  __shared__ double2 red[step];
+  const int t = threadIdx.x;
+  const long end = (long)n * W;
+  double2 v = make_double2(0.0, 0.0);
+  if (t < step) {
+    long e = t;
+    for (; e + 3 * step < end; e += 4 * step) {
+      double2 x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = p[e + j * step];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v = cadd(v, x[j]);
+    }
+    for (; e < end; e += step) v = cadd(v, p[e]);
+    red[t] = v;
+  }
+  __syncthreads();
+  v = make_double2(0.0, 0.0);
+  if (t < W)
+#pragma unroll 4
+    for (int k = 0; k < S; ++k) v = cadd(v, red[k * W + t]);
+  return v;
 }
 
 // Static Liouvillian of the free-energy Hessian (QSpaceHessian,
@@ -565,7 +627,7 @@ __device__ __forceinline__ double static_lambda(double w1, double w2, double n1,
 // R <- w^2 R - f_pert, W <- W / Lambda + d2v (QSH:605-692).  Block 0: R
 // sector; block 1 + p: the W block of pair p.
 template <int NB>
-__global__ void q_finish_static(const double2* __restrict__ psi, int ld, double2* __restrict__ out,
+__global__ void __launch_bounds__(256) q_finish_static(const double2* __restrict__ psi, int ld, double2* __restrict__ out,
                                 const int* __restrict__ active, const int* __restrict__ iqp,
                                 const int* __restrict__ npairs, const int* __restrict__ pq1,
                                 const int* __restrict__ pq2, const int* __restrict__ offa, int MP,
@@ -579,14 +641,11 @@ __global__ void q_finish_static(const double2* __restrict__ psi, int ld, double2
   const double2* ps = psi + (long)c * ld;
   double2* po = out + (long)c * ld;
   if (blk == 0) {
+    const double2 f = slice_sum<NB>(fpart + (long)c * ntile * NB, do_anh ? ntile : 0);
     if (t >= NB) return;
     const int qp = iqp[c];
     double2 o = make_double2(0.0, 0.0);
-    if (do_anh) {
-      double2 f = make_double2(0.0, 0.0);
-      for (int k = 0; k < ntile; ++k) f = cadd(f, fpart[((long)c * ntile + k) * NB + t]);
-      o = csc(f, -inv_norm);
-    }
+    if (do_anh) o = csc(f, -inv_norm);
     if (do_harm) {
       const double w = wq[qp * NB + t];
       o = cadd(o, csc(ps[t], w * w));
@@ -595,18 +654,16 @@ __global__ void q_finish_static(const double2* __restrict__ psi, int ld, double2
     return;
   }
   const int p = blk - 1;
-  if (p >= npairs[c] || t >= NB * NB) return;
+  if (p >= npairs[c]) return;
+  double2 d = slice_sum<NB * NB>(dpart + ((long)c * MP + p) * nch * NB * NB, do_anh ? nch : 0);
+  if (t >= NB * NB) return;
   const int i = t / NB, j = t % NB;
   const int q1 = pq1[c * MP + p], q2 = pq2[c * MP + p];
   const int full = q1 < q2;
   if (!full && i > j) return;
   const int e = offa[c * MP + p] + (full ? i * NB + j : tri_index(i, j, NB));
   double2 o = make_double2(0.0, 0.0);
-  if (do_anh) {
-    const double2* dp = dpart + ((long)c * MP + p) * nch * NB * NB + t;
-    for (int k = 0; k < nch; ++k) o = cadd(o, dp[(long)k * NB * NB]);
-    o = csc(o, inv_norm);
-  }
+  if (do_anh) o = csc(d, inv_norm);
   if (do_harm) {
     const double lam = static_lambda(wq[q1 * NB + i], wq[q2 * NB + j], nbose[q1 * NB + i],
                                      nbose[q2 * NB + j], valid[q1 * NB + i], valid[q2 * NB + j],
@@ -616,9 +673,11 @@ __global__ void q_finish_static(const double2* __restrict__ psi, int ld, double2
   po[e] = o;
 }
 
-// block 0: R sector; block 1 + p: pair p
+// block 0: R sector; block 1 + p: pair p.  A chain of dependent loads per entry when
+// one thread adds the partials (125 us at 8 chains on 2x2x2 with 375 of them); 8 us
+// in slices.
 template <int NB>
-__global__ void q_finish(const double2* __restrict__ psi, int ld, double2* __restrict__ out,
+__global__ void __launch_bounds__(256) q_finish(const double2* __restrict__ psi, int ld, double2* __restrict__ out,
                          const int* __restrict__ active, const int* __restrict__ iqp,
                          const int* __restrict__ npairs, const int* __restrict__ pq1,
                          const int* __restrict__ pq2, const int* __restrict__ offa,
@@ -632,10 +691,9 @@ __global__ void q_finish(const double2* __restrict__ psi, int ld, double2* __res
   const double2* ps = psi + (long)c * ld;
   double2* po = out + (long)c * ld;
   if (blk == 0) {
+    const double2 f = slice_sum<NB>(fpart + (long)c * ntile * NB, do_anh ? ntile : 0);
     if (t >= NB) return;
     const int qp = iqp[c];
-    double2 f = make_double2(0.0, 0.0);
-    for (int k = 0; k < ntile; ++k) f = cadd(f, fpart[((long)c * ntile + k) * NB + t]);
     double2 o = make_double2(0.0, 0.0);
     if (do_anh) o = csc(f, inv_norm);
     if (do_harm && valid[qp * NB + t]) {
@@ -646,7 +704,9 @@ __global__ void q_finish(const double2* __restrict__ psi, int ld, double2* __res
     return;
   }
   const int p = blk - 1;
-  if (p >= npairs[c] || t >= NB * NB) return;
+  if (p >= npairs[c]) return;
+  double2 d = slice_sum<NB * NB>(dpart + ((long)c * MP + p) * nch * NB * NB, do_anh ? nch : 0);
+  if (t >= NB * NB) return;
   const int i = t / NB, j = t % NB;
   const int q1 = pq1[c * MP + p], q2 = pq2[c * MP + p];
   const int full = q1 < q2;
@@ -658,9 +718,6 @@ __global__ void q_finish(const double2* __restrict__ psi, int ld, double2* __res
                                  valid[q1 * NB + i], valid[q2 * NB + j]);
   double2 oa = make_double2(0.0, 0.0), ob = make_double2(0.0, 0.0);
   if (do_anh) {
-    double2 d = make_double2(0.0, 0.0);
-    const double2* dp = dpart + ((long)c * MP + p) * nch * NB * NB + t;
-    for (int k = 0; k < nch; ++k) d = cadd(d, dp[(long)k * NB * NB]);
     d = csc(d, inv_norm);
     oa = csc(d, sqrt(-0.5 * f.chim));
     ob = csc(d, -sqrt(0.5 * f.chip));
@@ -734,6 +791,17 @@ static size_t slab_units(int nq, int nb, int T) {
   return 2 * (size_t)nq * (nb * T + 1) + 2 * (size_t)kD2vChains * T;
 }
 
+template <typename Fn>
+static void with_slab(int T, Fn fn) {
+  switch (T) {
+    case 1: fn(std::integral_constant<int, 1>{}); break;
+    case 2: fn(std::integral_constant<int, 2>{}); break;
+    case 4: fn(std::integral_constant<int, 4>{}); break;
+    case 8: fn(std::integral_constant<int, 8>{}); break;
+    default: fn(std::integral_constant<int, 16>{}); break;
+  }
+}
+
 static int log2_pow2(int T) {
   int lg = 0;
   while ((1 << lg) < T) ++lg;
@@ -778,11 +846,11 @@ static int build_slabs(QCtx* q) {
 // d2v chunk (configurations per workgroup) that gives `rounds` rounds of
 // slab workgroups on the device (n_item_blocks workgroups per chunk, two
 // resident workgroups per CU: two buffers of half the CU's LDS and 256
-// threads at up to 256 VGPRs), at least 8 slabs.
+// threads at up to 256 VGPRs), at least 4 slabs.
 static int slab_chunk(const QCtx* q, int n_item_blocks, int rounds) {
   const long slots = 2L * q->n_cu * rounds;
   const long nch = std::max(1L, slots / std::max(1, n_item_blocks));
-  const long chunk = std::max<long>(8L * q->slabT, (q->N + nch - 1) / nch);
+  const long chunk = std::max<long>(4L * q->slabT, (q->N + nch - 1) / nch);
   return (int)((chunk + q->slabT - 1) / q->slabT * q->slabT);
 }
 
@@ -859,7 +927,7 @@ static int build_batch(QCtx* q, int C, const int* iq_pert, const int* pair_map, 
         }
       h_bs.push_back((int)h_items.size());
     };
-    partition(kD2vThreads);
+    partition(kD2vThreads / d2v_slices(b.slabT));
     const int nfull = (int)h_bs.size() - 1;      // then the same count of even workgroups
     partition(((int)h_items.size() + nfull - 1) / nfull);
     b.n_items = (int)h_items.size();
@@ -946,9 +1014,11 @@ static void launch_L_nb(QCtx* q, QBatch& b, const double2* psi, double2* out, in
                        C, ngroups, b.ntile, ignore_v4 ? 0 : 1, b.wc, b.wd, b.fpart);
     if (b.slabT) {
       const int nblk2 = (b.nch + 7) / 8 * 8 * b.nib;
-      hipLaunchKernelGGL(q_d2v_slab<NB>, dim3(nblk2), dim3(kD2vThreads), 0, s, q->S, q->N, nq,
-                         b.active, b.items, b.blk_start, b.nib, MP, b.wc, b.wd,
-                         log2_pow2(b.slabT), b.chunk, b.nch, b.dpart);
+      with_slab(b.slabT, [&](auto T) {
+        hipLaunchKernelGGL((q_d2v_slab<NB, decltype(T)::value>), dim3(nblk2), dim3(kD2vThreads), 0,
+                           s, q->S, q->N, nq, b.active, b.items, b.blk_start, b.nib, MP, b.wc,
+                           b.wd, b.chunk, b.nch, b.dpart);
+      });
     } else {
       hipLaunchKernelGGL(q_d2v<NB>, dim3(b.maxp, C, b.nch), dim3(256), 0, s, q->X, q->Y, q->N,
                          q->fY, b.active, b.npairs, b.pq1, b.pq2, MP, b.wc, b.wd, b.chunk, b.nch,
@@ -956,12 +1026,12 @@ static void launch_L_nb(QCtx* q, QBatch& b, const double2* psi, double2* out, in
     }
   }
   if (static_op)
-    hipLaunchKernelGGL(q_finish_static<NB>, dim3(MP + 1, C), dim3(64), 0, s, psi, b.ld, out,
+    hipLaunchKernelGGL(q_finish_static<NB>, dim3(MP + 1, C), dim3(256), 0, s, psi, b.ld, out,
                        b.active, b.iqp, b.npairs, b.pq1, b.pq2, b.offa, MP, q->wq, q->nbose,
                        q->valid, q->T > 1e-12 ? RY_TO_K / q->T : 0.0, b.fpart, b.ntile, b.dpart,
                        b.nch, 1.0 / q->neff, ignore_harmonic ? 0 : 1, do_anh);
   else
-    hipLaunchKernelGGL(q_finish<NB>, dim3(MP + 1, C), dim3(64), 0, s, psi, b.ld, out, b.active,
+    hipLaunchKernelGGL(q_finish<NB>, dim3(MP + 1, C), dim3(256), 0, s, psi, b.ld, out, b.active,
                        b.iqp, b.npairs, b.pq1, b.pq2, b.offa, b.offb, MP, q->wq, q->nbose,
                        q->valid, b.fpart, b.ntile, b.dpart, b.nch, 1.0 / q->neff,
                        ignore_harmonic ? 0 : 1, do_anh);
