@@ -164,7 +164,7 @@ struct Ctx {
   double* R1 = nullptr;     // [kMaxChains, np]
   double* Y1 = nullptr;     // [kMaxChains, np, np]
   double* coef = nullptr;   // [kMaxChains, Mp, 4] (c1, c2, alpha, beta)
-  double* zpart = nullptr;  // [kMaxChains, ksplit, np, np]
+  double* zpart = nullptr;  // [kMaxChains, ksplit] partial tiles of the outer GEMM
   double* fpart = nullptr;  // [kMaxChains, ksplit, np]
   double* f_out = nullptr;  // [kMaxChains, np]
   double* d2v_out = nullptr;// [kMaxChains, np, np]

@@ -62,15 +62,29 @@ __global__ void symmetrize_out(const double* __restrict__ zsum_all, const double
 
 static double bose(double w, double T) { return T > 0 ? 1.0 / (std::exp(w * RY_TO_K / T) - 1.0) : 0.0; }
 
-static int choose_ksplit(int ntile, long Mp) {
-  // aim at ~6 workgroups per CU for the outer GEMM, multiple of 8 (one per XCD)
-  const int target = 1536;
-  int ks = (target + ntile * ntile - 1) / (ntile * ntile);
-  ks = round_up(ks, 8);
-  ks = std::min(ks, 128);
-  // at least 256 images per split
-  while (ks > 8 && (long)ks * 256 > Mp) ks -= 8;
-  return std::max(ks, 8);
+// doubles of the outer GEMM's partial tiles, per chain
+static size_t zpart_size(int n, int ksplit) {
+  const F64Tiles t = f64_tiles(n);
+  const size_t zl = 16 * (size_t)t.ntile * t.cb;
+  return zl * zl * ksplit;
+}
+
+// K split of the FP64 outer GEMM, a multiple of 8 (one range per XCD): with several
+// tiles up to 128 ranges of at least 256 images, about 6 work-groups per CU.  A
+// single tile (at most 128 modes) has one work-group per range and is bound by the
+// latency of a range's chunks: up to 512 ranges of at least 32 images, a power of two
+// so that the slices of their sum are even (45 modes, 2000 images: 8 ranges 20.8 us,
+// 64 ranges 5.9; 96000 images: 128 ranges 57, 512 ranges 24).
+static int choose_ksplit(int n, long Mp) {
+  const int t = f64_tiles(n).ntile, t2 = t * t;
+  if (t == 1) {
+    int ks = 8;
+    while (ks < 512 && ks * 64L <= Mp) ks *= 2;
+    return ks;
+  }
+  int ks = std::min(128, round_up((1536 + t2 - 1) / t2, 8));
+  while (ks > 8 && ks * 256L > Mp) ks -= 8;
+  return ks;
 }
 
 // run the perturbed averages for nc chains whose padded inputs are in c->R1/c->Y1;
@@ -174,7 +188,7 @@ int tdscha_ctx_create(tdscha_ctx** out, int n_modes, int n_configs, const double
   TDS_REQUIRE(ne != 0.0, 2, "tdscha_ctx_create: sum of weights is zero");
   const int np = c->np;
   const long Mp = c->Mp;
-  c->ksplit = choose_ksplit(np / kTile, Mp);
+  c->ksplit = choose_ksplit(n_modes, Mp);
 
   auto fail = [&](void) { tdscha_ctx_destroy(reinterpret_cast<tdscha_ctx*>(c)); return -1; };
 #define ALLOC(ptr, bytes)                                                 \
@@ -195,7 +209,7 @@ int tdscha_ctx_create(tdscha_ctx** out, int n_modes, int n_configs, const double
   ALLOC(c->R1, sizeof(double) * kMaxChains * np);
   ALLOC(c->Y1, sizeof(double) * kMaxChains * (long)np * np);
   ALLOC(c->coef, sizeof(double) * kMaxChains * Mp * 4);
-  ALLOC(c->zpart, sizeof(double) * kMaxChains * (long)c->ksplit * np * np);
+  ALLOC(c->zpart, sizeof(double) * kMaxChains * zpart_size(n_modes, c->ksplit));
   ALLOC(c->fpart, sizeof(double) * kMaxChains * (long)c->ksplit * np);
   ALLOC(c->f_out, sizeof(double) * kMaxChains * np);
   ALLOC(c->d2v_out, sizeof(double) * kMaxChains * (long)np * np);
@@ -527,7 +541,7 @@ int tdscha_set_ksplit(tdscha_ctx* ctx, int ksplit) {
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   TDS_CHECK_HIP(hipStreamSynchronize(c->stream));
   double *zp = nullptr, *fp = nullptr;
-  TDS_CHECK_HIP(hipMalloc((void**)&zp, sizeof(double) * kMaxChains * (size_t)ksplit * c->np * c->np));
+  TDS_CHECK_HIP(hipMalloc((void**)&zp, sizeof(double) * kMaxChains * zpart_size(c->n, ksplit)));
   TDS_CHECK_HIP(hipMalloc((void**)&fp, sizeof(double) * kMaxChains * (size_t)ksplit * c->np));
   (void)hipFree(c->zpart);
   (void)hipFree(c->fpart);
@@ -566,7 +580,7 @@ int tdscha_autotune(tdscha_ctx* ctx, int n_chains, int precision, int reps, int*
       const int ks = cand[i];
       int rc;
       if (precision == PREC_FP64) {
-        if ((long)ks * 256 > c->Mp) continue;
+        if ((long)ks * 32 > c->Mp) continue;
         rc = tdscha_set_ksplit(ctx, ks);
       } else {
         if ((long)ks * 4 > c->Mp / 16) continue;

@@ -354,7 +354,8 @@ __global__ __launch_bounds__(256, CB > 5 ? 2 : 3) void outer_f64(
   const int ks = xcd + 8 * (rest / t2);
   const int tm = tile / ntile, tn = tile % ntile;
   const double* coef = coef_all + (long)chain * Mp * 4;
-  double* zpart = zpart_all + ((long)chain * ksplit + ks) * np * np;
+  const int zl = ntile * T;   // partials hold the tiles only
+  double* zpart = zpart_all + ((long)chain * ksplit + ks) * zl * zl;
   double* fpart = fpart_all + ((long)chain * ksplit + ks) * np;
   const int mu0 = tm * T, nu0 = tn * T;
 
@@ -493,7 +494,7 @@ __global__ __launch_bounds__(256, CB > 5 ? 2 : 3) void outer_f64(
 #pragma unroll
   for (int i = 0; i < CB; ++i) {
     const int mu = mu0 + (CB % 2 ? 16 * i + drow : 16 * (i & ~1) + 2 * drow + (i & 1));
-    double* z = zpart + (long)mu * np + nu0 + 4 * CB * wave + lq;
+    double* z = zpart + (long)mu * zl + nu0 + 4 * CB * wave + lq;
 #pragma unroll
     for (int g = 0; g < NF; ++g)
 #pragma unroll
@@ -523,21 +524,21 @@ __global__ __launch_bounds__(256, CB > 5 ? 2 : 3) void outer_f64(
 }
 
 // sum the K-split partials in a fixed order, rows and columns below n: 64
-// elements per work-group, the partials in 4 slices of 8 loads in flight each,
+// elements per work-group, the partials in 4 or 16 slices of 8 loads in flight each,
 // combined in LDS; grid (ceil(n / 64), n + 1, chains), the last row the f sums
-__global__ __launch_bounds__(256) void reduce_ksplit(const double* __restrict__ zpart_all,
-                                                     const double* __restrict__ fpart_all, int n,
-                                                     int np, int ksplit,
-                                                     double* __restrict__ zsum_all,
-                                                     double* __restrict__ f_all, double norm) {
+template <int SL>
+__global__ __launch_bounds__(64 * SL) void reduce_ksplit(const double* __restrict__ zpart_all,
+                                                         const double* __restrict__ fpart_all,
+                                                         int n, int np, int zl, int ksplit,
+                                                         double* __restrict__ zsum_all,
+                                                         double* __restrict__ f_all, double norm) {
   const int chain = blockIdx.z, row = blockIdx.y;
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;
-  const long nn = (long)np * np;
+  const int t = threadIdx.x & 63, c = blockIdx.x * 64 + t, sl = threadIdx.x >> 6;
   const bool isf = row == n;
-  const long stride = isf ? np : nn;
+  const long stride = isf ? np : (long)zl * zl;
   const double* p = isf ? fpart_all + (long)chain * ksplit * np + c
-                        : zpart_all + (long)chain * ksplit * nn + (long)row * np + c;
-  const int per = (ksplit + 3) / 4;
+                        : zpart_all + (long)chain * ksplit * stride + (long)row * zl + c;
+  const int per = (ksplit + SL - 1) / SL;
   const int lo = sl * per, hi = lo + per < ksplit ? lo + per : ksplit;
   double s = 0.0;
   if (c < n) {
@@ -551,15 +552,18 @@ __global__ __launch_bounds__(256) void reduce_ksplit(const double* __restrict__ 
     }
     for (; k < hi; ++k) s += p[k * stride];
   }
-  __shared__ double red[4][64];
-  red[sl][threadIdx.x & 63] = s;
+  __shared__ double red[SL][64];
+  red[sl][t] = s;
   __syncthreads();
   if (sl == 0 && c < n) {
-    const double t = (red[0][c & 63] + red[1][c & 63]) + (red[2][c & 63] + red[3][c & 63]);
+    double v = 0.0;
+#pragma unroll
+    for (int q = 0; q < SL; q += 4)
+      v += (red[q][t] + red[q + 1][t]) + (red[q + 2][t] + red[q + 3][t]);
     if (isf)
-      f_all[(long)chain * np + c] = t * norm;
+      f_all[(long)chain * np + c] = v * norm;
     else
-      zsum_all[(long)chain * nn + (long)row * np + c] = t;
+      zsum_all[(long)chain * np * np + (long)row * np + c] = v;
   }
 }
 
@@ -614,8 +618,16 @@ void launch_outer_f64(const F64Rows& r, int n, int np, int nc, const double* coe
 
 void launch_reduce_f64(int n, int np, int nc, int ksplit, const double* zpart,
                        const double* fpart, double* zsum, double* f, double norm, hipStream_t s) {
-  hipLaunchKernelGGL(reduce_ksplit, dim3((n + 63) / 64, n + 1, nc), dim3(256), 0, s, zpart, fpart,
-                     n, np, ksplit, zsum, f, norm);
+  const F64Tiles t = f64_tiles(n);
+  const int zl = t.ntile * 16 * t.cb;
+  const dim3 g((n + 63) / 64, n + 1, nc);
+  // a single tile has few work-groups and many splits
+  if (t.ntile == 1)
+    hipLaunchKernelGGL(reduce_ksplit<16>, g, dim3(1024), 0, s, zpart, fpart, n, np, zl, ksplit,
+                       zsum, f, norm);
+  else
+    hipLaunchKernelGGL(reduce_ksplit<4>, g, dim3(256), 0, s, zpart, fpart, n, np, zl, ksplit,
+                       zsum, f, norm);
 }
 
 int launch_pa_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev) {
