@@ -69,6 +69,7 @@ struct LanczosState {
   int nslice = 1;            // element slices of the projections
   int jsplit = 1;            // basis-vector ranges of the update
   int jchunk = 1;
+  bool one_wg = false;       // the recurrence of a step in one work-group per chain
 };
 
 static void free_state(LanczosState& s) {
@@ -316,6 +317,116 @@ __global__ void lanczos_init(const double* __restrict__ part, long ps,
   qcur[c * len + i] = v;
 }
 
+// The whole recurrence of one step for a short chain (len <= 1024 kShortE), one
+// work-group per chain: a_k, the residual, Gram-Schmidt with its conditional second
+// pass, b_k, the next vector and the commit.  The residual stays in registers, its
+// masked copy and the coefficients in LDS; the basis is read from L2 twice per pass,
+// which bounds it (about 100 GB/s for one work-group).  As separate kernels the step is
+// fifteen launches of about 4 us each.  Whole step at 45 modes (2115 entries) and 500
+// images, separate / here: 30 steps 89 / 46 us, 100 steps 97 / 68, 300 steps 102 / 155,
+// so the line is drawn at kShortWork entries of the whole basis.
+constexpr int kShortE = 6;
+constexpr int kShortBasis = 1536;
+constexpr long kShortWork = 300000;
+
+__global__ __launch_bounds__(1024) void lanczos_short(
+    const double* __restrict__ mask, const double* __restrict__ Lq, long len, int kmax, double tol,
+    int reorth, int* __restrict__ kk, int* __restrict__ active, const int* __restrict__ cap,
+    int* __restrict__ ndone, double* __restrict__ a, double* __restrict__ b, double* Qall,
+    double* qall) {
+  const int c = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (!active[c]) return;
+  const int k = kk[c], n = (int)len;
+  __shared__ double rm[1024 * kShortE], coef[kShortBasis], red[16];
+  double* Q = Qall + (long)c * (kmax + 1) * len;
+  double* qc = qall + c * len;
+  auto block_sum = [&](double v) {
+    v = wave_sum64(v);
+    if (lane == 0) red[wave] = v;
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) s += red[w];
+    __syncthreads();
+    return s;
+  };
+  double m[kShortE], q[kShortE], r[kShortE], v = 0.0;
+#pragma unroll
+  for (int e = 0; e < kShortE; ++e) {
+    const int i = t + 1024 * e;
+    m[e] = i < n ? mask[i] : 0.0;
+    q[e] = i < n ? qc[i] : 0.0;
+    r[e] = i < n ? Lq[c * len + i] : 0.0;
+    v += q[e] * r[e] * m[e];
+  }
+  const double ak = block_sum(v);
+  const double bo = k > 0 ? b[c * kmax + k - 1] : 0.0;
+  v = 0.0;
+#pragma unroll
+  for (int e = 0; e < kShortE; ++e) {
+    const int i = t + 1024 * e;
+    r[e] -= ak * q[e];
+    if (k > 0 && i < n) r[e] -= bo * Q[(long)(k - 1) * len + i];
+    v += r[e] * r[e] * m[e];
+  }
+  double norm = block_sum(v);
+  for (int pass = 0; reorth && pass < 2; ++pass) {
+    const double before = norm;
+#pragma unroll
+    for (int e = 0; e < kShortE; ++e)
+      if (t + 1024 * e < n) rm[t + 1024 * e] = r[e] * m[e];
+    __syncthreads();
+    for (int j = wave; j <= k; j += 16) {
+      const double* Qj = Q + (long)j * len;
+      double s = 0.0;
+#pragma unroll 8
+      for (int i = lane; i < n; i += 64) s += Qj[i] * rm[i];
+      s = wave_sum64(s);
+      if (lane == 0) coef[j] = s;
+    }
+    __syncthreads();
+    double u[kShortE];
+#pragma unroll
+    for (int e = 0; e < kShortE; ++e) u[e] = 0.0;
+#pragma unroll 4
+    for (int j = 0; j <= k; ++j) {
+      const double cj = coef[j];
+#pragma unroll
+      for (int e = 0; e < kShortE; ++e)
+        if (t + 1024 * e < n) u[e] += cj * Q[(long)j * len + t + 1024 * e];
+    }
+    v = 0.0;
+#pragma unroll
+    for (int e = 0; e < kShortE; ++e) {
+      r[e] -= u[e];
+      v += r[e] * r[e] * m[e];
+    }
+    norm = block_sum(v);
+    if (!(norm < 0.5 * before)) break;   // (as second_pass_flags)
+  }
+  const double bk = sqrt(norm);
+  const bool small = !(fabs(bk) >= tol), stop = small || k + 1 >= cap[c];
+  if (!stop)
+#pragma unroll
+    for (int e = 0; e < kShortE; ++e) {
+      const int i = t + 1024 * e;
+      if (i < n) {
+        const double x = r[e] / bk;
+        Q[(long)(k + 1) * len + i] = x;
+        qc[i] = x;
+      }
+    }
+  if (t == 0) {
+    a[c * kmax + k] = ak;
+    ndone[c] = k + 1;
+    if (!small) b[c * kmax + k] = bk;
+    if (stop)
+      active[c] = 0;
+    else
+      kk[c] = k + 1;
+  }
+}
+
 static void lanczos_step(Ctx* c, LanczosState& st, int reorth, int precision, int ignore_harmonic,
                          int ignore_v3, int ignore_v4, double tol, hipStream_t s) {
   const long len = st.len;
@@ -325,6 +436,11 @@ static void lanczos_step(Ctx* c, LanczosState& st, int reorth, int precision, in
   const dim3 gr(kRedBlocks, nc);
   apply_L_groups(c, nc, len, st.qcur, st.Lq, 1, 0, ignore_harmonic, ignore_v3, ignore_v4, 0,
                  0.0, precision, s, st.plans.empty() ? nullptr : &st.plans);
+  if (st.one_wg) {
+    hipLaunchKernelGGL(lanczos_short, dim3(nc), dim3(1024), 0, s, st.mask, st.Lq, len, kmax, tol,
+                       reorth, st.k, st.active, st.cap, st.ndone, st.a, st.b, st.Q, st.qcur);
+    return;
+  }
   hipLaunchKernelGGL(dot_partial, gr, dim3(kRedThreads), 0, s, st.qcur, len, st.Lq, len, st.mask,
                      len, st.part, ps, 0);
   hipLaunchKernelGGL(lanczos_residual, gv, dim3(256), 0, s, st.part, ps, st.Q, st.qcur, st.Lq,
@@ -805,6 +921,10 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
       }
       general = general || !st.plans.back().ok;
     }
+  bool planned = false;
+  for (const OrbPlan& p : st.plans) planned = planned || p.ok;
+  st.one_wg = !planned && len <= 1024 * kShortE && n_steps < kShortBasis &&
+              len * n_steps <= kShortWork;
   if (general && precision != PREC_FP64) {
     rc = ensure_split(c, precision);  // allocations must precede graph capture
     if (rc) {

@@ -1261,11 +1261,137 @@ static void reorth_pass(QLanczos& l, QBatch& b, hipStream_t s) {
                      l.kmax, l.cont, l.k, l.r);
 }
 
+// The recurrence of one step for a short chain (ld <= 1024 kQShortE) in one
+// work-group per chain: everything from a_k to the next vector, with r in registers,
+// its masked copy and the coefficients in LDS and the basis from L2.  As separate
+// kernels the step is eleven launches of about 4.7 us each: 250 us per step with the
+// L application for 8 chains on 2x2x2, 200 us here.  The line against the separate
+// kernels is the one of the mode-space recurrence (kQShortWork doubles of the basis).
+constexpr int kQShortE = 3;
+constexpr int kQShortBasis = 1024;
+constexpr long kQShortWork = 300000;
+
+__global__ __launch_bounds__(1024) void ql_short(
+    const double2* __restrict__ Lq, const double* __restrict__ mask, int ld, int kmax, double tol,
+    int* __restrict__ active, int* __restrict__ nextc, int* __restrict__ kk,
+    const int* __restrict__ cap, int* __restrict__ ndone, double* __restrict__ a,
+    double* __restrict__ bb, double* __restrict__ cc, double2* Qall, double2* qall) {
+  const int c = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int nt = blockDim.x, nw = nt >> 6;
+  if (!active[c]) return;
+  const int k = kk[c];
+  __shared__ double2 rm[1024 * kQShortE];
+  __shared__ double coef[kQShortBasis], red[16];
+  double2* Q = Qall + (long)c * (kmax + 1) * ld;
+  double2* qc = qall + (long)c * ld;
+  auto block_sum = [&](double v) {
+    v = wave_sum(v);
+    if (lane == 0) red[wave] = v;
+    __syncthreads();
+    double s = 0.0;
+    for (int w = 0; w < nw; ++w) s += red[w];
+    __syncthreads();
+    return s;
+  };
+  const double2 zero = make_double2(0.0, 0.0);
+  double2 q[kQShortE], r[kQShortE];
+  double m[kQShortE], v = 0.0;
+#pragma unroll
+  for (int e = 0; e < kQShortE; ++e) {
+    const int i = t + nt * e;
+    const bool in = i < ld;
+    m[e] = in ? mask[(long)c * ld + i] : 0.0;
+    q[e] = in ? qc[i] : zero;
+    r[e] = in ? Lq[(long)c * ld + i] : zero;
+    v += m[e] * (q[e].x * r[e].x + q[e].y * r[e].y);
+  }
+  const double ak = block_sum(v);
+  const double cp = k > 0 ? cc[c * kmax + k - 1] : 0.0;
+  v = 0.0;
+#pragma unroll
+  for (int e = 0; e < kQShortE; ++e) {
+    const int i = t + nt * e;
+    r[e] = make_double2(r[e].x - ak * q[e].x, r[e].y - ak * q[e].y);
+    if (k > 0 && i < ld) {
+      const double2 qm = Q[(long)(k - 1) * ld + i];
+      r[e] = make_double2(r[e].x - cp * qm.x, r[e].y - cp * qm.y);
+    }
+    v += m[e] * (r[e].x * r[e].x + r[e].y * r[e].y);
+  }
+  // stop tests of QL:1083-1095 and the step cap (ql_decide)
+  const double b = sqrt(block_sum(v));
+  const bool conv = !(fabs(b) >= tol) || nextc[c], stop = conv || k + 1 >= cap[c];
+  __syncthreads();   // every thread has read the chain's state
+  if (t == 0) {
+    a[c * kmax + k] = ak;
+    ndone[c] = k + 1;
+    if (!conv) bb[c * kmax + k] = cc[c * kmax + k] = b;
+    if (stop) active[c] = 0;
+  }
+  if (stop) return;
+  const double inv = 1.0 / b;
+#pragma unroll
+  for (int e = 0; e < kQShortE; ++e) r[e] = csc(r[e], inv);
+  for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+    for (int e = 0; e < kQShortE; ++e)
+      if (t + nt * e < ld) rm[t + nt * e] = csc(r[e], m[e]);
+    __syncthreads();
+    for (int j = wave; j <= k; j += nw) {
+      const double2* Qj = Q + (long)j * ld;
+      double s = 0.0;
+#pragma unroll 8
+      for (int i = lane; i < ld; i += 64) {
+        const double2 x = Qj[i], y = rm[i];
+        s += x.x * y.x + x.y * y.y;
+      }
+      s = wave_sum(s);
+      if (lane == 0) coef[j] = s;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int j = 0; j <= k; ++j) {
+      const double cj = coef[j];
+#pragma unroll
+      for (int e = 0; e < kQShortE; ++e)
+        if (t + nt * e < ld) {
+          const double2 x = Q[(long)j * ld + t + nt * e];
+          r[e] = make_double2(r[e].x - cj * x.x, r[e].y - cj * x.y);
+        }
+    }
+  }
+  v = 0.0;
+#pragma unroll
+  for (int e = 0; e < kQShortE; ++e) v += m[e] * (r[e].x * r[e].x + r[e].y * r[e].y);
+  const double nrm = sqrt(block_sum(v));
+  const bool small = !(nrm >= tol);
+  const double sc = small ? 1.0 : 1.0 / nrm;
+#pragma unroll
+  for (int e = 0; e < kQShortE; ++e) {
+    const int i = t + nt * e;
+    if (i < ld) {
+      const double2 x = csc(r[e], sc);
+      Q[(long)(k + 1) * ld + i] = x;
+      qc[i] = x;
+    }
+  }
+  if (t == 0) {
+    nextc[c] = small ? 1 : 0;
+    kk[c] = k + 1;
+  }
+}
+
 static void ql_step(QCtx* q, QBatch& b, QLanczos& l, double tol, int ih, int i3, int i4,
                     hipStream_t s) {
   const int ld = b.ld, C = b.C;
   const dim3 gv((ld + 255) / 256, C);
   launch_L(q, b, l.qcur, l.Lq, ih, i3, i4, s);
+  if (ld <= 1024 * kQShortE && l.kmax < kQShortBasis && 2L * ld * l.kmax <= kQShortWork) {
+    hipLaunchKernelGGL(ql_short, dim3(C), dim3(ld <= 256 * kQShortE ? 256 : 1024), 0, s, l.Lq,
+                       l.mask, ld, l.kmax, tol, b.active, l.nextc, l.k, l.cap, l.ndone, l.a, l.bb,
+                       l.cc, l.Q, l.qcur);
+    return;
+  }
   hipLaunchKernelGGL(ql_dot, dim3(C), dim3(256), 0, s, l.qcur, l.Lq, l.mask, ld, b.active, l.scal,
                      0);
   hipLaunchKernelGGL(ql_residual, gv, dim3(256), 0, s, l.Lq, l.qcur, l.Q, ld, l.kmax, b.active,
