@@ -11,6 +11,7 @@
 // Every reduction is a fixed-order loop or tree (no atomics), so training is
 // reproducible.  Parameters are one contiguous FP32 array
 //   [W0 (d1 x d0), b0 (d1), W1 (d2 x d1), b1 (d2), ...], W row-major [out][in].
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -21,6 +22,7 @@ namespace tdscha {
 
 constexpr int kCfOut = 10;   // a_inf, b_inf, da[4], db[4]
 constexpr int kCfTail = 4;
+constexpr int kCfBlocks = 2048;   // work-groups of the spectral loss that fill the chip
 
 struct Mlp {
   int n_layers = 0;              // linear layers = n_hidden + 1
@@ -34,7 +36,8 @@ struct Mlp {
   float* m2 = nullptr;
   float* act = nullptr;          // [n_layers + 1][max_batch][max_dim] layer outputs (act[0] = input)
   float* pre = nullptr;          // [n_layers][max_batch][max_dim] pre-activations
-  float* dz = nullptr;           // [2][max_batch][max_dim] backward ping-pong
+  float* dz = nullptr;           // fused: [n_layers][max_batch][max_dim], the gradient at
+                                 // each layer's output; else [2] of them in turn
   float* target = nullptr;       // [max_batch][n_out] (kind 0)
   float* wout = nullptr;         // [n_out] loss weights (kind 0)
   float* loss_part = nullptr;    // [max_batch]
@@ -51,7 +54,9 @@ struct Mlp {
   double* cf_w = nullptr;        // [n_w]
   double* cf_mean = nullptr;     // [10]
   double* cf_std = nullptr;      // [10]
+  double* cf_part = nullptr;     // [samples x slices <= max_batch + kCfBlocks][11]
   long step = 0;                 // Adam steps taken
+  bool fused = false;            // all layers of a pass in one kernel
   hipStream_t stream = nullptr;
 };
 
@@ -87,6 +92,160 @@ __global__ void mlp_linear_fwd(const float* __restrict__ X, const float* __restr
   }
 }
 
+// Small networks (at most kFuseLayers layers of at most kFuseDim): every layer of a
+// pass in one kernel, a work-group per R batch rows, its activations in LDS.  The
+// weights pass through LDS in panels of 128 of the summed index by 128 outputs, the
+// next panel (of the next layer too) in registers meanwhile.  The sums run in the order
+// of the kernels above.  Bound by the latency of a panel; the separate kernels were 3
+// to 5 launches of 4.6 to 5.6 us per pass (64 rows of 80-128-128-128-10: forward 22 ->
+// 19 us, input gradients 16 -> 12 us; one row: forward 21 -> 15 us).
+constexpr int kFuseLayers = 8;
+constexpr int kFuseDim = 256;
+constexpr int kFusePanel = 128;
+constexpr int kFuseThreads = 512;
+
+struct MlpShape {
+  int layers, ld;                      // ld: row stride of activations
+  long stride;                         // of a layer's activations
+  int dim[kFuseLayers + 1];
+  long w[kFuseLayers], b[kFuseLayers];
+  int tile[kFuseLayers + 1];           // first 16 x 16 weight tile of a layer
+};
+
+template <int R>
+constexpr int fused_lds() {
+  return (kFusePanel * (kFusePanel + 1) + 2 * R * kFuseDim) * (int)sizeof(float);
+}
+
+// Panels of `steps` layers in turn; sizes(s) = (nk, no) and weights pw(s) of step s:
+// W(k, o) at pw[o * nk + k] (KC) or pw[k * no + o].  done(s, o, row, sum) takes the sum
+// over k of output o, row = t / 128 + 4 r, from x = xs[s & 1]; columns of x from nk on
+// are zero.  Thread: output t % 128 of a panel, rows t / 128 + 4 r.
+template <int R, bool KC, typename Sizes, typename Weights, typename Done>
+__device__ __forceinline__ void fused_layers(int steps, Sizes sizes, Weights weights, Done done,
+                                             float (*xs)[R][kFuseDim],
+                                             float (*ws)[kFusePanel + 1]) {
+  constexpr int P = kFusePanel, E = P * P / kFuseThreads, RT = R / 4;
+  const int t = threadIdx.x, lo = t & 127, hi = t >> 7;
+  float v[E];
+  auto fetch = [&](int s, int o0, int k0) {
+    const int2 z = sizes(s);
+    const float* pw = weights(s);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {   // clamped, so that every load can be in flight
+      const int k = min(k0 + (KC ? lo : hi + 4 * e), z.x - 1);
+      const int o = min(o0 + (KC ? hi + 4 * e : lo), z.y - 1);
+      v[e] = KC ? pw[o * z.x + k] : pw[k * z.y + o];
+    }
+  };
+  float acc[RT];
+  int s = 0, o0 = 0, k0 = 0;
+  fetch(0, 0, 0);
+  while (s < steps) {
+    const int2 z = sizes(s);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int k = KC ? lo : hi + 4 * e, o = KC ? hi + 4 * e : lo;
+      ws[k][o] = k0 + k < z.x && o0 + o < z.y ? v[e] : 0.f;
+    }
+    __syncthreads();
+    int s1 = s, o1 = o0, k1 = k0 + P;
+    if (k1 >= z.x) {
+      k1 = 0;
+      o1 += P;
+    }
+    if (o1 >= z.y) {
+      o1 = 0;
+      ++s1;
+    }
+    if (s1 < steps) fetch(s1, o1, k1);
+    if (k0 == 0)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) acc[r] = 0.f;
+    const int ke = min(P, z.x - k0);
+    for (int kb = 0; kb < ke; kb += 8)
+#pragma unroll
+      for (int k = kb; k < kb + 8; ++k) {
+        const float w = ws[k][lo];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r] += xs[s & 1][hi + 4 * r][k0 + k] * w;
+      }
+    if (k1 == 0)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) done(s, o0 + lo, hi + 4 * r, acc[r]);
+    s = s1;
+    o0 = o1;
+    k0 = k1;
+  }
+}
+
+// forward of rows idx[..] (or the rows themselves) of x; keep: store every layer's
+// pre-activations and activations, else the last layer's output only
+template <int R>
+__global__ __launch_bounds__(kFuseThreads) void mlp_fused_fwd(
+    MlpShape m, const float* __restrict__ params, const float* __restrict__ x, int xld,
+    const int* __restrict__ idx, int B, int keep, float* __restrict__ act,
+    float* __restrict__ pre) {
+  extern __shared__ float fsh[];
+  auto ws = reinterpret_cast<float(*)[kFusePanel + 1]>(fsh);
+  auto xs = reinterpret_cast<float(*)[R][kFuseDim]>(fsh + kFusePanel * (kFusePanel + 1));
+  const int b0 = blockIdx.x * R;
+  for (int e = threadIdx.x; e < R * kFuseDim; e += kFuseThreads) {
+    const int r = e / kFuseDim, i = e % kFuseDim, b = b0 + r;
+    const bool in = b < B && i < m.dim[0];
+    const float v = in ? x[(long)(idx ? idx[b] : b) * xld + i] : 0.f;
+    xs[0][r][i] = v;
+    if (keep && in) act[(long)b * m.ld + i] = v;
+  }
+  fused_layers<R, true>(
+      m.layers, [&](int l) { return make_int2(m.dim[l], m.dim[l + 1]); },
+      [&](int l) { return params + m.w[l]; },
+      [&](int l, int o, int row, float sum) {
+        const bool last = l + 1 == m.layers, in = o < m.dim[l + 1];
+        const float z = sum + (in ? params[m.b[l] + o] : 0.f), y = last ? z : silu(z);
+        xs[(l + 1) & 1][row][o] = y;
+        const int b = b0 + row;
+        if (b < B && in && (keep || last)) {
+          const long e = (long)b * m.ld + o;
+          if (keep) pre[l * m.stride + e] = z;
+          act[(l + 1) * m.stride + e] = y;
+        }
+      },
+      xs, ws);
+}
+
+// gradients at the outputs of layers layers - 2 .. 0 from the one at the last
+template <int R>
+__global__ __launch_bounds__(kFuseThreads) void mlp_fused_bwd_x(MlpShape m,
+                                                                const float* __restrict__ params,
+                                                                const float* __restrict__ pre,
+                                                                int B, float* __restrict__ dz) {
+  extern __shared__ float fsh[];
+  auto ws = reinterpret_cast<float(*)[kFusePanel + 1]>(fsh);
+  auto xs = reinterpret_cast<float(*)[R][kFuseDim]>(fsh + kFusePanel * (kFusePanel + 1));
+  const int b0 = blockIdx.x * R, L = m.layers;
+  for (int e = threadIdx.x; e < R * kFuseDim; e += kFuseThreads) {
+    const int r = e / kFuseDim, i = e % kFuseDim, b = b0 + r;
+    xs[0][r][i] = b < B && i < m.dim[L] ? dz[(L - 1) * m.stride + (long)b * m.ld + i] : 0.f;
+  }
+  // step s: through layer l = L - 1 - s to the output of layer l - 1
+  fused_layers<R, false>(
+      L - 1, [&](int s) { return make_int2(m.dim[L - s], m.dim[L - 1 - s]); },
+      [&](int s) { return params + m.w[L - 1 - s]; },
+      [&](int s, int i, int row, float sum) {
+        const int b = b0 + row, l = L - 1 - s;
+        float g = 0.f;
+        if (b < B && i < m.dim[l]) {
+          const long e = (l - 1) * m.stride + (long)b * m.ld + i;
+          g = sum * dsilu(pre[e]);
+          dz[e] = g;
+        }
+        xs[(s + 1) & 1][row][i] = g;
+      },
+      xs, ws);
+}
+
 // kind 0: dY = 2 w (Y - T) / B, loss_part = sum_o w (Y - T)^2 / B
 __global__ void mlp_mse_grad(const float* __restrict__ Y, const float* __restrict__ T,
                              const float* __restrict__ w, float* __restrict__ dY,
@@ -109,12 +268,13 @@ __device__ __forceinline__ cplx cmul(cplx a, cplx b) {
   return {a.r * b.r - a.i * b.i, a.r * b.i + a.i * b.r};
 }
 __device__ __forceinline__ cplx cinv(cplx z) {
-  const double d = z.r * z.r + z.i * z.i;
-  return {z.r / d, -z.i / d};
+  const double d = 1.0 / (z.r * z.r + z.i * z.i);
+  return {z.r * d, -z.i * d};
 }
 __device__ __forceinline__ cplx cscale(cplx a, double s) { return {a.r * s, a.i * s}; }
 
-// kind 1: one block per sample, threads stride over the frequency grid.
+// kind 1: a slice of the frequency grid of one sample per block (grid.x samples,
+// grid.y slices; cf_loss_sum adds the slices).
 // Tail: terminator root from (A, B) = b0 (p0, p1) as in the reference's
 // terminator (no smearing in its discriminant, smaller-modulus root, ties to
 // the minus root), then the four predicted levels a_j = b0 (p0 + p_{2+j}),
@@ -125,9 +285,9 @@ __global__ void __launch_bounds__(256) cf_loss_kernel(
     const float* __restrict__ Y, int ld, const int* __restrict__ idx,
     const double* __restrict__ chains, const double* __restrict__ ref,
     const double* __restrict__ wgrid, int n_w, int K, double eta,
-    const double* __restrict__ out_mean, const double* __restrict__ out_std, double scale,
-    float* __restrict__ dY, float* __restrict__ loss_part) {
-  __shared__ double red[kCfOut + 1][256];
+    const double* __restrict__ out_mean, const double* __restrict__ out_std,
+    double* __restrict__ part) {
+  __shared__ double red[kCfOut + 1][4];
   const int bi = blockIdx.x;
   const long row = idx[bi];
   const double* ch = chains + row * (2 * K + 2);
@@ -143,7 +303,7 @@ __global__ void __launch_bounds__(256) cf_loss_kernel(
 #pragma unroll
   for (int o = 0; o < kCfOut; ++o) gacc[o] = 0.0;
   const double A = b0 * p[0], Bt = b0 * p[1];
-  for (int k = threadIdx.x; k < n_w; k += blockDim.x) {
+  for (int k = blockIdx.y * 256 + threadIdx.x; k < n_w; k += 256 * gridDim.y) {
     const double om = wgrid[k];
     const double w2 = om * om, sm = 2.0 * om * eta;
     // terminator root and its derivatives
@@ -196,12 +356,24 @@ __global__ void __launch_bounds__(256) cf_loss_kernel(
       g = gn;
     }
     // the chain's own levels
+    // (eight levels' coefficients loaded at once: one wait per eight)
     cplx D = {1.0, 0.0};
-    for (int i = K - 1; i >= 0; --i) {
-      const double bi2 = bv[i] * bv[i];
-      const cplx gn = cinv({av[i] + w2 - bi2 * g.r, sm - bi2 * g.i});
-      D = cscale(cmul(D, cmul(gn, gn)), bi2);
-      g = gn;
+    for (int i0 = K - 1; i0 >= 0; i0 -= 8) {
+      double la[8], lb[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int i = i0 - e > 0 ? i0 - e : 0;
+        la[e] = av[i];
+        lb[e] = bv[i];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (i0 - e < 0) break;
+        const double bi2 = lb[e] * lb[e];
+        const cplx gn = cinv({la[e] + w2 - bi2 * g.r, sm - bi2 * g.i});
+        D = cscale(cmul(D, cmul(gn, gn)), bi2);
+        g = gn;
+      }
     }
     // Wigner convention: spectrum = -Im(G)
     const double r = -g.i * inv_s - rf[k];
@@ -213,32 +385,47 @@ __global__ void __launch_bounds__(256) cf_loss_kernel(
       gacc[o] -= c * t.i;
     }
   }
-  red[0][threadIdx.x] = lsum;
+  // sums over the grid: a wave, then the four waves in order
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int o = 0; o < kCfOut; ++o) red[o + 1][threadIdx.x] = gacc[o];
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
+  for (int q = 0; q <= kCfOut; ++q) {
+    double v = q ? gacc[q - 1] : lsum;
 #pragma unroll
-      for (int q = 0; q <= kCfOut; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + s];
-    }
-    __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if (lane == 0) red[q][wave] = v;
   }
-  if (threadIdx.x == 0) {
-    loss_part[bi] = (float)(scale * red[0][0] / n_w);
-#pragma unroll
-    for (int o = 0; o < kCfOut; ++o)
-      dY[(long)bi * ld + o] = (float)(scale * red[o + 1][0] / n_w * out_std[o]);
+  __syncthreads();
+  if (threadIdx.x <= kCfOut) {
+    const int q = threadIdx.x;
+    part[((long)bi * gridDim.y + blockIdx.y) * (kCfOut + 1) + q] =
+        (red[q][0] + red[q][1]) + (red[q][2] + red[q][3]);
   }
 }
 
+// slices of cf_loss_kernel in order: loss and gradient of sample blockIdx.x
+__global__ void cf_loss_sum(const double* __restrict__ part, int slices, int n_w, int ld,
+                            const double* __restrict__ out_std, double scale,
+                            float* __restrict__ dY, float* __restrict__ loss_part) {
+  const int bi = blockIdx.x, q = threadIdx.x;
+  if (q > kCfOut) return;
+  const double* p = part + (long)bi * slices * (kCfOut + 1) + q;
+  double v = 0.0;
+#pragma unroll 8
+  for (int k = 0; k < slices; ++k) v += p[k * (kCfOut + 1)];
+  if (q == 0)
+    loss_part[bi] = (float)(scale * v / n_w);
+  else
+    dY[(long)bi * ld + q - 1] = (float)(scale * v / n_w * out_std[q - 1]);
+}
+
 // dW[o][i] = sum_b dZ[b][o] Ain[b][i]; db[o] = sum_b dZ[b][o] (fixed order in b)
-__global__ void mlp_linear_bwd_w(const float* __restrict__ dZ, const float* __restrict__ Ain,
-                                 float* __restrict__ dW, float* __restrict__ db, int B, int in,
-                                 int out, int ld) {
+__device__ __forceinline__ void bwd_w_tile(const float* __restrict__ dZ,
+                                           const float* __restrict__ Ain, float* __restrict__ dW,
+                                           float* __restrict__ db, int B, int in, int out, int ld,
+                                           int bx, int by) {
   __shared__ float zs[16][17], as[16][17];
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int o = blockIdx.y * 16 + ty, i = blockIdx.x * 16 + tx;
+  const int o = by * 16 + ty, i = bx * 16 + tx;
   float s = 0.f, sb = 0.f;
   for (int b0 = 0; b0 < B; b0 += 16) {
     const int zb = b0 + tx;
@@ -254,7 +441,23 @@ __global__ void mlp_linear_bwd_w(const float* __restrict__ dZ, const float* __re
     __syncthreads();
   }
   if (o < out && i < in) dW[(long)o * in + i] = s;
-  if (o < out && blockIdx.x == 0 && tx == 0) db[o] = sb;
+  if (o < out && bx == 0 && tx == 0) db[o] = sb;
+}
+
+__global__ void mlp_linear_bwd_w(const float* __restrict__ dZ, const float* __restrict__ Ain,
+                                 float* __restrict__ dW, float* __restrict__ db, int B, int in,
+                                 int out, int ld) {
+  bwd_w_tile(dZ, Ain, dW, db, B, in, out, ld, blockIdx.x, blockIdx.y);
+}
+
+// the weight gradients of every layer in one launch
+__global__ void mlp_fused_bwd_w(MlpShape m, const float* __restrict__ dz,
+                                const float* __restrict__ act, float* __restrict__ grads, int B) {
+  int l = 0;
+  while ((int)blockIdx.x >= m.tile[l + 1]) ++l;
+  const int q = blockIdx.x - m.tile[l], nx = (m.dim[l] + 15) / 16;
+  bwd_w_tile(dz + l * m.stride, act + l * m.stride, grads + m.w[l], grads + m.b[l], B, m.dim[l],
+             m.dim[l + 1], m.ld, q % nx, q / nx);
 }
 
 // dZprev[b][i] = (sum_o dZ[b][o] W[o][i]) * SiLU'(Zprev[b][i])
@@ -306,6 +509,61 @@ __global__ void mlp_gather(const float* __restrict__ dx, const float* __restrict
 static float* act_l(Mlp* m, int l) { return m->act + (long)l * m->max_batch * m->max_dim; }
 static float* pre_l(Mlp* m, int l) { return m->pre + (long)l * m->max_batch * m->max_dim; }
 
+// the fused kernels use more than 64 KB of the CU's 160 KB of LDS
+static bool fused_ready() {
+  auto allow = [](const void* f, int bytes) {
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+  };
+  const bool ok = allow((const void*)mlp_fused_fwd<4>, fused_lds<4>()) &&
+                  allow((const void*)mlp_fused_fwd<8>, fused_lds<8>()) &&
+                  allow((const void*)mlp_fused_bwd_x<4>, fused_lds<4>()) &&
+                  allow((const void*)mlp_fused_bwd_x<8>, fused_lds<8>());
+  if (!ok) (void)hipGetLastError();
+  return ok;
+}
+
+static MlpShape shape(const Mlp* m) {
+  MlpShape h;
+  h.layers = m->n_layers;
+  h.ld = m->max_dim;
+  h.stride = (long)m->max_batch * m->max_dim;
+  h.tile[0] = 0;
+  for (int l = 0; l < m->n_layers; ++l) {
+    h.dim[l] = m->dims[l];
+    h.w[l] = m->w_off[l];
+    h.b[l] = m->b_off[l];
+    h.tile[l + 1] = h.tile[l] + ((m->dims[l] + 15) / 16) * ((m->dims[l + 1] + 15) / 16);
+  }
+  h.dim[m->n_layers] = m->dims[m->n_layers];
+  return h;
+}
+
+// fused forward of rows of x (row stride xld); 4 rows to a work-group until every CU
+// has four of them, then 8
+static void forward_fused(Mlp* m, int B, const float* x, int xld, const int* idx, int keep) {
+  const MlpShape h = shape(m);
+  if (B <= 4096)
+    hipLaunchKernelGGL(mlp_fused_fwd<4>, dim3((B + 3) / 4), dim3(kFuseThreads), fused_lds<4>(),
+                       m->stream, h, m->params, x, xld, idx, B, keep, m->act, m->pre);
+  else
+    hipLaunchKernelGGL(mlp_fused_fwd<8>, dim3((B + 7) / 8), dim3(kFuseThreads), fused_lds<8>(),
+                       m->stream, h, m->params, x, xld, idx, B, keep, m->act, m->pre);
+}
+
+static void backward_fused(Mlp* m, int B) {
+  const MlpShape h = shape(m);
+  if (m->n_layers > 1) {
+    if (B <= 4096)
+      hipLaunchKernelGGL(mlp_fused_bwd_x<4>, dim3((B + 3) / 4), dim3(kFuseThreads), fused_lds<4>(),
+                         m->stream, h, m->params, m->pre, B, m->dz);
+    else
+      hipLaunchKernelGGL(mlp_fused_bwd_x<8>, dim3((B + 7) / 8), dim3(kFuseThreads), fused_lds<8>(),
+                         m->stream, h, m->params, m->pre, B, m->dz);
+  }
+  hipLaunchKernelGGL(mlp_fused_bwd_w, dim3(h.tile[m->n_layers]), dim3(256), 0, m->stream, h, m->dz,
+                     m->act, m->grads, B);
+}
+
 static void forward(Mlp* m, int B) {
   const int ld = m->max_dim;
   for (int l = 0; l < m->n_layers; ++l) {
@@ -320,13 +578,19 @@ static void forward(Mlp* m, int B) {
 // loss partials and the gradient with respect to the network outputs
 static void loss_head(Mlp* m, int kind, int B) {
   const int ld = m->max_dim, L = m->n_layers;
+  float* dz = m->dz + (m->fused ? (long)(L - 1) * m->max_batch * ld : 0);
   if (kind == 0) {
     hipLaunchKernelGGL(mlp_mse_grad, dim3((B + 255) / 256), dim3(256), 0, m->stream,
-                       act_l(m, L), m->target, m->wout, m->dz, m->loss_part, B, m->dims[L], ld);
+                       act_l(m, L), m->target, m->wout, dz, m->loss_part, B, m->dims[L], ld);
   } else {
-    hipLaunchKernelGGL(cf_loss_kernel, dim3(B), dim3(256), 0, m->stream, act_l(m, L), ld, m->idx,
-                       m->data_ch, m->data_ref, m->cf_w, m->cf_nw, m->cf_K, m->cf_eta,
-                       m->cf_mean, m->cf_std, m->cf_scale / B, m->dz, m->loss_part);
+    // slices of 256 frequencies while they fill the chip (64 samples of 2000: 60 us
+    // with one block each, 17 us in eight, and 4 us to add them)
+    const int slices = std::min((m->cf_nw + 255) / 256, (kCfBlocks + B - 1) / B);
+    hipLaunchKernelGGL(cf_loss_kernel, dim3(B, slices), dim3(256), 0, m->stream, act_l(m, L), ld,
+                       m->idx, m->data_ch, m->data_ref, m->cf_w, m->cf_nw, m->cf_K, m->cf_eta,
+                       m->cf_mean, m->cf_std, m->cf_part);
+    hipLaunchKernelGGL(cf_loss_sum, dim3(B), dim3(64), 0, m->stream, m->cf_part, slices, m->cf_nw,
+                       ld, m->cf_std, m->cf_scale / B, dz, m->loss_part);
   }
 }
 
@@ -395,6 +659,15 @@ static int upload_data(Mlp* m, int kind, long n, const float* x, const float* t,
 // one minibatch: gather rows idx[0..B), forward, loss head, backward
 static void batch_pass(Mlp* m, int kind, int B) {
   const int n_in = m->dims[0], n_out = m->dims[m->n_layers];
+  if (m->fused) {
+    if (kind == 0)
+      hipLaunchKernelGGL(mlp_gather, dim3(B), dim3(128), 0, m->stream, (const float*)nullptr,
+                         m->data_t, m->idx, B, 0, n_out, m->max_dim, (float*)nullptr, m->target);
+    forward_fused(m, B, m->data_x, n_in, m->idx, 1);
+    loss_head(m, kind, B);
+    backward_fused(m, B);
+    return;
+  }
   hipLaunchKernelGGL(mlp_gather, dim3(B), dim3(128), 0, m->stream, m->data_x,
                      kind == 0 ? m->data_t : nullptr, m->idx, B, n_in, n_out, m->max_dim,
                      act_l(m, 0), m->target);
@@ -464,7 +737,8 @@ int tdscha_mlp_create(tdscha_mlp** out, int n_in, int width, int n_hidden, int n
   for (int d : m->dims) m->max_dim = d > m->max_dim ? d : m->max_dim;
   const long act_n = (long)(m->n_layers + 1) * max_batch * m->max_dim;
   const long pre_n = (long)m->n_layers * max_batch * m->max_dim;
-  const long dz_n = 2L * max_batch * m->max_dim;
+  m->fused = m->n_layers <= kFuseLayers && m->max_dim <= kFuseDim && fused_ready();
+  const long dz_n = (m->fused ? m->n_layers : 2L) * max_batch * m->max_dim;
   auto fail = [&]() {
     tdscha_mlp_destroy(reinterpret_cast<tdscha_mlp*>(m));
     return -1;
@@ -512,7 +786,8 @@ void tdscha_mlp_destroy(tdscha_mlp* h) {
   if (m->stream) hipStreamSynchronize(m->stream);
   void* ptrs[] = {m->params,  m->grads,  m->m1,      m->m2,       m->act,  m->pre,
                   m->dz,      m->target, m->wout,    m->loss_part, m->idx, m->data_x,
-                  m->data_t,  m->data_ch, m->data_ref, m->cf_w,    m->cf_mean, m->cf_std};
+                  m->data_t,  m->data_ch, m->data_ref, m->cf_w,    m->cf_mean, m->cf_std,
+                  m->cf_part};
   for (void* p : ptrs)
     if (p) hipFree(p);
   if (m->stream) hipStreamDestroy(m->stream);
@@ -567,6 +842,9 @@ int tdscha_mlp_set_cf_loss(tdscha_mlp* h, int K, int n_w, const double* w, doubl
   m->cf_w = nullptr;
   if (!m->cf_mean) TDS_CHECK_HIP(hipMalloc((void**)&m->cf_mean, sizeof(double) * kCfOut));
   if (!m->cf_std) TDS_CHECK_HIP(hipMalloc((void**)&m->cf_std, sizeof(double) * kCfOut));
+  if (!m->cf_part)
+    TDS_CHECK_HIP(hipMalloc((void**)&m->cf_part, sizeof(double) * (kCfOut + 1) *
+                                                     ((size_t)m->max_batch + kCfBlocks)));
   TDS_CHECK_HIP(hipMalloc((void**)&m->cf_w, sizeof(double) * n_w));
   TDS_CHECK_HIP(hipMemcpy(m->cf_w, w, sizeof(double) * n_w, hipMemcpyHostToDevice));
   TDS_CHECK_HIP(hipMemcpy(m->cf_mean, out_mean, sizeof(double) * kCfOut, hipMemcpyHostToDevice));
@@ -588,7 +866,10 @@ int tdscha_mlp_forward(tdscha_mlp* h, int batch, const float* x, float* y) {
     TDS_CHECK_HIP(hipMemcpy2DAsync(act_l(m, 0), sizeof(float) * m->max_dim,
                                    x + (long)b0 * n_in, sizeof(float) * n_in,
                                    sizeof(float) * n_in, B, hipMemcpyHostToDevice, m->stream));
-    forward(m, B);
+    if (m->fused)
+      forward_fused(m, B, act_l(m, 0), m->max_dim, nullptr, 0);
+    else
+      forward(m, B);
     TDS_CHECK_HIP(hipGetLastError());
     TDS_CHECK_HIP(hipMemcpy2DAsync(y + (long)b0 * n_out, sizeof(float) * n_out,
                                    act_l(m, m->n_layers), sizeof(float) * m->max_dim,
