@@ -382,6 +382,10 @@ int tdscha_mlp_get_params(tdscha_mlp* net, float* params_out);
 int tdscha_mlp_set_params(tdscha_mlp* net, const float* params, int reset_optimizer);
 /* Inference: y [batch, n_out] from x [batch, n_in] (host arrays). */
 int tdscha_mlp_forward(tdscha_mlp* net, int batch, const float* x, float* y);
+/* The same rows through n_nets networks of equal input and output sizes side by side:
+ * y [n_nets][batch][n_out]. */
+int tdscha_mlp_forward_many(int n_nets, tdscha_mlp* const* nets, int batch, const float* x,
+                            float* y);
 /* Loss kind 0: sum_o w_o (y_o - t_o)^2 averaged over the batch (w defaults to 1). */
 int tdscha_mlp_set_mse_weights(tdscha_mlp* net, const float* w);
 /*

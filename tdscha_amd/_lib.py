@@ -95,6 +95,7 @@ def _signatures(L):
     L.tdscha_mlp_get_params.argtypes = [_vp, _vp]
     L.tdscha_mlp_set_params.argtypes = [_vp, _vp, C.c_int]
     L.tdscha_mlp_forward.argtypes = [_vp, C.c_int, _vp, _vp]
+    L.tdscha_mlp_forward_many.argtypes = [C.c_int, _vp, C.c_int, _vp, _vp]
     L.tdscha_mlp_set_mse_weights.argtypes = [_vp, _vp]
     L.tdscha_mlp_set_cf_loss.argtypes = [_vp, C.c_int, C.c_int, _vp, C.c_double, _vp, _vp,
                                          C.c_double]

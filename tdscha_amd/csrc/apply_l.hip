@@ -9,6 +9,7 @@
 // pairs p in row-major upper-triangle order (row r <= col c), w_a = w[c],
 // w_b = w[r] (DL:2339-2346).
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <vector>
 
@@ -684,15 +685,21 @@ int tdscha_apply_L(tdscha_ctx* ctx, int n_vec, const double* psi, double* out, i
   int rc = setup_pairs(c);
   if (rc) return rc;
   const long len = c->n + (long)c->n * (c->n + 1);
-  TDS_CHECK_HIP(hipMemcpyAsync(c->psi_dev, psi, sizeof(double) * n_vec * len,
-                               hipMemcpyHostToDevice, c->stream));
+  const size_t bytes = sizeof(double) * n_vec * len;
+  const bool pinned = c->pinned && bytes <= kPinned;
+  double* in = pinned ? reinterpret_cast<double*>(c->pinned) : c->psi_dev;
+  double* res = pinned ? reinterpret_cast<double*>(c->pinned + kPinned) : c->psi_out_dev;
+  if (pinned)
+    std::memcpy(in, psi, bytes);
+  else
+    TDS_CHECK_HIP(hipMemcpyAsync(in, psi, bytes, hipMemcpyHostToDevice, c->stream));
   TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0, 1 or 2");
-  rc = apply_L_dev(c, n_vec, c->psi_dev, c->psi_out_dev, use_wigner, transpose, ignore_harmonic,
-                   ignore_v3, ignore_v4, reverse, shift, precision, c->stream, nullptr, psi);
+  rc = apply_L_dev(c, n_vec, in, res, use_wigner, transpose, ignore_harmonic, ignore_v3,
+                   ignore_v4, reverse, shift, precision, c->stream, nullptr, psi);
   if (rc) return rc;
-  TDS_CHECK_HIP(hipMemcpyAsync(out, c->psi_out_dev, sizeof(double) * n_vec * len,
-                               hipMemcpyDeviceToHost, c->stream));
+  if (!pinned) TDS_CHECK_HIP(hipMemcpyAsync(out, res, bytes, hipMemcpyDeviceToHost, c->stream));
   TDS_CHECK_HIP(hipStreamSynchronize(c->stream));
+  if (pinned) std::memcpy(out, res, bytes);
   return 0;
 }
 

@@ -2,6 +2,8 @@
 // (Modules/DynamicalLanczos.py:5032-5162), one thread per frequency, FP64.
 #include <hip/hip_complex.h>
 
+#include <vector>
+
 #include "common.hpp"
 #include "../../include/tdscha_amd.h"
 
@@ -95,24 +97,27 @@ extern "C" int tdscha_continued_fraction(int n_a, const double* a, int n_b, cons
     bm *= sign;
     cm *= sign;
   }
-  const int nbb = n_b > 0 ? n_b : 1;
-  double *da = nullptr, *db = nullptr, *dc = nullptr, *dw = nullptr, *dout = nullptr;
-  TDS_CHECK_HIP(hipMalloc((void**)&da, sizeof(double) * n_a));
-  TDS_CHECK_HIP(hipMalloc((void**)&db, sizeof(double) * nbb));
-  TDS_CHECK_HIP(hipMalloc((void**)&dc, sizeof(double) * nbb));
-  TDS_CHECK_HIP(hipMalloc((void**)&dw, sizeof(double) * n_w));
-  TDS_CHECK_HIP(hipMalloc((void**)&dout, sizeof(double) * 2 * n_w));
-  TDS_CHECK_HIP(hipMemcpy(da, a, sizeof(double) * n_a, hipMemcpyHostToDevice));
-  if (n_b > 0) {
-    TDS_CHECK_HIP(hipMemcpy(db, b, sizeof(double) * n_b, hipMemcpyHostToDevice));
-    TDS_CHECK_HIP(hipMemcpy(dc, c ? c : b, sizeof(double) * n_b, hipMemcpyHostToDevice));
+  // one allocation and one copy each way: [a, b, c, w] in, [out] behind them
+  const size_t nin = (size_t)n_a + 2 * n_b + n_w;
+  std::vector<double> in;
+  in.reserve(nin);
+  in.insert(in.end(), a, a + n_a);
+  in.insert(in.end(), b, b + n_b);
+  in.insert(in.end(), c ? c : b, (c ? c : b) + n_b);
+  in.insert(in.end(), w, w + n_w);
+  double* da = nullptr;
+  TDS_CHECK_HIP(hipMalloc((void**)&da, sizeof(double) * (nin + 2 * (size_t)n_w)));
+  double *db = da + n_a, *dc = db + n_b, *dw = dc + n_b, *dout = dw + n_w;
+  hipError_t e = hipMemcpy(da, in.data(), sizeof(double) * nin, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(cfrac_kernel, dim3((n_w + 127) / 128), dim3(128), 0, 0, da, db, dc, n_a,
+                       c ? 1 : 0, dw, n_w, use_wigner, use_terminator, am, bm, cm, smearing,
+                       smooth_ramp, sign, shift, modulus, dout);
+    e = hipGetLastError();
   }
-  TDS_CHECK_HIP(hipMemcpy(dw, w, sizeof(double) * n_w, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(cfrac_kernel, dim3((n_w + 127) / 128), dim3(128), 0, 0, da, db, dc, n_a,
-                     c ? 1 : 0, dw, n_w, use_wigner, use_terminator, am, bm, cm, smearing,
-                     smooth_ramp, sign, shift, modulus, dout);
-  TDS_CHECK_HIP(hipGetLastError());
-  TDS_CHECK_HIP(hipMemcpy(gf_out, dout, sizeof(double) * 2 * n_w, hipMemcpyDeviceToHost));
-  (void)hipFree(da); (void)hipFree(db); (void)hipFree(dc); (void)hipFree(dw); (void)hipFree(dout);
+  if (e == hipSuccess)
+    e = hipMemcpy(gf_out, dout, sizeof(double) * 2 * n_w, hipMemcpyDeviceToHost);
+  (void)hipFree(da);
+  TDS_CHECK_HIP(e);
   return 0;
 }

@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace tdscha {
@@ -64,6 +65,25 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Arrays carved from one allocation (256-byte aligned): add() each, allocate total()
+// bytes, assign() the base.
+class Carve {
+ public:
+  template <typename T>
+  void add(T** p, size_t count) {
+    parts_.push_back({reinterpret_cast<void**>(p), total_});
+    total_ += (sizeof(T) * count + 255) / 256 * 256;
+  }
+  size_t total() const { return total_; }
+  void assign(void* base) const {
+    for (const auto& q : parts_) *q.first = static_cast<char*>(base) + q.second;
+  }
+
+ private:
+  std::vector<std::pair<void**, size_t>> parts_;
+  size_t total_ = 0;
+};
+
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -88,6 +108,11 @@ struct SplitStore {
   float* colw = nullptr;   // [3, np] 1/su, 1/sf, fpsi in FP32 (weights epilogue)
   bool ready = false;
 };
+
+// Host calls up to this size pass their vectors through pinned memory that the kernels
+// access: a copy each way is a launch of its own (4 to 5 us on the device, 16 atoms:
+// 82 -> 40 us per call).  Longer vectors are copied.
+constexpr size_t kPinned = 65536;
 
 // Orbit form of the averages (orbit.hip)
 constexpr int kProbe = 8;            // probe configurations of the rank search
@@ -160,6 +185,9 @@ struct Ctx {
   double* fy = nullptr;     // [np]
   double* fpsi = nullptr;   // [np]
   double* w = nullptr;      // [np]
+  // pinned host memory that the kernels read and write directly, for calls whose
+  // vectors take at most kPinned bytes each way (null: no such call)
+  char* pinned = nullptr;   // [2 kPinned]: in, out
   // per-call buffers
   double* R1 = nullptr;     // [kMaxChains, np]
   double* Y1 = nullptr;     // [kMaxChains, np, np]

@@ -216,6 +216,13 @@ int tdscha_ctx_create(tdscha_ctx** out, int n_modes, int n_configs, const double
   ALLOC(c->stage_in, sizeof(double) * kMaxChains * ((long)n_modes + (long)n_modes * n_modes));
   ALLOC(c->stage_out, sizeof(double) * kMaxChains * ((long)n_modes + (long)n_modes * n_modes));
 
+  // (the rotation form adds to its outputs: not over the bus)
+  if (!c->rotate && sizeof(double) * ((size_t)n_modes * (n_modes + 2)) <= kPinned &&
+      hipHostMalloc((void**)&c->pinned, 2 * kPinned) != hipSuccess) {
+    (void)hipGetLastError();
+    c->pinned = nullptr;
+  }
+
   // thermal factors (padded modes get zero)
   std::vector<double> hfy(np, 0.0), hfp(np, 0.0), hw(np, 0.0);
   for (int m = 0; m < n_modes; ++m) {
@@ -371,6 +378,7 @@ void tdscha_ctx_destroy(tdscha_ctx* ctx) {
     for (void* p : sp)
       if (p) hipFree(p);
   }
+  if (c->pinned) (void)hipHostFree(c->pinned);
   orbit_free(c);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
@@ -440,19 +448,32 @@ int tdscha_perturb_averages_batched(tdscha_ctx* ctx, int n_chains, const double*
   TDS_REQUIRE(n_chains >= 1 && n_chains <= kMaxChains, 2, "n_chains must be in [1, 8]");
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   const size_t n = c->n, nn = n * n;
-  double* dR = c->stage_in;
-  double* dY = c->stage_in + (size_t)n_chains * n;
-  double* df = c->stage_out;
-  double* dd = c->stage_out + (size_t)n_chains * n;
-  TDS_CHECK_HIP(hipMemcpyAsync(dR, R1, sizeof(double) * n_chains * n, hipMemcpyHostToDevice, c->stream));
-  TDS_CHECK_HIP(hipMemcpyAsync(dY, Y1, sizeof(double) * n_chains * nn, hipMemcpyHostToDevice, c->stream));
+  const size_t br = sizeof(double) * n_chains * n, by = sizeof(double) * n_chains * nn;
+  const bool pinned = c->pinned && br + by <= kPinned;
+  double* dR = pinned ? reinterpret_cast<double*>(c->pinned) : c->stage_in;
+  double* dY = dR + (size_t)n_chains * n;
+  double* df = pinned ? reinterpret_cast<double*>(c->pinned + kPinned) : c->stage_out;
+  double* dd = df + (size_t)n_chains * n;
+  if (pinned) {
+    std::memcpy(dR, R1, br);
+    std::memcpy(dY, Y1, by);
+  } else {
+    TDS_CHECK_HIP(hipMemcpyAsync(dR, R1, br, hipMemcpyHostToDevice, c->stream));
+    TDS_CHECK_HIP(hipMemcpyAsync(dY, Y1, by, hipMemcpyHostToDevice, c->stream));
+  }
   TDS_REQUIRE(apply_d4 == 0 || apply_d4 == 1, 2, "the apply_d4 value passed must be either 0 or 1");
   TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0 (FP64), 1 (FP16x2) or 2 (BF16x2)");
   int rc = perturb_averages_dev(c, n_chains, dR, dY, apply_d4, precision, df, dd, c->stream, R1);
   if (rc) return rc;
-  TDS_CHECK_HIP(hipMemcpyAsync(f_out, df, sizeof(double) * n_chains * n, hipMemcpyDeviceToHost, c->stream));
-  TDS_CHECK_HIP(hipMemcpyAsync(d2v_out, dd, sizeof(double) * n_chains * nn, hipMemcpyDeviceToHost, c->stream));
+  if (!pinned) {
+    TDS_CHECK_HIP(hipMemcpyAsync(f_out, df, br, hipMemcpyDeviceToHost, c->stream));
+    TDS_CHECK_HIP(hipMemcpyAsync(d2v_out, dd, by, hipMemcpyDeviceToHost, c->stream));
+  }
   TDS_CHECK_HIP(hipStreamSynchronize(c->stream));
+  if (pinned) {
+    std::memcpy(f_out, df, br);
+    std::memcpy(d2v_out, dd, by);
+  }
   return 0;
 }
 

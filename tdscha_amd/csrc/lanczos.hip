@@ -64,6 +64,7 @@ struct LanczosState {
   int* cap = nullptr;        // [nc]
   int* ndone = nullptr;      // [nc] number of a coefficients
   int* stepno = nullptr;     // steps taken by the run
+  void* mem = nullptr;       // the arrays above
   std::vector<OrbPlan> plans;  // per group of kMaxChains chains (empty: general form)
   double* upart = nullptr;   // [nc, jsplit, len] basis-range partial updates (short vectors)
   int nslice = 1;            // element slices of the projections
@@ -73,10 +74,7 @@ struct LanczosState {
 };
 
 static void free_state(LanczosState& s) {
-  void* p[] = {s.Q, s.qcur, s.Lq, s.r, s.mask, s.part, s.coef, s.a, s.b, s.scal, s.k, s.active,
-               s.cap, s.ndone, s.upart, s.act2, s.stepno};
-  for (void* x : p)
-    if (x) (void)hipFree(x);
+  if (s.mem) (void)hipFree(s.mem);
   for (OrbPlan& q : s.plans) orbit_plan_free(q);
 }
 
@@ -834,30 +832,33 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
   st.len = n + (long)n * (n + 1);
   const long len = st.len;
   const size_t qbytes = sizeof(double) * (size_t)n_chains * (n_steps + 1) * len;
-  bool ok = hipMalloc((void**)&st.Q, qbytes) == hipSuccess &&
-            hipMalloc((void**)&st.qcur, sizeof(double) * n_chains * len) == hipSuccess &&
-            hipMalloc((void**)&st.Lq, sizeof(double) * n_chains * len) == hipSuccess &&
-            hipMalloc((void**)&st.r, sizeof(double) * n_chains * len) == hipSuccess &&
-            hipMalloc((void**)&st.mask, sizeof(double) * len) == hipSuccess &&
-            hipMalloc((void**)&st.part, sizeof(double) * n_chains * (n_steps + 1) * kRedBlocks) == hipSuccess &&
-            hipMalloc((void**)&st.coef, sizeof(double) * n_chains * (n_steps + 1)) == hipSuccess &&
-            hipMalloc((void**)&st.a, sizeof(double) * n_chains * n_steps) == hipSuccess &&
-            hipMalloc((void**)&st.b, sizeof(double) * n_chains * n_steps) == hipSuccess &&
-            hipMalloc((void**)&st.scal, sizeof(double) * n_chains * 4) == hipSuccess &&
-            hipMalloc((void**)&st.k, sizeof(int) * n_chains) == hipSuccess &&
-            hipMalloc((void**)&st.active, sizeof(int) * n_chains) == hipSuccess &&
-            hipMalloc((void**)&st.act2, sizeof(int) * n_chains) == hipSuccess &&
-            hipMalloc((void**)&st.cap, sizeof(int) * n_chains) == hipSuccess &&
-            hipMalloc((void**)&st.ndone, sizeof(int) * n_chains) == hipSuccess &&
-            hipMalloc((void**)&st.stepno, sizeof(int)) == hipSuccess;
   // projections: element slices of >= 4096 entries (at most 64); updates of
   // short vectors split over ranges of basis vectors so that enough
   // work-groups run
   st.nslice = (int)std::max(1L, std::min(64L, len / 4096));
   st.jsplit = len < 32768 ? std::max(1, std::min(16, (n_steps + 1) / 32)) : 1;
   st.jchunk = (n_steps + 1 + st.jsplit - 1) / st.jsplit;
-  if (ok && st.jsplit > 1)
-    ok = hipMalloc((void**)&st.upart, sizeof(double) * n_chains * st.jsplit * len) == hipSuccess;
+  const size_t nc = n_chains, ncs = nc * n_steps;
+  Carve carve;
+  carve.add(&st.Q, nc * (n_steps + 1) * len);
+  carve.add(&st.qcur, nc * len);
+  carve.add(&st.Lq, nc * len);
+  carve.add(&st.r, nc * len);
+  carve.add(&st.mask, len);
+  carve.add(&st.part, nc * (n_steps + 1) * kRedBlocks);
+  carve.add(&st.coef, nc * (n_steps + 1));
+  carve.add(&st.a, ncs);
+  carve.add(&st.b, ncs);
+  carve.add(&st.scal, nc * 4);
+  carve.add(&st.k, nc);
+  carve.add(&st.active, nc);
+  carve.add(&st.act2, nc);
+  carve.add(&st.cap, nc);
+  carve.add(&st.ndone, nc);
+  carve.add(&st.stepno, 1);
+  if (st.jsplit > 1) carve.add(&st.upart, nc * st.jsplit * len);
+  bool ok = hipMalloc(&st.mem, carve.total()) == hipSuccess;
+  if (ok) carve.assign(st.mem);
   if (!ok) {
     free_state(st);
     set_error("tdscha_lanczos_run: device allocation failed");

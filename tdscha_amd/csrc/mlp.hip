@@ -13,6 +13,8 @@
 //   [W0 (d1 x d0), b0 (d1), W1 (d2 x d1), b1 (d2), ...], W row-major [out][in].
 #include <algorithm>
 #include <cmath>
+#include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -40,7 +42,7 @@ struct Mlp {
                                  // each layer's output; else [2] of them in turn
   float* target = nullptr;       // [max_batch][n_out] (kind 0)
   float* wout = nullptr;         // [n_out] loss weights (kind 0)
-  float* loss_part = nullptr;    // [max_batch]
+  float* loss_part = nullptr;    // [max_batch], in the pinned memory
   int* idx = nullptr;            // [max_batch] rows of the data arrays in use
   // data arrays (device): either one batch (direct calls) or a training set
   float* data_x = nullptr;       // [n][n_in]
@@ -57,6 +59,9 @@ struct Mlp {
   double* cf_part = nullptr;     // [samples x slices <= max_batch + kCfBlocks][11]
   long step = 0;                 // Adam steps taken
   bool fused = false;            // all layers of a pass in one kernel
+  char* pinned = nullptr;        // host memory the kernels access: small inputs (kPinned
+                                 // bytes), outputs (kPinned), losses (max_batch)
+  char* staged = nullptr;        // [kPinned] device copy of small inputs
   hipStream_t stream = nullptr;
 };
 
@@ -180,12 +185,12 @@ __device__ __forceinline__ void fused_layers(int steps, Sizes sizes, Weights wei
   }
 }
 
-// forward of rows idx[..] (or the rows themselves) of x; keep: store every layer's
-// pre-activations and activations, else the last layer's output only
+// forward of rows idx[..] (or the rows themselves) of x: the last layer's output to
+// y_out [B][n_out], or (null) every layer's pre-activations and activations
 template <int R>
 __global__ __launch_bounds__(kFuseThreads) void mlp_fused_fwd(
     MlpShape m, const float* __restrict__ params, const float* __restrict__ x, int xld,
-    const int* __restrict__ idx, int B, int keep, float* __restrict__ act,
+    const int* __restrict__ idx, int B, float* __restrict__ y_out, float* __restrict__ act,
     float* __restrict__ pre) {
   extern __shared__ float fsh[];
   auto ws = reinterpret_cast<float(*)[kFusePanel + 1]>(fsh);
@@ -196,7 +201,7 @@ __global__ __launch_bounds__(kFuseThreads) void mlp_fused_fwd(
     const bool in = b < B && i < m.dim[0];
     const float v = in ? x[(long)(idx ? idx[b] : b) * xld + i] : 0.f;
     xs[0][r][i] = v;
-    if (keep && in) act[(long)b * m.ld + i] = v;
+    if (!y_out && in) act[(long)b * m.ld + i] = v;
   }
   fused_layers<R, true>(
       m.layers, [&](int l) { return make_int2(m.dim[l], m.dim[l + 1]); },
@@ -206,10 +211,13 @@ __global__ __launch_bounds__(kFuseThreads) void mlp_fused_fwd(
         const float z = sum + (in ? params[m.b[l] + o] : 0.f), y = last ? z : silu(z);
         xs[(l + 1) & 1][row][o] = y;
         const int b = b0 + row;
-        if (b < B && in && (keep || last)) {
+        if (b >= B || !in) return;
+        if (!y_out) {
           const long e = (long)b * m.ld + o;
-          if (keep) pre[l * m.stride + e] = z;
+          pre[l * m.stride + e] = z;
           act[(l + 1) * m.stride + e] = y;
+        } else if (last) {
+          y_out[(long)b * m.dim[l + 1] + o] = y;
         }
       },
       xs, ws);
@@ -289,7 +297,7 @@ __global__ void __launch_bounds__(256) cf_loss_kernel(
     double* __restrict__ part) {
   __shared__ double red[kCfOut + 1][4];
   const int bi = blockIdx.x;
-  const long row = idx[bi];
+  const long row = idx ? idx[bi] : bi;
   const double* ch = chains + row * (2 * K + 2);
   const double* av = ch;
   const double* bv = ch + K;
@@ -500,10 +508,17 @@ __global__ void mlp_gather(const float* __restrict__ dx, const float* __restrict
                            float* __restrict__ x, float* __restrict__ t) {
   const int b = blockIdx.x;
   if (b >= B) return;
-  const long r = idx[b];
+  const long r = idx ? idx[b] : b;
   for (int i = threadIdx.x; i < n_in; i += blockDim.x) x[(long)b * ld + i] = dx[r * n_in + i];
   if (dt)
     for (int o = threadIdx.x; o < n_out; o += blockDim.x) t[(long)b * n_out + o] = dt[r * n_out + o];
+}
+
+// rows of stride ld to contiguous ones
+__global__ void mlp_rows(const float* __restrict__ y, int B, int n, int ld,
+                         float* __restrict__ out) {
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < (long)B * n) out[e] = y[e / n * ld + e % n];
 }
 
 static float* act_l(Mlp* m, int l) { return m->act + (long)l * m->max_batch * m->max_dim; }
@@ -538,16 +553,17 @@ static MlpShape shape(const Mlp* m) {
   return h;
 }
 
-// fused forward of rows of x (row stride xld); 4 rows to a work-group until every CU
+// fused forward of rows of x (y: see mlp_fused_fwd); 4 rows to a work-group until every CU
 // has four of them, then 8
-static void forward_fused(Mlp* m, int B, const float* x, int xld, const int* idx, int keep) {
+static void forward_fused(Mlp* m, int B, const float* x, const int* idx, float* y) {
+  const int xld = m->dims[0];
   const MlpShape h = shape(m);
   if (B <= 4096)
     hipLaunchKernelGGL(mlp_fused_fwd<4>, dim3((B + 3) / 4), dim3(kFuseThreads), fused_lds<4>(),
-                       m->stream, h, m->params, x, xld, idx, B, keep, m->act, m->pre);
+                       m->stream, h, m->params, x, xld, idx, B, y, m->act, m->pre);
   else
     hipLaunchKernelGGL(mlp_fused_fwd<8>, dim3((B + 7) / 8), dim3(kFuseThreads), fused_lds<8>(),
-                       m->stream, h, m->params, x, xld, idx, B, keep, m->act, m->pre);
+                       m->stream, h, m->params, x, xld, idx, B, y, m->act, m->pre);
 }
 
 static void backward_fused(Mlp* m, int B) {
@@ -575,8 +591,15 @@ static void forward(Mlp* m, int B) {
   }
 }
 
+// device arrays of a pass: rows idx[0 .. B) (null: the first B rows) of each
+struct MlpData {
+  const float *x = nullptr, *t = nullptr;
+  const double *ch = nullptr, *ref = nullptr;
+  const int* idx = nullptr;
+};
+
 // loss partials and the gradient with respect to the network outputs
-static void loss_head(Mlp* m, int kind, int B) {
+static void loss_head(Mlp* m, const MlpData& d, int kind, int B) {
   const int ld = m->max_dim, L = m->n_layers;
   float* dz = m->dz + (m->fused ? (long)(L - 1) * m->max_batch * ld : 0);
   if (kind == 0) {
@@ -587,7 +610,7 @@ static void loss_head(Mlp* m, int kind, int B) {
     // with one block each, 17 us in eight, and 4 us to add them)
     const int slices = std::min((m->cf_nw + 255) / 256, (kCfBlocks + B - 1) / B);
     hipLaunchKernelGGL(cf_loss_kernel, dim3(B, slices), dim3(256), 0, m->stream, act_l(m, L), ld,
-                       m->idx, m->data_ch, m->data_ref, m->cf_w, m->cf_nw, m->cf_K, m->cf_eta,
+                       d.idx, d.ch, d.ref, m->cf_w, m->cf_nw, m->cf_K, m->cf_eta,
                        m->cf_mean, m->cf_std, m->cf_part);
     hipLaunchKernelGGL(cf_loss_sum, dim3(B), dim3(64), 0, m->stream, m->cf_part, slices, m->cf_nw,
                        ld, m->cf_std, m->cf_scale / B, dz, m->loss_part);
@@ -631,49 +654,59 @@ static int ensure(T** p, long* cap, long n) {
   return 0;
 }
 
-// Upload n rows of data for the given loss kind to the device data arrays
-// (synchronous: the host arrays may be released on return).
+// Upload n rows of data for the given loss kind to the device arrays (the host arrays
+// may be released on return).  What fits goes through the pinned memory in one copy.
 static int upload_data(Mlp* m, int kind, long n, const float* x, const float* t,
-                       const double* chains, const double* ref) {
+                       const double* chains, const double* ref, MlpData* d) {
   const int n_in = m->dims[0], n_out = m->dims[m->n_layers];
   TDS_CHECK_HIP(hipStreamSynchronize(m->stream));
-  int rc = ensure(&m->data_x, &m->data_cap_x, n * n_in);
+  size_t used = 0;
+  auto place = [&](auto** dev, long* cap, const auto* host, auto** out, size_t count) -> int {
+    const size_t bytes = sizeof(*host) * count;
+    if (used + bytes <= kPinned) {
+      std::memcpy(m->pinned + used, host, bytes);
+      *out = reinterpret_cast<std::remove_reference_t<decltype(*out)>>(m->staged + used);
+      used += (bytes + 255) / 256 * 256;
+      return 0;
+    }
+    const int rc = ensure(dev, cap, (long)count);
+    if (rc) return rc;
+    TDS_CHECK_HIP(hipMemcpy(*dev, host, bytes, hipMemcpyHostToDevice));
+    *out = *dev;
+    return 0;
+  };
+  int rc = place(&m->data_x, &m->data_cap_x, x, &d->x, (size_t)n * n_in);
   if (rc) return rc;
-  TDS_CHECK_HIP(hipMemcpy(m->data_x, x, sizeof(float) * n * n_in, hipMemcpyHostToDevice));
   if (kind == 0) {
-    rc = ensure(&m->data_t, &m->data_cap_t, n * n_out);
-    if (rc) return rc;
-    TDS_CHECK_HIP(hipMemcpy(m->data_t, t, sizeof(float) * n * n_out, hipMemcpyHostToDevice));
+    rc = place(&m->data_t, &m->data_cap_t, t, &d->t, (size_t)n * n_out);
   } else {
-    const long nch = n * (2L * m->cf_K + 2), nref = n * (long)m->cf_nw;
-    rc = ensure(&m->data_ch, &m->data_cap_ch, nch);
+    rc = place(&m->data_ch, &m->data_cap_ch, chains, &d->ch, (size_t)n * (2L * m->cf_K + 2));
     if (rc) return rc;
-    rc = ensure(&m->data_ref, &m->data_cap_ref, nref);
-    if (rc) return rc;
-    TDS_CHECK_HIP(hipMemcpy(m->data_ch, chains, sizeof(double) * nch, hipMemcpyHostToDevice));
-    TDS_CHECK_HIP(hipMemcpy(m->data_ref, ref, sizeof(double) * nref, hipMemcpyHostToDevice));
+    rc = place(&m->data_ref, &m->data_cap_ref, ref, &d->ref, (size_t)n * m->cf_nw);
   }
+  if (rc) return rc;
+  if (used)
+    TDS_CHECK_HIP(hipMemcpyAsync(m->staged, m->pinned, std::min(used, kPinned),
+                                 hipMemcpyHostToDevice, m->stream));
   return 0;
 }
 
-// one minibatch: gather rows idx[0..B), forward, loss head, backward
-static void batch_pass(Mlp* m, int kind, int B) {
+// one minibatch: gather rows, forward, loss head, backward
+static void batch_pass(Mlp* m, const MlpData& d, int kind, int B) {
   const int n_in = m->dims[0], n_out = m->dims[m->n_layers];
-  if (m->fused) {
-    if (kind == 0)
-      hipLaunchKernelGGL(mlp_gather, dim3(B), dim3(128), 0, m->stream, (const float*)nullptr,
-                         m->data_t, m->idx, B, 0, n_out, m->max_dim, (float*)nullptr, m->target);
-    forward_fused(m, B, m->data_x, n_in, m->idx, 1);
-    loss_head(m, kind, B);
+  if (kind == 0 || !m->fused)
+    hipLaunchKernelGGL(mlp_gather, dim3(B), dim3(128), 0, m->stream, d.x,
+                       kind == 0 ? d.t : nullptr, d.idx, B, m->fused ? 0 : n_in, n_out,
+                       m->max_dim, act_l(m, 0), m->target);
+  if (m->fused)
+    forward_fused(m, B, d.x, d.idx, nullptr);
+  else
+    forward(m, B);
+  loss_head(m, d, kind, B);
+  if (m->fused)
     backward_fused(m, B);
-    return;
-  }
-  hipLaunchKernelGGL(mlp_gather, dim3(B), dim3(128), 0, m->stream, m->data_x,
-                     kind == 0 ? m->data_t : nullptr, m->idx, B, n_in, n_out, m->max_dim,
-                     act_l(m, 0), m->target);
-  forward(m, B);
-  loss_head(m, kind, B);
-  backward(m, B);
+  else
+    backward(m, B);
 }
 
 static int check_kind(Mlp* m, int kind, const float* t, const double* chains, const double* ref) {
@@ -687,21 +720,50 @@ static int check_kind(Mlp* m, int kind, const float* t, const double* chains, co
   return 0;
 }
 
-static int identity_idx(Mlp* m, int B) {
-  std::vector<int> id(B);
-  for (int i = 0; i < B; ++i) id[i] = i;
-  TDS_CHECK_HIP(hipMemcpy(m->idx, id.data(), sizeof(int) * B, hipMemcpyHostToDevice));
+// sum of the pass's losses (waits for the stream)
+static int read_loss(Mlp* m, int B, double* loss) {
+  TDS_CHECK_HIP(hipStreamSynchronize(m->stream));
+  double s = 0.0;
+  for (int b = 0; b < B; ++b) s += m->loss_part[b];
+  *loss = s;
   return 0;
 }
 
-static int read_loss(Mlp* m, int B, float* loss) {
-  std::vector<float> lp(B);
-  TDS_CHECK_HIP(hipMemcpyAsync(lp.data(), m->loss_part, sizeof(float) * B, hipMemcpyDeviceToHost,
-                               m->stream));
+// up to max_batch rows, contiguous on the host, through the pinned memory where they
+// fit; the kernels read and write it directly
+static int forward_start(Mlp* m, int B, const float* x, float* y) {
+  const size_t bx = sizeof(float) * B * m->dims[0], by = sizeof(float) * B * m->dims[m->n_layers];
+  const float* dx = reinterpret_cast<const float*>(m->pinned);
+  if (m->fused && bx <= kPinned) {
+    std::memcpy(m->pinned, x, bx);
+  } else {
+    const int rc = ensure(&m->data_x, &m->data_cap_x, (long)B * m->dims[0]);
+    if (rc) return rc;
+    TDS_CHECK_HIP(hipMemcpyAsync(m->data_x, x, bx, hipMemcpyHostToDevice, m->stream));
+    dx = m->data_x;
+  }
+  const bool out = by <= kPinned;
+  float* dy = out ? reinterpret_cast<float*>(m->pinned + kPinned) : m->target;
+  if (m->fused) {
+    forward_fused(m, B, dx, nullptr, dy);
+  } else {
+    hipLaunchKernelGGL(mlp_gather, dim3(B), dim3(128), 0, m->stream, dx, (const float*)nullptr,
+                       (const int*)nullptr, B, m->dims[0], 0, m->max_dim, act_l(m, 0),
+                       (float*)nullptr);
+    forward(m, B);
+    const long n = (long)B * m->dims[m->n_layers];
+    hipLaunchKernelGGL(mlp_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream,
+                       act_l(m, m->n_layers), B, m->dims[m->n_layers], m->max_dim, dy);
+  }
+  TDS_CHECK_HIP(hipGetLastError());
+  if (!out) TDS_CHECK_HIP(hipMemcpyAsync(y, dy, by, hipMemcpyDeviceToHost, m->stream));
+  return 0;
+}
+
+static int forward_end(Mlp* m, int B, float* y) {
   TDS_CHECK_HIP(hipStreamSynchronize(m->stream));
-  double s = 0.0;
-  for (float v : lp) s += v;
-  *loss = (float)s;
+  const size_t by = sizeof(float) * B * m->dims[m->n_layers];
+  if (by <= kPinned) std::memcpy(y, m->pinned + kPinned, by);
   return 0;
 }
 
@@ -753,11 +815,13 @@ int tdscha_mlp_create(tdscha_mlp** out, int n_in, int width, int n_hidden, int n
       hipMalloc((void**)&m->dz, sizeof(float) * dz_n) != hipSuccess ||
       hipMalloc((void**)&m->target, sizeof(float) * max_batch * n_out) != hipSuccess ||
       hipMalloc((void**)&m->wout, sizeof(float) * n_out) != hipSuccess ||
-      hipMalloc((void**)&m->loss_part, sizeof(float) * max_batch) != hipSuccess ||
+      hipHostMalloc((void**)&m->pinned, 2 * kPinned + sizeof(float) * max_batch) != hipSuccess ||
+      hipMalloc((void**)&m->staged, kPinned) != hipSuccess ||
       hipMalloc((void**)&m->idx, sizeof(int) * max_batch) != hipSuccess) {
     set_error("tdscha_mlp_create: device allocation failed");
     return fail();
   }
+  m->loss_part = reinterpret_cast<float*>(m->pinned + 2 * kPinned);
   // zero once so padded columns of the activations stay finite
   if (hipMemset(m->act, 0, sizeof(float) * act_n) != hipSuccess ||
       hipMemset(m->pre, 0, sizeof(float) * pre_n) != hipSuccess ||
@@ -785,11 +849,12 @@ void tdscha_mlp_destroy(tdscha_mlp* h) {
   Mlp* m = reinterpret_cast<Mlp*>(h);
   if (m->stream) hipStreamSynchronize(m->stream);
   void* ptrs[] = {m->params,  m->grads,  m->m1,      m->m2,       m->act,  m->pre,
-                  m->dz,      m->target, m->wout,    m->loss_part, m->idx, m->data_x,
+                  m->dz,      m->target, m->wout,    m->staged, m->idx, m->data_x,
                   m->data_t,  m->data_ch, m->data_ref, m->cf_w,    m->cf_mean, m->cf_std,
                   m->cf_part};
   for (void* p : ptrs)
     if (p) hipFree(p);
+  if (m->pinned) hipHostFree(m->pinned);
   if (m->stream) hipStreamDestroy(m->stream);
   delete m;
 }
@@ -859,22 +924,40 @@ int tdscha_mlp_set_cf_loss(tdscha_mlp* h, int K, int n_w, const double* w, doubl
 int tdscha_mlp_forward(tdscha_mlp* h, int batch, const float* x, float* y) {
   TDS_REQUIRE(h && x && y, 2, "tdscha_mlp_forward: NULL argument");
   TDS_REQUIRE(batch >= 0, 2, "tdscha_mlp_forward: negative batch");
-  Mlp* m = reinterpret_cast<Mlp*>(h);
-  const int n_in = m->dims[0], n_out = m->dims[m->n_layers];
-  for (int b0 = 0; b0 < batch; b0 += m->max_batch) {
-    const int B = batch - b0 < m->max_batch ? batch - b0 : m->max_batch;
-    TDS_CHECK_HIP(hipMemcpy2DAsync(act_l(m, 0), sizeof(float) * m->max_dim,
-                                   x + (long)b0 * n_in, sizeof(float) * n_in,
-                                   sizeof(float) * n_in, B, hipMemcpyHostToDevice, m->stream));
-    if (m->fused)
-      forward_fused(m, B, act_l(m, 0), m->max_dim, nullptr, 0);
-    else
-      forward(m, B);
-    TDS_CHECK_HIP(hipGetLastError());
-    TDS_CHECK_HIP(hipMemcpy2DAsync(y + (long)b0 * n_out, sizeof(float) * n_out,
-                                   act_l(m, m->n_layers), sizeof(float) * m->max_dim,
-                                   sizeof(float) * n_out, B, hipMemcpyDeviceToHost, m->stream));
-    TDS_CHECK_HIP(hipStreamSynchronize(m->stream));
+  return tdscha_mlp_forward_many(1, &h, batch, x, y);
+}
+
+int tdscha_mlp_forward_many(int n_nets, tdscha_mlp* const* nets, int batch, const float* x,
+                            float* y) {
+  TDS_REQUIRE(n_nets >= 0 && (n_nets == 0 || nets) && x && y, 2,
+              "tdscha_mlp_forward_many: NULL argument");
+  TDS_REQUIRE(batch >= 0, 2, "tdscha_mlp_forward: negative batch");
+  for (int k = 0; k < n_nets; ++k) {
+    TDS_REQUIRE(nets[k], 2, "tdscha_mlp_forward_many: NULL network");
+    const Mlp *m = reinterpret_cast<const Mlp*>(nets[k]), *f = reinterpret_cast<const Mlp*>(nets[0]);
+    TDS_REQUIRE(m->dims[0] == f->dims[0] && m->dims[m->n_layers] == f->dims[f->n_layers], 2,
+                "tdscha_mlp_forward_many: networks of different inputs or outputs");
+    for (int j = 0; j < k; ++j)
+      TDS_REQUIRE(nets[j] != nets[k], 2, "tdscha_mlp_forward_many: the same network twice");
+  }
+  // each network's rows max_batch at a time, the networks of a round side by side
+  for (int done = 0, left = n_nets ? batch : 0; left > 0;) {
+    int step = left;
+    for (int k = 0; k < n_nets; ++k)
+      step = std::min(step, reinterpret_cast<const Mlp*>(nets[k])->max_batch);
+    int rc = 0;
+    for (int pass = 0; pass < 2; ++pass)
+      for (int k = 0; k < n_nets; ++k) {
+        Mlp* m = reinterpret_cast<Mlp*>(nets[k]);
+        const long n_out = m->dims[m->n_layers];
+        float* yk = y + (k * (long)batch + done) * n_out;
+        const int r = pass ? forward_end(m, step, yk)
+                           : forward_start(m, step, x + (long)done * m->dims[0], yk);
+        if (r) rc = r;
+      }
+    if (rc) return rc;
+    done += step;
+    left -= step;
   }
   return 0;
 }
@@ -886,16 +969,18 @@ int tdscha_mlp_loss_grad(tdscha_mlp* h, int kind, int batch, const float* x, con
   TDS_REQUIRE(batch > 0 && batch <= m->max_batch, 2, "tdscha_mlp_loss_grad: batch out of range");
   int rc = check_kind(m, kind, target, chains, ref);
   if (rc) return rc;
-  rc = upload_data(m, kind, batch, x, target, chains, ref);
+  MlpData d;
+  rc = upload_data(m, kind, batch, x, target, chains, ref, &d);
   if (rc) return rc;
-  rc = identity_idx(m, batch);
-  if (rc) return rc;
-  batch_pass(m, kind, batch);
+  batch_pass(m, d, kind, batch);
   TDS_CHECK_HIP(hipGetLastError());
   if (grad)
     TDS_CHECK_HIP(hipMemcpyAsync(grad, m->grads, sizeof(float) * m->n_params,
                                  hipMemcpyDeviceToHost, m->stream));
-  return read_loss(m, batch, loss);
+  double sum = 0.0;
+  rc = read_loss(m, batch, &sum);
+  if (!rc) *loss = (float)sum;
+  return rc;
 }
 
 int tdscha_mlp_adam_step(tdscha_mlp* h, int kind, int batch, const float* x, const float* target,
@@ -906,16 +991,16 @@ int tdscha_mlp_adam_step(tdscha_mlp* h, int kind, int batch, const float* x, con
   TDS_REQUIRE(batch > 0 && batch <= m->max_batch, 2, "tdscha_mlp_adam_step: batch out of range");
   int rc = check_kind(m, kind, target, chains, ref);
   if (rc) return rc;
-  rc = upload_data(m, kind, batch, x, target, chains, ref);
+  MlpData d;
+  rc = upload_data(m, kind, batch, x, target, chains, ref, &d);
   if (rc) return rc;
-  rc = identity_idx(m, batch);
-  if (rc) return rc;
-  batch_pass(m, kind, batch);
+  batch_pass(m, d, kind, batch);
   adam(m, lr, beta1, beta2, eps);
   TDS_CHECK_HIP(hipGetLastError());
-  if (loss) return read_loss(m, batch, loss);
-  TDS_CHECK_HIP(hipStreamSynchronize(m->stream));
-  return 0;
+  double sum = 0.0;
+  rc = read_loss(m, batch, &sum);
+  if (!rc && loss) *loss = (float)sum;
+  return rc;
 }
 
 int tdscha_mlp_train(tdscha_mlp* h, int kind, long n_samples, const float* x, const float* target,
@@ -929,8 +1014,10 @@ int tdscha_mlp_train(tdscha_mlp* h, int kind, long n_samples, const float* x, co
               2, "tdscha_mlp_train: need 0 < batch <= max_batch, batch <= n_samples, epochs > 0");
   int rc = check_kind(m, kind, target, chains, ref);
   if (rc) return rc;
-  rc = upload_data(m, kind, n_samples, x, target, chains, ref);
+  MlpData d;
+  rc = upload_data(m, kind, n_samples, x, target, chains, ref, &d);
   if (rc) return rc;
+  d.idx = m->idx;
   // per-epoch permutation on the host (splitmix64-driven Fisher-Yates); the
   // last n_samples % batch rows of each permutation sit the epoch out
   std::vector<int> perm(n_samples);
@@ -943,7 +1030,6 @@ int tdscha_mlp_train(tdscha_mlp* h, int kind, long n_samples, const float* x, co
     return z ^ (z >> 31);
   };
   const long n_batches = n_samples / batch;
-  std::vector<float> lp(batch);
   for (int ep = 0; ep < epochs; ++ep) {
     for (long i = 0; i < n_samples; ++i) perm[i] = (int)i;
     for (long i = n_samples - 1; i > 0; --i) {
@@ -956,14 +1042,14 @@ int tdscha_mlp_train(tdscha_mlp* h, int kind, long n_samples, const float* x, co
     for (long bi = 0; bi < n_batches; ++bi) {
       TDS_CHECK_HIP(hipMemcpyAsync(m->idx, perm.data() + bi * batch, sizeof(int) * batch,
                                    hipMemcpyHostToDevice, m->stream));
-      batch_pass(m, kind, batch);
+      batch_pass(m, d, kind, batch);
       adam(m, lr, beta1, beta2, eps);
       // one synchronisation per batch, which also keeps the pageable index
       // upload from racing the next permutation
-      TDS_CHECK_HIP(hipMemcpyAsync(lp.data(), m->loss_part, sizeof(float) * batch,
-                                   hipMemcpyDeviceToHost, m->stream));
-      TDS_CHECK_HIP(hipStreamSynchronize(m->stream));
-      for (float v : lp) ep_loss += v;
+      double sum = 0.0;
+      rc = read_loss(m, batch, &sum);
+      if (rc) return rc;
+      ep_loss += sum;
     }
     TDS_CHECK_HIP(hipGetLastError());
     if (epoch_loss) epoch_loss[ep] = (float)(ep_loss / n_batches);

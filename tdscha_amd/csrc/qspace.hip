@@ -30,7 +30,9 @@
 // All sums are fixed-order trees or loops: results do not depend on timing.
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -67,10 +69,22 @@ struct QCtx {
   int d2v_chunk = 0;        // configurations per workgroup of q_d2v (0 = automatic)
   int reorth_jtile = 16;    // basis vectors per workgroup of the reorthogonalisation dots
   hipStream_t stream = nullptr;
+  // device and pinned memory of a batch, kept for the next call (as large as the
+  // largest batch so far); `busy` while a batch uses it, another batch at that time
+  // allocates its own
+  void* work = nullptr;
+  void* pinned = nullptr;
+  size_t work_size = 0, pinned_size = 0;
+  std::atomic<bool> busy{false};
 };
 
 // Chain tables and work buffers of one batch.
 struct QBatch {
+  QCtx* owner = nullptr;    // whose kept memory this batch uses
+  void* mem = nullptr;      // or its own
+  double2* psi = nullptr;   // [C][ld] input and output of a single application
+  double2* out = nullptr;
+  double2* host = nullptr;  // pinned, [C][ld] (with psi)
   int C = 0, MP = 0, maxp = 0, ld = 0, nch = 1, ntile = 1;
   std::vector<int> h_len, h_np;
   int* iqp = nullptr;       // [C]
@@ -767,12 +781,54 @@ __global__ void q_expand(const double2* __restrict__ X, const double2* __restric
 
 // ------------------------------------------------------------ batch setup
 static void free_batch(QBatch& b) {
-  void* p[] = {b.iqp,   b.npairs, b.pq1, b.pq2, b.offa, b.offb,  b.partner, b.apair,
-               b.aorient, b.active, b.alpha, b.R1, b.wc,  b.wd,   b.fpart, b.dpart,
-               b.items, b.blk_start};
-  for (void* x : p)
-    if (x) (void)hipFree(x);
+  if (b.owner) {
+    (void)hipStreamSynchronize(b.owner->stream);   // (a failed run may still use it)
+    b.owner->busy.store(false, std::memory_order_release);
+  } else {
+    if (b.mem) (void)hipFree(b.mem);
+    if (b.host) (void)hipHostFree(b.host);
+  }
   b = QBatch();
+}
+
+// device memory of `size` bytes and pinned memory of `host` bytes for a batch: the
+// context's, if no other batch has it, else its own
+static bool take_memory(QCtx* q, size_t size, size_t host, QBatch& b) {
+  void *mem = nullptr, *pin = nullptr;
+  if (!q->busy.exchange(true, std::memory_order_acquire)) {
+    b.owner = q;
+    if (q->work_size < size) {
+      if (q->work) (void)hipFree(q->work);
+      q->work_size = 0;
+      q->work = nullptr;
+      if (hipMalloc(&q->work, size) != hipSuccess) {
+        q->work = nullptr;
+        return false;
+      }
+      q->work_size = size;
+    }
+    if (q->pinned_size < host) {
+      if (q->pinned) (void)hipHostFree(q->pinned);
+      q->pinned_size = 0;
+      q->pinned = nullptr;
+      if (hipHostMalloc(&q->pinned, host) != hipSuccess) {
+        q->pinned = nullptr;
+        return false;
+      }
+      q->pinned_size = host;
+    }
+    mem = q->work;
+    pin = q->pinned;
+  } else {
+    if (hipMalloc(&mem, size) != hipSuccess) return false;
+    if (host && hipHostMalloc(&pin, host) != hipSuccess) {
+      (void)hipFree(mem);
+      return false;
+    }
+  }
+  b.mem = mem;
+  b.host = host ? static_cast<double2*>(pin) : nullptr;
+  return true;
 }
 
 static int choose_chunk(const QCtx* q, int C, int MP_used) {
@@ -856,7 +912,7 @@ static int slab_chunk(const QCtx* q, int n_item_blocks, int rounds) {
 
 // Host tables from the pair maps; ld_min forces a minimum stride.
 static int build_batch(QCtx* q, int C, const int* iq_pert, const int* pair_map, QBatch& b,
-                       int ld_min = 0, bool static_layout = false) {
+                       int ld_min = 0, bool static_layout = false, bool with_psi = false) {
   const int nq = q->nq, nb = q->nb;
   b.C = C;
   b.MP = nq;
@@ -944,46 +1000,52 @@ static int build_batch(QCtx* q, int C, const int* iq_pert, const int* pair_map, 
   b.nch = (q->N + chunk - 1) / chunk;
   b.chunk = chunk;
   const size_t nbb = (size_t)nb * nb;
-  bool ok = hipMalloc((void**)&b.iqp, sizeof(int) * C) == hipSuccess &&
-            hipMalloc((void**)&b.npairs, sizeof(int) * C) == hipSuccess &&
-            hipMalloc((void**)&b.pq1, sizeof(int) * C * nq) == hipSuccess &&
-            hipMalloc((void**)&b.pq2, sizeof(int) * C * nq) == hipSuccess &&
-            hipMalloc((void**)&b.offa, sizeof(int) * C * nq) == hipSuccess &&
-            hipMalloc((void**)&b.offb, sizeof(int) * C * nq) == hipSuccess &&
-            hipMalloc((void**)&b.partner, sizeof(int) * C * nq) == hipSuccess &&
-            hipMalloc((void**)&b.apair, sizeof(int) * C * nq) == hipSuccess &&
-            hipMalloc((void**)&b.aorient, sizeof(int) * C * nq) == hipSuccess &&
-            hipMalloc((void**)&b.active, sizeof(int) * C) == hipSuccess &&
-            hipMalloc((void**)&b.alpha, sizeof(double2) * C * nq * nbb) == hipSuccess &&
-            hipMalloc((void**)&b.R1, sizeof(double2) * C * nb) == hipSuccess &&
-            hipMalloc((void**)&b.wc, sizeof(double2) * (size_t)C * q->N) == hipSuccess &&
-            hipMalloc((void**)&b.wd, sizeof(double2) * (size_t)C * q->N) == hipSuccess &&
-            hipMalloc((void**)&b.fpart, sizeof(double2) * (size_t)C * b.ntile * nb) == hipSuccess &&
-            hipMalloc((void**)&b.dpart, sizeof(double2) * (size_t)C * nq * b.nch * nbb) == hipSuccess &&
-            (!b.slabT ||
-             (hipMalloc((void**)&b.items, sizeof(int4) * (size_t)b.n_items) == hipSuccess &&
-              hipMalloc((void**)&b.blk_start, sizeof(int) * (size_t)(b.nib + 1)) == hipSuccess));
-  if (!ok) {
+  // one allocation; the tables first, uploaded by one copy
+  Carve carve;
+  std::vector<std::pair<const void*, size_t>> tables;
+  auto table = [&](auto** p, const auto& v) {
+    carve.add(p, v.size());
+    tables.push_back({v.data(), sizeof(v[0]) * v.size()});
+  };
+  const std::vector<int> ones(C, 1);
+  table(&b.iqp, h_iqp);
+  table(&b.npairs, h_np);
+  table(&b.pq1, h_pq1);
+  table(&b.pq2, h_pq2);
+  table(&b.offa, h_offa);
+  table(&b.offb, h_offb);
+  table(&b.partner, h_part);
+  table(&b.apair, h_apair);
+  table(&b.aorient, h_orient);
+  table(&b.active, ones);
+  if (b.slabT) {
+    table(&b.items, h_items);
+    table(&b.blk_start, h_bs);
+  }
+  std::vector<char> packed(carve.total());
+  carve.add(&b.alpha, (size_t)C * nq * nbb);
+  carve.add(&b.R1, (size_t)C * nb);
+  carve.add(&b.wc, (size_t)C * q->N);
+  carve.add(&b.wd, (size_t)C * q->N);
+  carve.add(&b.fpart, (size_t)C * b.ntile * nb);
+  carve.add(&b.dpart, (size_t)C * nq * b.nch * nbb);
+  if (with_psi) {
+    carve.add(&b.psi, (size_t)C * b.ld);
+    carve.add(&b.out, (size_t)C * b.ld);
+  }
+  if (!take_memory(q, carve.total(), with_psi ? sizeof(double2) * C * b.ld : 0, b)) {
     free_batch(b);
     set_error("q-space: device allocation failed");
     return -1;
   }
-  std::vector<int> ones(C, 1);
-  ok = hipMemcpy(b.iqp, h_iqp.data(), sizeof(int) * C, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.npairs, h_np.data(), sizeof(int) * C, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.pq1, h_pq1.data(), sizeof(int) * C * nq, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.pq2, h_pq2.data(), sizeof(int) * C * nq, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.offa, h_offa.data(), sizeof(int) * C * nq, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.offb, h_offb.data(), sizeof(int) * C * nq, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.partner, h_part.data(), sizeof(int) * C * nq, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.apair, h_apair.data(), sizeof(int) * C * nq, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.aorient, h_orient.data(), sizeof(int) * C * nq, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(b.active, ones.data(), sizeof(int) * C, hipMemcpyHostToDevice) == hipSuccess &&
-       (!b.slabT ||
-        (hipMemcpy(b.items, h_items.data(), sizeof(int4) * (size_t)b.n_items,
-                   hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(b.blk_start, h_bs.data(), sizeof(int) * (size_t)(b.nib + 1),
-                   hipMemcpyHostToDevice) == hipSuccess));
+  carve.assign(b.mem);
+  size_t at = 0;
+  for (const auto& t : tables) {
+    std::memcpy(packed.data() + at, t.first, t.second);
+    at += (t.second + 255) / 256 * 256;
+  }
+  const bool ok =
+      hipMemcpy(b.mem, packed.data(), packed.size(), hipMemcpyHostToDevice) == hipSuccess;
   if (!ok) {
     free_batch(b);
     set_error("q-space: table upload failed");
@@ -1048,6 +1110,7 @@ static void launch_L(QCtx* q, QBatch& b, const double2* psi, double2* out, int i
 // ------------------------------------------------------- Hermitian Lanczos
 struct QLanczos {
   int kmax = 0;
+  void* mem = nullptr;      // the arrays below
   double2* Q = nullptr;     // [C][kmax+1][ld]
   double2* qcur = nullptr;  // [C][ld]
   double2* Lq = nullptr;
@@ -1066,10 +1129,7 @@ struct QLanczos {
 };
 
 static void free_ql(QLanczos& l) {
-  void* p[] = {l.Q, l.qcur, l.Lq, l.r, l.mask, l.coef, l.a, l.bb, l.cc, l.scal, l.k, l.cont,
-               l.nextc, l.cap, l.ndone};
-  for (void* x : p)
-    if (x) (void)hipFree(x);
+  if (l.mem) (void)hipFree(l.mem);
   l = QLanczos();
 }
 
@@ -1575,9 +1635,10 @@ void tdscha_qctx_destroy(tdscha_qctx* ctx) {
   if (!ctx) return;
   QCtx* q = reinterpret_cast<QCtx*>(ctx);
   if (q->stream) (void)hipStreamSynchronize(q->stream);
-  void* p[] = {q->X, q->Y, q->rho, q->wq, q->nbose, q->valid, q->fY, q->fP, q->S};
+  void* p[] = {q->X, q->Y, q->rho, q->wq, q->nbose, q->valid, q->fY, q->fP, q->S, q->work};
   for (void* x : p)
     if (x) (void)hipFree(x);
+  if (q->pinned) (void)hipHostFree(q->pinned);
   if (q->stream) (void)hipStreamDestroy(q->stream);
   delete q;
 }
@@ -1744,42 +1805,35 @@ static int apply_L_host(tdscha_qctx* ctx, int n_chains, const int* iq_pert,
   TDS_REQUIRE(n_chains >= 1 && n_chains <= kQMaxChains, 2, "n_chains must be in [1, 256]");
   QCtx* q = reinterpret_cast<QCtx*>(ctx);
   QBatch b;
-  int rc = build_batch(q, n_chains, iq_pert, q_pair_map, b, 0, static_op);
+  int rc = build_batch(q, n_chains, iq_pert, q_pair_map, b, 0, static_op, true);
   if (rc) return rc;
   const int C = n_chains, ld = b.ld;
-  double2 *dpsi = nullptr, *dout = nullptr;
-  std::vector<double2> hp((size_t)C * ld, make_double2(0.0, 0.0));
+  const size_t bytes = sizeof(double2) * C * ld;
   long pos = 0;
   for (int c = 0; c < C; ++c) {
-    for (int e = 0; e < b.h_len[c]; ++e)
-      hp[(size_t)c * ld + e] = make_double2(psi[2 * (pos + e)], psi[2 * (pos + e) + 1]);
-    pos += b.h_len[c];
+    const int len = b.h_len[c];
+    std::memcpy(b.host + (size_t)c * ld, psi + 2 * pos, sizeof(double2) * len);
+    std::fill(b.host + (size_t)c * ld + len, b.host + (size_t)(c + 1) * ld,
+              make_double2(0.0, 0.0));
+    pos += len;
   }
   hipStream_t s = q->stream;
-  bool ok = hipMalloc((void**)&dpsi, sizeof(double2) * C * ld) == hipSuccess &&
-            hipMalloc((void**)&dout, sizeof(double2) * C * ld) == hipSuccess &&
-            hipMemcpy(dpsi, hp.data(), sizeof(double2) * C * ld, hipMemcpyHostToDevice) == hipSuccess &&
-            hipMemset(dout, 0, sizeof(double2) * C * ld) == hipSuccess;
+  bool ok = hipMemcpyAsync(b.psi, b.host, bytes, hipMemcpyHostToDevice, s) == hipSuccess;
   if (ok) {
-    launch_L(q, b, dpsi, dout, ignore_harmonic, ignore_v3, ignore_v4, s, static_op);
-    ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess &&
-         hipMemcpy(hp.data(), dout, sizeof(double2) * C * ld, hipMemcpyDeviceToHost) == hipSuccess;
+    launch_L(q, b, b.psi, b.out, ignore_harmonic, ignore_v3, ignore_v4, s, static_op);
+    ok = hipGetLastError() == hipSuccess &&
+         hipMemcpyAsync(b.host, b.out, bytes, hipMemcpyDeviceToHost, s) == hipSuccess &&
+         hipStreamSynchronize(s) == hipSuccess;
   }
-  if (dpsi) (void)hipFree(dpsi);
-  if (dout) (void)hipFree(dout);
-  const std::vector<int> lens = b.h_len;
+  pos = 0;
+  for (int c = 0; ok && c < C; ++c) {
+    std::memcpy(out + 2 * pos, b.host + (size_t)c * ld, sizeof(double2) * b.h_len[c]);
+    pos += b.h_len[c];
+  }
   free_batch(b);
   if (!ok) {
     set_error("tdscha_qspace_apply_L: device execution failed");
     return -1;
-  }
-  pos = 0;
-  for (int c = 0; c < C; ++c) {
-    for (int e = 0; e < lens[c]; ++e) {
-      out[2 * (pos + e)] = hp[(size_t)c * ld + e].x;
-      out[2 * (pos + e) + 1] = hp[(size_t)c * ld + e].y;
-    }
-    pos += lens[c];
   }
   return 0;
 }
@@ -1801,21 +1855,25 @@ int tdscha_qspace_lanczos_run(tdscha_qctx* ctx, int n_chains, const int* iq_pert
   QLanczos l;
   l.kmax = kmax;
   const size_t qn = (size_t)C * (kmax + 1) * ld;
-  bool ok = hipMalloc((void**)&l.Q, sizeof(double2) * qn) == hipSuccess &&
-            hipMalloc((void**)&l.qcur, sizeof(double2) * C * ld) == hipSuccess &&
-            hipMalloc((void**)&l.Lq, sizeof(double2) * C * ld) == hipSuccess &&
-            hipMalloc((void**)&l.r, sizeof(double2) * C * ld) == hipSuccess &&
-            hipMalloc((void**)&l.mask, sizeof(double) * C * ld) == hipSuccess &&
-            hipMalloc((void**)&l.coef, sizeof(double) * C * (kmax + 1)) == hipSuccess &&
-            hipMalloc((void**)&l.a, sizeof(double) * C * kmax) == hipSuccess &&
-            hipMalloc((void**)&l.bb, sizeof(double) * C * kmax) == hipSuccess &&
-            hipMalloc((void**)&l.cc, sizeof(double) * C * kmax) == hipSuccess &&
-            hipMalloc((void**)&l.scal, sizeof(double) * C * 4) == hipSuccess &&
-            hipMalloc((void**)&l.k, sizeof(int) * C) == hipSuccess &&
-            hipMalloc((void**)&l.cont, sizeof(int) * C) == hipSuccess &&
-            hipMalloc((void**)&l.nextc, sizeof(int) * C) == hipSuccess &&
-            hipMalloc((void**)&l.cap, sizeof(int) * C) == hipSuccess &&
-            hipMalloc((void**)&l.ndone, sizeof(int) * C) == hipSuccess;
+  Carve carve;   // l.Lq to l.cc start from zero, with one fill
+  carve.add(&l.Q, qn);
+  carve.add(&l.Lq, (size_t)C * ld);
+  carve.add(&l.a, (size_t)C * kmax);
+  carve.add(&l.bb, (size_t)C * kmax);
+  carve.add(&l.cc, (size_t)C * kmax);
+  const size_t zeroed = carve.total();
+  carve.add(&l.qcur, (size_t)C * ld);
+  carve.add(&l.r, (size_t)C * ld);
+  carve.add(&l.mask, (size_t)C * ld);
+  carve.add(&l.coef, (size_t)C * (kmax + 1));
+  carve.add(&l.scal, (size_t)C * 4);
+  carve.add(&l.k, C);
+  carve.add(&l.cont, C);
+  carve.add(&l.nextc, C);
+  carve.add(&l.cap, C);
+  carve.add(&l.ndone, C);
+  bool ok = hipMalloc(&l.mem, carve.total()) == hipSuccess;
+  if (ok) carve.assign(l.mem);
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1846,11 +1904,7 @@ int tdscha_qspace_lanczos_run(tdscha_qctx* ctx, int n_chains, const int* iq_pert
   ok = hipMemcpy(l.r, hp.data(), sizeof(double2) * C * ld, hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(l.mask, hm.data(), sizeof(double) * C * ld, hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(l.cap, hcap.data(), sizeof(int) * C, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemset(l.Q, 0, sizeof(double2) * qn) == hipSuccess &&
-       hipMemset(l.Lq, 0, sizeof(double2) * C * ld) == hipSuccess &&
-       hipMemset(l.a, 0, sizeof(double) * C * kmax) == hipSuccess &&
-       hipMemset(l.bb, 0, sizeof(double) * C * kmax) == hipSuccess &&
-       hipMemset(l.cc, 0, sizeof(double) * C * kmax) == hipSuccess;
+       hipMemset(l.mem, 0, zeroed) == hipSuccess;
   if (!ok) return fail("upload failed");
   hipLaunchKernelGGL(q_fill_int, dim3((C + 63) / 64), dim3(64), 0, s, l.k, C, 0);
   hipLaunchKernelGGL(q_fill_int, dim3((C + 63) / 64), dim3(64), 0, s, l.cont, C, 1);

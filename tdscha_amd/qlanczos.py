@@ -71,11 +71,23 @@ class QSpaceEngine:
                    "tdscha_qspace_psi_size")
         return n.value
 
+    def _psi_sizes(self, pms):
+        """psi_size of every row of pms, or None where a row is no pair map."""
+        q = np.arange(self.n_q)
+        if pms.shape[1:] != (self.n_q,) or np.any((pms < 0) | (pms >= self.n_q)):
+            return None
+        if np.any(np.take_along_axis(pms, pms, 1) != q):
+            return None
+        nb = self.n_bands
+        return (nb + 2 * nb * nb * np.sum(q < pms, axis=1)
+                + nb * (nb + 1) * np.sum(q == pms, axis=1))
+
     def _check_lengths(self, pms, psis):
         if len(psis) != len(pms):
             raise ValueError("one pair map and one psi per chain")
+        sizes = self._psi_sizes(pms)
         for i, p in enumerate(psis):
-            n = self.psi_size(pms[i])
+            n = self.psi_size(pms[i]) if sizes is None else sizes[i]
             if len(p) != n:
                 raise ValueError("chain %d: psi of %d entries, its layout has %d"
                                  % (i, len(p), n))

@@ -197,6 +197,17 @@ class Network:
             pass
 
 
+def forward_many(nets, x):
+    """Outputs (M, n, n_out) of M networks of one shape for the same rows, the
+    networks side by side on the device."""
+    x = np.atleast_2d(np.ascontiguousarray(x, dtype=np.float32))
+    y = np.empty((len(nets), x.shape[0], nets[0].shape[3]), np.float32)
+    h = (C.c_void_p * len(nets))(*[n.h for n in nets])
+    _lib.check(_lib.lib().tdscha_mlp_forward_many(len(nets), h, x.shape[0], _p(x), _p(y)),
+               "tdscha_mlp_forward_many")
+    return y
+
+
 class LearnedTerminator:
     """Ensemble of tail-predicting networks plus the normalisation they need.
 
@@ -250,7 +261,8 @@ class LearnedTerminator:
         """Tail parameters (n, 10) in units of |b_0| (ensemble mean) and the
         ensemble variance of the standardised asymptote (n,)."""
         x = self.standardise(a, b)
-        zs = np.array([net.forward(x) for net in self.nets()], np.float64)   # (M, n, 10)
+        nets = self.nets()
+        zs = (forward_many(nets, x) if nets else np.array([])).astype(np.float64)   # (M, n, 10)
         p = self.out_mean + self.out_std * zs.mean(0)
         var = zs[:, :, :2].var(0).mean(1) if len(zs) > 1 else np.zeros(len(x))
         return p, var
