@@ -126,6 +126,7 @@ constexpr double kOrbWorthUs = 500.0;
 
 struct OrbPlan {
   bool ok = false;
+  int prec = 0;            // of its averages
   int nc = 0, npairs = 0;
   struct Round {
     int chain0, chains, first, count;
@@ -138,6 +139,8 @@ struct OrbPlan {
   int2 *pairs = nullptr, *clean = nullptr;
   double* C = nullptr;
 };
+
+struct Ctx;
 
 struct Orbit {
   bool usable = false;     // tables built
@@ -158,6 +161,9 @@ struct Orbit {
   double *R1 = nullptr, *Y1 = nullptr;    // [kOrbPairs, np(, np)] rotated inputs
   double *Rb = nullptr, *Yb = nullptr;    // [2 kMaxChains, np(, np)] unpacked vectors
   double *coef = nullptr, *zpart = nullptr, *fpart = nullptr, *z = nullptr, *f = nullptr;
+  // the configurations as a context of their own, with what the split precisions need
+  // (made at the first plan in one of them); its inputs and outputs are set per pass
+  Ctx* sub = nullptr;
   OrbPlan plan[1];                        // of the synchronous entries
 };
 

@@ -18,6 +18,7 @@ __global__ void expand_images(const double*, const double*, const double*, const
                               int, int, long, double*, double*, double*);
 int launch_pa_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev);
 int launch_pa_split(Ctx* c, int nc, int apply_d4, int prec, hipStream_t s, hipEvent_t* ev);
+void free_split(Ctx* c);
 int set_ksplit_split(Ctx* c, int ks);
 int default_ksplit_split(Ctx* c);
 int rot_setup(Ctx* c, const double* X_dev, const double* Y_dev, const double* rho_dev);
@@ -363,21 +364,16 @@ void tdscha_ctx_destroy(tdscha_ctx* ctx) {
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   if (c->stream) hipStreamSynchronize(c->stream);
   void* ptrs[] = {c->U, c->F, c->rho_img, c->fy, c->fpsi, c->w, c->R1, c->Y1, c->coef, c->zpart,
-                  c->fpart, c->f_out, c->d2v_out, c->Y1h, c->Y1l, c->ysc, c->ysc3, c->bsc, c->cmax,
+                  c->fpart, c->f_out, c->d2v_out, c->bsc,
                   c->pair_ca, c->pair_cb, c->pair_sm, c->pair_sp, c->pair_harm_a, c->pair_harm_b,
                   c->pair_row, c->pair_col, c->std_coef, c->inv_coef, c->yw, c->reaw, c->pols, c->inv_perms, c->rep_dof, c->jrep, c->ju, c->rep_sum,
                   c->tproj, c->cart_tmp, c->cart_tmp2, c->mode_tmp, c->psi_dev, c->psi_out_dev,
-                  c->stage_in, c->stage_out, c->f_fin, c->d2v_fin, c->f_proj, c->epi,
-                  c->coef32, c->wpart, c->zpart32, c->fpart_s, c->sbsc, c->pmax,
+                  c->stage_in, c->stage_out, c->f_fin, c->d2v_fin, c->f_proj,
                   c->rt_cols, c->rt_d, c->rt_bs, c->rt_pstart, c->rt_sr, c->rt_sc, c->R1_base, c->Y1_base, c->rot_t1,
                   c->rot_t2, c->rot_f};
   for (void* p : ptrs)
     if (p) hipFree(p);
-  for (auto& s : c->split) {
-    void* sp[] = {s.Uh, s.Ul, s.FA, s.UA32, s.UhT, s.UlT, s.XT, s.YT, s.su, s.sf, s.umax, s.fmax, s.colw};
-    for (void* p : sp)
-      if (p) hipFree(p);
-  }
+  free_split(c);
   if (c->pinned) (void)hipHostFree(c->pinned);
   orbit_free(c);
   if (c->stream) hipStreamDestroy(c->stream);

@@ -47,6 +47,9 @@ __global__ void expand_images(const double*, const double*, const double*, const
                               int, int, long, double*, double*, double*);
 __global__ void rot_copy_configs(const double* X, const double* Y, const double* rho, int n, int np,
                                  long N, long Mp, double* U, double* F, double* rho_img);
+int ensure_split(Ctx* c, int prec);
+void free_split(Ctx* c);
+int launch_pa_split(Ctx* c, int nc, int apply_d4, int prec, hipStream_t s, hipEvent_t* ev);
 int rot_panels(const int* bs, const int* d, int n, int np, int* start, int* nreal);
 
 constexpr int kOP = 32;          // modes of a panel (whole blocks)
@@ -655,6 +658,10 @@ int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const in
 
 void orbit_free(Ctx* c) {
   Orbit& o = c->orb;
+  if (o.sub) {
+    free_split(o.sub);
+    delete o.sub;   // (its rows, inputs and outputs belong to this struct)
+  }
   if (o.arena) (void)hipFree(o.arena);
   if (o.work) (void)hipFree(o.work);
   if (o.pout) (void)hipHostFree(o.pout);
@@ -810,6 +817,35 @@ bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld) {
   return true;
 }
 
+// the split images of the configurations; false = no room
+static bool split_ready(Ctx* c, int prec) {
+  Orbit& o = c->orb;
+  if (!o.sub) {
+    Ctx* s = new Ctx();
+    s->device = c->device;
+    s->stream = c->stream;
+    s->n = c->n;
+    s->np = c->np;
+    s->N = c->N;
+    s->n_syms = 1;
+    s->M = c->N;
+    s->Mp = o.Mp;
+    s->n_eff = c->n_eff;
+    s->row_lo = 0;
+    s->row_hi = c->N;
+    s->U = o.U;
+    s->F = o.F;
+    s->rho_img = o.rho;
+    s->fy = c->fy;
+    s->fpsi = c->fpsi;
+    o.sub = s;
+  }
+  if (ensure_split(o.sub, prec) == 0) return true;
+  (void)hipGetLastError();
+  free_split(o.sub);
+  return false;
+}
+
 // Plan of nc chains whose padded inputs are in c->R1, c->Y1 (waits for the
 // stream): p.ok false = use the general form.
 int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p) {
@@ -846,8 +882,10 @@ int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p) {
     Call.insert(Call.end(), C.begin(), C.end());
   }
   const double full = estimate_us(nc * pass_flop(c, (double)c->N * ns), prec);
-  const double orb = estimate_us(pairs.size() * pass_flop(c, c->N), PREC_FP64) + 150.0;
+  const double orb = estimate_us(pairs.size() * pass_flop(c, c->N), prec) + 200.0;
   if (orb > 0.8 * full) return 0;
+  if (prec != PREC_FP64 && !split_ready(c, prec)) return 0;
+  p.prec = prec;
   p.nc = nc;
   p.npairs = (int)pairs.size();
   // rounds of the clean-up: whole chains, at most kOrbPairs pairs each
@@ -906,13 +944,28 @@ int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* 
   const OrbPanels pn = panels(c);
   hipLaunchKernelGGL(orb_in, dim3(o.npanel * o.npanel, P), dim3(256), 0, s, pn, p.pairs, c->Y1,
                      c->R1, np, (const int*)nullptr, 0, o.Y1, o.R1);
-  const F64Rows rows{o.U, o.F, o.rho, o.Mp};
-  launch_weights_f64(rows, n, np, P, o.Y1, o.R1, c->fy, c->fpsi, apply_d4, 0,
-                     (c->N + 63) / 64, 0, c->N, o.coef, s);
-  const long ke = round_up_l(c->N, 8);
-  launch_outer_f64(rows, n, np, P, o.coef, c->fy, ks, 0, ke, round_up_l((ke + ks - 1) / ks, 8), 0,
-                   o.zpart, o.fpart, s);
-  launch_reduce_f64(n, np, P, ks, o.zpart, o.fpart, o.z, o.f, 1.0 / c->n_eff, s);
+  if (p.prec != PREC_FP64) {
+    // the split kernels on the configurations, in groups of 6 pairs (they take three
+    // at a time).  128 atoms x 20000, 9 pairs: 0.40 ms for 2.0 in FP64; against FP64
+    // results the error is below that of the split average over the images (d2v
+    // 1e-7 for 7e-7 in FP16x2, 1.3e-6 for 1.5e-6 in BF16x2 at 12000 configurations)
+    for (int p0 = 0; p0 < P; p0 += 6) {
+      o.sub->R1 = o.R1 + (long)p0 * np;
+      o.sub->Y1 = o.Y1 + (long)p0 * np * np;
+      o.sub->f_out = o.f + (long)p0 * np;
+      o.sub->d2v_out = o.z + (long)p0 * np * np;
+      const int rc = launch_pa_split(o.sub, std::min(6, P - p0), apply_d4, p.prec, s, nullptr);
+      if (rc) return rc;
+    }
+  } else {
+    const F64Rows rows{o.U, o.F, o.rho, o.Mp};
+    launch_weights_f64(rows, n, np, P, o.Y1, o.R1, c->fy, c->fpsi, apply_d4, 0, (c->N + 63) / 64,
+                       0, c->N, o.coef, s);
+    const long ke = round_up_l(c->N, 8);
+    launch_outer_f64(rows, n, np, P, o.coef, c->fy, ks, 0, ke, round_up_l((ke + ks - 1) / ks, 8),
+                     0, o.zpart, o.fpart, s);
+    launch_reduce_f64(n, np, P, ks, o.zpart, o.fpart, o.z, o.f, 1.0 / c->n_eff, s);
+  }
   hipLaunchKernelGGL(orb_out<true>, dim3(o.npanel * (o.npanel + 1) / 2, p.nc), dim3(512), 0, s, pn,
                      p.mats, p.C, o.z, o.f, c->fy, n, np, 1.0 / o.nsym,
                      1.0 / (c->n_eff * o.nsym), (const int*)nullptr, 0, (const int*)nullptr, f_dev,

@@ -1006,6 +1006,25 @@ int ensure_split(Ctx* c, int prec) {
   return 0;
 }
 
+// the split images and workspaces of every precision
+void free_split(Ctx* c) {
+  auto drop = [](auto** p) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+  };
+  for (SplitStore& s : c->split) {
+    for (void** p : {&s.Uh, &s.Ul, &s.UhT, &s.UlT}) drop(p);
+    for (float** p : {&s.FA, &s.UA32, &s.XT, &s.YT, &s.colw}) drop(p);
+    for (double** p : {&s.su, &s.sf, &s.umax, &s.fmax}) drop(p);
+    s.ready = false;
+  }
+  drop(&c->Y1h);
+  drop(&c->Y1l);
+  for (float** p : {&c->epi, &c->coef32, &c->zpart32}) drop(p);
+  for (double** p : {&c->ysc, &c->ysc3, &c->cmax, &c->pmax, &c->wpart, &c->fpart_s, &c->sbsc})
+    drop(p);
+}
+
 template <typename H, int NC, bool FOLD>
 static void launch_weights(Ctx* c, const SplitStore& st, int chain0, hipStream_t s) {
   const int np = c->np;

@@ -109,10 +109,13 @@ def test_averages(L, N, gamma, form):
     p.close()
 
 
-@pytest.mark.parametrize("prec", [0, 1, 2])
-def test_averages_of_many_images(prec):
-    """Enough images that the split precisions take the orbit form (in FP64): against
-    the FP64 average over the whole range of the images."""
+@pytest.mark.parametrize("rotate", [False, True])
+@pytest.mark.parametrize("prec, tol", [(0, 1e-9), (1, 1e-6), (2, 1e-5)])
+def test_averages_of_many_images(prec, tol, rotate):
+    """Enough images that the split precisions take the orbit form (7 pairs and more:
+    two groups): against the FP64 average over the whole range of the images, within
+    the accuracy of the split products (2^-22 and 2^-17 per term, as the other split
+    tests), and no further from it than the general form in the same precision."""
     from tdscha_amd.engine import Engine
     from tdscha_amd.rocksalt import Ensemble, RockSalt
     ens = Ensemble(RockSalt(L=3), 300.0, 11000, seed=5)
@@ -120,11 +123,15 @@ def test_averages_of_many_images(prec):
     v = (ens.ir_vector() / np.sqrt(ens.m)) @ ens.pols
     R, Y = sector_perturbations(ms, v, 8)
     eng = Engine(ens.X, ens.Y, ens.w, np.ones(ens.N), 300.0, ms.symmetries, ms.degenerate_space,
-                 ms.sym_block_id)
+                 ms.sym_block_id, rotate=rotate)
     f, d = eng.perturb_averages_batched(R, Y, 1, prec)
-    fo, do = eng.perturb_averages_range(R, Y, 1, ens.N * ms.symmetries[0].shape[0], 1, 0)
+    M = ens.N * ms.symmetries[0].shape[0]
+    fo, do = eng.perturb_averages_range(R, Y, 1, M, 1, 0)
+    fg, dg = eng.perturb_averages_range(R, Y, 1, M, 1, prec)
     eng.close()
-    assert rel(f, fo) < 1e-9 and rel(d, do) < 1e-9
+    assert rel(f, fo) < tol and rel(d, do) < tol
+    if prec:
+        assert rel(f, fo) + rel(d, do) < rel(fg, fo) + rel(dg, do)
 
 
 @pytest.mark.parametrize("wigner, transpose", [(True, False), (False, False), (False, True)])
