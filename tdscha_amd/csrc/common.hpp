@@ -65,6 +65,31 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// FP64 matrix products of 4 x 4 x 4 blocks
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+
+// v of the lane 4 R lanes before, cyclic within a row of 16 lanes
+template <int R>
+__device__ __forceinline__ double rot4(double v) {
+  if constexpr (R == 0) return v;
+  constexpr int ctrl = 0x120 + 4 * R;   // row_ror:4R
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// acc += A B for a 16 x 16 block, 4 of the K index: A[i][k] i = lane % 16,
+// B[k][j] j = lane % 16, k = lane / 16; acc[r] of a lane is the element of row
+// 4 q + lane / 16, column 4 ((q - r) % 4) + lane % 4 (q = lane / 4 % 4)
+__device__ __forceinline__ void mma16(double a, double b, double (&acc)[4]) {
+  acc[0] = mfma4(a, b, acc[0]);
+  acc[1] = mfma4(a, rot4<1>(b), acc[1]);
+  acc[2] = mfma4(a, rot4<2>(b), acc[2]);
+  acc[3] = mfma4(a, rot4<3>(b), acc[3]);
+}
+
 // Arrays carved from one allocation (256-byte aligned): add() each, allocate total()
 // bytes, assign() the base.
 class Carve {
@@ -127,7 +152,7 @@ constexpr double kOrbWorthUs = 500.0;
 struct OrbPlan {
   bool ok = false;
   int prec = 0;            // of its averages
-  int nc = 0, npairs = 0;
+  int nc = 0, npairs = 0, rank = 0;   // chains, pairs, largest rank of a chain
   struct Round {
     int chain0, chains, first, count;
   };

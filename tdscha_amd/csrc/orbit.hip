@@ -55,30 +55,6 @@ int rot_panels(const int* bs, const int* d, int n, int np, int* start, int* nrea
 constexpr int kOP = 32;          // modes of a panel (whole blocks)
 constexpr int kOLd = kOP + 1;
 
-static __device__ __forceinline__ double mfma4(double a, double b, double c) {
-  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-
-// v of the lane 4 R lanes before, cyclic within a row of 16 lanes
-template <int R>
-static __device__ __forceinline__ double rot4(double v) {
-  if constexpr (R == 0) return v;
-  constexpr int ctrl = 0x120 + 4 * R;   // row_ror:4R
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-
-// acc += A B for a 16 x 16 block, 4 of the K index: A[i][k] i = lane % 16,
-// B[k][j] j = lane % 16, k = lane / 16; acc[r] of a lane is the element of row
-// 4 q + lane / 16, column 4 ((q - r) % 4) + lane % 4 (q = lane / 4 % 4)
-static __device__ __forceinline__ void mma16(double a, double b, double (&acc)[4]) {
-  acc[0] = mfma4(a, b, acc[0]);
-  acc[1] = mfma4(a, rot4<1>(b), acc[1]);
-  acc[2] = mfma4(a, rot4<2>(b), acc[2]);
-  acc[3] = mfma4(a, rot4<3>(b), acc[3]);
-}
-
 // ------------------------------------------------------------------- the probe
 // row-dots of 16 probe rows over 16 columns of V = U Y1, a quarter of the K index
 // per wave (the dots are linear in V); grid (rows / 16, ceil(n / 16), chains):
@@ -215,12 +191,15 @@ __global__ __launch_bounds__(256) void orb_in(OrbPanels pn, const int2* __restri
 // sums, results to f_out, d_out (both halves).  Else D_k the symmetric inputs,
 // results to the packed vectors x [chain][n + 2 P] (matrix m = 2 chain + sector; R
 // with sector 0), in which case the kernel runs only on every `every`-th step.
-// grid (panel pairs pi <= pj, matrices); per symmetry a wave combines D in
-// registers (its 16 rows), and the product with S_pj^T passes through LDS.  Bound by
-// the latency of that chain over the symmetries (few tiles): two groups of four waves
-// take every other one, 97 instead of 128 us at 159 modes, 185 (171) us at 381.
-template <bool AVG>
-__global__ __launch_bounds__(512) void orb_out(
+// RM: largest rank of the plan (3, or kOrbRank).  grid (panel pairs pi <= pj, then
+// panels for f; matrices); per symmetry a wave combines D in registers (its 16 rows),
+// and the product with S_pj^T passes through LDS.  Bound by the latency of that chain:
+// two groups of four waves take every other symmetry, every load is unconditional,
+// rank 3 leaves two work-groups to a CU, and f has work-groups of its own (with
+// conditional loads and f behind its diagonal tile: 97 us for three matrices of 159
+// modes and 185 of 381; 59 and 101 now).
+template <bool AVG, int RM>
+__global__ __launch_bounds__(512, RM > 3 ? 2 : 4) void orb_out(
     OrbPanels pn, const int4* __restrict__ mats, const double* __restrict__ C,
     const double* __restrict__ Zb, const double* __restrict__ fb, const double* __restrict__ fy,
     int n, int np, double normf, double normd, const int* __restrict__ kk, int every,
@@ -229,52 +208,97 @@ __global__ __launch_bounds__(512) void orb_out(
   const int m = blockIdx.y;
   const int4 mt = mats[m];
   if (!AVG && !active[m >> 1]) return;
+  const int ntile = pn.npanel * (pn.npanel + 1) / 2;
+  const bool isf = (int)blockIdx.x >= ntile;
   int pj = 0, pi = blockIdx.x;
-  while (pi > pj) pi -= ++pj;   // pair (pi, pj), pi <= pj
+  if (isf)
+    pi = pj = blockIdx.x - ntile;
+  else
+    while (pi > pj) pi -= ++pj;   // pair (pi, pj), pi <= pj
   const int r0 = pn.start[pi], h = pn.start[pi + 1] - r0;
   const int q0 = pn.start[pj], w = pn.start[pj + 1] - q0;
-  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, half = threadIdx.x >> 8;
+  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
+  const int half = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
   const int wr = 16 * (wave >> 1), wc = 16 * (wave & 1);
   const int lr = lane & 15, lg = lane >> 4, lq = lane & 3, lb = (lane >> 2) & 3;
   __shared__ double T[2][2][kOP][kOLd];
   const long nn = (long)np * np;
   const int rank = mt.y;
-  double d[kOrbRank][8];
+  const double* Cm = C + (long)mt.z * pn.nsym * kOrbRank;
+  if (isf) {
+    // f of a panel, sixteen symmetries at a time: h_j = sum_k C_jk f_k in LDS, then
+    // S_j h_j, thread = (mode, symmetry)
+    if (!AVG && (m & 1)) return;
+    double(*hs)[kOP] = reinterpret_cast<double(*)[kOP]>(&T[0][0][0][0]);   // [16][32]
+    double(*part)[kOP] = reinterpret_cast<double(*)[kOP]>(&T[1][0][0][0]); // [16][32]
+    const int t = threadIdx.x & 31, sl = threadIdx.x >> 5;
+    const double* St = pn.ST + (long)pi * pn.nsym * kOP * kOP + t;
+    double fk[RM], v = 0.0;
 #pragma unroll
-  for (int k = 0; k < kOrbRank; ++k)
+    for (int k = 0; k < RM; ++k) {
+      const double f = fb[(long)(mt.x + min(k, rank - 1)) * np + r0 + min(t, h - 1)];
+      fk[k] = k < rank && t < h ? f : 0.0;
+    }
+    for (int j0 = 0; j0 < pn.nsym; j0 += 16) {
+      const int j = min(j0 + sl, pn.nsym - 1);
+      double st[kOP], x = 0.0;
+#pragma unroll
+      for (int b = 0; b < kOP; ++b) st[b] = St[((long)j * kOP + b) * kOP];
+#pragma unroll
+      for (int k = 0; k < RM; ++k) x += Cm[j * kOrbRank + k] * fk[k];   // (zero from rank on)
+      __syncthreads();
+      hs[sl][t] = j0 + sl < pn.nsym ? x : 0.0;
+      __syncthreads();
+#pragma unroll
+      for (int b = 0; b < kOP; ++b) v += st[b] * hs[sl][b];
+    }
+    part[sl][t] = v;
+    __syncthreads();
+    if ((int)threadIdx.x < h) {
+      double f = 0.0;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) f += part[q][t];
+      if (AVG)
+        f_out[(long)m * n + r0 + t] = normf * f;
+      else
+        d_out[(m >> 1) * (n + (long)n * (n + 1)) + r0 + t] = normf * f;
+    }
+    return;
+  }
+  // (loads clamped to the tile, not conditional: all of them in flight)
+  double d[RM][8];
+#pragma unroll
+  for (int k = 0; k < RM; ++k) {
+    const double* z = Zb + (long)(mt.x + min(k, rank - 1)) * nn;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
       const int a = wr + lr, b = 4 * ks + lg;
-      double v = 0.0;
-      if (k < rank && a < h && b < w) {
-        const double* z = Zb + (long)(mt.x + k) * nn;
-        v = z[(long)(r0 + a) * np + q0 + b];
-        if (AVG) v = fy[r0 + a] * v + fy[q0 + b] * z[(long)(q0 + b) * np + r0 + a];
-      }
-      d[k][ks] = v;
+      const int ga = r0 + min(a, h - 1), gb = q0 + min(b, w - 1);
+      double v = z[(long)ga * np + gb];
+      if (AVG) v = fy[ga] * v + fy[gb] * z[(long)gb * np + ga];
+      d[k][ks] = k < rank && a < h && b < w ? v : 0.0;
     }
-  const double* Cm = C + (long)mt.z * pn.nsym * kOrbRank;
+  }
   const double* Ti = pn.ST + (long)pi * pn.nsym * kOP * kOP + wr + lr;
   const double* Tj = pn.ST + (long)pj * pn.nsym * kOP * kOP + wc + lr;
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  // the halves take every other symmetry (weight zero past the last)
   for (int jj = 0; jj < pn.nsym; jj += 2) {
-    // the halves take every other symmetry (weight zero past the last)
-    const bool in = jj + half < pn.nsym;
-    const int j = in ? jj + half : 0;
+    const int jc = min(jj + half, pn.nsym - 1);
+    const long o = (long)jc * kOP * kOP + lg * kOP;
     double sj[8], si[8], mm[8];
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      sj[ks] = Tj[(long)j * kOP * kOP + (4 * ks + lg) * kOP];
-      si[ks] = Ti[(long)j * kOP * kOP + (4 * ks + lg) * kOP];
+      sj[ks] = Tj[o + 4 * ks * kOP];
+      si[ks] = Ti[o + 4 * ks * kOP];
       mm[ks] = 0.0;
     }
 #pragma unroll
-    for (int k = 0; k < kOrbRank; ++k)
-      if (k < rank) {
-        const double c = in ? Cm[j * kOrbRank + k] : 0.0;
+    for (int k = 0; k < RM; ++k) {   // (zero from rank on)
+      const double c = jj + half < pn.nsym ? Cm[jc * kOrbRank + k] : 0.0;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) mm[ks] += c * d[k][ks];
-      }
+      for (int ks = 0; ks < 8; ++ks) mm[ks] += c * d[k][ks];
+    }
     double t[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) mma16(mm[ks], sj[ks], t);
@@ -311,42 +335,6 @@ __global__ __launch_bounds__(512) void orb_out(
       const long p = (long)gr * n - (long)gr * (gr - 1) / 2 + (gc - gr);
       d_out[(m >> 1) * len + n + (m & 1) * P + p] = v;
     }
-  }
-  if (pi != pj || !(AVG || (m & 1) == 0)) return;
-  // f of the panel: thread = (mode, every sixteenth symmetry), f_k in LDS
-  __syncthreads();
-  double(*fs)[kOP] = reinterpret_cast<double(*)[kOP]>(&T[0][0][0][0]);   // [kOrbRank][32]
-  double(*part)[kOP] = reinterpret_cast<double(*)[kOP]>(&T[1][0][0][0]); // [16][32]
-  const int t = threadIdx.x & 31, sl = threadIdx.x >> 5;
-  if (sl < rank) fs[sl][t] = t < h ? fb[(long)(mt.x + sl) * np + r0 + t] : 0.0;
-  __syncthreads();
-  const double* St = pn.ST + (long)pi * pn.nsym * kOP * kOP + t;
-  double v = 0.0;
-  for (int j = sl; j < pn.nsym; j += 16) {
-    double g[kOrbRank];
-#pragma unroll
-    for (int k = 0; k < kOrbRank; ++k) g[k] = 0.0;
-#pragma unroll 8
-    for (int b = 0; b < kOP; ++b) {
-      const double st = St[((long)j * kOP + b) * kOP];
-#pragma unroll
-      for (int k = 0; k < kOrbRank; ++k)
-        if (k < rank) g[k] += st * fs[k][b];
-    }
-#pragma unroll
-    for (int k = 0; k < kOrbRank; ++k)
-      if (k < rank) v += Cm[j * kOrbRank + k] * g[k];
-  }
-  part[sl][t] = v;
-  __syncthreads();
-  if ((int)threadIdx.x < h) {
-    double f = 0.0;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) f += part[q][t];
-    if (AVG)
-      f_out[(long)m * n + r0 + t] = normf * f;
-    else
-      d_out[(m >> 1) * len + r0 + t] = normf * f;
   }
 }
 
@@ -888,6 +876,8 @@ int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p) {
   p.prec = prec;
   p.nc = nc;
   p.npairs = (int)pairs.size();
+  p.rank = 0;
+  for (const int4& m : mats) p.rank = std::max(p.rank, m.y);
   // rounds of the clean-up: whole chains, at most kOrbPairs pairs each
   p.rounds.clear();
   for (int ch = 0, at = 0; ch < nc;) {
@@ -966,8 +956,8 @@ int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* 
                      0, o.zpart, o.fpart, s);
     launch_reduce_f64(n, np, P, ks, o.zpart, o.fpart, o.z, o.f, 1.0 / c->n_eff, s);
   }
-  hipLaunchKernelGGL(orb_out<true>, dim3(o.npanel * (o.npanel + 1) / 2, p.nc), dim3(512), 0, s, pn,
-                     p.mats, p.C, o.z, o.f, c->fy, n, np, 1.0 / o.nsym,
+  const auto out = p.rank <= 3 ? orb_out<true, 3> : orb_out<true, kOrbRank>;
+  hipLaunchKernelGGL(out, dim3(o.npanel * (o.npanel + 3) / 2, p.nc), dim3(512), 0, s, pn, p.mats, p.C, o.z, o.f, c->fy, n, np, 1.0 / o.nsym,
                      1.0 / (c->n_eff * o.nsym), (const int*)nullptr, 0, (const int*)nullptr, f_dev,
                      d2v_dev);
   TDS_CHECK_HIP(hipGetLastError());
@@ -988,7 +978,8 @@ int orbit_clean(Ctx* c, const OrbPlan& p, double* x, const int* kk, const int* a
   for (const OrbPlan::Round& r : p.rounds) {
     hipLaunchKernelGGL(orb_in, dim3(o.npanel * o.npanel, r.count), dim3(256), 0, s, pn,
                        p.clean + r.first, o.Yb, o.Rb, np, kk, kOrbClean, o.Y1, o.R1);
-    hipLaunchKernelGGL(orb_out<false>, dim3(o.npanel * (o.npanel + 1) / 2, 2 * r.chains),
+    const auto out = p.rank <= 3 ? orb_out<false, 3> : orb_out<false, kOrbRank>;
+    hipLaunchKernelGGL(out, dim3(o.npanel * (o.npanel + 3) / 2, 2 * r.chains),
                        dim3(512), 0, s, pn, p.cmats + 2 * r.chain0, p.C, o.Y1, o.R1, c->fy, n, np,
                        1.0 / o.nsym, 1.0 / o.nsym, kk, kOrbClean, active + r.chain0,
                        (double*)nullptr, x + r.chain0 * len);

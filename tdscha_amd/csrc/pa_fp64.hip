@@ -84,10 +84,6 @@ __global__ void expand_images(const double* __restrict__ X, const double* __rest
 // tiles of 80 columns, where whole 128-column tiles would do 1.6 times the
 // work of a GEMM side and 2.6 times that of the outer product).
 // ---------------------------------------------------------------------------
-static __device__ __forceinline__ double mfma4(double a, double b, double c) {
-  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
-
 // CB consecutive doubles from p[o] on (16-byte pieces where CB is even).  The
 // LDS reads of both kernels form each address with one index: the compiler
 // knows which LDS array a read may touch only through short pointer
@@ -112,16 +108,6 @@ static __device__ __forceinline__ void read_run(const double* p, long o, double 
 typedef __attribute__((address_space(3))) double* lds_d;
 static __device__ __forceinline__ void copy16(const double* g, lds_d l) {
   __builtin_amdgcn_global_load_lds((gbl_ptr_t)g, (lds_ptr_t)l, 16, 0, 0);
-}
-
-// v of the lane 4 R lanes before, cyclic within a row of 16 lanes
-template <int R>
-static __device__ __forceinline__ double rot4(double v) {
-  if constexpr (R == 0) return v;
-  constexpr int ctrl = 0x120 + 4 * R;   // row_ror:4R
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
 }
 
 // acc[i][r] += A_i x B, 16 rows per i: block q of lane's column group q - r
