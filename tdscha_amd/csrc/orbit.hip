@@ -426,60 +426,64 @@ static double dot(const double* x, const double* y, int n) {
 }
 
 // Whether the S_j are closed under multiplication: p.S_i S_j z equals p.S_k z for
-// one k for two independent random pairs (p, z), to 1e-9 of their size.  Fills
-// the list of generators.
+// one k for two independent random pairs (p, z), to 1e-9 of their size.  Elements
+// become generators until the products with them reach the whole list; every one of
+// these products has to be in the list (then the list is the group they generate).
 static bool closed(Ctx* c) {
   Orbit& o = c->orb;
   const int ns = o.nsym, n = c->n;
   std::mt19937_64 g(12345);
   std::normal_distribution<double> nd;
-  std::vector<double> A[2], B[2], ref(2 * (size_t)ns);
+  std::vector<double> A[2], z[2], ref(2 * (size_t)ns), sz(n);
   for (int t = 0; t < 2; ++t) {
-    std::vector<double> p(n), z(n);
+    std::vector<double> p(n);
+    z[t].resize(n);
     for (double& v : p) v = nd(g);
-    for (double& v : z) v = nd(g);
+    for (double& v : z[t]) v = nd(g);
     A[t].resize((size_t)ns * n);
-    B[t].resize((size_t)ns * n);
     for (int j = 0; j < ns; ++j) {
-      apply_s(c, o.syms, j, true, p.data(), A[t].data() + (size_t)j * n);
-      apply_s(c, o.syms, j, false, z.data(), B[t].data() + (size_t)j * n);
-      ref[2 * (size_t)j + t] = dot(p.data(), B[t].data() + (size_t)j * n, n);
+      double* a = A[t].data() + (size_t)j * n;
+      apply_s(c, o.syms, j, true, p.data(), a);
+      ref[2 * (size_t)j + t] = dot(a, z[t].data(), n);
     }
   }
   const double tol = 1e-9 * n;
-  std::vector<int> order(ns), table((size_t)ns * ns);
+  std::vector<int> order(ns);
   for (int j = 0; j < ns; ++j) order[j] = j;
   std::sort(order.begin(), order.end(),
             [&](int a, int b) { return ref[2 * (size_t)a] < ref[2 * (size_t)b]; });
-  for (int i = 0; i < ns; ++i)
-    for (int j = 0; j < ns; ++j) {
-      double v[2];
-      for (int t = 0; t < 2; ++t)
-        v[t] = dot(A[t].data() + (size_t)i * n, B[t].data() + (size_t)j * n, n);
-      auto it = std::lower_bound(order.begin(), order.end(), v[0] - tol,
-                                 [&](int a, double x) { return ref[2 * (size_t)a] < x; });
-      int hit = -1;
-      for (; it != order.end() && ref[2 * (size_t)*it] <= v[0] + tol && hit < 0; ++it)
-        if (std::fabs(ref[2 * (size_t)*it + 1] - v[1]) <= tol) hit = *it;
-      if (hit < 0) return false;
-      table[(size_t)i * ns + j] = hit;
-    }
-  // generators: add elements until their products reach the whole list
+  std::vector<double> gz[2];   // S_q z of each generator q
+  auto product = [&](int i, int q) {
+    double v[2];
+    for (int t = 0; t < 2; ++t)
+      v[t] = dot(A[t].data() + (size_t)i * n, gz[t].data() + (size_t)q * n, n);
+    auto it = std::lower_bound(order.begin(), order.end(), v[0] - tol,
+                               [&](int a, double x) { return ref[2 * (size_t)a] < x; });
+    for (; it != order.end() && ref[2 * (size_t)*it] <= v[0] + tol; ++it)
+      if (std::fabs(ref[2 * (size_t)*it + 1] - v[1]) <= tol) return *it;
+    return -1;
+  };
   std::vector<char> in(ns, 0);
   std::vector<int> sub;
   o.gens.clear();
   for (int j = 0; j < ns; ++j) {
     if (in[j]) continue;
+    for (int t = 0; t < 2; ++t) {
+      apply_s(c, o.syms, j, false, z[t].data(), sz.data());
+      gz[t].insert(gz[t].end(), sz.begin(), sz.end());
+    }
     o.gens.push_back(j);
     in[j] = 1;
     sub.push_back(j);
     for (size_t a = 0; a < sub.size(); ++a)
-      for (int q : o.gens)
-        for (int k : {table[(size_t)sub[a] * ns + q], table[(size_t)q * ns + sub[a]]})
-          if (!in[k]) {
-            in[k] = 1;
-            sub.push_back(k);
-          }
+      for (size_t q = 0; q < o.gens.size(); ++q) {
+        const int k = product(sub[a], (int)q);
+        if (k < 0) return false;
+        if (!in[k]) {
+          in[k] = 1;
+          sub.push_back(k);
+        }
+      }
   }
   return true;
 }

@@ -47,6 +47,8 @@ constexpr int kQWeightsChains = 2;   // chains per q_weights workgroup
 constexpr int kD2vChains = 15;       // chains per slab q_d2v workgroup
 constexpr int kSlabBytes = 65536;    // LDS of one slab q_d2v workgroup (two buffers)
 constexpr int kD2vThreads = 256;     // threads (items) per slab q_d2v workgroup
+constexpr int kMmaUnits = 3584;      // entries of one LDS buffer of q_d2v_mma
+constexpr int kMmaGroups = 3;        // groups of four items per wave of q_d2v_mma
 
 struct QCtx {
   int nq = 0, nb = 0, N = 0;
@@ -62,6 +64,7 @@ struct QCtx {
   double* fP = nullptr;     // [nq][nb]
   double2* S = nullptr;     // slab images of (fY X, Y) for q_d2v_slab
   int slabT = 0;            // configurations per slab (0: no slab images)
+  bool mma = false;         // the slabs are q_d2v_mma's
   int d2v_form = 1;         // 1: q_d2v_slab when slab images exist, 0: q_d2v
   int n_cu = 256;           // compute units of the context's device
   // tile choices (autotuner)
@@ -567,6 +570,156 @@ __global__ void __launch_bounds__(kD2vThreads) __attribute__((amdgpu_waves_per_e
   }
 }
 
+// The blocks on the FP64 matrix instructions (6 bands): as real matrices the block of
+// an item is r (12 x K) times Q (K x 12), K the configurations, for each of the two
+// products; a 4 x 4 x 4 instruction takes four items at once (its four blocks) and
+// four configurations, nine of them the 12 x 12 entries.  The same FP64 work as a
+// thread per item, but 9 accumulators instead of 72 and each operand read once per
+// four lanes' worth of configurations, so that a CU has 16 waves instead of 8, no lane
+// without an item but in the last group, and slabs of at least four configurations.
+// Sixteen waves: `slices` of the slab's steps of four configurations (fixed by T, so
+// that a chain's sums do not depend on its batch) times 16 / slices columns, groups of
+// items dealt to the columns in turn.  64 chains on 4x4x4: 859 us with a thread per
+// item, MMA64 us; 8 chains on 2x2x2 with 48 images: 61, MMA8 us.
+constexpr int mma_slices(int T) { return T / 4; }
+constexpr int mma_cap(int T) { return 16 / mma_slices(T) * kMmaGroups * 4; }
+
+template <int T>
+__global__ __launch_bounds__(1024) void q_d2v_mma(
+    const double2* __restrict__ S, int N, int nq, const int* __restrict__ active,
+    const int4* __restrict__ items, const int* __restrict__ blk_start, int nib, int MP,
+    const double2* __restrict__ wc, const double2* __restrict__ wd, int chunk, int nch,
+    double2* __restrict__ dpart) {
+  constexpr int NB = 6, SR = NB * T + 1, NSL = mma_slices(T), NCOL = 16 / NSL, G = kMmaGroups;
+  __shared__ double2 bufA[kMmaUnits], bufB[kMmaUnits];
+  // equal numbers of workgroups on the XCDs (one fits a CU: an XCD with one too many
+  // would take twice the time), the item blocks of a chunk side by side
+  const int total = nib * nch, per = (total + 7) >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (id >= total) return;
+  const int ch = id / nib, ib = id - ch * nib;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int slice = wave % NSL, col = wave / NSL;
+  const int i = lane & 3, blk = (lane >> 2) & 3, k = lane >> 4, sgn = i & 1;
+  const int i0 = blk_start[ib], i1 = blk_start[ib + 1], ni = i1 - i0, ng = (ni + 3) / 4;
+  const int c_lo = items[i0].x, ncb = items[i1 - 1].x - c_lo + 1;
+  bool any = false;
+  for (int c = 0; c < ncb; ++c) any |= active[c_lo + c] != 0;
+  if (!any) return;
+  // entries of a slab, the weights behind them, both in whole copies of 64 entries
+  const int U = 2 * nq * SR, U64 = (U + 63) / 64, nW = ncb * 2 * T, W64 = (nW + 63) / 64;
+  const int oy = nq * SR * 2;   // from x to y, in doubles
+  int ox1[G], ox2[G], ow[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int4 it = items[i0 + min(4 * (g * NCOL + col) + blk, ni - 1)];
+    const int o = ((i >> 1) * T + 4 * slice + k) * 2 + sgn;
+    ox1[g] = it.z * SR * 2 + o;
+    ox2[g] = it.w * SR * 2 + o;
+    ow[g] = U64 * 64 + (it.x - c_lo) * 2 * T + 4 * slice + k;
+  }
+  const int lo = ch * chunk, hi = min(N, lo + chunk);
+  // (every lane takes part in each copy; those past the end repeat the last entry)
+  auto issue = [&](int s0, double2* dst) {
+    const double2* src = S + (long)(s0 / T) * U;
+    for (int q = wave; q < U64; q += 16) dma16(src + min(q * 64 + lane, U - 1), dst + q * 64);
+    for (int q = wave; q < W64; q += 16) {
+      const int e = min(q * 64 + lane, nW - 1);
+      const int j = e % T, h = (e / T) & 1, c = c_lo + e / (2 * T);
+      dma16((h ? wd : wc) + (long)c * N + min(s0 + j, N - 1), dst + (U64 + q) * 64);
+    }
+  };
+  double acc[G][3][3];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b) acc[g][a][b] = 0.0;
+  // the other half (imaginary for real) of the complex entry: lane ^ 1
+  auto other = [](double v) {
+    const int a = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xf, 0xf, true);
+    const int b = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xf, 0xf, true);
+    return __hiloint2double(b, a);
+  };
+  auto accumulate = [&](const double2* img) {
+    const double* d = reinterpret_cast<const double*>(img);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (g * NCOL + col >= ng) break;
+      double x1[3], y1[3], Q1[3], Q2[3];
+      const double2 c1 = img[ow[g]], c2 = img[ow[g] + T];
+      const double c1y = sgn ? -c1.y : c1.y, c2y = sgn ? -c2.y : c2.y;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        // -Q1 = conj(wc) r22 + conj(wd) r12, -Q2 = conj(wc) r12
+        const double x = d[ox2[g] + 4 * a * T], y = d[ox2[g] + oy + 4 * a * T];
+        const double xo = other(x), yo = other(y);
+        Q2[a] = __builtin_fma(c1y, xo, c1.x * x);
+        Q1[a] = __builtin_fma(c2y, xo,
+                              __builtin_fma(c2.x, x, __builtin_fma(c1y, yo, c1.x * y)));
+        x1[a] = d[ox1[g] + 4 * a * T];
+        y1[a] = d[ox1[g] + oy + 4 * a * T];
+      }
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = 0; b < 3; ++b) acc[g][a][b] = mfma4(x1[a], Q1[b], acc[g][a][b]);
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = 0; b < 3; ++b) acc[g][a][b] = mfma4(y1[a], Q2[b], acc[g][a][b]);
+    }
+  };
+  issue(lo, bufA);
+  for (int s0 = lo; s0 < hi; s0 += 2 * T) {
+    TDS_WAIT_VMCNT(0);
+    lds_barrier();                     // slab s0 in bufA; bufB free
+    if (s0 + T < hi) issue(s0 + T, bufB);
+    accumulate(bufA);
+    if (s0 + T >= hi) break;
+    TDS_WAIT_VMCNT(0);
+    lds_barrier();                     // slab s0 + T in bufB; bufA free
+    if (s0 + 2 * T < hi) issue(s0 + 2 * T, bufA);
+    accumulate(bufB);
+  }
+  if constexpr (NSL > 1) {   // the slices in order, three accumulators at a time
+    double* red = reinterpret_cast<double*>(bufA);   // [wave][3][64]
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        lds_barrier();
+#pragma unroll
+        for (int b = 0; b < 3; ++b) red[(wave * 3 + b) * 64 + lane] = acc[g][a][b];
+        lds_barrier();
+        if (slice == 0)
+#pragma unroll
+          for (int q = 1; q < NSL; ++q)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) acc[g][a][b] += red[((wave + q) * 3 + b) * 64 + lane];
+      }
+    if (slice) return;
+  }
+  // D: column lane % 4, item lane / 4 % 4, row lane / 16: complex entry (a, b) from the
+  // four real ones (2 a + s, 2 b + s')
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int at = 4 * (g * NCOL + col) + blk;
+    const int4 it = items[i0 + min(at, ni - 1)];
+    const bool mine = at < ni && !(lane & 17) && active[it.x] != 0;
+    double2* o = dpart + (((long)it.x * MP + it.y) * nch + ch) * NB * NB;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b) {
+        const double v = acc[g][a][b];
+        const double re = v + __shfl_xor(v, 17), im = __shfl_xor(v, 16) - __shfl_xor(v, 1);
+        if (mine) o[(2 * a + (lane >> 5)) * NB + 2 * b + ((lane >> 1) & 1)] = make_double2(-re, -im);
+      }
+  }
+}
+
 // Sum over k of p[k W + t], k < n, for t < W of a 256-thread workgroup: the
 // entries in 256 / W slices, four loads in flight each, the slices added in LDS in
 // a fixed order.
@@ -864,7 +1017,15 @@ static int log2_pow2(int T) {
   return lg;
 }
 
-static int slab_configs(int nq, int nb) {
+static int slab_configs(int nq, int nb, bool* mma) {
+  // q_d2v_mma: 16, 8 or 4 configurations, whole copies of 64 entries
+  *mma = false;
+  if (nb == 6)
+    for (int T = 16; T >= 4; T >>= 1)
+      if ((2 * nq * (6 * T + 1) + 63) / 64 * 64 + (2 * kD2vChains * T + 63) / 64 * 64 <= kMmaUnits) {
+        *mma = true;
+        return T;
+      }
   int T = 16;
   while (T > 0 && slab_units(nq, nb, T) * sizeof(double2) > (size_t)kSlabBytes / 2) T >>= 1;
   return T;
@@ -875,7 +1036,7 @@ static int slab_configs(int nq, int nb) {
 static int build_slabs(QCtx* q) {
   if (q->S) (void)hipFree(q->S);
   q->S = nullptr;
-  q->slabT = slab_configs(q->nq, q->nb);
+  q->slabT = slab_configs(q->nq, q->nb, &q->mma);
   if (!q->slabT) return 0;
   const int lg = log2_pow2(q->slabT);
   const long nslab = (q->N + q->slabT - 1) / q->slabT;
@@ -904,7 +1065,7 @@ static int build_slabs(QCtx* q) {
 // resident workgroups per CU: two buffers of half the CU's LDS and 256
 // threads at up to 256 VGPRs), at least 4 slabs.
 static int slab_chunk(const QCtx* q, int n_item_blocks, int rounds) {
-  const long slots = 2L * q->n_cu * rounds;
+  const long slots = (q->mma ? 1L : 2L) * q->n_cu * rounds;
   const long nch = std::max(1L, slots / std::max(1, n_item_blocks));
   const long chunk = std::max<long>(4L * q->slabT, (q->N + nch - 1) / nch);
   return (int)((chunk + q->slabT - 1) / q->slabT * q->slabT);
@@ -983,7 +1144,7 @@ static int build_batch(QCtx* q, int C, const int* iq_pert, const int* pair_map, 
         }
       h_bs.push_back((int)h_items.size());
     };
-    partition(kD2vThreads / d2v_slices(b.slabT));
+    partition(q->mma ? mma_cap(b.slabT) : kD2vThreads / d2v_slices(b.slabT));
     const int nfull = (int)h_bs.size() - 1;      // then the same count of even workgroups
     partition(((int)h_items.size() + nfull - 1) / nfull);
     b.n_items = (int)h_items.size();
@@ -1075,12 +1236,15 @@ static void launch_L_nb(QCtx* q, QBatch& b, const double2* psi, double2* out, in
                        q->rho, q->N, nq, q->fY, q->fP, b.active, b.iqp, b.partner, b.alpha, b.R1,
                        C, ngroups, b.ntile, ignore_v4 ? 0 : 1, b.wc, b.wd, b.fpart);
     if (b.slabT) {
-      const int nblk2 = (b.nch + 7) / 8 * 8 * b.nib;
-      with_slab(b.slabT, [&](auto T) {
-        hipLaunchKernelGGL((q_d2v_slab<NB, decltype(T)::value>), dim3(nblk2), dim3(kD2vThreads), 0,
-                           s, q->S, q->N, nq, b.active, b.items, b.blk_start, b.nib, MP, b.wc,
-                           b.wd, b.chunk, b.nch, b.dpart);
-      });
+      const int nblk2 = q->mma ? (b.nch * b.nib + 7) / 8 * 8 : (b.nch + 7) / 8 * 8 * b.nib;
+      auto run = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(nblk2), dim3(threads), 0, s, q->S, q->N, nq, b.active,
+                           b.items, b.blk_start, b.nib, MP, b.wc, b.wd, b.chunk, b.nch, b.dpart);
+      };
+      if (q->mma)
+        run(b.slabT == 16 ? q_d2v_mma<16> : b.slabT == 8 ? q_d2v_mma<8> : q_d2v_mma<4>, 1024);
+      else
+        with_slab(b.slabT, [&](auto T) { run(q_d2v_slab<NB, decltype(T)::value>, kD2vThreads); });
     } else {
       hipLaunchKernelGGL(q_d2v<NB>, dim3(b.maxp, C, b.nch), dim3(256), 0, s, q->X, q->Y, q->N,
                          q->fY, b.active, b.npairs, b.pq1, b.pq2, MP, b.wc, b.wd, b.chunk, b.nch,
