@@ -43,7 +43,6 @@ namespace tdscha {
 
 constexpr int kQMaxChains = 256;
 constexpr int kQMaxQ = 512;
-constexpr int kQWeightsChains = 2;   // chains per q_weights workgroup
 constexpr int kD2vChains = 15;       // chains per slab q_d2v workgroup
 constexpr int kSlabBytes = 65536;    // LDS of one slab q_d2v workgroup (two buffers)
 constexpr int kD2vThreads = 256;     // threads (items) per slab q_d2v workgroup
@@ -96,7 +95,6 @@ struct QBatch {
   int* pq2 = nullptr;
   int* offa = nullptr;
   int* offb = nullptr;
-  int* partner = nullptr;   // [C][nq]
   int* apair = nullptr;     // [C][nq]
   int* aorient = nullptr;   // [C][nq]
   int* active = nullptr;    // [C]
@@ -222,118 +220,125 @@ __device__ __forceinline__ bool xcd_tile(int b, int ngroups, int ntile, int& til
   return tile < ntile;
 }
 
-// One thread per configuration and CB chains per workgroup: the own-q
-// vectors x_q and fP_q y_q are loaded once for the CB chains, each chain
-// then loads its partner x_{q_pert - q} and applies its oriented alpha block,
-// which is the same for every thread (scalar loads).
-template <int NB, int CB>
+// One thread per configuration, one chain per workgroup.  The oriented alpha block of a
+// pair's second q-point is the conjugate transpose of the first one's: each pair is
+// taken once, with 24 vectors in flight and its block (the same for every thread) read
+// once, from LDS, for both products,
+//   bu1 = A x2, bu2 = A^H x1,   tot += 2 Re x1^H bu1,
+//   bfw += fP1 y1 . conj(bu1) + fP2 y2 . conj(bu2).
+// Bound by the L2 reads and their latency.  64 chains on 4x4x4 / 8 chains on 2x2x2 with
+// 48 images: 1095 / 59 us with a q-point at a time, two chains a workgroup and scalar
+// loads of the blocks (more than the scalar registers hold); 871 / 52 us.
+template <int NB>
 __global__ void __launch_bounds__(256) q_weights(
     const double2* __restrict__ X, const double2* __restrict__ Y, const double* __restrict__ rho,
     int N, int nq, const double* __restrict__ fY, const double* __restrict__ fP,
-    const int* __restrict__ active, const int* __restrict__ iqp,
-    const int* __restrict__ partner, const double2* __restrict__ alq,
-    const double2* __restrict__ R1, int C, int ngroups, int ntile, int apply_v4,
-    double2* __restrict__ wc, double2* __restrict__ wd, double2* __restrict__ fpart) {
-  __shared__ double red[4][CB][2 * NB];
-  int tile, g;
-  if (!xcd_tile(blockIdx.x, ngroups, ntile, tile, g)) return;
+    const int* __restrict__ active, const int* __restrict__ iqp, const int* __restrict__ npairs,
+    const int* __restrict__ pq1, const int* __restrict__ pq2, int MP,
+    const double2* __restrict__ alq, const double2* __restrict__ R1, int C, int ntile,
+    int apply_v4, double2* __restrict__ wc, double2* __restrict__ wd,
+    double2* __restrict__ fpart) {
+  constexpr int PB = 16;   // pairs whose blocks are in LDS at a time
+  __shared__ double2 As[PB][NB * NB];
+  __shared__ double red[4][2 * NB];
+  int tile, c;
+  if (!xcd_tile(blockIdx.x, C, ntile, tile, c)) return;
+  if (!active[c]) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int c0 = g * CB;
-  unsigned act = 0;
-#pragma unroll
-  for (int k = 0; k < CB; ++k)
-    if (c0 + k < C && active[c0 + k]) act |= 1u << k;
-  if (!act) return;
   const int i = tile * blockDim.x + t;
   const bool in = i < N;
-  double2 tot[CB], bfw[CB];
-#pragma unroll
-  for (int k = 0; k < CB; ++k) tot[k] = bfw[k] = make_double2(0.0, 0.0);
-  if (in) {
-    for (int q = 0; q < nq; ++q) {
-      double2 xq[NB], yq[NB];
-#pragma unroll
-      for (int v = 0; v < NB; ++v) {
-        xq[v] = X[((long)q * NB + v) * N + i];
-        yq[v] = csc(Y[((long)q * NB + v) * N + i], fP[q * NB + v]);
-      }
-#pragma unroll
-      for (int k = 0; k < CB; ++k) {
-        if (!((act >> k) & 1u)) continue;
-        const int c = c0 + k;
-        const int q2 = partner[c * nq + q];
-        const double2* A = alq + ((long)c * nq + q) * NB * NB;
-        double2 x2[NB];
-#pragma unroll
-        for (int v = 0; v < NB; ++v) x2[v] = X[((long)q2 * NB + v) * N + i];
-#pragma unroll
-        for (int v1 = 0; v1 < NB; ++v1) {
-          double2 bu = cmul(A[v1 * NB], x2[0]);
-#pragma unroll
-          for (int v2 = 1; v2 < NB; ++v2) bu = cmac(bu, A[v1 * NB + v2], x2[v2]);
-          tot[k] = cmacj(tot[k], bu, xq[v1]);      // conj(x) bu
-          bfw[k] = cmacj(bfw[k], yq[v1], bu);      // conj(bu) fP y
-        }
-      }
+  const int il = min(i, N - 1);   // (what lanes past the end sum is not used)
+  double2 tot = make_double2(0.0, 0.0), bfw = tot;
+  const int np = npairs[c];
+  for (int p = 0; p < np; ++p) {
+    if (p % PB == 0) {
+      __syncthreads();
+      for (int e = t; e < min(PB, np - p) * NB * NB; e += blockDim.x)
+        As[e / (NB * NB)][e % (NB * NB)] =
+            alq[((long)c * nq + pq1[c * MP + p + e / (NB * NB)]) * NB * NB + e % (NB * NB)];
+      __syncthreads();
     }
-  }
-  const double r = in ? rho[i] : 0.0;
-#pragma unroll
-  for (int k = 0; k < CB; ++k) {
-    if (!((act >> k) & 1u)) continue;
-    const int c = c0 + k;
-    const int qp = iqp[c];
-    double2 fc[NB];
-#pragma unroll
-    for (int v = 0; v < NB; ++v) fc[v] = make_double2(0.0, 0.0);
-    if (in) {
-      double2 wR = make_double2(0.0, 0.0), wRf = make_double2(0.0, 0.0);
-      double2 xp[NB], yp[NB];
-#pragma unroll
-      for (int v = 0; v < NB; ++v) {
-        xp[v] = X[((long)qp * NB + v) * N + i];
-        yp[v] = Y[((long)qp * NB + v) * N + i];
-        const double2 r1 = R1[c * NB + v];
-        wR = cadd(wR, csc(cmulcj(xp[v], r1), fY[qp * NB + v]));
-        wRf = cadd(wRf, cmulcj(yp[v], r1));
-      }
-      wR = csc(wR, r / 3.0);
-      wRf = csc(wRf, r / 3.0);
-      const double2 w1 = csc(tot[k], -0.5 * r / 3.0);
-      const double2 w2 = csc(bfw[k], -r / 3.0);
-#pragma unroll
-      for (int v = 0; v < NB; ++v)
-        fc[v] = cadd(cmul(w1, yp[v]), csc(cmul(w2, xp[v]), fY[qp * NB + v]));
-      double2 c1 = wR, c2 = wRf;
-      if (apply_v4) {
-        c1 = cadd(c1, csc(tot[k], -r / 8.0));
-        c2 = cadd(c2, csc(bfw[k], -r / 4.0));
-      }
-      wc[(long)c * N + i] = c1;
-      wd[(long)c * N + i] = c2;
-    }
-    // fixed-order reduction of the f_pert contributions: waves, then the
-    // workgroup's waves in order
+    const int q1 = pq1[c * MP + p], q2 = pq2[c * MP + p];
+    const double2* A = As[p % PB];
+    double2 x1[NB], y1[NB], x2[NB], y2[NB];
 #pragma unroll
     for (int v = 0; v < NB; ++v) {
-      const double sx = wave_sum(fc[v].x), sy = wave_sum(fc[v].y);
-      if (lane == 0) {
-        red[wv][k][2 * v] = sx;
-        red[wv][k][2 * v + 1] = sy;
+      x1[v] = X[((long)q1 * NB + v) * N + il];
+      x2[v] = X[((long)q2 * NB + v) * N + il];
+      y1[v] = Y[((long)q1 * NB + v) * N + il];
+      y2[v] = Y[((long)q2 * NB + v) * N + il];
+    }
+    double2 b2[NB], t1 = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int v = 0; v < NB; ++v) b2[v] = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int v1 = 0; v1 < NB; ++v1) {
+      double2 b1 = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int v2 = 0; v2 < NB; ++v2) {
+        const double2 e = A[v1 * NB + v2];
+        b1 = cmac(b1, e, x2[v2]);
+        b2[v2] = cmacj(b2[v2], x1[v1], e);   // conj(A[v1][v2]) x1[v1]
       }
+      t1 = cmacj(t1, b1, x1[v1]);                                  // conj(x) bu
+      bfw = cmacj(bfw, csc(y1[v1], fP[q1 * NB + v1]), b1);         // conj(bu) fP y
+    }
+    if (q1 == q2) {
+      tot = cadd(tot, t1);
+    } else {
+      tot.x += 2.0 * t1.x;
+#pragma unroll
+      for (int v = 0; v < NB; ++v) bfw = cmacj(bfw, csc(y2[v], fP[q2 * NB + v]), b2[v]);
+    }
+  }
+  const int qp = iqp[c];
+  double2 fc[NB];
+#pragma unroll
+  for (int v = 0; v < NB; ++v) fc[v] = make_double2(0.0, 0.0);
+  if (in) {
+    const double r = rho[i];
+    double2 wR = make_double2(0.0, 0.0), wRf = make_double2(0.0, 0.0);
+    double2 xp[NB], yp[NB];
+#pragma unroll
+    for (int v = 0; v < NB; ++v) {
+      xp[v] = X[((long)qp * NB + v) * N + i];
+      yp[v] = Y[((long)qp * NB + v) * N + i];
+      const double2 r1 = R1[c * NB + v];
+      wR = cadd(wR, csc(cmulcj(xp[v], r1), fY[qp * NB + v]));
+      wRf = cadd(wRf, cmulcj(yp[v], r1));
+    }
+    wR = csc(wR, r / 3.0);
+    wRf = csc(wRf, r / 3.0);
+    const double2 w1 = csc(tot, -0.5 * r / 3.0);
+    const double2 w2 = csc(bfw, -r / 3.0);
+#pragma unroll
+    for (int v = 0; v < NB; ++v)
+      fc[v] = cadd(cmul(w1, yp[v]), csc(cmul(w2, xp[v]), fY[qp * NB + v]));
+    if (apply_v4) {
+      wR = cadd(wR, csc(tot, -r / 8.0));
+      wRf = cadd(wRf, csc(bfw, -r / 4.0));
+    }
+    wc[(long)c * N + i] = wR;
+    wd[(long)c * N + i] = wRf;
+  }
+  // fixed-order reduction of the f_pert contributions: waves, then the
+  // workgroup's waves in order
+#pragma unroll
+  for (int v = 0; v < NB; ++v) {
+    const double sx = wave_sum(fc[v].x), sy = wave_sum(fc[v].y);
+    if (lane == 0) {
+      red[wv][2 * v] = sx;
+      red[wv][2 * v + 1] = sy;
     }
   }
   __syncthreads();
-  if (t < CB * NB) {
-    const int k = t / NB, v = t % NB;
-    if ((act >> k) & 1u) {
-      double sx = 0.0, sy = 0.0;
-      for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-        sx += red[w][k][2 * v];
-        sy += red[w][k][2 * v + 1];
-      }
-      fpart[((long)(c0 + k) * ntile + tile) * NB + v] = make_double2(sx, sy);
+  if (t < NB) {
+    double sx = 0.0, sy = 0.0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
+      sx += red[w][2 * t];
+      sy += red[w][2 * t + 1];
     }
+    fpart[((long)c * ntile + tile) * NB + t] = make_double2(sx, sy);
   }
 }
 
@@ -580,7 +585,7 @@ __global__ void __launch_bounds__(kD2vThreads) __attribute__((amdgpu_waves_per_e
 // Sixteen waves: `slices` of the slab's steps of four configurations (fixed by T, so
 // that a chain's sums do not depend on its batch) times 16 / slices columns, groups of
 // items dealt to the columns in turn.  64 chains on 4x4x4: 859 us with a thread per
-// item, MMA64 us; 8 chains on 2x2x2 with 48 images: 61, MMA8 us.
+// item, 708 us; 8 chains on 2x2x2 with 48 images: 61, 41 us.
 constexpr int mma_slices(int T) { return T / 4; }
 constexpr int mma_cap(int T) { return 16 / mma_slices(T) * kMmaGroups * 4; }
 
@@ -1078,7 +1083,7 @@ static int build_batch(QCtx* q, int C, const int* iq_pert, const int* pair_map, 
   b.C = C;
   b.MP = nq;
   std::vector<int> h_iqp(C), h_np(C), h_pq1((size_t)C * nq, 0), h_pq2((size_t)C * nq, 0),
-      h_offa((size_t)C * nq, 0), h_offb((size_t)C * nq, 0), h_part((size_t)C * nq),
+      h_offa((size_t)C * nq, 0), h_offb((size_t)C * nq, 0),
       h_apair((size_t)C * nq), h_orient((size_t)C * nq), h_len(C);
   int maxp = 0;
   for (int c = 0; c < C; ++c) {
@@ -1102,7 +1107,6 @@ static int build_batch(QCtx* q, int C, const int* iq_pert, const int* pair_map, 
         }
         ++np;
       }
-    for (int i = 0; i < nq; ++i) h_part[(size_t)c * nq + i] = pm[i];
     int off = nb;
     for (int p = 0; p < np; ++p) {
       h_offa[(size_t)c * nq + p] = off;
@@ -1175,7 +1179,6 @@ static int build_batch(QCtx* q, int C, const int* iq_pert, const int* pair_map, 
   table(&b.pq2, h_pq2);
   table(&b.offa, h_offa);
   table(&b.offb, h_offb);
-  table(&b.partner, h_part);
   table(&b.apair, h_apair);
   table(&b.aorient, h_orient);
   table(&b.active, ones);
@@ -1229,12 +1232,10 @@ static void launch_L_nb(QCtx* q, QBatch& b, const double2* psi, double2* out, in
       hipLaunchKernelGGL(q_unpack<NB>, dim3(nq, C), dim3(64), 0, s, psi, b.ld, b.active, b.pq1,
                          b.pq2, b.offa, b.offb, MP, nq, b.apair, b.aorient, q->wq, q->nbose,
                          q->valid, ignore_v3, b.alpha, b.R1);
-    constexpr int CB = kQWeightsChains;
-    const int ngroups = (C + CB - 1) / CB;
-    const int nblk = (b.ntile + 7) / 8 * 8 * ngroups;
-    hipLaunchKernelGGL((q_weights<NB, CB>), dim3(nblk), dim3(q->weights_tile), 0, s, q->X, q->Y,
-                       q->rho, q->N, nq, q->fY, q->fP, b.active, b.iqp, b.partner, b.alpha, b.R1,
-                       C, ngroups, b.ntile, ignore_v4 ? 0 : 1, b.wc, b.wd, b.fpart);
+    hipLaunchKernelGGL(q_weights<NB>, dim3((b.ntile + 7) / 8 * 8 * C), dim3(q->weights_tile), 0, s,
+                       q->X, q->Y, q->rho, q->N, nq, q->fY, q->fP, b.active, b.iqp, b.npairs,
+                       b.pq1, b.pq2, MP, b.alpha, b.R1, C, b.ntile, ignore_v4 ? 0 : 1, b.wc, b.wd,
+                       b.fpart);
     if (b.slabT) {
       const int nblk2 = q->mma ? (b.nch * b.nib + 7) / 8 * 8 : (b.nch + 7) / 8 * 8 * b.nib;
       auto run = [&](auto kernel, int threads) {
