@@ -19,8 +19,6 @@
 namespace tdscha {
 
 int run_pa(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_dev, hipStream_t s);
-bool orbit_translations(Ctx* c, int n_cart, const double* pols, int n_cells, const int* inv_perms,
-                        const double* proj);
 
 // coefficient rows of c->std_coef
 enum { SC_X = 0, SC_Y = 1, SC_X1 = 2, SC_Y1 = 3 };
@@ -656,8 +654,7 @@ int tdscha_set_translations(tdscha_ctx* ctx, int n_cart, const double* pols, int
   TDS_CHECK_HIP(hipMemcpy(c->tproj, tT.data(), sizeof(double) * (long)n * n,
                           hipMemcpyHostToDevice));
   c->n_cells = n_cells;
-  c->orb.trans_ok = c->orb.usable && c->orb.group &&
-                    orbit_translations(c, n_cart, pols, n_cells, inv_perms, trans_projector);
+  c->orb.trans = -1;
   return 0;
 }
 

@@ -169,8 +169,9 @@ struct Ctx;
 
 struct Orbit {
   bool usable = false;     // tables built
-  bool group = false;      // the symmetries are closed under multiplication
-  bool trans_ok = false;   // the translation average commutes with them
+  // found by the first Lanczos run (-1: not yet)
+  int group = -1;          // the symmetries are closed under multiplication
+  int trans = -1;          // the translation average commutes with them
   int nsym = 1, npanel = 0, rows = 0;
   long Mp = 0;
   std::vector<double> syms;               // host copy of the symmetry blocks
@@ -311,6 +312,7 @@ int ensure_split(Ctx* c, int prec);
 
 void orbit_plan_free(OrbPlan& p);
 bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld);
+int orbit_sector(Ctx* c, bool* ok);
 int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p);
 int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
                  hipStream_t s);

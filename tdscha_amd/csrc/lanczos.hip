@@ -907,7 +907,14 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
     return fail("initialisation failed");
   // orbit form per group of chains, from the start vectors: an operator that
   // commutes with the symmetry group keeps their relation
-  const bool sector = !ignore_v3 && c->orb.group && (c->n_cells == 0 || c->orb.trans_ok);
+  bool sector = false;
+  for (int c0 = 0; !ignore_v3 && c0 < n_chains; c0 += kMaxChains)
+    sector = sector || orbit_worth(c, std::min(kMaxChains, n_chains - c0), precision,
+                                   psi0 + (long)c0 * len, len);
+  if (sector && orbit_sector(c, &sector)) {
+    free_state(st);
+    return -1;
+  }
   bool general = !sector;
   if (sector)
     for (int c0 = 0; c0 < n_chains; c0 += kMaxChains) {

@@ -491,7 +491,7 @@ static bool closed(Ctx* c) {
 // Whether the translation average commutes with the group's generators, on random
 // vectors: the mean projector (proj z against its rotation), and the second
 // moment over the permutations that the average of d2v applies.
-bool orbit_translations(Ctx* c, int n_cart, const double* pols, int n_cells, const int* inv_perms,
+static bool orbit_translations(Ctx* c, int n_cart, const double* pols, int n_cells, const int* inv_perms,
                         const double* proj) {
   const Orbit& o = c->orb;
   const int n = c->n;
@@ -533,6 +533,30 @@ bool orbit_translations(Ctx* c, int n_cart, const double* pols, int n_cells, con
     if (!(std::fabs(s1 - s2) <= 1e-9 * (std::fabs(s1) + std::fabs(s2)))) return false;
   }
   return true;
+}
+
+// Whether the operator commutes with the symmetries: they form a group, which commutes
+// with the translation average.  Checked once per context, by its first Lanczos run
+// that may use it (1.3 ms on the host at 381 modes).
+int orbit_sector(Ctx* c, bool* ok) {
+  Orbit& o = c->orb;
+  if (o.group < 0) o.group = closed(c);
+  if (o.group && c->n_cells > 0 && o.trans < 0) {
+    const size_t n = c->n, nc = c->n_cart;
+    std::vector<double> pols(nc * n), pt(n * n), proj(n * n);
+    std::vector<int> perms((size_t)c->n_cells * nc);
+    TDS_CHECK_HIP(hipMemcpy(pols.data(), c->pols, sizeof(double) * pols.size(),
+                            hipMemcpyDeviceToHost));
+    TDS_CHECK_HIP(hipMemcpy(pt.data(), c->tproj, sizeof(double) * pt.size(),
+                            hipMemcpyDeviceToHost));
+    TDS_CHECK_HIP(hipMemcpy(perms.data(), c->inv_perms, sizeof(int) * perms.size(),
+                            hipMemcpyDeviceToHost));
+    for (size_t a = 0; a < n; ++a)   // (kept transposed on the device)
+      for (size_t b = 0; b < n; ++b) proj[a * n + b] = pt[b * n + a];
+    o.trans = orbit_translations(c, c->n_cart, pols.data(), c->n_cells, perms.data(), proj.data());
+  }
+  *ok = o.group && (c->n_cells == 0 || o.trans);
+  return 0;
 }
 
 static double estimate_us(double flop, int prec) {
@@ -579,7 +603,6 @@ int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const in
   start[nreal] = n;
   const size_t ntab = (size_t)nreal * n_syms * kOP * kOP;
   o.syms = syms;
-  o.group = closed(c);
   // probe configurations: thermal amplitudes for x; forces of the same weight
   // in s2 = u.Y1.(fpsi f) as x has in s1
   std::mt19937_64 g(2024);
