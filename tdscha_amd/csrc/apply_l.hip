@@ -123,20 +123,6 @@ __global__ void prepare_pert(const double* __restrict__ psi_all, long len, int n
   if (e < np) R1p[(long)chain * np + e] = (e < n) ? psi[e] : 0.0;
 }
 
-// final (normalised, unpadded) f and d2v from the K-split sums
-__global__ void finalize_pa(const double* __restrict__ zsum_all, const double* __restrict__ fsum,
-                            const double* __restrict__ fy, int n, int np, double norm,
-                            double* __restrict__ f_all, double* __restrict__ d2v_all) {
-  const int chain = blockIdx.y;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) f_all[(long)chain * n + e] = fsum[(long)chain * np + e];
-  if (e >= (long)n * n) return;
-  const int mu = (int)(e / n), nu = (int)(e % n);
-  const double* z = zsum_all + (long)chain * np * np;
-  d2v_all[(long)chain * n * n + e] =
-      norm * (fy[mu] * z[(long)mu * np + nu] + fy[nu] * z[(long)nu * np + mu]);
-}
-
 // C = op(A) op(B), FP64, batched (blockIdx.z), on v_mfma_f64_16x16x4f64.
 // A 32 x 32 output tile per work-group; the four waves split each 64-deep K
 // chunk (16 rows each) and their partial tiles are summed in LDS in wave
@@ -357,60 +343,181 @@ int project_translations(Ctx* c, int nc, hipStream_t s) {
 }
 
 // out = [L1 + L_anh](psi), then reverse/shift
-__global__ void assemble_out(const double* __restrict__ psi_all, long len, int n,
-                             const double* __restrict__ w, const double* __restrict__ f_all,
-                             const double* __restrict__ d2v_all, const int* __restrict__ prow,
-                             const int* __restrict__ pcol, const double* __restrict__ sm,
-                             const double* __restrict__ sp, const double* __restrict__ ha,
-                             const double* __restrict__ hb, const double* __restrict__ sc,
-                             const double* __restrict__ yw, const double* __restrict__ reaw,
-                             int use_wigner, int transpose, int harmonic, int anharmonic,
-                             int reverse, double shift, double* __restrict__ out_all) {
-  const int chain = blockIdx.y;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// what the entries of L psi need beside psi and the averages
+struct OutForm {
+  int n;
+  long P;   // n (n + 1) / 2 mode pairs
+  const double *w, *sm, *sp, *ha, *hb, *sc, *yw, *reaw;
+  const int *prow, *pcol;
+  int use_wigner, transpose, harmonic, anharmonic, reverse;
+  double shift;
+};
+
+__device__ __forceinline__ double out_mode(const OutForm& o, int e, double psi, double f) {
+  const double wm = o.w[e];
+  double v = 0.0;
+  if (o.harmonic) v = o.use_wigner ? -(psi * wm) * wm : (psi * wm) * wm;
+  if (o.anharmonic) v += o.use_wigner ? f : -f;
+  if (o.reverse) v = -v;
+  return v + o.shift * psi;
+}
+
+// pair p = (r, col) of the first (secA) or second sector; pa, pb: psi's two sectors at p
+__device__ __forceinline__ double out_pair(const OutForm& o, long p, int r, int col, bool secA,
+                                           double pa, double pb, double d) {
+  const long P = o.P;
+  double v = 0.0;
+  if (o.use_wigner) {
+    if (o.harmonic) v = secA ? o.ha[p] * pa : o.hb[p] * pb;
+    if (o.anharmonic) v += secA ? o.sm[p] * d : -o.sp[p] * d;
+  } else {
+    if (o.harmonic) {
+      const double X = o.sc[SC_X * P + p], Y = o.sc[SC_Y * P + p];
+      const double X1 = o.sc[SC_X1 * P + p], Y1 = o.sc[SC_Y1 * P + p];
+      if (!o.transpose)
+        v = secA ? (-X * pa - Y * pb) : (-X1 * pa - Y1 * pb);
+      else
+        v = secA ? (-X * pa - X1 * pb) : (-Y * pa - Y1 * pb);
+    }
+    if (o.anharmonic) {
+      double pert;
+      if (!o.transpose)
+        pert = secA ? d * (o.yw[r] + o.yw[col]) : d * (o.reaw[r] + o.reaw[col]);
+      else
+        pert = secA ? 0.5 * d / (o.yw[r] * o.yw[col]) * (r == col ? 1.0 : 2.0) : 0.0;
+      v -= pert;
+    }
+  }
+  if (o.reverse) v = -v;
+  return v + o.shift * (secA ? pa : pb);
+}
+
+__global__ void assemble_out(const double* __restrict__ psi_all, long len,
+                             const double* __restrict__ f_all, const double* __restrict__ d2v_all,
+                             OutForm o, double* __restrict__ out_all) {
+  const int chain = blockIdx.y, n = o.n;
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x, P = o.P;
   if (e >= len) return;
   const double* psi = psi_all + chain * len;
-  const double* f = f_all + (long)chain * n;
-  const double* d2v = d2v_all + (long)chain * n * n;
-  const long P = (long)n * (n + 1) / 2;
-  double v = 0.0;
+  double v;
   if (e < n) {
-    const double wm = w[e];
-    if (harmonic) v = use_wigner ? -(psi[e] * wm) * wm : (psi[e] * wm) * wm;
-    if (anharmonic) v += use_wigner ? f[e] : -f[e];
+    v = out_mode(o, (int)e, psi[e], f_all[(long)chain * n + e]);
   } else {
     const bool secA = e < n + P;
     const long p = secA ? e - n : e - n - P;
-    const int r = prow[p], col = pcol[p];
-    const double pa = psi[n + p], pb = psi[n + P + p];
-    if (use_wigner) {
-      if (harmonic) v = secA ? ha[p] * pa : hb[p] * pb;
-      if (anharmonic) {
-        const double d = d2v[(long)r * n + col];
-        v += secA ? sm[p] * d : -sp[p] * d;
-      }
-    } else {
-      if (harmonic) {
-        const double X = sc[SC_X * P + p], Y = sc[SC_Y * P + p];
-        const double X1 = sc[SC_X1 * P + p], Y1 = sc[SC_Y1 * P + p];
-        if (!transpose)
-          v = secA ? (-X * pa - Y * pb) : (-X1 * pa - Y1 * pb);
-        else
-          v = secA ? (-X * pa - X1 * pb) : (-Y * pa - Y1 * pb);
-      }
-      if (anharmonic) {
-        const double d = d2v[(long)r * n + col];
-        double pert;
-        if (!transpose)
-          pert = secA ? d * (yw[r] + yw[col]) : d * (reaw[r] + reaw[col]);
-        else
-          pert = secA ? 0.5 * d / (yw[r] * yw[col]) * (r == col ? 1.0 : 2.0) : 0.0;
-        v -= pert;
-      }
+    const int r = o.prow[p], col = o.pcol[p];
+    v = out_pair(o, p, r, col, secA, psi[n + p], psi[n + P + p],
+                 d2v_all[((long)chain * n + r) * n + col]);
+  }
+  out_all[chain * len + e] = v;
+}
+
+// The end of an FP64 call whose modes fit one tile (at most 128), in one launch: the
+// K-split partials summed in a fixed order, d2v symmetrised and normalised, and, with
+// OUT, the entries of L psi.  A work-group takes an 8 x 8 block of Z and its mirror
+// image, the partials in 16 slices, 16 loads in flight per thread; the last
+// ceil(n / 64) work-groups of a chain take f.  Bound by launches and latency: sums,
+// symmetrisation and assembly as kernels of their own took 4.2 + 3.4 + 3.7 us and their
+// gaps at 45 modes and 64 partials, one kernel takes 5.0 us.
+template <bool OUT>
+__global__ __launch_bounds__(1024) void finish_f64(
+    const double* __restrict__ zpart_all, const double* __restrict__ fpart_all, int n, int np,
+    int zl, int ks, const double* __restrict__ fy, double norm, double* __restrict__ f_all,
+    double* __restrict__ d2v_all, const double* __restrict__ psi_all, long len, OutForm o,
+    double* __restrict__ out_all) {
+  const int chain = blockIdx.y, t = threadIdx.x & 63, sl = threadIdx.x >> 6;
+  const int nt = (n + 7) / 8, nblk = nt * (nt + 1) / 2;
+  const bool isf = (int)blockIdx.x >= nblk;
+  const long zz = (long)zl * zl, P = o.P;
+  int ti = 0, b = blockIdx.x;
+  if (!isf)
+    for (; b >= nt - ti; ++ti) b -= nt - ti;
+  const int tj = ti + b, mu = 8 * ti + (t >> 3), nu = 8 * tj + (t & 7);
+  const int fe = 64 * ((int)blockIdx.x - nblk) + t;
+  const double* psi = psi_all + (long)chain * len;
+  const bool mine = sl == 0 && (isf ? fe < n : mu <= nu && nu < n);
+  const long p = (long)mu * n - (long)mu * (mu - 1) / 2 + (nu - mu);
+  double pa = 0.0, pb = 0.0;
+  if (OUT && mine) {   // on their way while the partials are summed
+    pa = psi[isf ? fe : n + p];
+    if (!isf) pb = psi[n + P + p];
+  }
+  const double* z1;
+  const double* z2;
+  long stride;
+  if (isf) {
+    z1 = z2 = fpart_all + (long)chain * ks * np + (fe < n ? fe : 0);
+    stride = np;
+  } else {
+    const double* z = zpart_all + (long)chain * ks * zz;
+    z1 = z + (long)mu * zl + nu;
+    z2 = z + (long)(8 * tj + (t >> 3)) * zl + 8 * ti + (t & 7);
+    stride = zz;
+  }
+  const int per = (ks + 15) / 16, lo = sl * per, hi = lo + per < ks ? lo + per : ks;
+  double s1 = 0.0, s2 = 0.0;
+  for (int k = lo; k < hi; k += 8) {
+    double v1[8], v2[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {   // (a load behind a condition would wait by itself)
+      const long q = (k + j < hi ? k + j : hi - 1) * stride;
+      v1[j] = z1[q];
+      v2[j] = z2[q];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      s1 += k + j < hi ? v1[j] : 0.0;
+      s2 += k + j < hi ? v2[j] : 0.0;
     }
   }
-  if (reverse) v = -v;
-  out_all[chain * len + e] = v + shift * psi[e];
+  __shared__ double red[2][16][64];
+  red[0][sl][t] = s1;
+  red[1][sl][t] = s2;
+  __syncthreads();
+  if (!mine) return;
+  const int tt = isf ? t : (t & 7) * 8 + (t >> 3);   // this element's mirror image
+  double a = 0.0, m = 0.0;
+#pragma unroll
+  for (int q = 0; q < 16; q += 4) {
+    a += (red[0][q][t] + red[0][q + 1][t]) + (red[0][q + 2][t] + red[0][q + 3][t]);
+    m += (red[1][q][tt] + red[1][q + 1][tt]) + (red[1][q + 2][tt] + red[1][q + 3][tt]);
+  }
+  if (isf) {
+    if (OUT)
+      out_all[chain * len + fe] = out_mode(o, fe, pa, a * norm);
+    else
+      f_all[(long)chain * n + fe] = a * norm;
+    return;
+  }
+  const double d = norm * (fy[mu] * a + fy[nu] * m);
+  if (OUT) {
+    out_all[chain * len + n + p] = out_pair(o, p, mu, nu, true, pa, pb, d);
+    out_all[chain * len + n + P + p] = out_pair(o, p, mu, nu, false, pa, pb, d);
+  } else {
+    double* v = d2v_all + (long)chain * n * n;
+    v[(long)mu * n + nu] = d;
+    v[(long)nu * n + mu] = d;
+  }
+}
+
+static OutForm out_form(const Ctx* c, int use_wigner, int transpose, int harmonic, int anharmonic,
+                        int reverse, double shift) {
+  return {c->n, (long)c->n * (c->n + 1) / 2, c->w, c->pair_sm, c->pair_sp, c->pair_harm_a,
+          c->pair_harm_b, c->std_coef, c->yw, c->reaw, c->pair_row, c->pair_col, use_wigner,
+          transpose, harmonic, anharmonic, reverse, shift};
+}
+
+template <bool OUT>
+static void launch_finish(Ctx* c, int nc, double* f, double* d2v, const double* psi, long len,
+                          const OutForm& o, double* out, hipStream_t s) {
+  const int nt = (c->n + 7) / 8;
+  hipLaunchKernelGGL(finish_f64<OUT>, dim3(nt * (nt + 1) / 2 + (c->n + 63) / 64, nc), dim3(1024),
+                     0, s, c->zpart, c->fpart, c->n, c->np, 16 * f64_tiles(c->n).cb, c->ksplit,
+                     c->fy, 1.0 / (c->n_eff * c->n_syms), f, d2v, psi, len, o, out);
+}
+
+void launch_finish_averages(Ctx* c, int nc, double* f, double* d2v, hipStream_t s) {
+  launch_finish<false>(c, nc, f, d2v, nullptr, 0, OutForm{}, nullptr, s);
 }
 
 // R1, Y1 of the vectors, padded, into c->R1, c->Y1
@@ -434,6 +541,8 @@ int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, 
   const long P = (long)n * (n + 1) / 2;
   const long len = n + 2 * P;
   const int anharmonic = ignore_v3 ? 0 : 1;
+  const OutForm o = out_form(c, use_wigner, transpose, ignore_harmonic ? 0 : 1, anharmonic,
+                             reverse, shift);
   if (anharmonic) {
     launch_prepare_pert(c, nc, psi, use_wigner, transpose, s);
     const int d4 = ignore_v4 ? 0 : 1;
@@ -442,8 +551,15 @@ int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, 
       if (rc) return rc;
       plan = &c->orb.plan[0];
     }
-    rc = plan && plan->ok ? run_pa_orbit(c, *plan, d4, c->f_fin, c->d2v_fin, s)
-                          : run_pa(c, nc, d4, precision, c->f_fin, c->d2v_fin, s);
+    const bool orbit = plan && plan->ok;
+    if (!orbit && c->n_cells == 0 && finish_in_one(c, precision)) {
+      launch_sums_fp64(c, nc, d4, s, nullptr);
+      launch_finish<true>(c, nc, nullptr, nullptr, psi, len, o, out, s);
+      TDS_CHECK_HIP(hipGetLastError());
+      return 0;
+    }
+    rc = orbit ? run_pa_orbit(c, *plan, d4, c->f_fin, c->d2v_fin, s)
+               : run_pa(c, nc, d4, precision, c->f_fin, c->d2v_fin, s);
     if (rc) return rc;
     if (c->n_cells > 0) {
       rc = project_translations(c, nc, s);
@@ -452,10 +568,7 @@ int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, 
   }
   const double* f_src = (anharmonic && c->n_cells > 0) ? c->f_proj : c->f_fin;
   hipLaunchKernelGGL(assemble_out, dim3((unsigned)((len + 255) / 256), nc), dim3(256), 0, s, psi,
-                     len, n, c->w, f_src, c->d2v_fin, c->pair_row, c->pair_col, c->pair_sm,
-                     c->pair_sp, c->pair_harm_a, c->pair_harm_b, c->std_coef, c->yw, c->reaw,
-                     use_wigner, transpose, ignore_harmonic ? 0 : 1, anharmonic, reverse, shift,
-                     out);
+                     len, f_src, c->d2v_fin, o, out);
   TDS_CHECK_HIP(hipGetLastError());
   return 0;
 }

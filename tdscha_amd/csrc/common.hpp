@@ -340,5 +340,13 @@ void launch_outer_f64(const F64Rows& r, int n, int np, int nc, const double* coe
                       double* zpart, double* fpart, hipStream_t s);
 void launch_reduce_f64(int n, int np, int nc, int ksplit, const double* zpart,
                        const double* fpart, double* zsum, double* f, double norm, hipStream_t s);
+void launch_sums_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev);
+// One tile of modes (the image form): sums and output in one launch up to 256 partials.
+// Its work-groups read whole 8 x 8 blocks of every partial (45 modes: 64 partials
+// 5.0 us, 512 13.3); sums and symmetrisation as two kernels take about 10 us.
+inline bool finish_in_one(const Ctx* c, int prec) {
+  return prec == PREC_FP64 && !c->rotate && f64_tiles(c->n).ntile == 1 && c->ksplit <= 256;
+}
+void launch_finish_averages(Ctx* c, int nc, double* f, double* d2v, hipStream_t s);
 
 }  // namespace tdscha

@@ -93,6 +93,12 @@ static int choose_ksplit(int n, long Mp) {
 int run_pa(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_dev, hipStream_t s) {
   if (c->rotate) return run_pa_rot(c, nc, apply_d4, prec, f_dev, d2v_dev, s);
   int rc;
+  if (finish_in_one(c, prec)) {
+    launch_sums_fp64(c, nc, apply_d4, s, nullptr);
+    launch_finish_averages(c, nc, f_dev, d2v_dev, s);
+    TDS_CHECK_HIP(hipGetLastError());
+    return 0;
+  }
   if (prec == PREC_FP64) {
     rc = launch_pa_fp64(c, nc, apply_d4, s, nullptr);
   } else {

@@ -616,7 +616,8 @@ void launch_reduce_f64(int n, int np, int nc, int ksplit, const double* zpart,
                        zsum, f, norm);
 }
 
-int launch_pa_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev) {
+// weights and K-split partials of c->R1/c->Y1
+void launch_sums_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev) {
   const F64Rows rows{c->U, c->F, c->rho_img, c->Mp};
   // image range [row_lo, row_hi): whole 64-row tiles of the weights kernel
   // (rows outside the range get zero coefficients), and the outer GEMM's K
@@ -632,6 +633,10 @@ int launch_pa_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev) 
   launch_outer_f64(rows, c->n, c->np, nc, c->coef, c->fy, c->ksplit, kb, ke, rps, 0, c->zpart,
                    c->fpart, s);
   if (ev) (void)hipEventRecord(ev[2], s);
+}
+
+int launch_pa_fp64(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* ev) {
+  launch_sums_fp64(c, nc, apply_d4, s, ev);
   // zsum -> c->d2v_out (padded), normalised f -> c->f_out
   launch_reduce_f64(c->n, c->np, nc, c->ksplit, c->zpart, c->fpart, c->d2v_out, c->f_out,
                     1.0 / (c->n_eff * c->n_syms), s);
