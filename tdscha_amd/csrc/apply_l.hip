@@ -530,11 +530,12 @@ void launch_prepare_pert(Ctx* c, int nc, const double* psi, int use_wigner, int 
 }
 
 // plan: the orbit form of these vectors (a Lanczos run's); psi_host: the host's copy
-// of psi, where one may be looked for (waits for the stream)
+// of psi, where one may be looked for (waits for the stream); prepared: R1 and Y1 are in
+// place already (a short chain's)
 int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, int transpose,
                 int ignore_harmonic, int ignore_v3, int ignore_v4, int reverse, double shift,
                 int precision, hipStream_t s, const OrbPlan* plan,
-                const double* psi_host) {
+                const double* psi_host, bool prepared) {
   int rc = setup_pairs(c);
   if (rc) return rc;
   const int n = c->n;
@@ -544,7 +545,7 @@ int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, 
   const OutForm o = out_form(c, use_wigner, transpose, ignore_harmonic ? 0 : 1, anharmonic,
                              reverse, shift);
   if (anharmonic) {
-    launch_prepare_pert(c, nc, psi, use_wigner, transpose, s);
+    if (!prepared) launch_prepare_pert(c, nc, psi, use_wigner, transpose, s);
     const int d4 = ignore_v4 ? 0 : 1;
     if (!plan && psi_host && orbit_worth(c, nc, precision, psi_host, len)) {
       rc = orbit_plan(c, nc, precision, s, c->orb.plan[0]);
@@ -782,7 +783,7 @@ int tdscha_apply_L_dev(tdscha_ctx* ctx, int n_vec, const double* psi_dev, double
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : c->stream;
   return apply_L_dev(c, n_vec, psi_dev, out_dev, use_wigner, transpose, ignore_harmonic, ignore_v3,
-                     ignore_v4, reverse, shift, precision, s, nullptr, nullptr);
+                     ignore_v4, reverse, shift, precision, s, nullptr, nullptr, false);
 }
 
 int tdscha_apply_L(tdscha_ctx* ctx, int n_vec, const double* psi, double* out, int use_wigner,
@@ -805,7 +806,7 @@ int tdscha_apply_L(tdscha_ctx* ctx, int n_vec, const double* psi, double* out, i
     TDS_CHECK_HIP(hipMemcpyAsync(in, psi, bytes, hipMemcpyHostToDevice, c->stream));
   TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0, 1 or 2");
   rc = apply_L_dev(c, n_vec, in, res, use_wigner, transpose, ignore_harmonic, ignore_v3,
-                   ignore_v4, reverse, shift, precision, c->stream, nullptr, psi);
+                   ignore_v4, reverse, shift, precision, c->stream, nullptr, psi, false);
   if (rc) return rc;
   if (!pinned) TDS_CHECK_HIP(hipMemcpyAsync(out, res, bytes, hipMemcpyDeviceToHost, c->stream));
   TDS_CHECK_HIP(hipStreamSynchronize(c->stream));
