@@ -1,8 +1,8 @@
 """GPU: the d2v blocks and the final sums of the q-space application in slices.
 
-Grids of 1, 8 and 27 q-points with 6 or 3 bands give every slab length that shares an
-item between threads (16, 8 and 4 configurations: 8, 4 and 2 threads), 64 q-points the
-one that does not;
+Grids of 1, 8 and 27 q-points with 6 or 3 bands give every slab length (16, 8 and 4
+configurations) in both forms, matrix instructions (6 bands) and a thread per item (3
+bands), 64 q-points the longest item lists;
 configuration counts below one slab, at its edges and with several chunks; batches
 with fewer items than a work-group and more.  Against the direct form of d2v (one
 pair and chunk per work-group) on the same engine: FP64 sums of the same terms in
