@@ -236,7 +236,6 @@ struct Ctx {
   double* ysc = nullptr;    // [kMaxChains] power-of-two scale of split Y1
   double* ysc3 = nullptr;   // [kMaxChains] scale of the folded fY R1 column
   double* bsc = nullptr;    // [kMaxChains, np] column scale of split B
-  double* cmax = nullptr;   // [kMaxChains, 2] max|c1|, max|c2| (device)
   double* pmax = nullptr;   // [kMaxChains, kPartBlocks, 2] per-block maxima of the split prep
   float* epi = nullptr;     // [kMaxChains, 2, np] fY R1 and R1 (weights epilogue)
   float* coef32 = nullptr;  // [Mp/16, kMaxChains, 4, 16] FP32 coefficients for the outer GEMM

@@ -185,41 +185,46 @@ __global__ void split_images(const double* __restrict__ U, const double* __restr
 }
 
 // ------------------------------------------------------------ per-call prep
+// The preparation takes its chain-wide maxima from the block maxima of the kernel
+// before, in every work-group that needs them: as kernels of their own the three
+// scales (Y1, the folded column, B) were launches of 2 to 5 us each (one chain of 45
+// modes over 5238 configurations, whole call: 92 -> 82 us).
+
+// maximum over a work-group of 256; red: 4 entries
+__device__ __forceinline__ double block_max256(double v, double* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+  __syncthreads();   // (red may still be read)
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+}
+
 // One power-of-two scale per chain for the split Y1: sy with
 // max_jk |Y1[j][k] / su[k]| * sy < 2^12.  Block maxima over slices of Y1
-// (grid kYmaxBlocks x chains), then one block per chain.
+// (grid kYmaxBlocks x chains); prep_y takes the maximum of these, one per lane.
 constexpr int kYmaxBlocks = 64;
 __global__ void ymax_part_kernel(const double* __restrict__ Y1all, const double* __restrict__ su,
                                  int np, double* __restrict__ pmax) {
   const int chain = blockIdx.y;
   const double* Y = Y1all + (long)chain * np * np;
-  const long nn = (long)np * np, per = (nn + gridDim.x - 1) / gridDim.x;
-  const long lo = blockIdx.x * per, hi = lo + per < nn ? lo + per : nn;
-  __shared__ double red[256];
+  const int nn = np * np, per = (nn + gridDim.x - 1) / gridDim.x;
+  const int lo = blockIdx.x * per, hi = min(lo + per, nn);
+  __shared__ double red[4];
   double mx = 0.0;
-  for (long e = lo + threadIdx.x; e < hi; e += blockDim.x) mx = fmax(mx, fabs(Y[e] / su[e % np]));
-  red[threadIdx.x] = mx;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + o]);
-    __syncthreads();
+  for (int e0 = lo + threadIdx.x; e0 < hi; e0 += 4 * 256) {
+    double y[4], u[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {   // (clamped: an entry twice leaves the maximum as it is)
+      const int e = min(e0 + 256 * k, hi - 1);
+      y[k] = Y[e];
+      u[k] = su[e % np];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mx = fmax(mx, fabs(y[k] / u[k]));
   }
-  if (threadIdx.x == 0) pmax[((long)chain * kPartBlocks + blockIdx.x) * 2] = red[0];
-}
-
-__global__ void ymax_kernel(const double* __restrict__ pmax, int nblocks, double* __restrict__ ysc) {
-  const int chain = blockIdx.x;
-  __shared__ double red[64];
-  double mx = 0.0;
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x)
-    mx = fmax(mx, pmax[((long)chain * kPartBlocks + b) * 2]);
-  red[threadIdx.x] = mx;
-  __syncthreads();
-  for (int o = 32; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + o]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) ysc[chain] = pow2_scale(red[0]);
+  mx = block_max256(mx, red);
+  if (threadIdx.x == 0) pmax[((long)chain * kPartBlocks + blockIdx.x) * 2] = mx;
 }
 
 // When the modes are padded (n < np), the fp16 path lets the row-dot
@@ -227,35 +232,34 @@ __global__ void ymax_kernel(const double* __restrict__ pmax, int nblocks, double
 // of its own per chain (sy3: max_k |fY R1 / su| sy3 < 2^12), and the
 // accumulator of that column is s3 sy3 (the padding of U and F keeps it out
 // of the other row-dots).
-__global__ void foldmax_kernel(const double* __restrict__ R1all, const double* __restrict__ su,
-                               const double* __restrict__ fy, int np, double* __restrict__ ysc3) {
-  const int chain = blockIdx.x;
-  __shared__ double red[256];
-  double mx = 0.0;
-  for (int k = threadIdx.x; k < np; k += blockDim.x)
-    mx = fmax(mx, fabs(fy[k] * R1all[(long)chain * np + k] / su[k]));
-  red[threadIdx.x] = mx;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + o]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) ysc3[chain] = pow2_scale(red[0]);
-}
-
+//
 // YB[c] block (column tile, K step) holds Y1[c][j][k] sy / su[k] split hi/lo
 // (and, with ysc3 given, fY R1 sy3 / su in the last column); per-chain
 // epilogue column factors (fY R1, R1) in FP32.  One block per (column j,
-// chain).
+// chain); column 0 writes sy, the last one sy3.
 template <typename H>
 __global__ void prep_y(const double* __restrict__ Y1all, const double* __restrict__ R1all,
                        const double* __restrict__ su, const double* __restrict__ fy, int np,
-                       const double* __restrict__ ysc, const double* __restrict__ ysc3,
-                       u16* __restrict__ YBh, u16* __restrict__ YBl, float* __restrict__ epw) {
+                       const double* __restrict__ pmax, double* __restrict__ ysc,
+                       double* __restrict__ ysc3, u16* __restrict__ YBh, u16* __restrict__ YBl,
+                       float* __restrict__ epw) {
   const int j = blockIdx.x, chain = blockIdx.y;
   const double* Y = Y1all + ((long)chain * np + j) * np;
   const bool fold = ysc3 != nullptr && j == np - 1;
-  const double sy = fold ? ysc3[chain] : ysc[chain];
+  static_assert(kYmaxBlocks == 64, "a block maximum per lane");
+  double mx = pmax[((long)chain * kPartBlocks + (threadIdx.x & 63)) * 2];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if (j == 0 && threadIdx.x == 0) ysc[chain] = pow2_scale(mx);
+  if (fold) {
+    __shared__ double red[4];
+    mx = 0.0;
+    for (int k = threadIdx.x; k < np; k += blockDim.x)
+      mx = fmax(mx, fabs(fy[k] * R1all[(long)chain * np + k] / su[k]));
+    mx = block_max256(mx, red);
+    if (threadIdx.x == 0) ysc3[chain] = pow2_scale(mx);
+  }
+  const double sy = pow2_scale(mx);
   const int nct = np / kBR, nkc = np / kBK;
   const long base = ((long)chain * nct + j / kBR) * nkc * kBE;
   for (int k = threadIdx.x; k < np; k += blockDim.x) {
@@ -597,60 +601,36 @@ __global__ void finalize_coef(const double* __restrict__ part, const double* __r
 }
 
 // One power-of-two B scale per chain: sb with max_nu (max|c1| fmx[nu] +
-// max|c2| fY[nu] umx[nu] / 2) * sb < 2^12, written for every nu (the
-// reduction undoes it per column).  One block per chain.
-__global__ void bscale_kernel(const double* __restrict__ pmax, int nblocks,
-                              const double* __restrict__ umx, const double* __restrict__ fmx,
-                              const double* __restrict__ fy, int np, double* __restrict__ cmax,
-                              double* __restrict__ sb_all) {
-  const int chain = blockIdx.x;
-  __shared__ double red[256], red2[256];
-  // max |c1|, max |c2| over the coefficient blocks
+// max|c2| fY[nu] umx[nu] / 2) * sb < 2^12, from the block maxima of finalize_coef
+// (every work-group finds it), written for every nu by the first (the reduction undoes
+// it per column); c1 and c2 of the coefficient blocks times it (exact).
+__global__ void scale_coef_kernel(const double* __restrict__ pmax, int nblocks,
+                                  const double* __restrict__ umx, const double* __restrict__ fmx,
+                                  const double* __restrict__ fy, int np, long nsub,
+                                  double* __restrict__ sb_all, float* __restrict__ coefB) {
+  const int chain = blockIdx.y;
+  __shared__ double red[4];
   double m1 = 0.0, m2 = 0.0;
   for (int bk = threadIdx.x; bk < nblocks; bk += blockDim.x) {
     const double* pm = pmax + ((long)chain * kPartBlocks + bk) * 2;
     m1 = fmax(m1, pm[0]);
     m2 = fmax(m2, pm[1]);
   }
-  red[threadIdx.x] = m1;
-  red2[threadIdx.x] = m2;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + o]);
-      red2[threadIdx.x] = fmax(red2[threadIdx.x], red2[threadIdx.x + o]);
-    }
-    __syncthreads();
-  }
-  const double a = red[0], b = 0.5 * red2[0];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    cmax[chain * 2 + 0] = a;
-    cmax[chain * 2 + 1] = red2[0];
-  }
+  const double a = block_max256(m1, red), b = 0.5 * block_max256(m2, red);
   double mx = 0.0;
   for (int nu = threadIdx.x; nu < np; nu += blockDim.x)
     mx = fmax(mx, a * fmx[nu] + b * fy[nu] * umx[nu]);
-  red[threadIdx.x] = mx;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + o]);
-    __syncthreads();
+  const double sbd = pow2_scale(block_max256(mx, red));
+  if (blockIdx.x == 0)
+    for (int nu = threadIdx.x; nu < np; nu += blockDim.x) sb_all[(long)chain * np + nu] = sbd;
+  const float sb = (float)sbd;
+  // (step, image) pairs
+  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < nsub * kBK;
+       e += (long)gridDim.x * blockDim.x) {
+    float* cb = coefB + ((e / kBK) * kMaxChains + chain) * 4 * kBK + e % kBK;
+    cb[0] *= sb;
+    cb[kBK] *= sb;
   }
-  const double sb = pow2_scale(red[0]);
-  for (int nu = threadIdx.x; nu < np; nu += blockDim.x) sb_all[(long)chain * np + nu] = sb;
-}
-
-// c1 and c2 of the coefficient blocks times the chain's B scale (exact)
-__global__ void scale_coef_kernel(const double* __restrict__ sb_all, int np, long nsub,
-                                  float* __restrict__ coefB) {
-  const int chain = blockIdx.y;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;   // (step, image) pair
-  if (e >= nsub * kBK) return;
-  const float sb = (float)sb_all[(long)chain * np];
-  float* cb = coefB + ((e / kBK) * kMaxChains + chain) * 4 * kBK + e % kBK;
-  cb[0] *= sb;
-  cb[kBK] *= sb;
 }
 
 // ------------------------------------------------------------- outer GEMM
@@ -972,7 +952,6 @@ int ensure_split(Ctx* c, int prec) {
     TDS_CHECK_HIP(hipMalloc((void**)&c->epi, sizeof(float) * kMaxChains * 2 * np));
     TDS_CHECK_HIP(hipMalloc((void**)&c->ysc, sizeof(double) * kMaxChains));
     TDS_CHECK_HIP(hipMalloc((void**)&c->ysc3, sizeof(double) * kMaxChains));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->cmax, sizeof(double) * kMaxChains * 2));
     TDS_CHECK_HIP(hipMalloc((void**)&c->pmax, sizeof(double) * kMaxChains * kPartBlocks * 2));
     TDS_CHECK_HIP(hipMalloc((void**)&c->coef32, sizeof(float) * kMaxChains * Mp * 4));
     TDS_CHECK_HIP(hipMalloc((void**)&c->wpart, sizeof(double) * kMaxChains * (np / kBR) * Mp * 4));
@@ -1021,7 +1000,7 @@ void free_split(Ctx* c) {
   drop(&c->Y1h);
   drop(&c->Y1l);
   for (float** p : {&c->epi, &c->coef32, &c->zpart32}) drop(p);
-  for (double** p : {&c->ysc, &c->ysc3, &c->cmax, &c->pmax, &c->wpart, &c->fpart_s, &c->sbsc})
+  for (double** p : {&c->ysc, &c->ysc3, &c->pmax, &c->wpart, &c->fpart_s, &c->sbsc})
     drop(p);
 }
 
@@ -1056,17 +1035,14 @@ static int launch_all(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* e
   if (ev) (void)hipEventRecord(ev[0], s);
   hipLaunchKernelGGL(ymax_part_kernel, dim3(kYmaxBlocks, nc), dim3(256), 0, s, c->Y1, st.su, np,
                      c->pmax);
-  hipLaunchKernelGGL(ymax_kernel, dim3(nc), dim3(64), 0, s, c->pmax, kYmaxBlocks, c->ysc);
   // with padded modes the row-dot s3 rides the fp16 GEMM in the last padding
   // column (hi/lo products good to ~2^-22, like the FP32 sums they replace);
   // bf16 hi/lo carries ~2^-17, and s3 dominates c1, so the bf16 path keeps
   // the FP32 row-dot (its spectrum error would grow fivefold)
   const bool fold = c->n < np && std::is_same<H, _Float16>::value;
-  if (fold)
-    hipLaunchKernelGGL(foldmax_kernel, dim3(nc), dim3(256), 0, s, c->R1, st.su, c->fy, np,
-                       c->ysc3);
   hipLaunchKernelGGL(prep_y<H>, dim3(np, nc), dim3(256), 0, s, c->Y1, c->R1, st.su, c->fy, np,
-                     c->ysc, fold ? c->ysc3 : nullptr, (u16*)c->Y1h, (u16*)c->Y1l, c->epi);
+                     c->pmax, c->ysc, fold ? c->ysc3 : nullptr, (u16*)c->Y1h, (u16*)c->Y1l,
+                     c->epi);
   // chains in groups of up to 3 per pass
   for (int c0 = 0; c0 < nc;) {
     const int g = nc - c0 >= 3 ? 3 : nc - c0;
@@ -1092,10 +1068,9 @@ static int launch_all(Ctx* c, int nc, int apply_d4, hipStream_t s, hipEvent_t* e
                      c->rho_img, c->ysc, fold ? c->ysc3 : nullptr, Mp, nct, apply_d4, c->row_lo,
                      c->row_hi,
                      (double*)nullptr, c->coef32, c->pmax);
-  hipLaunchKernelGGL(bscale_kernel, dim3(nc), dim3(256), 0, s, c->pmax, fin_blocks, st.umax,
-                     st.fmax, c->fy, np, c->cmax, c->sbsc);
-  hipLaunchKernelGGL(scale_coef_kernel, dim3((unsigned)((Mp + 255) / 256), nc), dim3(256), 0, s,
-                     c->sbsc, np, Mp / kBK, c->coef32);
+  hipLaunchKernelGGL(scale_coef_kernel, dim3((unsigned)std::min(512L, fin_blocks_l), nc), dim3(256),
+                     0, s, c->pmax, fin_blocks, st.umax, st.fmax, c->fy, np, Mp / kBK, c->sbsc,
+                     c->coef32);
   if (ev) (void)hipEventRecord(ev[1], s);
   for (int c0 = 0; c0 < nc;) {
     const int g = nc - c0 >= 3 ? 3 : nc - c0;
