@@ -61,6 +61,11 @@ void tdscha_ctx_destroy(tdscha_ctx* ctx);
 int tdscha_ctx_info(const tdscha_ctx* ctx, int* n_modes, int* n_modes_padded, long* n_images,
                     long* n_images_padded, int* ksplit);
 
+/* How many chains of the context's last perturbed averages, L application or Lanczos
+ * run took the orbit form (averages over the configurations for the few independent
+ * rotations of a perturbation, instead of over all images). */
+int tdscha_orbit_chains(const tdscha_ctx* ctx, int* n_chains);
+
 /*
  * Number of image ranges the outer-product GEMM is split into (a multiple of
  * 8, one slice per XCD in turn); each range is summed in FP64 afterwards in a

@@ -31,6 +31,7 @@ def _signatures(L):
     L.tdscha_ctx_destroy.argtypes = [_vp]
     L.tdscha_ctx_destroy.restype = None
     L.tdscha_ctx_info.argtypes = [_vp, _ip, _ip, C.POINTER(C.c_long), C.POINTER(C.c_long), _ip]
+    L.tdscha_orbit_chains.argtypes = [_vp, _ip]
     L.tdscha_synchronize.argtypes = [_vp]
     L.tdscha_perturb_averages.argtypes = [_vp, _vp, _vp, C.c_int, _vp, _vp]
     L.tdscha_perturb_averages_dev.argtypes = [_vp, C.c_int, _vp, _vp, C.c_int, C.c_int, _vp, _vp, _vp]

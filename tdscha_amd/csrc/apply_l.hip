@@ -548,9 +548,10 @@ int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, 
     if (!prepared) launch_prepare_pert(c, nc, psi, use_wigner, transpose, s);
     const int d4 = ignore_v4 ? 0 : 1;
     if (!plan && psi_host && orbit_worth(c, nc, precision, psi_host, len)) {
-      rc = orbit_plan(c, nc, precision, s, c->orb.plan[0]);
+      rc = orbit_plan(c, nc, precision, nullptr, s, c->orb.plan[0]);
       if (rc) return rc;
       plan = &c->orb.plan[0];
+      if (plan->ok) c->orb.chains = nc;
     }
     const bool orbit = plan && plan->ok;
     if (!orbit && c->n_cells == 0 && finish_in_one(c, precision)) {
@@ -782,6 +783,7 @@ int tdscha_apply_L_dev(tdscha_ctx* ctx, int n_vec, const double* psi_dev, double
   TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0, 1 or 2");
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   hipStream_t s = stream ? reinterpret_cast<hipStream_t>(stream) : c->stream;
+  c->orb.chains = 0;
   return apply_L_dev(c, n_vec, psi_dev, out_dev, use_wigner, transpose, ignore_harmonic, ignore_v3,
                      ignore_v4, reverse, shift, precision, s, nullptr, nullptr, false);
 }
@@ -805,6 +807,7 @@ int tdscha_apply_L(tdscha_ctx* ctx, int n_vec, const double* psi, double* out, i
   else
     TDS_CHECK_HIP(hipMemcpyAsync(in, psi, bytes, hipMemcpyHostToDevice, c->stream));
   TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0, 1 or 2");
+  c->orb.chains = 0;
   rc = apply_L_dev(c, n_vec, in, res, use_wigner, transpose, ignore_harmonic, ignore_v3,
                    ignore_v4, reverse, shift, precision, c->stream, nullptr, psi, false);
   if (rc) return rc;

@@ -169,6 +169,7 @@ struct Ctx;
 
 struct Orbit {
   bool usable = false;     // tables built
+  int chains = 0;          // chains of the last call or run that took the form
   // found by the first Lanczos run (-1: not yet)
   int group = -1;          // the symmetries are closed under multiplication
   int trans = -1;          // the translation average commutes with them
@@ -312,7 +313,7 @@ int ensure_split(Ctx* c, int prec);
 void orbit_plan_free(OrbPlan& p);
 bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld);
 int orbit_sector(Ctx* c, bool* ok);
-int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p);
+int orbit_plan(Ctx* c, int nc, int prec, const double* x, hipStream_t s, OrbPlan& p);
 int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
                  hipStream_t s);
 int orbit_clean(Ctx* c, const OrbPlan& p, double* x, const int* kk, const int* active,

@@ -120,13 +120,17 @@ static int perturb_averages_dev(Ctx* c, int nc, const double* R1_dev, const doub
                                 hipStream_t s, const double* R_host) {
   const long nn = (long)c->np * c->np;
   dim3 g((unsigned)((nn + 255) / 256), nc);
+  c->orb.chains = 0;
   hipLaunchKernelGGL(pad_inputs, g, dim3(256), 0, s, R1_dev, Y1_dev, c->n, c->np, c->R1, c->Y1);
   TDS_CHECK_HIP(hipGetLastError());
   if (R_host && orbit_worth(c, nc, prec, R_host, c->n)) {
     OrbPlan& p = c->orb.plan[0];
-    const int rc = orbit_plan(c, nc, prec, s, p);
+    const int rc = orbit_plan(c, nc, prec, nullptr, s, p);
     if (rc) return rc;
-    if (p.ok) return run_pa_orbit(c, p, apply_d4, f_dev, d2v_dev, s);
+    if (p.ok) {
+      c->orb.chains = nc;
+      return run_pa_orbit(c, p, apply_d4, f_dev, d2v_dev, s);
+    }
   }
   return run_pa(c, nc, apply_d4, prec, f_dev, d2v_dev, s);
 }
@@ -397,6 +401,12 @@ int tdscha_ctx_info(const tdscha_ctx* ctx, int* n_modes, int* n_modes_padded, lo
   if (n_images) *n_images = c->M * (c->rotate ? c->rot_nsym : 1);
   if (n_images_padded) *n_images_padded = c->Mp;
   if (ksplit) *ksplit = c->ksplit;
+  return 0;
+}
+
+int tdscha_orbit_chains(const tdscha_ctx* ctx, int* n_chains) {
+  TDS_REQUIRE(ctx && n_chains, 2, "tdscha_orbit_chains: NULL pointer");
+  *n_chains = reinterpret_cast<const Ctx*>(ctx)->orb.chains;
   return 0;
 }
 

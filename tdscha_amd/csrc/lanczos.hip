@@ -743,6 +743,7 @@ int tdscha_lanczos_run_biconjugate(tdscha_ctx* ctx, int n_chains, const double* 
               "tdscha_lanczos_run_biconjugate: NULL pointer");
   TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0, 1 or 2");
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
+  c->orb.chains = 0;
   int rc = setup_pairs(c);
   if (rc) return rc;
   if (precision != PREC_FP64) {
@@ -864,6 +865,7 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
   TDS_REQUIRE(precision >= 0 && precision <= 2, 2, "precision must be 0, 1 or 2");
   TDS_REQUIRE(reorth == 0 || reorth == 1, 2, "reorth must be 0 or 1");
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
+  c->orb.chains = 0;
   int rc = setup_pairs(c);
   if (rc) return rc;
   const int n = c->n;
@@ -962,8 +964,7 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
       const int g = std::min(kMaxChains, n_chains - c0);
       st.plans.emplace_back();
       if (orbit_worth(c, g, precision, psi0 + (long)c0 * len, len)) {
-        launch_prepare_pert(c, g, st.qcur + (long)c0 * len, 1, 0, s);
-        if (orbit_plan(c, g, precision, s, st.plans.back())) {
+        if (orbit_plan(c, g, precision, st.qcur + (long)c0 * len, s, st.plans.back())) {
           free_state(st);
           return -1;
         }
@@ -971,7 +972,10 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
       general = general || !st.plans.back().ok;
     }
   bool planned = false;
-  for (const OrbPlan& p : st.plans) planned = planned || p.ok;
+  for (const OrbPlan& p : st.plans) {
+    planned = planned || p.ok;
+    if (p.ok) c->orb.chains += p.nc;
+  }
   st.one_wg = !planned && len <= 1024 * kShortE && n_steps < kShortBasis &&
               len * n_steps <= kShortWork;
   if (st.one_wg && n_chains <= kMaxChains && !ignore_v3 && !c->rotate) {

@@ -25,7 +25,10 @@
 //
 // A Lanczos run whose operator commutes with the symmetries (they form a group
 // and the translation average commutes with them, both checked numerically)
-// keeps the relation C of its start vector.  Rounding leaves that sector and
+// keeps the relation C of its start vector, which is the one of all three parts of
+// the packed vector: R and both pair sectors, A and B.  (Y1 = ca A - cb B alone would
+// not do: ca is zero for pairs of equal frequencies, and for every pair at T = 0, and
+// A and B can cancel.)  Rounding leaves that sector and
 // the three-term recurrence amplifies it (about 5-fold per step), so the residual is
 // projected back every kOrbClean steps with the same two kernels (0.2 ms for three
 // chains of 381 modes).  Spectra of the three IR chains, equal by symmetry, after 200
@@ -708,7 +711,7 @@ static bool ensure(Ctx* c) {
   if (o.work) return true;
   const size_t np = c->np, nn = np * np;
   const int ks = orb_ksplit(c), ncol = (c->n + 15) / 16;
-  const size_t count[] = {(size_t)kMaxChains * ncol * o.rows * 4,
+  const size_t count[] = {2 * (size_t)kMaxChains * ncol * o.rows * 4,
                           kOrbPairs * np, kOrbPairs * nn,
                           2 * kMaxChains * np, 2 * kMaxChains * nn,
                           kOrbPairs * (size_t)o.Mp * 4,
@@ -717,7 +720,7 @@ static bool ensure(Ctx* c) {
   double** dst[] = {&o.ppart, &o.R1, &o.Y1, &o.Rb, &o.Yb, &o.coef, &o.zpart, &o.fpart, &o.z, &o.f};
   size_t at = 0;
   for (size_t k : count) at += (k + 31) / 32 * 32;
-  const size_t nout = (size_t)kMaxChains * o.rows * 4;
+  const size_t nout = 2 * (size_t)kMaxChains * o.rows * 4;
   if (hipMalloc((void**)&o.work, sizeof(double) * at) != hipSuccess) o.work = nullptr;
   if (o.work && hipHostMalloc((void**)&o.pout, sizeof(double) * nout) != hipSuccess) {
     (void)hipFree(o.work);
@@ -738,26 +741,47 @@ static bool ensure(Ctx* c) {
 
 // ----------------------------------------------------------------- the relation
 // Rank and relation of one chain from its row-dots s[rows][4]: rows j of W hold
-// the 4 kProbe functionals, scaled so that what weighs F (s1, s3) and what weighs
-// U (s2, s4) have unit size.  Pivoted Gram-Schmidt; rank 0 = no use.
-static int relation(const double* s, int ns, std::vector<int>& piv, std::vector<double>& C) {
-  constexpr int K = 4 * kProbe;
-  std::vector<double> W((size_t)ns * K);
-  double g[2] = {0.0, 0.0};
+// the functionals of `dots`, each group of them scaled to unit size (a group that is
+// zero throughout obeys any relation).  Pivoted Gram-Schmidt; rank 0 = no use.
+struct Dots {
+  const double* s;   // row-dots [kProbe][ns][4] of one matrix
+  int q;             // which of the four
+  double weight;
+  int group;
+};
+
+static int relation(const std::vector<Dots>& dots, int ns, std::vector<int>& piv,
+                    std::vector<double>& C) {
+  const int nd = (int)dots.size(), K = nd * kProbe;
+  std::vector<double> W((size_t)ns * K), g(nd, 0.0);
   for (int j = 0; j < ns; ++j)
-    for (int i = 0; i < kProbe; ++i) {
-      const double* q = s + ((size_t)i * ns + j) * 4;
-      double* w = W.data() + (size_t)j * K + 4 * i;
-      w[0] = q[0] / 6.0;
-      w[1] = q[2] / 3.0;
-      w[2] = q[1] / 3.0;
-      w[3] = q[3] / 3.0;
-      g[0] += w[0] * w[0] + w[1] * w[1];
-      g[1] += w[2] * w[2] + w[3] * w[3];
+    for (int i = 0; i < kProbe; ++i)
+      for (int d = 0; d < nd; ++d) {
+        const double w = dots[d].weight * dots[d].s[((size_t)i * ns + j) * 4 + dots[d].q];
+        W[(size_t)j * K + nd * i + d] = w;
+        g[dots[d].group] = std::max(g[dots[d].group], std::fabs(w));
+        if (!std::isfinite(w)) return 0;
+      }
+  // by the largest entry (whose square may be out of range), then by the sum of squares
+  std::vector<double> q(nd, 0.0);
+  bool some = false;
+  for (int d = 0; d < nd; ++d) {
+    if (g[d] > 0.0 && g[d] < 1e-290) return 0;   // (few digits left)
+    some = some || g[d] > 0.0;
+    if (g[d] == 0.0) g[d] = 1.0;
+  }
+  if (!some) return 0;
+  for (int j = 0; j < ns; ++j)
+    for (int e = 0; e < K; ++e) {
+      double& w = W[(size_t)j * K + e];
+      w /= g[dots[e % nd].group];
+      q[dots[e % nd].group] += w * w;
     }
-  if (!(g[0] > 0.0) || !(g[1] > 0.0) || !std::isfinite(g[0]) || !std::isfinite(g[1])) return 0;
   for (int j = 0; j < ns; ++j)
-    for (int e = 0; e < K; ++e) W[(size_t)j * K + e] /= std::sqrt(g[(e & 3) >> 1] / ns);
+    for (int e = 0; e < K; ++e) {
+      const double t = q[dots[e % nd].group];
+      if (t > 0.0) W[(size_t)j * K + e] /= std::sqrt(t / ns);
+    }
   std::vector<double> V = W, Q;
   piv.clear();
   double top = 0.0;
@@ -775,13 +799,13 @@ static int relation(const double* s, int ns, std::vector<int>& piv, std::vector<
     piv.push_back(best);
     const size_t r = piv.size() - 1;
     Q.resize((r + 1) * K);
-    double* q = Q.data() + r * K;
-    for (int e = 0; e < K; ++e) q[e] = V[(size_t)best * K + e] / nrm[best];
+    double* qr = Q.data() + r * K;
+    for (int e = 0; e < K; ++e) qr[e] = V[(size_t)best * K + e] / nrm[best];
     for (int j = 0; j < ns; ++j)   // twice: the second pass takes what rounding left
       for (int pass = 0; pass < 2; ++pass) {
         double* v = V.data() + (size_t)j * K;
-        const double t = dot(v, q, K);
-        for (int e = 0; e < K; ++e) v[e] -= t * q[e];
+        const double t = dot(v, qr, K);
+        for (int e = 0; e < K; ++e) v[e] -= t * qr[e];
       }
   }
   // W_j = sum_k C_jk W_piv[k]: with W Q^T = A, C A_piv = A (A_piv lower triangular)
@@ -864,9 +888,10 @@ static bool split_ready(Ctx* c, int prec) {
   return false;
 }
 
-// Plan of nc chains whose padded inputs are in c->R1, c->Y1 (waits for the
-// stream): p.ok false = use the general form.
-int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p) {
+// Plan of nc chains (waits for the stream): p.ok false = use the general form.  x null:
+// of the averages of the padded inputs in c->R1, c->Y1.  Else of a run from the packed
+// vectors x (device): the relation holds for R and for each of the two pair sectors.
+int orbit_plan(Ctx* c, int nc, int prec, const double* x, hipStream_t s, OrbPlan& p) {
   Orbit& o = c->orb;
   p.ok = false;
   const bool first = !o.work;
@@ -879,16 +904,31 @@ int orbit_plan(Ctx* c, int nc, int prec, hipStream_t s, OrbPlan& p) {
   const int ncol = (c->n + 15) / 16, rows4 = o.rows * 4, ns = o.nsym;
   std::vector<int> piv;
   std::vector<double> C, Call;
-  hipLaunchKernelGGL(orb_probe, dim3(o.rows / 16, ncol, nc), dim3(256), 0, s, o.pu, o.pf, c->Y1,
-                     c->R1, c->fy, c->fpsi, c->np, round_up(c->n, 16), o.rows, o.ppart);
-  hipLaunchKernelGGL(orb_probe_sum, dim3((rows4 + 255) / 256, nc), dim3(256), 0, s, o.ppart, ncol,
+  const int nm = x ? 2 * nc : nc;   // matrices
+  if (x) {
+    const long nn = (long)c->np * c->np;
+    hipLaunchKernelGGL(orb_unpack, dim3((unsigned)((nn + 255) / 256), nm), dim3(256), 0, s, x, c->n,
+                       c->np, (const int*)nullptr, 0, o.Yb, o.Rb);
+  }
+  hipLaunchKernelGGL(orb_probe, dim3(o.rows / 16, ncol, nm), dim3(256), 0, s, o.pu, o.pf,
+                     x ? o.Yb : c->Y1, x ? o.Rb : c->R1, c->fy, c->fpsi, c->np, round_up(c->n, 16),
+                     o.rows, o.ppart);
+  hipLaunchKernelGGL(orb_probe_sum, dim3((rows4 + 255) / 256, nm), dim3(256), 0, s, o.ppart, ncol,
                      rows4, o.pout);
   TDS_CHECK_HIP(hipGetLastError());
   TDS_CHECK_HIP(hipStreamSynchronize(s));
   std::vector<int2> pairs, clean;
   std::vector<int4> mats, cmats;
   for (int ch = 0; ch < nc; ++ch) {
-    const int r = relation(o.pout + (size_t)ch * rows4, ns, piv, C);
+    const double *m0 = o.pout + (size_t)(x ? 2 * ch : ch) * rows4, *m1 = m0 + rows4;
+    // s1, s2 of a matrix and s3, s4 of a vector; the averages weigh F by s1 and s3, U by
+    // s2 and s4
+    const int r = x ? relation({{m0, 2, 1.0, 0}, {m0, 3, 1.0, 1}, {m0, 0, 1.0, 2},
+                                {m0, 1, 1.0, 3}, {m1, 0, 1.0, 4}, {m1, 1, 1.0, 5}},
+                               ns, piv, C)
+                    : relation({{m0, 0, 1.0 / 6.0, 0}, {m0, 2, 1.0 / 3.0, 0},
+                                {m0, 1, 1.0 / 3.0, 1}, {m0, 3, 1.0 / 3.0, 1}},
+                               ns, piv, C);
     if (r == 0 || (int)pairs.size() + r > kOrbPairs) return 0;
     mats.push_back(int4{(int)pairs.size(), r, ch, 0});
     for (int k = 0; k < r; ++k) pairs.push_back(int2{ch, piv[k]});

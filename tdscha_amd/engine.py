@@ -102,6 +102,12 @@ class Engine:
     def synchronize(self):
         _lib.check(self._L.tdscha_synchronize(self.ctx), "tdscha_synchronize")
 
+    def orbit_chains(self):
+        """Chains of the last averages, L application or run that took the orbit form."""
+        n = C.c_int(0)
+        _lib.check(self._L.tdscha_orbit_chains(self.ctx, C.byref(n)), "tdscha_orbit_chains")
+        return n.value
+
     # -- perturbed averages ------------------------------------------------
     def perturb_averages(self, R1, Y1, apply_d4=1):
         """Host FP64 call: returns (f_pert_av[n], d2v_pert_av[n, n])."""

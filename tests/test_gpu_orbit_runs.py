@@ -1,0 +1,116 @@
+"""GPU: which start vectors of a Lanczos run take the orbit form.  The relation of a
+run has to hold for R and for each pair sector, A and B, of the packed vector: Y1 =
+ca A - cb B alone says nothing of A where ca is zero (pairs of equal frequencies, and
+every pair at T = 0), nor of A and B that cancel.
+
+Reference: the general form, in a context without symmetries whose configurations are
+the images.  Tolerance 1e-8 on the coefficients of 8 steps: rounding of 1e-15 grows by
+about 5 per step where it leaves the symmetry sector."""
+import copy
+
+import numpy as np
+import pytest
+
+from tests.test_rotation_form import dense_syms
+
+pytestmark = pytest.mark.gpu
+
+AXES = ((1.0, 0.0, 0.0), (0.0, 1.0, 0.0), (0.3, -0.5, 0.8))
+STEPS = 8
+
+
+class System:
+    """54 atoms with the point group of a cubic crystal (the images of one chain are
+    enough work for the orbit form), and the same images as configurations."""
+
+    def __init__(self, T=300.0, N=3000, weights=None, L=3, gamma=True):
+        from tdscha_amd.lanczos import Lanczos
+        from tdscha_amd.rocksalt import Ensemble, RockSalt
+        ens = Ensemble(RockSalt(L=L), T, N, seed=L)
+        ms = ens.symmetries(True, gamma_only=gamma)
+        self.ens, self.ms, self.n, self.T = ens, ms, len(ens.w), T
+        rho = np.ones(N) if weights is None else weights
+        self.S = S = dense_syms(ms.symmetries, ms.degenerate_space, self.n)
+        one = copy.copy(ms)
+        one.symmetries = [np.ones((1, 1, 1))] * self.n
+        one.degenerate_space = [np.array([i], dtype=np.int32) for i in range(self.n)]
+        one.sym_block_id = np.arange(self.n, dtype=np.int32)
+        sides = ((ens.X, ens.Y, rho, ms),
+                 (np.concatenate([ens.X @ s.T for s in S]),
+                  np.concatenate([ens.Y @ s.T for s in S]), np.tile(rho, len(S)), one))
+        self.sides = []
+        for X, Y, r, m in sides:
+            lanc = Lanczos(ens)
+            lanc.X, lanc.Y, lanc.rho, lanc.N = X, Y, r, len(X)
+            lanc.N_eff = float(np.sum(r))
+            lanc.gamma_only = gamma
+            lanc.init(symmetries=m)
+            self.sides.append(lanc)
+        self.row, self.col = np.triu_indices(self.n)
+
+    def ir(self):
+        r = np.array([(self.ens.ir_vector(pv) / np.sqrt(self.ens.m)) @ self.ens.pols
+                      for pv in AXES])
+        return r / np.linalg.norm(r, axis=1)[:, None]
+
+    def pack(self, R, A=None, B=None):
+        x = np.zeros((len(R), self.n + 2 * len(self.row)))
+        x[:, :self.n] = R
+        for k, M in ((0, A), (1, B)):
+            if M is not None:
+                lo = self.n + k * len(self.row)
+                x[:, lo:lo + len(self.row)] = M[:, self.row, self.col]
+        return x
+
+    def sector(self, r0, seed, nc):
+        """nc members of the symmetric matrices that rotate as the IR vector r0."""
+        rng = np.random.default_rng(seed)
+        chi = self.S @ r0 @ r0 / (r0 @ r0)
+        A = rng.normal(size=(self.n, self.n))
+        A = sum(c * (s @ (A + A.T) @ s.T) for c, s in zip(chi, self.S))
+        k = np.random.default_rng(0).integers(0, len(self.S), nc)
+        A = np.array([self.S[j].T @ A @ self.S[j] for j in k])
+        return A / np.linalg.norm(A[0]), np.array([self.S[j].T @ r0 for j in k])
+
+    def pair_factors(self):
+        """ca and cb of Y1 = ca A - cb B."""
+        w, T = self.ens.w, self.T
+        nb = 1.0 / (np.exp(w * 157887.32400374097 / T) - 1.0) if T > 0 else np.zeros(self.n)
+        wa, wb, na, nb_ = w[:, None], w[None], nb[:, None], nb[None]
+        w2x = 8 * wa * wb / ((1 + 2 * na) * (1 + 2 * nb_))
+        return (w2x * np.sqrt(np.maximum(0.0, -0.5 * (wa - wb) * (na - nb_) / (2 * wa * wb))),
+                w2x * np.sqrt(0.5 * (wa + wb) * (1 + na + nb_) / (2 * wa * wb)))
+
+    def check(self, x, orbit, **kw):
+        ref, _ = self.sides[1].run_FT_batched(x, STEPS)
+        out, _ = self.sides[0].run_FT_batched(x, STEPS, **kw)
+        assert self.sides[0].engine.orbit_chains() == orbit
+        for (a, b), (ao, bo) in zip(out, ref):
+            assert np.abs(a / ao - 1).max() < 1e-8 and np.abs(b / bo - 1).max() < 1e-8
+
+    def close(self):
+        for lanc in self.sides:
+            lanc.close()
+
+
+@pytest.mark.parametrize("T", [300.0, 0.0])
+def test_start_vectors(T):
+    p = System(T)
+    rng = np.random.default_rng(3)
+    R, z = p.ir(), np.zeros((3, p.n, p.n))
+    p.check(p.pack(R), 3)
+    # all three parts in the sector
+    A, r = p.sector(R[0], 5, 3)
+    B, _ = p.sector(R[0], 6, 3)
+    p.check(p.pack(r, A, B), 3)
+    # Y1 does not show it: a diagonal A without symmetry
+    D = z.copy()
+    D[:, np.arange(p.n), np.arange(p.n)] = rng.normal(size=(3, p.n)) / np.sqrt(p.n)
+    p.check(p.pack(R, D), 0)
+    # a general A (invisible at T = 0), and A and B that cancel in Y1
+    G = rng.normal(size=(3, p.n, p.n)) / p.n
+    G = G + G.transpose(0, 2, 1)
+    p.check(p.pack(R, G), 0)
+    ca, cb = p.pair_factors()
+    p.check(p.pack(R, G, ca / cb * G), 0)
+    p.close()
