@@ -143,7 +143,8 @@ constexpr size_t kPinned = 65536;
 constexpr int kProbe = 8;            // probe configurations of the rank search
 constexpr int kOrbRank = 6;          // largest orbit of a chain
 constexpr int kOrbPairs = 24;        // rotated perturbations of one pass
-constexpr double kOrbTol = 1e-12;    // accuracy of the relation
+constexpr double kOrbTol = 1e-13;    // accuracy of the relation
+constexpr double kOrbGain = 16.0;    // largest sum of its factors
 constexpr int kOrbClean = 2;         // Lanczos steps between projections on the sector
 // shortest general form (microseconds, estimated) for which the search, a wait
 // for the host of about 40 us and the rotations are worth trying

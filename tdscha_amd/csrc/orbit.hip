@@ -16,12 +16,14 @@
 // The rank is found for each call from the perturbation itself, not assumed: the
 // row-dots of the averages (s1 = u.Y1.u, s2 = u.Y1.(fpsi f), s3 = (fY u).R1,
 // s4 = f.R1) are evaluated on all images of kProbe random configurations of the
-// thermal amplitudes; a relation C that holds for these 4 kProbe functionals
-// to kOrbTol holds for the perturbation (random functionals: a remainder that
-// all of them miss has probability zero, and one that the 26 beyond the rank
-// understate tenfold 1e-26).  Otherwise the general form is used.  kOrbTol is the accuracy
-// to which the symmetry tables themselves are a representation (1e-12 on 381
-// modes).
+// thermal amplitudes: 2 kProbe functionals of R1 and as many of Y1.  A relation C that
+// holds for both to kOrbTol of each one's size holds for the perturbation (random
+// functionals: a remainder that all of them miss has probability zero, and one that
+// the 10 beyond the rank understate tenfold 1e-11).  Otherwise the general form is
+// used.  kOrbTol lies at the rounding of the symmetry tables: the images of an IR
+// vector are 1e-14, those of a Raman tensor 2e-14 from their span on 381 modes (the
+// tables are orthogonal to 1e-14).  The sum of |C| over an image, which the rounding of
+// the averages enters with, is 2 and 5 there, and at most kOrbGain.
 //
 // A Lanczos run whose operator commutes with the symmetries (they form a group
 // and the translation average commutes with them, both checked numerically)
@@ -740,48 +742,43 @@ static bool ensure(Ctx* c) {
 }
 
 // ----------------------------------------------------------------- the relation
-// Rank and relation of one chain from its row-dots s[rows][4]: rows j of W hold
-// the functionals of `dots`, each group of them scaled to unit size (a group that is
-// zero throughout obeys any relation).  Pivoted Gram-Schmidt; rank 0 = no use.
+// Rank and relation of one chain: row j of W holds the functionals of `dots` of the
+// image j, each kind scaled to unit size, so that the relation holds for every part of
+// the perturbation to kOrbTol of that part's own size (f comes from Y1 alone, and
+// without apply_d4 d2v from R1 alone).  A kind that is zero throughout obeys any
+// relation.  Pivoted Gram-Schmidt; rank 0 = no use.
 struct Dots {
-  const double* s;   // row-dots [kProbe][ns][4] of one matrix
+  const double* s;   // row-dots [kProbe][ns][4] of one matrix and vector
   int q;             // which of the four
-  double weight;
-  int group;
 };
 
 static int relation(const std::vector<Dots>& dots, int ns, std::vector<int>& piv,
                     std::vector<double>& C) {
   const int nd = (int)dots.size(), K = nd * kProbe;
-  std::vector<double> W((size_t)ns * K), g(nd, 0.0);
-  for (int j = 0; j < ns; ++j)
-    for (int i = 0; i < kProbe; ++i)
-      for (int d = 0; d < nd; ++d) {
-        const double w = dots[d].weight * dots[d].s[((size_t)i * ns + j) * 4 + dots[d].q];
-        W[(size_t)j * K + nd * i + d] = w;
-        g[dots[d].group] = std::max(g[dots[d].group], std::fabs(w));
-        if (!std::isfinite(w)) return 0;
-      }
-  // by the largest entry (whose square may be out of range), then by the sum of squares
-  std::vector<double> q(nd, 0.0);
+  std::vector<double> W((size_t)ns * K);
   bool some = false;
   for (int d = 0; d < nd; ++d) {
-    if (g[d] > 0.0 && g[d] < 1e-290) return 0;   // (few digits left)
-    some = some || g[d] > 0.0;
-    if (g[d] == 0.0) g[d] = 1.0;
+    // scaled by the largest entry (whose square may be out of range), then by the rms
+    double top = 0.0, sum = 0.0, sq = 0.0;
+    const double* p = dots[d].s + dots[d].q;
+    for (int e = 0; e < ns * kProbe; ++e) {
+      top = std::max(top, std::fabs(p[4 * e]));
+      sum += p[4 * e];
+    }
+    if (!std::isfinite(sum) || (top > 0.0 && top < 1e-290)) return 0;   // (too few digits)
+    if (top == 0.0) continue;
+    some = true;
+    for (int i = 0; i < kProbe; ++i)
+      for (int j = 0; j < ns; ++j) {
+        double& w = W[(size_t)j * K + d * kProbe + i];
+        w = p[4 * (i * ns + j)] / top;
+        sq += w * w;
+      }
+    const double inv = 1.0 / std::sqrt(sq / ns);
+    for (int j = 0; j < ns; ++j)
+      for (int i = 0; i < kProbe; ++i) W[(size_t)j * K + d * kProbe + i] *= inv;
   }
   if (!some) return 0;
-  for (int j = 0; j < ns; ++j)
-    for (int e = 0; e < K; ++e) {
-      double& w = W[(size_t)j * K + e];
-      w /= g[dots[e % nd].group];
-      q[dots[e % nd].group] += w * w;
-    }
-  for (int j = 0; j < ns; ++j)
-    for (int e = 0; e < K; ++e) {
-      const double t = q[dots[e % nd].group];
-      if (t > 0.0) W[(size_t)j * K + e] /= std::sqrt(t / ns);
-    }
   std::vector<double> V = W, Q;
   piv.clear();
   double top = 0.0;
@@ -794,7 +791,7 @@ static int relation(const std::vector<Dots>& dots, int ns, std::vector<int>& piv
     }
     if (piv.empty()) top = nrm[best];
     if (nrm[best] <= kOrbTol * top) break;
-    // a direction this weak would enter the relation with large factors
+    // (a direction this weak is known to too few digits)
     if (nrm[best] < 1e-3 * top || (int)piv.size() == kOrbRank) return 0;
     piv.push_back(best);
     const size_t r = piv.size() - 1;
@@ -822,6 +819,12 @@ static int relation(const std::vector<Dots>& dots, int ns, std::vector<int>& piv
       for (int l = k + 1; l < r; ++l) t -= C[(size_t)j * kOrbRank + l] * A[(size_t)piv[l] * r + k];
       C[(size_t)j * kOrbRank + k] = t / A[(size_t)piv[k] * r + k];
     }
+  // the rounding of the averages enters with the factors C
+  for (int j = 0; j < ns; ++j) {
+    double sum = 0.0;
+    for (int k = 0; k < r; ++k) sum += std::fabs(C[(size_t)j * kOrbRank + k]);
+    if (!(sum <= kOrbGain)) return 0;
+  }
   return r;
 }
 
@@ -921,14 +924,10 @@ int orbit_plan(Ctx* c, int nc, int prec, const double* x, hipStream_t s, OrbPlan
   std::vector<int4> mats, cmats;
   for (int ch = 0; ch < nc; ++ch) {
     const double *m0 = o.pout + (size_t)(x ? 2 * ch : ch) * rows4, *m1 = m0 + rows4;
-    // s1, s2 of a matrix and s3, s4 of a vector; the averages weigh F by s1 and s3, U by
-    // s2 and s4
-    const int r = x ? relation({{m0, 2, 1.0, 0}, {m0, 3, 1.0, 1}, {m0, 0, 1.0, 2},
-                                {m0, 1, 1.0, 3}, {m1, 0, 1.0, 4}, {m1, 1, 1.0, 5}},
-                               ns, piv, C)
-                    : relation({{m0, 0, 1.0 / 6.0, 0}, {m0, 2, 1.0 / 3.0, 0},
-                                {m0, 1, 1.0 / 3.0, 1}, {m0, 3, 1.0 / 3.0, 1}},
-                               ns, piv, C);
+    // s3, s4 of the vector (R or R1), s1, s2 of each matrix (A and B, or Y1)
+    std::vector<Dots> dots = {{m0, 2}, {m0, 3}, {m0, 0}, {m0, 1}};
+    if (x) dots.insert(dots.end(), {{m1, 0}, {m1, 1}});
+    const int r = relation(dots, ns, piv, C);
     if (r == 0 || (int)pairs.size() + r > kOrbPairs) return 0;
     mats.push_back(int4{(int)pairs.size(), r, ch, 0});
     for (int k = 0; k < r; ++k) pairs.push_back(int2{ch, piv[k]});
