@@ -433,10 +433,12 @@ static double dot(const double* x, const double* y, int n) {
   return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 }
 
-// Whether the S_j are closed under multiplication: p.S_i S_j z equals p.S_k z for
-// one k for two independent random pairs (p, z), to 1e-9 of their size.  Elements
-// become generators until the products with them reach the whole list; every one of
-// these products has to be in the list (then the list is the group they generate).
+// Whether the S_j are a group of orthogonal matrices (then S_j^T, which takes the
+// perturbation to its image, is one of them, and T_sym commutes with all).  Closed under
+// multiplication: p.S_i S_j z equals p.S_k z for one k for two independent random pairs
+// (p, z), to 1e-9 of their size.  Elements become generators until the products with
+// them reach the whole list; every one of these products has to be in the list (then
+// the list is the group they generate).
 static bool closed(Ctx* c) {
   Orbit& o = c->orb;
   const int ns = o.nsym, n = c->n;
@@ -492,6 +494,15 @@ static bool closed(Ctx* c) {
           sub.push_back(k);
         }
       }
+  }
+  // the generators orthogonal: S_q^T S_q z is z
+  std::vector<double> back(n);
+  double scale = 0.0;
+  for (double v : z[0]) scale = std::max(scale, std::fabs(v));
+  for (size_t q = 0; q < o.gens.size(); ++q) {
+    apply_s(c, o.syms, o.gens[q], true, gz[0].data() + q * n, back.data());
+    for (int m = 0; m < n; ++m)
+      if (!(std::fabs(back[m] - z[0][m]) <= 1e-9 * scale)) return false;
   }
   return true;
 }

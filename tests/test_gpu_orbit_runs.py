@@ -23,11 +23,13 @@ class System:
     """54 atoms with the point group of a cubic crystal (the images of one chain are
     enough work for the orbit form), and the same images as configurations."""
 
-    def __init__(self, T=300.0, N=3000, weights=None, L=3, gamma=True):
+    def __init__(self, T=300.0, N=3000, weights=None, trans=True, tables=None):
         from tdscha_amd.lanczos import Lanczos
         from tdscha_amd.rocksalt import Ensemble, RockSalt
-        ens = Ensemble(RockSalt(L=L), T, N, seed=L)
-        ms = ens.symmetries(True, gamma_only=gamma)
+        ens = Ensemble(RockSalt(L=3), T, N, seed=3)
+        ms = ens.symmetries(True, gamma_only=True)
+        if tables is not None:
+            ms = tables(ms)
         self.ens, self.ms, self.n, self.T = ens, ms, len(ens.w), T
         rho = np.ones(N) if weights is None else weights
         self.S = S = dense_syms(ms.symmetries, ms.degenerate_space, self.n)
@@ -43,7 +45,7 @@ class System:
             lanc = Lanczos(ens)
             lanc.X, lanc.Y, lanc.rho, lanc.N = X, Y, r, len(X)
             lanc.N_eff = float(np.sum(r))
-            lanc.gamma_only = gamma
+            lanc.gamma_only = trans
             lanc.init(symmetries=m)
             self.sides.append(lanc)
         self.row, self.col = np.triu_indices(self.n)
@@ -113,4 +115,28 @@ def test_start_vectors(T):
     p.check(p.pack(R, G), 0)
     ca, cb = p.pair_factors()
     p.check(p.pack(R, G, ca / cb * G), 0)
+    p.close()
+
+
+def skewed(ms):
+    """The same group in a basis of each degenerate block that is not orthonormal."""
+    rng = np.random.default_rng(9)
+    ms, blocks = copy.copy(ms), []
+    for s in ms.symmetries:
+        P = np.eye(s.shape[1]) + 0.2 * rng.normal(size=s.shape[1:]) / np.sqrt(s.shape[1])
+        blocks.append(P @ s @ np.linalg.inv(P))
+    ms.symmetries = blocks
+    return ms
+
+
+def test_tables_that_are_not_orthogonal():
+    """T_sym(S^T v) = S^-1 T_sym(v): a run leaves the span of the images S_j^T v, so it
+    stays in the general form; the averages themselves need no more than the span."""
+    p = System(trans=False, tables=skewed)
+    x = p.pack(p.ir())
+    p.check(x, 0)
+    y = p.sides[1].apply_L_batch(x)
+    out = p.sides[0].apply_L_batch(x)
+    assert p.sides[0].engine.orbit_chains() == 3
+    assert np.linalg.norm(out - y) < 1e-12 * np.linalg.norm(y)
     p.close()
