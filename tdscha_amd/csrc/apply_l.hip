@@ -18,7 +18,6 @@
 
 namespace tdscha {
 
-int run_pa(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_dev, hipStream_t s);
 
 // coefficient rows of c->std_coef
 enum { SC_X = 0, SC_Y = 1, SC_X1 = 2, SC_Y1 = 3 };
@@ -547,11 +546,12 @@ int apply_L_dev(Ctx* c, int nc, const double* psi, double* out, int use_wigner, 
   if (anharmonic) {
     if (!prepared) launch_prepare_pert(c, nc, psi, use_wigner, transpose, s);
     const int d4 = ignore_v4 ? 0 : 1;
-    if (!plan && psi_host && orbit_worth(c, nc, precision, psi_host, len)) {
-      rc = orbit_plan(c, nc, precision, nullptr, s, c->orb.plan[0]);
+    const unsigned mask = psi_host ? orbit_candidates(c, nc, precision, psi_host, len) : 0;
+    if (mask) {
+      rc = orbit_plan(c, nc, mask, precision, nullptr, s, c->orb.plan[0]);
       if (rc) return rc;
       plan = &c->orb.plan[0];
-      if (plan->ok) c->orb.chains = nc;
+      if (plan->ok) c->orb.chains = plan->chains;
     }
     const bool orbit = plan && plan->ok;
     if (!orbit && c->n_cells == 0 && finish_in_one(c, precision)) {

@@ -146,19 +146,26 @@ constexpr int kOrbPairs = 24;        // rotated perturbations of one pass
 constexpr double kOrbTol = 1e-13;    // accuracy of the relation
 constexpr double kOrbGain = 16.0;    // largest sum of its factors
 constexpr int kOrbClean = 2;         // Lanczos steps between projections on the sector
-// shortest general form (microseconds, estimated) for which the search, a wait
-// for the host of about 40 us and the rotations are worth trying
-constexpr double kOrbWorthUs = 500.0;
+// least time that the form saves (microseconds, estimated, one chain): the search, a wait
+// for the host of about 40 us and the rotations cost a call of one chain 150 to 200
+// (averages of one IR vector: 54 atoms x 6000, saving 500: 874 -> 285 us; 128 atoms x
+// 1000, 483: 807 -> 454)
+constexpr double kOrbWorthUs = 200.0;
 
 struct OrbPlan {
-  bool ok = false;
+  bool ok = false;         // some chain takes the form
   int prec = 0;            // of its averages
-  int nc = 0, npairs = 0, rank = 0;   // chains, pairs, largest rank of a chain
-  struct Round {
-    int chain0, chains, first, count;
+  int nc = 0, chains = 0, rank = 0;   // chains, those with an orbit, their largest rank
+  struct List {
+    int n, at[kMaxChains];
   };
-  std::vector<Round> rounds;   // passes of the clean-up
+  List others = {};        // the chains without, in the general form
+  struct Round {           // a pass: its first matrix and their number, its pairs
+    int mat, mats, pair, count;
+  };
+  std::vector<Round> rounds, clean_rounds;   // of the averages, of the clean-up
   std::vector<char> host;
+  double* general = nullptr;   // [kMaxChains, n], [kMaxChains, n, n] averages of `others`
   void* dev = nullptr;
   size_t cap = 0;
   int4 *mats = nullptr, *cmats = nullptr;
@@ -312,9 +319,12 @@ struct Ctx {
 int ensure_split(Ctx* c, int prec);
 
 void orbit_plan_free(OrbPlan& p);
-bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld);
+bool orbit_sized(const Ctx* c, int prec);
+unsigned orbit_candidates(const Ctx* c, int nc, int prec, const double* R, long ld);
 int orbit_sector(Ctx* c, bool* ok);
-int orbit_plan(Ctx* c, int nc, int prec, const double* x, hipStream_t s, OrbPlan& p);
+int orbit_plan(Ctx* c, int nc, unsigned mask, int prec, const double* x, hipStream_t s,
+               OrbPlan& p);
+int run_pa(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_dev, hipStream_t s);
 int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
                  hipStream_t s);
 int orbit_clean(Ctx* c, const OrbPlan& p, double* x, const int* kk, const int* active,

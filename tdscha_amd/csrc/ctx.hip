@@ -55,7 +55,8 @@ __global__ void symmetrize_out(const double* __restrict__ zsum_all, const double
   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e < n) f_all[(long)chain * n + e] = fsum[(long)chain * np + e];
   if (e >= (long)n * n) return;
-  const int mu = (int)(e / n), nu = (int)(e % n);
+  // (row <= column: d2v exactly symmetric, in this form as in the orbit form)
+  const int r = (int)(e / n), q = (int)(e % n), mu = min(r, q), nu = max(r, q);
   const double* z = zsum_all + (long)chain * np * np;
   d2v_all[(long)chain * n * n + e] =
       norm * (fy[mu] * z[(long)mu * np + nu] + fy[nu] * z[(long)nu * np + mu]);
@@ -123,12 +124,13 @@ static int perturb_averages_dev(Ctx* c, int nc, const double* R1_dev, const doub
   c->orb.chains = 0;
   hipLaunchKernelGGL(pad_inputs, g, dim3(256), 0, s, R1_dev, Y1_dev, c->n, c->np, c->R1, c->Y1);
   TDS_CHECK_HIP(hipGetLastError());
-  if (R_host && orbit_worth(c, nc, prec, R_host, c->n)) {
+  const unsigned mask = R_host ? orbit_candidates(c, nc, prec, R_host, c->n) : 0;
+  if (mask) {
     OrbPlan& p = c->orb.plan[0];
-    const int rc = orbit_plan(c, nc, prec, nullptr, s, p);
+    const int rc = orbit_plan(c, nc, mask, prec, nullptr, s, p);
     if (rc) return rc;
     if (p.ok) {
-      c->orb.chains = nc;
+      c->orb.chains = p.chains;
       return run_pa_orbit(c, p, apply_d4, f_dev, d2v_dev, s);
     }
   }

@@ -948,36 +948,38 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
                      st.part, ps, st.r, len, n_steps, st.Q, st.qcur);
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
     return fail("initialisation failed");
-  // orbit form per group of chains, from the start vectors: an operator that
-  // commutes with the symmetry group keeps their relation
-  bool sector = false;
-  for (int c0 = 0; !ignore_v3 && c0 < n_chains; c0 += kMaxChains)
-    sector = sector || orbit_worth(c, std::min(kMaxChains, n_chains - c0), precision,
-                                   psi0 + (long)c0 * len, len);
-  if (sector && orbit_sector(c, &sector)) {
-    free_state(st);
-    return -1;
-  }
-  bool general = !sector;
-  if (sector)
+  // orbit form, chain by chain, from the start vectors: an operator that commutes with
+  // the symmetry group keeps their relation.  Where the form may be taken, the step has
+  // room for its projection in all runs alike: separate kernels.
+  const bool short_run = len <= 1024 * kShortE && n_steps < kShortBasis &&
+                         len * n_steps <= kShortWork;
+  std::vector<unsigned> masks;
+  bool sector = false, general = false;
+  if (!ignore_v3 && orbit_sized(c, precision)) {
     for (int c0 = 0; c0 < n_chains; c0 += kMaxChains) {
-      const int g = std::min(kMaxChains, n_chains - c0);
-      st.plans.emplace_back();
-      if (orbit_worth(c, g, precision, psi0 + (long)c0 * len, len)) {
-        if (orbit_plan(c, g, precision, st.qcur + (long)c0 * len, s, st.plans.back())) {
-          free_state(st);
-          return -1;
-        }
-      }
-      general = general || !st.plans.back().ok;
+      masks.push_back(orbit_candidates(c, std::min(kMaxChains, n_chains - c0), precision,
+                                       psi0 + (long)c0 * len, len));
+      sector = sector || masks.back();
     }
-  bool planned = false;
-  for (const OrbPlan& p : st.plans) {
-    planned = planned || p.ok;
-    if (p.ok) c->orb.chains += p.nc;
+    if ((sector || short_run) && orbit_sector(c, &sector)) {
+      free_state(st);
+      return -1;
+    }
   }
-  st.one_wg = !planned && len <= 1024 * kShortE && n_steps < kShortBasis &&
-              len * n_steps <= kShortWork;
+  for (size_t g = 0; sector && g < masks.size(); ++g) {
+    st.plans.emplace_back();
+    OrbPlan& p = st.plans.back();
+    const int c0 = (int)g * kMaxChains, nc = std::min(kMaxChains, n_chains - c0);
+    if (masks[g] &&
+        orbit_plan(c, nc, masks[g], precision, st.qcur + (long)c0 * len, s, p)) {
+      free_state(st);
+      return -1;
+    }
+    general = general || !p.ok || p.others.n;
+    if (p.ok) c->orb.chains += p.chains;
+  }
+  general = general || !sector;
+  st.one_wg = !sector && short_run;
   if (st.one_wg && n_chains <= kMaxChains && !ignore_v3 && !c->rotate) {
     launch_prepare_pert(c, n_chains, st.qcur, 1, 0, s);
     st.next = {c->pair_ca, c->pair_cb, c->pair_row, c->pair_col, c->n, c->np, c->R1, c->Y1};

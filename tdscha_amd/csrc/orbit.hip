@@ -194,10 +194,10 @@ __global__ __launch_bounds__(256) void orb_in(OrbPanels pn, const int2* __restri
   }
 }
 
-// Matrix m = (first pair, rank, relation): sum_j S_j (sum_k C_jk D_k) S_j^T and
+// Matrix (first pair, rank, relation, m): sum_j S_j (sum_k C_jk D_k) S_j^T and
 // sum_j S_j sum_k C_jk f_k.  AVG: D_k = fY Z_k + (fY Z_k)^T of the raw outer
-// sums, results to f_out, d_out (both halves).  Else D_k the symmetric inputs,
-// results to the packed vectors x [chain][n + 2 P] (matrix m = 2 chain + sector; R
+// sums, results to f_out, d_out (both halves) of chain m.  Else D_k the symmetric inputs,
+// results to the packed vectors x [chain][n + 2 P] (m = 2 chain + sector; R
 // with sector 0), in which case the kernel runs only on every `every`-th step.
 // RM: largest rank of the plan (3, or kOrbRank).  grid (panel pairs pi <= pj, then
 // panels for f; matrices); per symmetry a wave combines D in registers (its 16 rows),
@@ -213,8 +213,8 @@ __global__ __launch_bounds__(512, RM > 3 ? 2 : 4) void orb_out(
     int n, int np, double normf, double normd, const int* __restrict__ kk, int every,
     const int* __restrict__ active, double* __restrict__ f_out, double* __restrict__ d_out) {
   if (every && (kk[0] % every) != every - 1) return;
-  const int m = blockIdx.y;
-  const int4 mt = mats[m];
+  const int4 mt = mats[blockIdx.y];
+  const int m = mt.w;
   if (!AVG && !active[m >> 1]) return;
   const int ntile = pn.npanel * (pn.npanel + 1) / 2;
   const bool isf = (int)blockIdx.x >= ntile;
@@ -578,21 +578,25 @@ int orbit_sector(Ctx* c, bool* ok) {
   return 0;
 }
 
-static double estimate_us(double flop, int prec) {
-  // sustained rates of the GEMM pairs: 55 TF/s in FP64, 300 TF/s (counted once,
-  // not three times) in the split precisions
-  return flop / (prec == PREC_FP64 ? 5.5e7 : 3e8);
+// Time of the GEMM pairs of one chain over `rows` images: 55 TF/s in FP64 (columns in
+// sixteens); the split kernels compute whole 128-column tiles, 270 TF/s (two chains of
+// 381 modes, counted once, not three times) to 500 TF/s (three of 159).
+static double estimate_us(const Ctx* c, double rows, int prec) {
+  const double w = round_up(c->n, prec == PREC_FP64 ? 16 : kTile);
+  return 4.0 * rows * w * w / (prec == PREC_FP64 ? 5.5e7 : 3.5e8);
 }
 
-static double pass_flop(const Ctx* c, double rows) {
-  const double n16 = round_up(c->n, 16);
-  return 4.0 * rows * n16 * n16;
+// Whether the form may save enough for one chain in this precision.  Per chain, so that
+// a chain's form, and with it its rounding, does not depend on its batch.
+bool orbit_sized(const Ctx* c, int prec) {
+  const Orbit& o = c->orb;
+  return o.usable && c->row_lo == 0 && c->row_hi == c->M &&
+         estimate_us(c, (double)c->N * (o.nsym - 1), prec) > kOrbWorthUs;
 }
 
 // The configurations, panel tables and probe rows; called at context creation
 // with the configurations still on the device.  Leaves c->orb.usable false where
-// the form does not apply or cannot pay (the general form of 8 chains under
-// kOrbWorthUs), or with more than 512 symmetries (the tables and the closure check
+// the form does not apply or cannot pay in any precision (orbit_sized), or with more than 512 symmetries (the tables and the closure check
 // grow with their number and its square).
 int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const int* block_modes,
                 const std::vector<double>& syms, const double* X_dev, const double* Y_dev,
@@ -600,8 +604,10 @@ int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const in
                 const int* d_bmo, const long* d_bso, const int* d_bm, const double* d_syms) {
   Orbit& o = c->orb;
   o.nsym = n_syms;
-  const double images = (double)c->N * n_syms;
-  if (n_syms < 4 || n_syms > 512 || estimate_us(8 * pass_flop(c, images), PREC_FP64) < kOrbWorthUs) return 0;
+  if (n_syms < 4 || n_syms > 512) return 0;
+  const double saved = (double)c->N * (n_syms - 1);
+  if (std::max(estimate_us(c, saved, PREC_FP64), estimate_us(c, saved, PREC_FP16X2)) <= kOrbWorthUs)
+    return 0;
   const int n = c->n, np = c->np;
   std::vector<double> fy(np);
   TDS_CHECK_HIP(hipMemcpy(fy.data(), c->fy, sizeof(double) * np, hipMemcpyDeviceToHost));
@@ -704,7 +710,10 @@ void orbit_free(Ctx* c) {
 
 void orbit_plan_free(OrbPlan& p) {
   if (p.dev) (void)hipFree(p.dev);
+  if (p.general) (void)hipFree(p.general);
   p.dev = nullptr;
+  p.general = nullptr;
+  p.cap = 0;
   p.ok = false;
 }
 
@@ -839,19 +848,18 @@ static int relation(const std::vector<Dots>& dots, int ns, std::vector<int>& piv
   return r;
 }
 
-// Whether to look for a plan: the general form is long enough, and the R vectors
-// (host, `ld` apart) do not rule it out: more than kOrbRank independent rotations
-// of one among the first symmetries.  This keeps the probe and the wait for it
-// away from perturbations of no symmetry (10 us of host work under the upload, for
-// 50 us).
-bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld) {
+// The chains (bit mask) to look for a plan of: the general form is long enough, and the
+// chain's R vector (host, `ld` apart) does not rule it out by more than kOrbRank
+// independent rotations among the first symmetries.  This keeps the probe and the wait
+// for it away from perturbations of no symmetry (10 us of host work under the upload,
+// for 50 us).
+unsigned orbit_candidates(const Ctx* c, int nc, int prec, const double* R, long ld) {
+  if (!orbit_sized(c, prec)) return 0;
   const Orbit& o = c->orb;
-  if (!o.usable || c->row_lo != 0 || c->row_hi != c->M ||
-      !(estimate_us(nc * pass_flop(c, (double)c->N * o.nsym), prec) > kOrbWorthUs))
-    return false;
   const int n = c->n;
+  unsigned mask = 0;
   std::vector<double> Q((size_t)(kOrbRank + 1) * n);
-  for (int ch = 0; R && ch < nc; ++ch) {
+  for (int ch = 0; ch < nc; ++ch) {
     int r = 0;
     for (int j = 0; j < std::min(o.nsym, kOrbRank + 2) && r <= kOrbRank; ++j) {
       double* v = Q.data() + (size_t)r * n;
@@ -868,9 +876,9 @@ bool orbit_worth(const Ctx* c, int nc, int prec, const double* R, long ld) {
       for (int m = 0; m < n; ++m) v[m] *= inv;
       ++r;
     }
-    if (r > kOrbRank) return false;
+    if (r <= kOrbRank) mask |= 1u << ch;
   }
-  return true;
+  return mask;
 }
 
 // the split images of the configurations; false = no room
@@ -902,10 +910,12 @@ static bool split_ready(Ctx* c, int prec) {
   return false;
 }
 
-// Plan of nc chains (waits for the stream): p.ok false = use the general form.  x null:
-// of the averages of the padded inputs in c->R1, c->Y1.  Else of a run from the packed
-// vectors x (device): the relation holds for R and for each of the two pair sectors.
-int orbit_plan(Ctx* c, int nc, int prec, const double* x, hipStream_t s, OrbPlan& p) {
+// Plan of nc chains (waits for the stream): the chains of `mask` that have a small orbit
+// take the form (p.ok: some do), the others the general one.  x null: the averages of
+// the padded inputs in c->R1, c->Y1.  Else a run from the packed vectors x (device):
+// the relation holds for R and for each of the two pair sectors.
+int orbit_plan(Ctx* c, int nc, unsigned mask, int prec, const double* x, hipStream_t s,
+               OrbPlan& p) {
   Orbit& o = c->orb;
   p.ok = false;
   const bool first = !o.work;
@@ -931,54 +941,71 @@ int orbit_plan(Ctx* c, int nc, int prec, const double* x, hipStream_t s, OrbPlan
                      rows4, o.pout);
   TDS_CHECK_HIP(hipGetLastError());
   TDS_CHECK_HIP(hipStreamSynchronize(s));
-  std::vector<int2> pairs, clean;
-  std::vector<int4> mats, cmats;
+  // chain by chain: rank and relation
+  p.nc = nc;
+  p.prec = prec;
+  p.chains = p.others.n = p.rank = 0;
+  std::vector<int> ranks(nc, 0);
+  std::vector<std::vector<int>> pivots(nc);
+  Call.assign((size_t)nc * ns * kOrbRank, 0.0);
+  const double full = estimate_us(c, (double)c->N * ns, prec);
   for (int ch = 0; ch < nc; ++ch) {
     const double *m0 = o.pout + (size_t)(x ? 2 * ch : ch) * rows4, *m1 = m0 + rows4;
     // s3, s4 of the vector (R or R1), s1, s2 of each matrix (A and B, or Y1)
     std::vector<Dots> dots = {{m0, 2}, {m0, 3}, {m0, 0}, {m0, 1}};
     if (x) dots.insert(dots.end(), {{m1, 0}, {m1, 1}});
-    const int r = relation(dots, ns, piv, C);
-    if (r == 0 || (int)pairs.size() + r > kOrbPairs) return 0;
-    mats.push_back(int4{(int)pairs.size(), r, ch, 0});
-    for (int k = 0; k < r; ++k) pairs.push_back(int2{ch, piv[k]});
-    for (int sec = 0; sec < 2; ++sec) {
-      // pairs of the clean-up, in rounds of whole chains (orbit_clean)
-      cmats.push_back(int4{0, r, ch, 0});
-      for (int k = 0; k < r; ++k) clean.push_back(int2{2 * ch + sec, piv[k]});
+    const int r = mask >> ch & 1 ? relation(dots, ns, piv, C) : 0;
+    if (r && full - estimate_us(c, (double)c->N * r, prec) > kOrbWorthUs) {
+      ranks[ch] = r;
+      pivots[ch] = piv;
+      std::copy(C.begin(), C.end(), Call.begin() + (size_t)ch * ns * kOrbRank);
+      p.rank = std::max(p.rank, r);
+      ++p.chains;
+    } else {
+      p.others.at[p.others.n++] = ch;
     }
-    Call.insert(Call.end(), C.begin(), C.end());
   }
-  const double full = estimate_us(nc * pass_flop(c, (double)c->N * ns), prec);
-  const double orb = estimate_us(pairs.size() * pass_flop(c, c->N), prec) + 200.0;
-  if (orb > 0.8 * full) return 0;
+  if (p.chains == 0) return 0;
   if (prec != PREC_FP64 && !split_ready(c, prec)) return 0;
-  p.prec = prec;
-  p.nc = nc;
-  p.npairs = (int)pairs.size();
-  p.rank = 0;
-  for (const int4& m : mats) p.rank = std::max(p.rank, m.y);
-  // rounds of the clean-up: whole chains, at most kOrbPairs pairs each
-  p.rounds.clear();
-  for (int ch = 0, at = 0; ch < nc;) {
-    int used = 0, c0 = ch;
-    while (ch < nc && used + 2 * mats[ch].y <= kOrbPairs) {
-      for (int sec = 0; sec < 2; ++sec) {
-        cmats[2 * ch + sec].x = used;
-        used += mats[ch].y;
-      }
-      ++ch;
+  if (p.others.n && !p.general) {   // what the other chains leave, before it is spread
+    const size_t count = kMaxChains * ((size_t)c->n + (size_t)c->n * c->n);
+    if (hipMalloc((void**)&p.general, sizeof(double) * count) != hipSuccess) {
+      (void)hipGetLastError();
+      p.general = nullptr;
+      return 0;
     }
-    p.rounds.push_back({c0, ch - c0, at, used});
-    at += used;
   }
+  // rounds of whole chains, at most kOrbPairs pairs each; of the clean-up, whose
+  // matrices are the two sectors of each chain
+  std::vector<int2> pairs, clean;
+  std::vector<int4> mats, cmats;
+  auto deal = [&](int sectors, std::vector<OrbPlan::Round>& rounds, std::vector<int2>& pr,
+                  std::vector<int4>& mt) {
+    rounds.clear();
+    for (int ch = 0; ch < nc; ++ch) {
+      if (!ranks[ch]) continue;
+      if (rounds.empty() || rounds.back().count + sectors * ranks[ch] > kOrbPairs)
+        rounds.push_back({(int)mt.size(), 0, (int)pr.size(), 0});
+      OrbPlan::Round& rd = rounds.back();
+      for (int sec = 0; sec < sectors; ++sec) {
+        const int m = sectors * ch + sec;
+        mt.push_back(int4{rd.count, ranks[ch], ch, m});
+        for (int q : pivots[ch]) pr.push_back(int2{m, q});
+        rd.count += ranks[ch];
+        ++rd.mats;
+      }
+    }
+  };
+  deal(1, p.rounds, pairs, mats);
+  deal(2, p.clean_rounds, clean, cmats);
   const size_t b0 = sizeof(int4) * (mats.size() + cmats.size()),
                b1 = sizeof(int2) * (pairs.size() + clean.size()), b2 = sizeof(double) * Call.size();
   const size_t need = b0 + b1 + b2;
   if (p.cap < need) {
-    orbit_plan_free(p);
+    if (p.dev) (void)hipFree(p.dev);
+    p.dev = nullptr;
     p.cap = 0;
-    const size_t most = sizeof(int4) * 3 * kMaxChains + sizeof(int2) * 3 * kOrbPairs +
+    const size_t most = sizeof(int4) * 3 * kMaxChains + sizeof(int2) * 3 * kMaxChains * kOrbRank +
                         sizeof(double) * kMaxChains * (size_t)ns * kOrbRank;
     TDS_CHECK_HIP(hipMalloc(&p.dev, std::max(most, need)));
     p.cap = std::max(most, need);
@@ -1006,40 +1033,74 @@ static OrbPanels panels(const Ctx* c) {
   return OrbPanels{o.start, o.npanel, o.nsym, o.S, o.ST};
 }
 
-// the perturbed averages of the plan's chains (inputs in c->R1, c->Y1)
+// the perturbed averages of the plan's chains with an orbit (inputs in c->R1, c->Y1)
+static int run_orbits(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
+                      hipStream_t s) {
+  Orbit& o = c->orb;
+  const int n = c->n, np = c->np, ks = orb_ksplit(c);
+  const OrbPanels pn = panels(c);
+  for (const OrbPlan::Round& rd : p.rounds) {
+    const int P = rd.count;
+    hipLaunchKernelGGL(orb_in, dim3(o.npanel * o.npanel, P), dim3(256), 0, s, pn, p.pairs + rd.pair,
+                       c->Y1, c->R1, np, (const int*)nullptr, 0, o.Y1, o.R1);
+    if (p.prec != PREC_FP64) {
+      // the split kernels on the configurations, in groups of 6 pairs (they take three
+      // at a time).  128 atoms x 20000, 9 pairs: 0.40 ms for 2.0 in FP64; against FP64
+      // results the error is below that of the split average over the images (d2v
+      // 1e-7 for 7e-7 in FP16x2, 1.3e-6 for 1.5e-6 in BF16x2 at 12000 configurations)
+      for (int p0 = 0; p0 < P; p0 += 6) {
+        o.sub->R1 = o.R1 + (long)p0 * np;
+        o.sub->Y1 = o.Y1 + (long)p0 * np * np;
+        o.sub->f_out = o.f + (long)p0 * np;
+        o.sub->d2v_out = o.z + (long)p0 * np * np;
+        const int rc = launch_pa_split(o.sub, std::min(6, P - p0), apply_d4, p.prec, s, nullptr);
+        if (rc) return rc;
+      }
+    } else {
+      const F64Rows rows{o.U, o.F, o.rho, o.Mp};
+      launch_weights_f64(rows, n, np, P, o.Y1, o.R1, c->fy, c->fpsi, apply_d4, 0, (c->N + 63) / 64,
+                         0, c->N, o.coef, s);
+      const long ke = round_up_l(c->N, 8);
+      launch_outer_f64(rows, n, np, P, o.coef, c->fy, ks, 0, ke, round_up_l((ke + ks - 1) / ks, 8),
+                       0, o.zpart, o.fpart, s);
+      launch_reduce_f64(n, np, P, ks, o.zpart, o.fpart, o.z, o.f, 1.0 / c->n_eff, s);
+    }
+    const auto out = p.rank <= 3 ? orb_out<true, 3> : orb_out<true, kOrbRank>;
+    hipLaunchKernelGGL(out, dim3(o.npanel * (o.npanel + 3) / 2, rd.mats), dim3(512), 0, s, pn,
+                       p.mats + rd.mat, p.C, o.z, o.f, c->fy, n, np, 1.0 / o.nsym,
+                       1.0 / (c->n_eff * o.nsym), (const int*)nullptr, 0, (const int*)nullptr,
+                       f_dev, d2v_dev);
+    TDS_CHECK_HIP(hipGetLastError());
+  }
+  return 0;
+}
+
+// dst[k] = src[at[k]] (GATHER; in place too: at[k] >= k, and an element is moved by one
+// thread) or dst[at[k]] = src[k], `per` doubles per chain
+template <bool GATHER>
+__global__ void orb_move(const double* src, double* dst, OrbPlan::List l, long per) {
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= per) return;
+  for (int k = 0; k < l.n; ++k)
+    dst[(GATHER ? k : l.at[k]) * per + e] = src[(GATHER ? l.at[k] : k) * per + e];
+}
+
+// the perturbed averages of the plan's chains (inputs in c->R1, c->Y1): those with an
+// orbit, then the others, which c->R1, c->Y1 are packed for
 int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
                  hipStream_t s) {
-  Orbit& o = c->orb;
-  const int n = c->n, np = c->np, P = p.npairs, ks = orb_ksplit(c);
-  const OrbPanels pn = panels(c);
-  hipLaunchKernelGGL(orb_in, dim3(o.npanel * o.npanel, P), dim3(256), 0, s, pn, p.pairs, c->Y1,
-                     c->R1, np, (const int*)nullptr, 0, o.Y1, o.R1);
-  if (p.prec != PREC_FP64) {
-    // the split kernels on the configurations, in groups of 6 pairs (they take three
-    // at a time).  128 atoms x 20000, 9 pairs: 0.40 ms for 2.0 in FP64; against FP64
-    // results the error is below that of the split average over the images (d2v
-    // 1e-7 for 7e-7 in FP16x2, 1.3e-6 for 1.5e-6 in BF16x2 at 12000 configurations)
-    for (int p0 = 0; p0 < P; p0 += 6) {
-      o.sub->R1 = o.R1 + (long)p0 * np;
-      o.sub->Y1 = o.Y1 + (long)p0 * np * np;
-      o.sub->f_out = o.f + (long)p0 * np;
-      o.sub->d2v_out = o.z + (long)p0 * np * np;
-      const int rc = launch_pa_split(o.sub, std::min(6, P - p0), apply_d4, p.prec, s, nullptr);
-      if (rc) return rc;
-    }
-  } else {
-    const F64Rows rows{o.U, o.F, o.rho, o.Mp};
-    launch_weights_f64(rows, n, np, P, o.Y1, o.R1, c->fy, c->fpsi, apply_d4, 0, (c->N + 63) / 64,
-                       0, c->N, o.coef, s);
-    const long ke = round_up_l(c->N, 8);
-    launch_outer_f64(rows, n, np, P, o.coef, c->fy, ks, 0, ke, round_up_l((ke + ks - 1) / ks, 8),
-                     0, o.zpart, o.fpart, s);
-    launch_reduce_f64(n, np, P, ks, o.zpart, o.fpart, o.z, o.f, 1.0 / c->n_eff, s);
-  }
-  const auto out = p.rank <= 3 ? orb_out<true, 3> : orb_out<true, kOrbRank>;
-  hipLaunchKernelGGL(out, dim3(o.npanel * (o.npanel + 3) / 2, p.nc), dim3(512), 0, s, pn, p.mats, p.C, o.z, o.f, c->fy, n, np, 1.0 / o.nsym,
-                     1.0 / (c->n_eff * o.nsym), (const int*)nullptr, 0, (const int*)nullptr, f_dev,
-                     d2v_dev);
+  int rc = run_orbits(c, p, apply_d4, f_dev, d2v_dev, s);
+  if (rc || p.others.n == 0) return rc;
+  const long n = c->n, np = c->np;
+  auto blocks = [](long count) { return dim3((unsigned)((count + 255) / 256)); };
+  hipLaunchKernelGGL(orb_move<true>, blocks(np), dim3(256), 0, s, c->R1, c->R1, p.others, np);
+  hipLaunchKernelGGL(orb_move<true>, blocks(np * np), dim3(256), 0, s, c->Y1, c->Y1, p.others,
+                     np * np);
+  double *f = p.general, *d = p.general + kMaxChains * n;
+  rc = run_pa(c, p.others.n, apply_d4, p.prec, f, d, s);
+  if (rc) return rc;
+  hipLaunchKernelGGL(orb_move<false>, blocks(n), dim3(256), 0, s, f, f_dev, p.others, n);
+  hipLaunchKernelGGL(orb_move<false>, blocks(n * n), dim3(256), 0, s, d, d2v_dev, p.others, n * n);
   TDS_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1054,15 +1115,13 @@ int orbit_clean(Ctx* c, const OrbPlan& p, double* x, const int* kk, const int* a
   const OrbPanels pn = panels(c);
   hipLaunchKernelGGL(orb_unpack, dim3((unsigned)((nn + 255) / 256), 2 * p.nc), dim3(256), 0, s, x,
                      n, np, kk, kOrbClean, o.Yb, o.Rb);
-  const long len = n + (long)n * (n + 1);
-  for (const OrbPlan::Round& r : p.rounds) {
+  for (const OrbPlan::Round& r : p.clean_rounds) {
     hipLaunchKernelGGL(orb_in, dim3(o.npanel * o.npanel, r.count), dim3(256), 0, s, pn,
-                       p.clean + r.first, o.Yb, o.Rb, np, kk, kOrbClean, o.Y1, o.R1);
+                       p.clean + r.pair, o.Yb, o.Rb, np, kk, kOrbClean, o.Y1, o.R1);
     const auto out = p.rank <= 3 ? orb_out<false, 3> : orb_out<false, kOrbRank>;
-    hipLaunchKernelGGL(out, dim3(o.npanel * (o.npanel + 3) / 2, 2 * r.chains),
-                       dim3(512), 0, s, pn, p.cmats + 2 * r.chain0, p.C, o.Y1, o.R1, c->fy, n, np,
-                       1.0 / o.nsym, 1.0 / o.nsym, kk, kOrbClean, active + r.chain0,
-                       (double*)nullptr, x + r.chain0 * len);
+    hipLaunchKernelGGL(out, dim3(o.npanel * (o.npanel + 3) / 2, r.mats), dim3(512), 0, s, pn,
+                       p.cmats + r.mat, p.C, o.Y1, o.R1, c->fy, n, np, 1.0 / o.nsym, 1.0 / o.nsym,
+                       kk, kOrbClean, active, (double*)nullptr, x);
   }
   TDS_CHECK_HIP(hipGetLastError());
   return 0;

@@ -178,7 +178,8 @@ __global__ void rot_out_left(RotTab tb, const double* __restrict__ T2,
 }
 
 // d2v[chain] += normd T1[k], f[chain] += normf F1[k] for the pairs of the pass
-// in order (one thread per element of the unpadded outputs)
+// in order (one thread per element of the unpadded outputs; the upper half of T1 for
+// both, so that d2v is exactly symmetric)
 __global__ void rot_accumulate(const double* __restrict__ T1, const double* __restrict__ F1,
                                int n, int np, int nsym, int p0, int g, double normf, double normd,
                                double* __restrict__ f_all, double* __restrict__ d2v_all) {
@@ -192,7 +193,7 @@ __global__ void rot_accumulate(const double* __restrict__ T1, const double* __re
 #pragma unroll
   for (int k = 0; k < kMaxChains; ++k) {
     const int kk = k < g ? k : g - 1;
-    t[k] = T1[(long)kk * nn + (long)r * np + q];
+    t[k] = T1[(long)kk * nn + (long)min(r, q) * np + max(r, q)];
     fv[k] = e < n ? F1[(long)kk * np + e] : 0.0;
   }
   int ch = p0 / nsym;

@@ -23,7 +23,8 @@ class System:
     """54 atoms with the point group of a cubic crystal (the images of one chain are
     enough work for the orbit form), and the same images as configurations."""
 
-    def __init__(self, T=300.0, N=3000, weights=None, trans=True, tables=None):
+    def __init__(self, T=300.0, N=3000, weights=None, trans=True, tables=None,
+                 reference=True, form="images"):
         from tdscha_amd.lanczos import Lanczos
         from tdscha_amd.rocksalt import Ensemble, RockSalt
         ens = Ensemble(RockSalt(L=3), T, N, seed=3)
@@ -41,11 +42,12 @@ class System:
                  (np.concatenate([ens.X @ s.T for s in S]),
                   np.concatenate([ens.Y @ s.T for s in S]), np.tile(rho, len(S)), one))
         self.sides = []
-        for X, Y, r, m in sides:
+        for X, Y, r, m in sides[:1 + reference]:
             lanc = Lanczos(ens)
             lanc.X, lanc.Y, lanc.rho, lanc.N = X, Y, r, len(X)
             lanc.N_eff = float(np.sum(r))
             lanc.gamma_only = trans
+            lanc.symmetry_form = form if m is ms else "images"
             lanc.init(symmetries=m)
             self.sides.append(lanc)
         self.row, self.col = np.triu_indices(self.n)
