@@ -142,3 +142,37 @@ def test_tables_that_are_not_orthogonal():
     assert p.sides[0].engine.orbit_chains() == 3
     assert np.linalg.norm(out - y) < 1e-12 * np.linalg.norm(y)
     p.close()
+
+
+def dropped(ms):
+    """47 of the 48 tables: closed under nothing."""
+    ms = copy.copy(ms)
+    ms.symmetries = [s[:-1] for s in ms.symmetries]
+    return ms
+
+
+def one_axis(ms):
+    """The translations along one axis only: their average is not cubic."""
+    ms = copy.copy(ms)
+    perms = np.array(ms.trans_cart_perms)
+    one = next(p for p in perms if not np.array_equal(p, np.arange(len(p))))
+    keep = [np.arange(len(one)), one, one[one]]
+    which = [next(i for i, p in enumerate(perms) if np.array_equal(p, k)) for k in keep]
+    ms.trans_cart_perms = [ms.trans_cart_perms[i] for i in which]
+    ms.trans_operators = [ms.trans_operators[i] for i in which]
+    ms.trans_projector = np.mean(ms.trans_operators, axis=0)
+    return ms
+
+
+@pytest.mark.parametrize("tables", [dropped, one_axis])
+def test_operators_that_do_not_commute(tables):
+    """The images of the IR vectors span three directions, so one application takes the
+    form; a run does not, since the operator does not keep them."""
+    p = System(tables=tables)
+    x = p.pack(p.ir())
+    p.check(x, 0)
+    y = p.sides[1].apply_L_batch(x)
+    out = p.sides[0].apply_L_batch(x)
+    assert p.sides[0].engine.orbit_chains() == 3
+    assert np.linalg.norm(out - y) < 1e-12 * np.linalg.norm(y)
+    p.close()
