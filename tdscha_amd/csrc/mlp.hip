@@ -209,7 +209,8 @@ __global__ __launch_bounds__(kFuseThreads) void mlp_fused_fwd(
       [&](int l, int o, int row, float sum) {
         const bool last = l + 1 == m.layers, in = o < m.dim[l + 1];
         const float z = sum + (in ? params[m.b[l] + o] : 0.f), y = last ? z : silu(z);
-        xs[(l + 1) & 1][row][o] = y;
+        // (zero past the layer's width whatever the sum: 0 x Inf is not)
+        xs[(l + 1) & 1][row][o] = in ? y : 0.f;
         const int b = b0 + row;
         if (b >= B || !in) return;
         if (!y_out) {
