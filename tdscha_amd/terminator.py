@@ -200,8 +200,14 @@ class Network:
 def forward_many(nets, x):
     """Outputs (M, n, n_out) of M networks of one shape for the same rows, the
     networks side by side on the device."""
-    x = np.atleast_2d(np.ascontiguousarray(x, dtype=np.float32))
-    y = np.empty((len(nets), x.shape[0], nets[0].shape[3]), np.float32)
+    x = np.ascontiguousarray(np.atleast_2d(x), dtype=np.float32)
+    for net in nets:
+        if x.shape[1] != net.dims[0] or net.dims[-1] != nets[0].dims[-1]:
+            raise ValueError("input has %d features, the network %d; outputs %d and %d"
+                             % (x.shape[1], net.dims[0], net.dims[-1], nets[0].dims[-1]))
+    if not nets:
+        raise ValueError("no networks")
+    y = np.empty((len(nets), x.shape[0], nets[0].dims[-1]), np.float32)
     h = (C.c_void_p * len(nets))(*[n.h for n in nets])
     _lib.check(_lib.lib().tdscha_mlp_forward_many(len(nets), h, x.shape[0], _p(x), _p(y)),
                "tdscha_mlp_forward_many")
