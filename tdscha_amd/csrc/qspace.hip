@@ -43,6 +43,7 @@ namespace tdscha {
 
 constexpr int kQMaxChains = 256;
 constexpr int kQMaxQ = 512;
+constexpr size_t kQKeep = 1L << 30;  // batch memory kept between calls
 constexpr int kD2vChains = 15;       // chains per slab q_d2v workgroup
 constexpr int kSlabBytes = 65536;    // LDS of one slab q_d2v workgroup (two buffers)
 constexpr int kD2vThreads = 256;     // threads (items) per slab q_d2v workgroup
@@ -72,8 +73,9 @@ struct QCtx {
   int reorth_jtile = 16;    // basis vectors per workgroup of the reorthogonalisation dots
   hipStream_t stream = nullptr;
   // device and pinned memory of a batch, kept for the next call (as large as the
-  // largest batch so far); `busy` while a batch uses it, another batch at that time
-  // allocates its own
+  // largest batch so far, at most kQKeep bytes each; 64 chains on 4x4x4 and 20000
+  // configurations take 0.1 GB); `busy` while a batch uses it, another batch at that
+  // time allocates its own
   void* work = nullptr;
   void* pinned = nullptr;
   size_t work_size = 0, pinned_size = 0;
@@ -940,8 +942,19 @@ __global__ void q_expand(const double2* __restrict__ X, const double2* __restric
 // ------------------------------------------------------------ batch setup
 static void free_batch(QBatch& b) {
   if (b.owner) {
-    (void)hipStreamSynchronize(b.owner->stream);   // (a failed run may still use it)
-    b.owner->busy.store(false, std::memory_order_release);
+    QCtx* q = b.owner;
+    (void)hipStreamSynchronize(q->stream);   // (a failed run may still use it)
+    if (q->work_size > kQKeep) {
+      (void)hipFree(q->work);
+      q->work = nullptr;
+      q->work_size = 0;
+    }
+    if (q->pinned_size > kQKeep) {
+      (void)hipHostFree(q->pinned);
+      q->pinned = nullptr;
+      q->pinned_size = 0;
+    }
+    q->busy.store(false, std::memory_order_release);
   } else {
     if (b.mem) (void)hipFree(b.mem);
     if (b.host) (void)hipHostFree(b.host);
