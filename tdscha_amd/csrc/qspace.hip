@@ -453,12 +453,13 @@ __global__ void q_slab_build(const double2* __restrict__ X, const double2* __res
 // depend on the copies into the other.  Each thread accumulates the 6x6
 // block of one (chain, pair) item, in configuration order; on small grids (long
 // slabs, few items) ns threads take an item, every ns-th configuration each, and
-// their blocks are added in LDS at the end (36 items at 8 chains on 2x2x2: 124 us with
-// one thread each, 61 us).  ns follows from the grid alone, so that a chain's
-// sums do not depend on its batch.  The item blocks
+// their blocks are added in LDS at the end (6 bands, 36 items at 8 chains on 2x2x2:
+// 124 us with one thread each, 61 us).  ns follows from the grid alone, so that a
+// chain's sums do not depend on its batch.  The item blocks
 // of one chunk run on one XCD and share the chunk through its L2.  T is known at
-// compile time so that the LDS offsets are immediates (64 chains on 4x4x4: 934 us
-// with a run-time T, 859 us).
+// compile time so that the LDS offsets are immediates (6 bands, 64 chains on 4x4x4:
+// 934 us with a run-time T, 859 us).  Three bands run here on every grid, six on those
+// whose slabs are too short for q_d2v_mma (more than 69 q-points).
 constexpr int kSlabUnits = kSlabBytes / 2 / (int)sizeof(double2);
 constexpr int d2v_slices(int T) { return T > 2 ? T / 2 : 1; }
 
@@ -1018,14 +1019,15 @@ static size_t slab_units(int nq, int nb, int T) {
   return 2 * (size_t)nq * (nb * T + 1) + 2 * (size_t)kD2vChains * T;
 }
 
-template <typename Fn>
+// (6 bands: grids whose slabs hold 4 configurations or more run q_d2v_mma)
+template <int NB, typename Fn>
 static void with_slab(int T, Fn fn) {
-  switch (T) {
-    case 1: fn(std::integral_constant<int, 1>{}); break;
-    case 2: fn(std::integral_constant<int, 2>{}); break;
-    case 4: fn(std::integral_constant<int, 4>{}); break;
-    case 8: fn(std::integral_constant<int, 8>{}); break;
-    default: fn(std::integral_constant<int, 16>{}); break;
+  if (T == 1) fn(std::integral_constant<int, 1>{});
+  if (T == 2) fn(std::integral_constant<int, 2>{});
+  if constexpr (NB != 6) {
+    if (T == 4) fn(std::integral_constant<int, 4>{});
+    if (T == 8) fn(std::integral_constant<int, 8>{});
+    if (T == 16) fn(std::integral_constant<int, 16>{});
   }
 }
 
@@ -1258,7 +1260,7 @@ static void launch_L_nb(QCtx* q, QBatch& b, const double2* psi, double2* out, in
       if (q->mma)
         run(b.slabT == 16 ? q_d2v_mma<16> : b.slabT == 8 ? q_d2v_mma<8> : q_d2v_mma<4>, 1024);
       else
-        with_slab(b.slabT, [&](auto T) { run(q_d2v_slab<NB, decltype(T)::value>, kD2vThreads); });
+        with_slab<NB>(b.slabT, [&](auto T) { run(q_d2v_slab<NB, decltype(T)::value>, kD2vThreads); });
     } else {
       hipLaunchKernelGGL(q_d2v<NB>, dim3(b.maxp, C, b.nch), dim3(256), 0, s, q->X, q->Y, q->N,
                          q->fY, b.active, b.npairs, b.pq1, b.pq2, MP, b.wc, b.wd, b.chunk, b.nch,
