@@ -64,7 +64,7 @@ int setup_pairs(Ctx* c) {
     rw[m] = 2 * wv[m] * nm * (nm + 1) / (2 * nm + 1);
   }
   auto up = [&](void** dst, const void* src, size_t bytes) -> int {
-    TDS_CHECK_HIP(hipMalloc(dst, bytes));
+    TDS_CHECK_HIP(dev_alloc(c, dst, bytes));
     TDS_CHECK_HIP(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
     return 0;
   };
@@ -82,10 +82,10 @@ int setup_pairs(Ctx* c) {
   rc |= up((void**)&c->reaw, rw.data(), sizeof(double) * c->np);
   if (rc) return -1;
   const long len = n + 2 * P;
-  TDS_CHECK_HIP(hipMalloc((void**)&c->psi_dev, sizeof(double) * kMaxChains * len));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->psi_out_dev, sizeof(double) * kMaxChains * len));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->f_fin, sizeof(double) * kMaxChains * n));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->d2v_fin, sizeof(double) * kMaxChains * (long)n * n));
+  TDS_CHECK_HIP(dev_alloc(c, &c->psi_dev, sizeof(double) * kMaxChains * len));
+  TDS_CHECK_HIP(dev_alloc(c, &c->psi_out_dev, sizeof(double) * kMaxChains * len));
+  TDS_CHECK_HIP(dev_alloc(c, &c->f_fin, sizeof(double) * kMaxChains * n));
+  TDS_CHECK_HIP(dev_alloc(c, &c->d2v_fin, sizeof(double) * kMaxChains * (long)n * n));
   return 0;
 }
 
@@ -622,7 +622,7 @@ static int setup_inverse(Ctx* c) {
       ic[2 * P + p] = x1n;
       ic[3 * P + p] = y1n;
     }
-  TDS_CHECK_HIP(hipMalloc((void**)&c->inv_coef, sizeof(double) * 4 * P));
+  TDS_CHECK_HIP(dev_alloc(c, &c->inv_coef, sizeof(double) * 4 * P));
   TDS_CHECK_HIP(hipMemcpy(c->inv_coef, ic.data(), sizeof(double) * 4 * P, hipMemcpyHostToDevice));
   return 0;
 }
@@ -741,10 +741,10 @@ int tdscha_set_translations(tdscha_ctx* ctx, int n_cart, const double* pols, int
         jt[J] = bt;
       }
       c->n_rep = (int)reps.size();
-      TDS_CHECK_HIP(hipMalloc((void**)&c->rep_dof, sizeof(int) * c->n_rep));
-      TDS_CHECK_HIP(hipMalloc((void**)&c->jrep, sizeof(int) * n_cart));
-      TDS_CHECK_HIP(hipMalloc((void**)&c->ju, sizeof(int) * n_cart));
-      TDS_CHECK_HIP(hipMalloc((void**)&c->rep_sum,
+      TDS_CHECK_HIP(dev_alloc(c, &c->rep_dof, sizeof(int) * c->n_rep));
+      TDS_CHECK_HIP(dev_alloc(c, &c->jrep, sizeof(int) * n_cart));
+      TDS_CHECK_HIP(dev_alloc(c, &c->ju, sizeof(int) * n_cart));
+      TDS_CHECK_HIP(dev_alloc(c, &c->rep_sum,
                               sizeof(double) * kMaxChains * (long)c->n_rep * n_cart));
       TDS_CHECK_HIP(hipMemcpy(c->rep_dof, reps.data(), sizeof(int) * c->n_rep,
                               hipMemcpyHostToDevice));
@@ -753,13 +753,13 @@ int tdscha_set_translations(tdscha_ctx* ctx, int n_cart, const double* pols, int
     }
   }
   c->n_cart = n_cart;
-  TDS_CHECK_HIP(hipMalloc((void**)&c->pols, sizeof(double) * (long)n_cart * n));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->inv_perms, sizeof(int) * (long)n_cells * n_cart));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->tproj, sizeof(double) * (long)n * n));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->cart_tmp, sizeof(double) * kMaxChains * (long)n_cart * n_cart));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->cart_tmp2, sizeof(double) * kMaxChains * (long)n_cart * n_cart));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->mode_tmp, sizeof(double) * kMaxChains * (long)n_cart * n));
-  TDS_CHECK_HIP(hipMalloc((void**)&c->f_proj, sizeof(double) * kMaxChains * n));
+  TDS_CHECK_HIP(dev_alloc(c, &c->pols, sizeof(double) * (long)n_cart * n));
+  TDS_CHECK_HIP(dev_alloc(c, &c->inv_perms, sizeof(int) * (long)n_cells * n_cart));
+  TDS_CHECK_HIP(dev_alloc(c, &c->tproj, sizeof(double) * (long)n * n));
+  TDS_CHECK_HIP(dev_alloc(c, &c->cart_tmp, sizeof(double) * kMaxChains * (long)n_cart * n_cart));
+  TDS_CHECK_HIP(dev_alloc(c, &c->cart_tmp2, sizeof(double) * kMaxChains * (long)n_cart * n_cart));
+  TDS_CHECK_HIP(dev_alloc(c, &c->mode_tmp, sizeof(double) * kMaxChains * (long)n_cart * n));
+  TDS_CHECK_HIP(dev_alloc(c, &c->f_proj, sizeof(double) * kMaxChains * n));
   TDS_CHECK_HIP(hipMemcpy(c->pols, pols, sizeof(double) * (long)n_cart * n, hipMemcpyHostToDevice));
   TDS_CHECK_HIP(hipMemcpy(c->inv_perms, inv_perms, sizeof(int) * (long)n_cells * n_cart,
                           hipMemcpyHostToDevice));

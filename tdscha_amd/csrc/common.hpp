@@ -186,6 +186,7 @@ struct Orbit {
   std::vector<double> syms;               // host copy of the symmetry blocks
   std::vector<int> gens;                  // generators of the group
   double* arena = nullptr;                // holds start, S, ST, pu, pf (and U, F, rho)
+  size_t arena_bytes = 0;
   int* start = nullptr;                   // [npanel + 1]
   double *S = nullptr, *ST = nullptr;     // [npanel, nsym, 32, 32] panels of S_j, transposed
   double *U = nullptr, *F = nullptr, *rho = nullptr;       // [Mp, np] the configurations
@@ -195,7 +196,7 @@ struct Orbit {
   double* pout = nullptr;                 // pinned host memory: its results
   double *R1 = nullptr, *Y1 = nullptr;    // [kOrbPairs, np(, np)] rotated inputs
   double *Rb = nullptr, *Yb = nullptr;    // [2 kMaxChains, np(, np)] unpacked vectors
-  double *coef = nullptr, *zpart = nullptr, *fpart = nullptr, *z = nullptr, *f = nullptr;
+  double *coef = nullptr, *z = nullptr, *f = nullptr;
   // the configurations as a context of their own, with what the split precisions need
   // (made at the first plan in one of them); its inputs and outputs are set per pass
   Ctx* sub = nullptr;
@@ -324,6 +325,12 @@ unsigned orbit_candidates(const Ctx* c, int nc, int prec, const double* R, long 
 int orbit_sector(Ctx* c, bool* ok);
 int orbit_plan(Ctx* c, int nc, unsigned mask, int prec, const double* x, hipStream_t s,
                OrbPlan& p);
+bool orbit_ready(Ctx* c, int prec, hipStream_t s);
+hipError_t dev_alloc(Ctx* c, void** p, size_t bytes);
+template <typename T>
+hipError_t dev_alloc(Ctx* c, T** p, size_t bytes) {
+  return dev_alloc(c, reinterpret_cast<void**>(p), bytes);
+}
 int run_pa(Ctx* c, int nc, int apply_d4, int prec, double* f_dev, double* d2v_dev, hipStream_t s);
 int run_pa_orbit(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, double* d2v_dev,
                  hipStream_t s);

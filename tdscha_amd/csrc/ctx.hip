@@ -576,8 +576,8 @@ int tdscha_set_ksplit(tdscha_ctx* ctx, int ksplit) {
   Ctx* c = reinterpret_cast<Ctx*>(ctx);
   TDS_CHECK_HIP(hipStreamSynchronize(c->stream));
   double *zp = nullptr, *fp = nullptr;
-  TDS_CHECK_HIP(hipMalloc((void**)&zp, sizeof(double) * kMaxChains * zpart_size(c->n, ksplit)));
-  TDS_CHECK_HIP(hipMalloc((void**)&fp, sizeof(double) * kMaxChains * (size_t)ksplit * c->np));
+  TDS_CHECK_HIP(dev_alloc(c, &zp, sizeof(double) * kMaxChains * zpart_size(c->n, ksplit)));
+  TDS_CHECK_HIP(dev_alloc(c, &fp, sizeof(double) * kMaxChains * (size_t)ksplit * c->np));
   (void)hipFree(c->zpart);
   (void)hipFree(c->fpart);
   c->zpart = zp;

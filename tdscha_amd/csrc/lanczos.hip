@@ -759,17 +759,17 @@ int tdscha_lanczos_run_biconjugate(tdscha_ctx* ctx, int n_chains, const double* 
   const size_t vb = sizeof(double) * n_chains * len;
   bool ok = true;
   double** vecs[] = {&st.q, &st.qprev, &st.p, &st.pprev, &st.Lq, &st.pL, &st.r, &st.s};
-  for (double** v : vecs) ok = ok && hipMalloc((void**)v, vb) == hipSuccess;
-  ok = ok && hipMalloc((void**)&st.ones, sizeof(double) * len) == hipSuccess &&
-       hipMalloc((void**)&st.part, sizeof(double) * n_chains * 4 * kRedBlocks) == hipSuccess &&
-       hipMalloc((void**)&st.a, sizeof(double) * n_chains * n_steps) == hipSuccess &&
-       hipMalloc((void**)&st.b, sizeof(double) * n_chains * n_steps) == hipSuccess &&
-       hipMalloc((void**)&st.c, sizeof(double) * n_chains * n_steps) == hipSuccess &&
-       hipMalloc((void**)&st.scal, sizeof(double) * n_chains * 8) == hipSuccess &&
-       hipMalloc((void**)&st.k, sizeof(int) * n_chains) == hipSuccess &&
-       hipMalloc((void**)&st.active, sizeof(int) * n_chains) == hipSuccess &&
-       hipMalloc((void**)&st.cap, sizeof(int) * n_chains) == hipSuccess &&
-       hipMalloc((void**)&st.ndone, sizeof(int) * n_chains) == hipSuccess;
+  for (double** v : vecs) ok = ok && dev_alloc(c, v, vb) == hipSuccess;
+  ok = ok && dev_alloc(c, &st.ones, sizeof(double) * len) == hipSuccess &&
+       dev_alloc(c, &st.part, sizeof(double) * n_chains * 4 * kRedBlocks) == hipSuccess &&
+       dev_alloc(c, &st.a, sizeof(double) * n_chains * n_steps) == hipSuccess &&
+       dev_alloc(c, &st.b, sizeof(double) * n_chains * n_steps) == hipSuccess &&
+       dev_alloc(c, &st.c, sizeof(double) * n_chains * n_steps) == hipSuccess &&
+       dev_alloc(c, &st.scal, sizeof(double) * n_chains * 8) == hipSuccess &&
+       dev_alloc(c, &st.k, sizeof(int) * n_chains) == hipSuccess &&
+       dev_alloc(c, &st.active, sizeof(int) * n_chains) == hipSuccess &&
+       dev_alloc(c, &st.cap, sizeof(int) * n_chains) == hipSuccess &&
+       dev_alloc(c, &st.ndone, sizeof(int) * n_chains) == hipSuccess;
   if (!ok) {
     free_bi(st);
     set_error("tdscha_lanczos_run_biconjugate: device allocation failed");
@@ -900,7 +900,7 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
   carve.add(&st.ndone, nc);
   carve.add(&st.stepno, 1);
   if (st.jsplit > 1) carve.add(&st.upart, nc * st.jsplit * len);
-  bool ok = hipMalloc(&st.mem, carve.total()) == hipSuccess;
+  bool ok = dev_alloc(c, &st.mem, carve.total()) == hipSuccess;
   if (ok) carve.assign(st.mem);
   if (!ok) {
     free_state(st);
@@ -989,6 +989,11 @@ int tdscha_lanczos_run(tdscha_ctx* ctx, int n_chains, const double* psi0, int n_
     if (rc) {
       free_state(st);
       return rc;
+    }
+    // (it may have taken the memory of the orbit form: then the general one for all)
+    if (c->orb.chains && !orbit_ready(c, precision, s)) {
+      for (OrbPlan& p : st.plans) p.ok = false;
+      c->orb.chains = 0;
     }
   }
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)

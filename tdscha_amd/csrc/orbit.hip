@@ -655,8 +655,10 @@ int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const in
   auto up = [](void* dst, const void* src, size_t bytes) {
     return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess;
   };
-  if (hipMalloc((void**)&o.arena, sizeof(double) * at) != hipSuccess) {
+  o.arena_bytes = sizeof(double) * at;
+  if (hipMalloc((void**)&o.arena, o.arena_bytes) != hipSuccess) {
     (void)hipGetLastError();   // no room: the general form serves every call
+    o.arena = nullptr;
     return 0;
   }
   o.S = o.arena + aS; o.ST = o.arena + aST;
@@ -696,12 +698,16 @@ int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const in
   return 0;
 }
 
+static void drop_sub(Orbit& o) {
+  if (!o.sub) return;
+  free_split(o.sub);
+  delete o.sub;   // (its rows, inputs and outputs belong to this struct)
+  o.sub = nullptr;
+}
+
 void orbit_free(Ctx* c) {
   Orbit& o = c->orb;
-  if (o.sub) {
-    free_split(o.sub);
-    delete o.sub;   // (its rows, inputs and outputs belong to this struct)
-  }
+  drop_sub(o);
   if (o.arena) (void)hipFree(o.arena);
   if (o.work) (void)hipFree(o.work);
   if (o.pout) (void)hipHostFree(o.pout);
@@ -726,31 +732,27 @@ static int orb_ksplit(const Ctx* c) {
   return ks;
 }
 
-// workspaces of the orbit form, at its first use; false = no room (the general form
-// serves this and every later call)
-static bool ensure(Ctx* c) {
+// workspaces of the orbit form (the partial sums are the context's, idle in these
+// calls); false = no room: the general form serves this call
+static bool ensure(Ctx* c, hipStream_t s) {
   Orbit& o = c->orb;
   if (o.work) return true;
   const size_t np = c->np, nn = np * np;
-  const int ks = orb_ksplit(c), ncol = (c->n + 15) / 16;
+  const int ncol = (c->n + 15) / 16;
   const size_t count[] = {2 * (size_t)kMaxChains * ncol * o.rows * 4,
                           kOrbPairs * np, kOrbPairs * nn,
                           2 * kMaxChains * np, 2 * kMaxChains * nn,
                           kOrbPairs * (size_t)o.Mp * 4,
-                          kOrbPairs * ks * nn, kOrbPairs * ks * np,
                           kOrbPairs * nn, kOrbPairs * np};
-  double** dst[] = {&o.ppart, &o.R1, &o.Y1, &o.Rb, &o.Yb, &o.coef, &o.zpart, &o.fpart, &o.z, &o.f};
+  double** dst[] = {&o.ppart, &o.R1, &o.Y1, &o.Rb, &o.Yb, &o.coef, &o.z, &o.f};
   size_t at = 0;
   for (size_t k : count) at += (k + 31) / 32 * 32;
   const size_t nout = 2 * (size_t)kMaxChains * o.rows * 4;
-  if (hipMalloc((void**)&o.work, sizeof(double) * at) != hipSuccess) o.work = nullptr;
-  if (o.work && hipHostMalloc((void**)&o.pout, sizeof(double) * nout) != hipSuccess) {
-    (void)hipFree(o.work);
-    o.work = o.pout = nullptr;
-  }
-  if (!o.work) {
+  if (!o.pout && hipHostMalloc((void**)&o.pout, sizeof(double) * nout) != hipSuccess)
+    o.pout = nullptr;
+  if (!o.pout || hipMalloc((void**)&o.work, sizeof(double) * at) != hipSuccess) {
     (void)hipGetLastError();
-    o.usable = false;
+    o.work = nullptr;
     return false;
   }
   at = 0;
@@ -758,7 +760,48 @@ static bool ensure(Ctx* c) {
     *dst[k] = o.work + at;
     at += (count[k] + 31) / 32 * 32;
   }
+  // the padding of the rotated inputs is never written
+  if (hipMemsetAsync(o.R1, 0, sizeof(double) * kOrbPairs * np, s) != hipSuccess ||
+      hipMemsetAsync(o.Y1, 0, sizeof(double) * kOrbPairs * nn, s) != hipSuccess ||
+      hipStreamSynchronize(s) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipFree(o.work);
+    o.work = nullptr;
+    return false;
+  }
   return true;
+}
+
+// Device memory of the context for anything but the orbit form, which gives way: first
+// its workspaces and split images (made again by the next call that has room for them),
+// then, where that is enough, its tables and configurations (the general form from then
+// on).  A plan's own arrays stay.
+hipError_t dev_alloc(Ctx* c, void** p, size_t bytes) {
+  Orbit& o = c->orb;
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && (o.work || o.sub)) {
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(c->stream);
+    drop_sub(o);
+    if (o.work) (void)hipFree(o.work);
+    o.work = nullptr;
+    e = hipMalloc(p, bytes);
+  }
+  size_t left = 0, all = 0;
+  if (e != hipSuccess && o.arena && hipMemGetInfo(&left, &all) == hipSuccess &&
+      left + o.arena_bytes >= bytes) {
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(o.arena);
+    o.arena = nullptr;
+    o.usable = false;
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+  }
+  return e;
 }
 
 // ----------------------------------------------------------------- the relation
@@ -910,6 +953,11 @@ static bool split_ready(Ctx* c, int prec) {
   return false;
 }
 
+// whether what the passes of a plan in this precision need is there (again)
+bool orbit_ready(Ctx* c, int prec, hipStream_t s) {
+  return c->orb.usable && ensure(c, s) && (prec == PREC_FP64 || split_ready(c, prec));
+}
+
 // Plan of nc chains (waits for the stream): the chains of `mask` that have a small orbit
 // take the form (p.ok: some do), the others the general one.  x null: the averages of
 // the padded inputs in c->R1, c->Y1.  Else a run from the packed vectors x (device):
@@ -918,13 +966,7 @@ int orbit_plan(Ctx* c, int nc, unsigned mask, int prec, const double* x, hipStre
                OrbPlan& p) {
   Orbit& o = c->orb;
   p.ok = false;
-  const bool first = !o.work;
-  if (!ensure(c)) return 0;
-  if (first) {   // the padding of the rotated inputs is never written
-    TDS_CHECK_HIP(hipMemsetAsync(o.R1, 0, sizeof(double) * kOrbPairs * c->np, s));
-    TDS_CHECK_HIP(hipMemsetAsync(o.Y1, 0, sizeof(double) * kOrbPairs * (size_t)c->np * c->np, s));
-    TDS_CHECK_HIP(hipStreamSynchronize(s));
-  }
+  if (!ensure(c, s)) return 0;
   const int ncol = (c->n + 15) / 16, rows4 = o.rows * 4, ns = o.nsym;
   std::vector<int> piv;
   std::vector<double> C, Call;
@@ -1060,10 +1102,17 @@ static int run_orbits(Ctx* c, const OrbPlan& p, int apply_d4, double* f_dev, dou
       const F64Rows rows{o.U, o.F, o.rho, o.Mp};
       launch_weights_f64(rows, n, np, P, o.Y1, o.R1, c->fy, c->fpsi, apply_d4, 0, (c->N + 63) / 64,
                          0, c->N, o.coef, s);
-      const long ke = round_up_l(c->N, 8);
-      launch_outer_f64(rows, n, np, P, o.coef, c->fy, ks, 0, ke, round_up_l((ke + ks - 1) / ks, 8),
-                       0, o.zpart, o.fpart, s);
-      launch_reduce_f64(n, np, P, ks, o.zpart, o.fpart, o.z, o.f, 1.0 / c->n_eff, s);
+      // as many pairs at once as the context's partial sums have room for (it holds
+      // kMaxChains ksplit of them, ksplit at least 8, ks at most 24)
+      const long ke = round_up_l(c->N, 8), rps = round_up_l((ke + ks - 1) / ks, 8);
+      const int most = kMaxChains * c->ksplit / ks;
+      for (int p0 = 0; p0 < P; p0 += most) {
+        const int g = std::min(most, P - p0);
+        launch_outer_f64(rows, n, np, g, o.coef + (long)p0 * o.Mp * 4, c->fy, ks, 0, ke, rps, 0,
+                         c->zpart, c->fpart, s);
+        launch_reduce_f64(n, np, g, ks, c->zpart, c->fpart, o.z + (long)p0 * np * np,
+                          o.f + (long)p0 * np, 1.0 / c->n_eff, s);
+      }
     }
     const auto out = p.rank <= 3 ? orb_out<true, 3> : orb_out<true, kOrbRank>;
     hipLaunchKernelGGL(out, dim3(o.npanel * (o.npanel + 3) / 2, rd.mats), dim3(512), 0, s, pn,

@@ -936,30 +936,30 @@ int ensure_split(Ctx* c, int prec) {
   TDS_REQUIRE(Mp % kBR == 0 && np % kBR == 0, 3, "split path: padded sizes must be multiples of 128");
   const size_t half_bytes = sizeof(u16) * (size_t)Mp * np;
   void** arr[] = {&st.Uh, &st.Ul, &st.UhT, &st.UlT};
-  for (void** p : arr) TDS_CHECK_HIP(hipMalloc(p, half_bytes));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.FA, 2 * half_bytes));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.UA32, 2 * half_bytes));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.XT, 2 * half_bytes));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.YT, 2 * half_bytes));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.su, sizeof(double) * np));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.sf, sizeof(double) * np));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.umax, sizeof(double) * np));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.fmax, sizeof(double) * np));
-  TDS_CHECK_HIP(hipMalloc((void**)&st.colw, sizeof(float) * 3 * np));
+  for (void** p : arr) TDS_CHECK_HIP(dev_alloc(c, p, half_bytes));
+  TDS_CHECK_HIP(dev_alloc(c, &st.FA, 2 * half_bytes));
+  TDS_CHECK_HIP(dev_alloc(c, &st.UA32, 2 * half_bytes));
+  TDS_CHECK_HIP(dev_alloc(c, &st.XT, 2 * half_bytes));
+  TDS_CHECK_HIP(dev_alloc(c, &st.YT, 2 * half_bytes));
+  TDS_CHECK_HIP(dev_alloc(c, &st.su, sizeof(double) * np));
+  TDS_CHECK_HIP(dev_alloc(c, &st.sf, sizeof(double) * np));
+  TDS_CHECK_HIP(dev_alloc(c, &st.umax, sizeof(double) * np));
+  TDS_CHECK_HIP(dev_alloc(c, &st.fmax, sizeof(double) * np));
+  TDS_CHECK_HIP(dev_alloc(c, &st.colw, sizeof(float) * 3 * np));
   if (!c->Y1h) {
-    TDS_CHECK_HIP(hipMalloc(&c->Y1h, sizeof(u16) * kMaxChains * (size_t)np * np));
-    TDS_CHECK_HIP(hipMalloc(&c->Y1l, sizeof(u16) * kMaxChains * (size_t)np * np));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->epi, sizeof(float) * kMaxChains * 2 * np));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->ysc, sizeof(double) * kMaxChains));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->ysc3, sizeof(double) * kMaxChains));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->pmax, sizeof(double) * kMaxChains * kPartBlocks * 2));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->coef32, sizeof(float) * kMaxChains * Mp * 4));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->wpart, sizeof(double) * kMaxChains * (np / kBR) * Mp * 4));
+    TDS_CHECK_HIP(dev_alloc(c, &c->Y1h, sizeof(u16) * kMaxChains * (size_t)np * np));
+    TDS_CHECK_HIP(dev_alloc(c, &c->Y1l, sizeof(u16) * kMaxChains * (size_t)np * np));
+    TDS_CHECK_HIP(dev_alloc(c, &c->epi, sizeof(float) * kMaxChains * 2 * np));
+    TDS_CHECK_HIP(dev_alloc(c, &c->ysc, sizeof(double) * kMaxChains));
+    TDS_CHECK_HIP(dev_alloc(c, &c->ysc3, sizeof(double) * kMaxChains));
+    TDS_CHECK_HIP(dev_alloc(c, &c->pmax, sizeof(double) * kMaxChains * kPartBlocks * 2));
+    TDS_CHECK_HIP(dev_alloc(c, &c->coef32, sizeof(float) * kMaxChains * Mp * 4));
+    TDS_CHECK_HIP(dev_alloc(c, &c->wpart, sizeof(double) * kMaxChains * (np / kBR) * Mp * 4));
     const int ks = choose_ksplit_split(np / kBR, Mp);
     c->ksplit_s = ks;
-    TDS_CHECK_HIP(hipMalloc((void**)&c->zpart32, sizeof(float) * kMaxChains * (size_t)ks * np * np));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->fpart_s, sizeof(double) * kMaxChains * (size_t)ks * np));
-    TDS_CHECK_HIP(hipMalloc((void**)&c->sbsc, sizeof(double) * kMaxChains * np));
+    TDS_CHECK_HIP(dev_alloc(c, &c->zpart32, sizeof(float) * kMaxChains * (size_t)ks * np * np));
+    TDS_CHECK_HIP(dev_alloc(c, &c->fpart_s, sizeof(double) * kMaxChains * (size_t)ks * np));
+    TDS_CHECK_HIP(dev_alloc(c, &c->sbsc, sizeof(double) * kMaxChains * np));
   }
   hipStream_t s = c->stream;
   TDS_CHECK_HIP(hipMemsetAsync(st.umax, 0, sizeof(double) * np, s));
@@ -1101,8 +1101,8 @@ int set_ksplit_split(Ctx* c, int ks) {
   TDS_CHECK_HIP(hipStreamSynchronize(c->stream));
   float* zp = nullptr;
   double* fp = nullptr;
-  TDS_CHECK_HIP(hipMalloc((void**)&zp, sizeof(float) * kMaxChains * (size_t)ks * c->np * c->np));
-  if (hipMalloc((void**)&fp, sizeof(double) * kMaxChains * (size_t)ks * c->np) != hipSuccess) {
+  TDS_CHECK_HIP(dev_alloc(c, &zp, sizeof(float) * kMaxChains * (size_t)ks * c->np * c->np));
+  if (dev_alloc(c, &fp, sizeof(double) * kMaxChains * (size_t)ks * c->np) != hipSuccess) {
     (void)hipFree(zp);
     set_error("set_ksplit_split: hipMalloc failed");
     return -1;

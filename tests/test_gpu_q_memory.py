@@ -3,12 +3,12 @@ that needs more than 1 GiB gives it back."""
 import numpy as np
 import pytest
 
+from tests.device_memory import free_bytes
+
 pytestmark = pytest.mark.gpu
 
 
 def test_kept_memory_is_bounded():
-    import torch
-
     from tdscha_amd import qspace as QS
     from tdscha_amd.qlanczos import QSpaceEngine
     rng = np.random.default_rng(0)
@@ -23,9 +23,9 @@ def test_kept_memory_is_bounded():
     psis = [(lambda n: rng.normal(size=n) + 1j * rng.normal(size=n))(eng.psi_size(pm))
             for pm in pms]
     small = eng.apply_L(iq[:3], pms[:3], psis[:3])
-    free = torch.cuda.mem_get_info()[0]
+    free = free_bytes()
     out = eng.apply_L(iq, pms, psis)
-    assert free - torch.cuda.mem_get_info()[0] < 1 << 30
+    assert free - free_bytes() < 1 << 30
     again = eng.apply_L(iq[:3], pms[:3], psis[:3])
     for a, b in zip(small, again):
         assert np.array_equal(a, b)
