@@ -234,11 +234,40 @@ def qspace_run(ens, seed=3, tol=1e-8, cap_range=(50, 400), per_chain=True, tiles
     return out
 
 
+def general_L(lanc, psis, precision, reps=0):
+    """L of the vectors through the device entry point, which averages over all
+    images (or rotated passes) whatever their symmetry, and its rate in
+    L-applications/s over `reps` calls (the chains and the host calls take the
+    few rotations of an IR vector instead)."""
+    from tdscha_amd import _lib
+    from tdscha_amd.engine import precision_code
+    lib, eng = _lib.lib(), lanc.engine
+    src, dst = _lib.DeviceBuffer.from_array(psis), _lib.DeviceBuffer(psis.shape)
+
+    def apply():
+        _lib.check(lib.tdscha_apply_L_dev(eng.ctx, len(psis), src.ptr, dst.ptr, 1, 0, 0, 0, 0, 0,
+                                          0.0, precision_code(precision), None), "apply_L_dev")
+
+    apply()
+    eng.synchronize()
+    t0 = time.perf_counter()
+    for _ in range(reps):
+        apply()
+    eng.synchronize()
+    rate = len(psis) * reps / (time.perf_counter() - t0)
+    out = dst.numpy()
+    src.free()
+    dst.free()
+    return out, rate
+
+
 def rotation_run(ens, psis, lanc_img, results, args):
     """The same chains with the symmetries applied by rotating operators
     (configurations only on the device): L-applications/s of the FP64 and
-    headline split paths, device bytes of the two ensembles, and how far the
-    rotated L and the first coefficients sit from the image form's."""
+    headline split paths (both run the IR chains on the rotations of the start
+    vectors, whatever the ensemble's form), of one general L in each form,
+    device bytes of the two ensembles, and how far the rotated L sits from the
+    image form's."""
     from tdscha_amd.lanczos import Lanczos
     lanc = Lanczos(ens)
     lanc.gamma_only = True
@@ -267,18 +296,17 @@ def rotation_run(ens, psis, lanc_img, results, args):
         if prec in results:
             img = results[prec]
             out[prec + "_vs_images"] = (n_l / wall) / (img["n_l"] / img["wall"])
-            da = 0.0
-            for (a1, _), (a0, _) in zip(chains, img["chains"]):
-                k = min(len(a1), len(a0))
-                da = max(da, float(np.max(np.abs(a1[:k] - a0[:k]) / np.abs(a0[:k]))))
-            out[prec + "_coeff_a_max_rel_diff_vs_images"] = da
         log("rotation form %s: %d steps x %d chains %.3fs -> %.1f L/s" % (
             prec, args.rotation_steps, nc, wall, n_l / wall))
-    lanc.precision = "fp64"
-    lanc_img.precision = "fp64"
-    Lr, Li = lanc.apply_L_batch(psis), lanc_img.apply_L_batch(psis)
-    out["fp64_Lv_rel_diff_vs_images"] = float(np.max(np.linalg.norm(Lr - Li, axis=1)
-                                                     / np.linalg.norm(Li, axis=1)))
+    for prec in dict.fromkeys(["fp64", args.precision]):
+        Lr, rate_r = general_L(lanc, psis, prec, reps=3)
+        Li, rate_i = general_L(lanc_img, psis, prec, reps=3)
+        out[prec + "_general_L_value"] = rate_r
+        out[prec + "_general_L_value_images"] = rate_i
+        out[prec + "_general_Lv_rel_diff_vs_images"] = float(
+            np.max(np.linalg.norm(Lr - Li, axis=1) / np.linalg.norm(Li, axis=1)))
+        log("rotation form %s, general L: %.1f L/s (images %.1f), L.v apart by %.1e" % (
+            prec, rate_r, rate_i, out[prec + "_general_Lv_rel_diff_vs_images"]))
     lanc.close()
     return out
 
@@ -425,7 +453,8 @@ def main():
             timed_run(prec, W)
         chains, wall, dev_ms = timed_run(prec, K)
         n_l = sum(len(a) for a, _ in chains)
-        results[prec] = dict(chains=chains, wall=wall, dev_ms=dev_ms, n_l=n_l)
+        results[prec] = dict(chains=chains, wall=wall, dev_ms=dev_ms, n_l=n_l,
+                             orbit=lanc.engine.orbit_chains())
         log("%s: %d steps x %d chains: wall %.3fs, device loop %.3fs -> %.1f L/s" % (
             prec, K, nc, wall, dev_ms / 1e3, n_l / wall))
 
@@ -464,13 +493,6 @@ def main():
                                                         precision=prec)[0]
                 log("%s: %d-step chains for the accuracy gate (untimed, %.1fs)" % (
                     prec, gate_steps, time.perf_counter() - t0))
-        # the FP64 chains again with another K split of the outer GEMM (same
-        # arithmetic, another summation order): how far FP64 itself carries
-        # the coefficients of this workload
-        ks0 = lanc.engine.ksplit
-        lanc.engine.set_ksplit(max(8, (ks0 // 2) // 8 * 8))
-        fp64_alt = lanc.run_FT_batched(psis, gate_steps, reorth=True, precision="fp64")[0]
-        lanc.engine.set_ksplit(ks0)
 
         def parting_step(ch1, ch0, thr=1e-6):
             """First step whose a or b differs by more than thr (relative)."""
@@ -483,12 +505,19 @@ def main():
                 first = min(first, int(bad[0]) if len(bad) else k)
             return first
 
-        fp64_parting = parting_step(fp64_alt, long_chains["fp64"])
-        fp64_spec = spec_error(fp64_alt, long_chains["fp64"])[0]
-        log("fp64 vs fp64 with K split %d instead of %d: coefficients part (1e-6) at step %d, "
-            "spectrum %.2e" % (max(8, (ks0 // 2) // 8 * 8), ks0, fp64_parting, fp64_spec))
+        # the x, y and z chains are equal by symmetry: how far rounding alone
+        # carries the FP64 coefficients and spectra of this workload
+        xyz = [long_chains["fp64"][i] for i in (1, 2)]
+        fp64_parting = parting_step(xyz, [long_chains["fp64"][0]] * 2)
+        fp64_spec = spec_error(xyz, [long_chains["fp64"][0]] * 2)[0]
+        log("fp64 chains of x, y and z: coefficients part (1e-6) at step %d, spectra %.2e" % (
+            fp64_parting, fp64_spec))
+        # one L application against the average over all images
         lanc.precision = "fp64"
-        L64 = lanc.apply_L_batch(psis)
+        L64, _ = general_L(lanc, psis, "fp64")
+        Lo = lanc.apply_L_batch(psis)
+        fp64_lv = float(np.max(np.linalg.norm(Lo - L64, axis=1) / np.linalg.norm(L64, axis=1)))
+        log("fp64 L.v over the rotations of the vectors vs over all images: %.1e" % fp64_lv)
         for prec in results:
             if prec == "fp64":
                 continue
@@ -510,8 +539,9 @@ def main():
                          "coeff_a_max_rel_err_first50": ea, "coeff_b_max_rel_err_first50": eb,
                          "coeff_parting_step_1e-6": parting_step(long_chains[prec],
                                                                  long_chains["fp64"]),
-                         "fp64_vs_fp64_other_ksplit_parting_step_1e-6": fp64_parting,
-                         "fp64_vs_fp64_other_ksplit_spectrum_linf_rel_err": fp64_spec,
+                         "fp64_xyz_chains_parting_step_1e-6": fp64_parting,
+                         "fp64_xyz_chains_spectrum_linf_rel_err": fp64_spec,
+                         "fp64_Lv_rel_diff_vs_all_images": fp64_lv,
                          "Lv_rel_l2_err": lv}
             log("%s vs FP64 on %d-step chains: spectrum %.2e (per chain %s), a %.2e, b %.2e "
                 "(first 50), coefficients part at step %d, L.v %.2e; %d-step timed chains: "
@@ -525,7 +555,9 @@ def main():
                                                             results["fp64"]["wall"])}
         bf16.update(acc.get("bf16x2", {}))
 
-    # per-kernel durations with HIP events on the library stream
+    # per-kernel durations of the average over all images (general perturbations; the
+    # IR chains above run the same kernels on the configurations), with HIP events on
+    # the library stream
     L = _lib.lib()
     prof = {}
     for prec in results:
@@ -544,7 +576,8 @@ def main():
     kname = ["weights_gemm", "outer_gemm"][dom]
     alg = 2.0 * M * n * n * nc                 # one contraction of 2 M n^2 per chain
     achieved = alg * PRODUCTS[args.precision] / (pm[dom] * 1e-3)
-    roof = {"bound": "mfma", "kernel": kname, "achieved": achieved / 1e12,
+    roof = {"bound": "mfma", "kernel": kname, "rows": "all images (general perturbations)",
+            "achieved": achieved / 1e12,
             "peak": PEAK[args.precision] / 1e12, "unit": "TFLOP/s",
             "frac": achieved / PEAK[args.precision],
             "traffic": profiled_traffic(kname, args.precision)}
@@ -594,7 +627,8 @@ def main():
                                "projector, 3 IR chains, Wigner, full reorthogonalisation" % (
                                    args.supercell, args.supercell, args.supercell,
                                    ens.model.nat, n, args.configs, lanc.n_syms),
-                   "chains": nc, "images": M, "precision": args.precision},
+                   "chains": nc, "chains_on_orbits": head["orbit"], "images": M,
+                   "precision": args.precision},
         "fp64_value": (results["fp64"]["n_l"] / results["fp64"]["wall"]) if "fp64" in results
         else None,
         "speedup_vs_fp64": (value / (results["fp64"]["n_l"] / results["fp64"]["wall"]))
