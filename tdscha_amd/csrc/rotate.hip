@@ -178,8 +178,9 @@ __global__ void rot_out_left(RotTab tb, const double* __restrict__ T2,
 }
 
 // d2v[chain] += normd T1[k], f[chain] += normf F1[k] for the pairs of the pass
-// in order (one thread per element of the unpadded outputs; the upper half of T1 for
-// both, so that d2v is exactly symmetric)
+// in order (one thread per element of the unpadded outputs).  The upper half of d2v is
+// summed; a chain's last pair writes it to the lower one too, so that d2v is exactly
+// symmetric (the lower half read from the upper one of T1 in every pass: 2 % of a call)
 __global__ void rot_accumulate(const double* __restrict__ T1, const double* __restrict__ F1,
                                int n, int np, int nsym, int p0, int g, double normf, double normd,
                                double* __restrict__ f_all, double* __restrict__ d2v_all) {
@@ -187,13 +188,15 @@ __global__ void rot_accumulate(const double* __restrict__ T1, const double* __re
   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (long)n * n) return;
   const int r = (int)(e / n), q = (int)(e % n);
+  if (r > q) return;
+  const long mirror = (long)q * n + r;
   // the pairs of one chain are consecutive: the running sums stay in
   // registers and go back when the chain changes (same order of additions)
   double t[kMaxChains], fv[kMaxChains];
 #pragma unroll
   for (int k = 0; k < kMaxChains; ++k) {
     const int kk = k < g ? k : g - 1;
-    t[k] = T1[(long)kk * nn + (long)min(r, q) * np + max(r, q)];
+    t[k] = T1[(long)kk * nn + (long)r * np + q];
     fv[k] = e < n ? F1[(long)kk * np + e] : 0.0;
   }
   int ch = p0 / nsym;
@@ -203,7 +206,7 @@ __global__ void rot_accumulate(const double* __restrict__ T1, const double* __re
     if (k < g) {
       const int c = (p0 + k) / nsym;
       if (c != ch) {
-        d2v_all[(long)ch * n * n + e] = dv;
+        d2v_all[(long)ch * n * n + e] = d2v_all[(long)ch * n * n + mirror] = dv;
         if (e < n) f_all[(long)ch * n + e] = fa;
         ch = c;
         dv = d2v_all[(long)ch * n * n + e];
@@ -214,6 +217,7 @@ __global__ void rot_accumulate(const double* __restrict__ T1, const double* __re
     }
   }
   d2v_all[(long)ch * n * n + e] = dv;
+  if ((p0 + g) % nsym == 0) d2v_all[(long)ch * n * n + mirror] = dv;
   if (e < n) f_all[(long)ch * n + e] = fa;
 }
 
