@@ -146,11 +146,13 @@ constexpr int kOrbPairs = 24;        // rotated perturbations of one pass
 constexpr double kOrbTol = 1e-13;    // accuracy of the relation
 constexpr double kOrbGain = 16.0;    // largest sum of its factors
 constexpr int kOrbClean = 2;         // Lanczos steps between projections on the sector
-// least time that the form saves (microseconds, estimated, one chain): the search, a wait
-// for the host of about 40 us and the rotations cost a call of one chain 150 to 200
-// (averages of one IR vector: 54 atoms x 6000, saving 500: 874 -> 285 us; 128 atoms x
-// 1000, 483: 807 -> 454)
-constexpr double kOrbWorthUs = 200.0;
+// least time that the form saves (microseconds, estimated, one chain; the kernels take
+// 1.5 to 2 times the estimate at these sizes): the search, a wait for the host of about
+// 40 us and the rotations cost a call of one chain 150 to 200.  Averages of one IR
+// vector, host arrays: 54 atoms x 2500 (estimate 209) general 434 us, orbit 247; 128
+// atoms x 450 (217) about 570, 460; just below the line, 54 x 2050 (172) and 128 x 360
+// (174), the general form takes 365 and 530.
+constexpr double kOrbWorthUs = 175.0;
 
 struct OrbPlan {
   bool ok = false;         // some chain takes the form
@@ -185,6 +187,7 @@ struct Orbit {
   long Mp = 0;
   std::vector<double> syms;               // host copy of the symmetry blocks
   std::vector<int> gens;                  // generators of the group
+  std::vector<double> look;               // [8][8][n] S_j p of orbit_candidates
   double* arena = nullptr;                // holds start, S, ST, pu, pf (and U, F, rho)
   size_t arena_bytes = 0;
   int* start = nullptr;                   // [npanel + 1]

@@ -13,7 +13,7 @@
 // (vector) perturbation of a cubic crystal, at most 6 for a Raman (tensor) one,
 // against 48 images.
 //
-// The rank is found for each call from the perturbation itself, not assumed: the
+// The rank is found for each chain and call from the perturbation itself: the
 // row-dots of the averages (s1 = u.Y1.u, s2 = u.Y1.(fpsi f), s3 = (fY u).R1,
 // s4 = f.R1) are evaluated on all images of kProbe random configurations of the
 // thermal amplitudes: 2 kProbe functionals of R1 and as many of Y1.  A relation C that
@@ -25,22 +25,27 @@
 // tables are orthogonal to 1e-14).  The sum of |C| over an image, which the rounding of
 // the averages enters with, is 2 and 5 there, and at most kOrbGain.
 //
-// A Lanczos run whose operator commutes with the symmetries (they form a group
-// and the translation average commutes with them, both checked numerically)
-// keeps the relation C of its start vector, which is the one of all three parts of
-// the packed vector: R and both pair sectors, A and B.  (Y1 = ca A - cb B alone would
-// not do: ca is zero for pairs of equal frequencies, and for every pair at T = 0, and
-// A and B can cancel.)  Rounding leaves that sector and
-// the three-term recurrence amplifies it (about 5-fold per step), so the residual is
-// projected back every kOrbClean steps with the same two kernels (0.2 ms for three
-// chains of 381 modes).  Spectra of the three IR chains, equal by symmetry, after 200
+// A Lanczos run whose operator commutes with the symmetries (they form a group of
+// orthogonal matrices and the translation average commutes with them, both checked
+// numerically) keeps the relation C of its start vector, which is the one of all three
+// parts of the packed vector: R and both pair sectors, A and B.  (Y1 = ca A - cb B alone
+// would not do: ca is zero for pairs of equal frequencies, and for every pair at T = 0,
+// and A and B can cancel.)  Rounding leaves that sector and the three-term recurrence
+// amplifies it (about 5-fold per step), so the residual is projected back every
+// kOrbClean steps with the same two kernels (0.2 ms for three chains of 381 modes).
+// Spectra of the three IR chains, equal by symmetry, after 200
 // FP64 steps at 128 atoms: apart by 3e-6 with a projection every third step, 1.2e-7
 // every second and every step (4e-8 in the general form).
 //
+// The given tables are a representation to their own rounding, 1e-14, and the form uses
+// that they are one: with exact arithmetic too, its averages of an IR vector are f 2e-15
+// and d2v 7e-15 from the sum over the tables verbatim at 54 atoms (the general form's
+// rounding: 6e-16), a whole application of L 1.7e-16 (1.5e-16).
+//
 // Measured, three IR vectors, one application of L in FP64 (host arrays in and out):
 // 128 atoms x 20000 configurations x 48: 9 averages over 20,096 rows instead of
-// three over 960,000 images, 29.1 -> 2.67 ms (weights 1.04, outer 1.04, rotations
-// 0.13 ms); 54 atoms x 5000 x 48: 1.70 -> 0.44 ms.
+// three over 960,000 images, 29.1 -> 2.63 ms (weights 1.04, outer 1.04, rotations
+// 0.13 ms); 54 atoms x 5000 x 48: 1.70 -> 0.42 ms.
 #include <algorithm>
 #include <cmath>
 #include <random>
@@ -62,6 +67,7 @@ int rot_panels(const int* bs, const int* d, int n, int np, int* start, int* nrea
 
 constexpr int kOP = 32;          // modes of a panel (whole blocks)
 constexpr int kOLd = kOP + 1;
+constexpr int kLook = 8;         // symmetries and functionals of orbit_candidates
 
 // ------------------------------------------------------------------- the probe
 // row-dots of 16 probe rows over 16 columns of V = U Y1, a quarter of the K index
@@ -583,7 +589,7 @@ int orbit_sector(Ctx* c, bool* ok) {
 // 381 modes, counted once, not three times) to 500 TF/s (three of 159).
 static double estimate_us(const Ctx* c, double rows, int prec) {
   const double w = round_up(c->n, prec == PREC_FP64 ? 16 : kTile);
-  return 4.0 * rows * w * w / (prec == PREC_FP64 ? 5.5e7 : 3.5e8);
+  return 4.0 * rows * w * w / (prec == PREC_FP64 ? 5.5e7 : 4e8);
 }
 
 // Whether the form may save enough for one chain in this precision.  Per chain, so that
@@ -628,6 +634,8 @@ int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const in
   start[nreal] = n;
   const size_t ntab = (size_t)nreal * n_syms * kOP * kOP;
   o.syms = syms;
+  const int look = std::min(n_syms, kLook);
+  o.look.resize((size_t)look * kLook * n);
   // probe configurations: thermal amplitudes for x; forces of the same weight
   // in s2 = u.Y1.(fpsi f) as x has in s1
   std::mt19937_64 g(2024);
@@ -638,6 +646,16 @@ int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const in
       px[(size_t)i * n + m] = nd(g) / std::sqrt(fy[m]);
       py[(size_t)i * n + m] = nd(g) * std::sqrt(fy[m]);
     }
+  // (symmetries drawn from the whole list: the first ones often leave an axis alone)
+  std::vector<int> pick(n_syms);
+  for (int j = 0; j < n_syms; ++j) pick[j] = j;
+  for (int j = 0; j < look; ++j) std::swap(pick[j], pick[j + g() % (n_syms - j)]);
+  std::vector<double> pv(n);
+  for (int i = 0; i < kLook; ++i) {
+    for (double& v : pv) v = nd(g);
+    for (int j = 0; j < look; ++j)
+      apply_s(c, o.syms, pick[j], false, pv.data(), o.look.data() + ((size_t)j * kLook + i) * n);
+  }
   o.rows = round_up(kProbe * n_syms, 16);
   // one allocation: tables, probe rows, and the inputs of the kernels that fill them
   size_t at = 0;
@@ -891,35 +909,38 @@ static int relation(const std::vector<Dots>& dots, int ns, std::vector<int>& piv
   return r;
 }
 
-// The chains (bit mask) to look for a plan of: the general form is long enough, and the
-// chain's R vector (host, `ld` apart) does not rule it out by more than kOrbRank
-// independent rotations among the first symmetries.  This keeps the probe and the wait
-// for it away from perturbations of no symmetry (10 us of host work under the upload,
-// for 50 us).
+// The chains (bit mask) to look for a plan of: the general form is long enough for the
+// rank that the chain's R vector (host, `ld` apart) shows at least.  R is looked at
+// through kLook random functionals p of its images under kLook random symmetries,
+// p.S_j^T R = (S_j p).R with S_j p from the context's creation.  This keeps the probe and
+// the wait for it away from perturbations of no symmetry and from calls at the line
+// (64 dots, 3 us at 381 modes, for 50 us).
 unsigned orbit_candidates(const Ctx* c, int nc, int prec, const double* R, long ld) {
   if (!orbit_sized(c, prec)) return 0;
   const Orbit& o = c->orb;
-  const int n = c->n;
+  const int n = c->n, rows = std::min(o.nsym, kLook);
+  const double full = estimate_us(c, (double)c->N * o.nsym, prec);
   unsigned mask = 0;
-  std::vector<double> Q((size_t)(kOrbRank + 1) * n);
   for (int ch = 0; ch < nc; ++ch) {
+    double Q[kLook][kLook];
     int r = 0;
-    for (int j = 0; j < std::min(o.nsym, kOrbRank + 2) && r <= kOrbRank; ++j) {
-      double* v = Q.data() + (size_t)r * n;
-      apply_s(c, o.syms, j, true, R + ch * ld, v);
-      const double whole = dot(v, v, n);
+    for (int j = 0; j < rows; ++j) {
+      double* v = Q[r];
+      for (int i = 0; i < kLook; ++i)
+        v[i] = dot(o.look.data() + ((size_t)j * kLook + i) * n, R + ch * ld, n);
+      const double whole = dot(v, v, kLook);
       for (int k = 0; k < r; ++k) {
-        const double* q = Q.data() + (size_t)k * n;
-        const double t = dot(v, q, n);
-        for (int m = 0; m < n; ++m) v[m] -= t * q[m];
+        const double t = dot(v, Q[k], kLook);
+        for (int m = 0; m < kLook; ++m) v[m] -= t * Q[k][m];
       }
-      const double rest = dot(v, v, n);
+      const double rest = dot(v, v, kLook);
       if (!(rest > 1e-12 * whole)) continue;   // (NaN: left to the probe)
       const double inv = 1.0 / std::sqrt(rest);
-      for (int m = 0; m < n; ++m) v[m] *= inv;
+      for (int m = 0; m < kLook; ++m) v[m] *= inv;
       ++r;
     }
-    if (r <= kOrbRank) mask |= 1u << ch;
+    if (r <= kOrbRank && full - estimate_us(c, (double)c->N * std::max(r, 1), prec) > kOrbWorthUs)
+      mask |= 1u << ch;
   }
   return mask;
 }
