@@ -41,6 +41,25 @@ def test_ranks_and_weights(form):
     p.close()
 
 
+def test_384_operations():
+    p = System(N=3000, full=True, trans=False)
+    a, b = (s.engine for s in p.sides)
+    Y = tensors(p, list(RANKS))
+    z = np.zeros((len(Y), p.n))
+    d = a.perturb_averages_batched(z, Y, 1)[1]     # (f of a tensor is zero by symmetry)
+    assert a.orbit_chains() == len(Y)
+    do = b.perturb_averages_batched(z, Y, 1)[1]
+    for k in range(len(Y)):
+        assert rel(d[k], do[k]) < 1e-12
+    Y, R = p.sector(p.ir()[0], 5, 3)
+    f, d = a.perturb_averages_batched(R, Y, 1)
+    assert a.orbit_chains() == 3
+    fo, do = b.perturb_averages_batched(R, Y, 1)
+    assert rel(f, fo) < 1e-12 and rel(d, do) < 1e-12
+    p.check(p.pack(p.ir()), 3)
+    p.close()
+
+
 @pytest.mark.parametrize("prec, tol", [("fp16x2", 1e-5), ("bf16x2", 1e-4)])
 def test_split_chains(prec, tol):
     p = System(N=7000)

@@ -20,15 +20,16 @@ STEPS = 8
 
 
 class System:
-    """54 atoms with the point group of a cubic crystal (the images of one chain are
-    enough work for the orbit form), and the same images as configurations."""
+    """54 atoms with the point group of a cubic crystal, or (full) 16 with the 384
+    operations of its supercell (the images of one chain are enough work for the orbit
+    form), and the same images as configurations."""
 
     def __init__(self, T=300.0, N=3000, weights=None, trans=True, tables=None,
-                 reference=True, form="images"):
+                 reference=True, form="images", full=False):
         from tdscha_amd.lanczos import Lanczos
         from tdscha_amd.rocksalt import Ensemble, RockSalt
-        ens = Ensemble(RockSalt(L=3), T, N, seed=3)
-        ms = ens.symmetries(True, gamma_only=True)
+        ens = Ensemble(RockSalt(L=2 if full else 3), T, N, seed=3)
+        ms = ens.symmetries(True, gamma_only=not full)
         if tables is not None:
             ms = tables(ms)
         self.ens, self.ms, self.n, self.T = ens, ms, len(ens.w), T
