@@ -602,8 +602,9 @@ bool orbit_sized(const Ctx* c, int prec) {
 
 // The configurations, panel tables and probe rows; called at context creation
 // with the configurations still on the device.  Leaves c->orb.usable false where
-// the form does not apply or cannot pay in any precision (orbit_sized), or with more than 512 symmetries (the tables and the closure check
-// grow with their number and its square).
+// the form does not apply or cannot pay in any precision (orbit_sized), or with more
+// than 512 symmetries (the tables and the closure check grow with their number and its
+// square).
 int orbit_setup(Ctx* c, int n_syms, int n_blocks, const int* block_dim, const int* block_modes,
                 const std::vector<double>& syms, const double* X_dev, const double* Y_dev,
                 const double* rho_dev, const int* d_mb, const int* d_mp, const int* d_bd,
